@@ -11,21 +11,22 @@
 //                       solute atoms in a fine cell grid (counting sort + scan)
 //   k_near_mark         cells within cutoff + radius of some solute atom
 //   k_prep_solvent_tiles  centre of every solvent molecule, key when near
-//   k_scan_rows, k_mol_scatter, k_chunk_table
-//                       near molecules sorted by the Morton key of their cell
-//                       per (frame, pass), cut into chunks of whole molecules,
-//                       one wavefront each
-//   k_fill_real         FP32 atoms of the near molecules in sorted order
-//   k_eval_tiles        per chunk: AABB, solute atoms within the cutoff of it
-//                       staged in LDS, FP32 minimum per atom (LDS broadcast),
-//                       segmented minimum per molecule, exact FP64 resolve,
-//                       LDS histograms
+//   k_scan_sums, k_scan_rows, k_mol_scatter, k_chunk_table
+//                       near molecules sorted by the Hilbert key of their cell
+//                       (the real pass; the random passes of a frame together),
+//                       cut into chunks of whole molecules, one wavefront each
+//   k_fill_real         atoms of the near molecules in sorted order, fixed point
+//   k_eval_tiles        per chunk: AABB, solute atoms within reach of it staged
+//                       in LDS, distances on the matrix cores, minimum and second
+//                       smallest per atom, minimum per molecule, records that
+//                       FP32 decides into LDS histograms
+//   k_resolve           the other molecules (about one in two hundred) in FP64
 //   k_bulk_compact      ordered list of bulk molecules (inbulk, src/mddf.jl:55-57)
 //   k_place_keys, k_place_near
 //                       Philox placement (src/rigid_body.jl:107-137): centres
 //                       of all slots, then the full placement of the slots whose
 //                       centre is near the solute, in sorted order
-//   then sort, chunk and k_eval_tiles again for the random passes.
+//   then sort, chunk, k_eval_tiles and k_resolve again for the random passes.
 //
 // "mols" -- many solute molecules (self MDDF, small solutes): molecule
 // centres in a cell list, one thread per solvent molecule evaluating all atom
@@ -34,11 +35,12 @@
 //
 // k_flush turns integer hits into FP64 accumulators times the frame weight.
 //
-// Exactness.  Candidate pairs are evaluated in FP32 from coordinates in the
-// frame of each molecule's cell.  Per atom (tiles) or molecule pair (mols) the
+// Exactness.  Candidate pairs are evaluated in FP32, from fixed-point fractions
+// of the cell (tiles: differences are exact) or from coordinates in the frame of
+// each molecule's cell (mols).  Per atom (tiles) or molecule pair (mols) the
 // kernels keep the best and second-best squared distance; when the gap exceeds
 // a guard band that bounds the FP32 error, the FP32 argmin is the FP64 argmin
-// and only that pair is recomputed in FP64 (the recorded distance).
+// and its d^2 decides the bin, in FP64 when the bin edge is within the guard.
 // Otherwise every pair near the minimum is recomputed in FP64.  Records,
 // indices and bins therefore equal those of an FP64 evaluation.
 #include <hip/hip_runtime.h>
@@ -88,9 +90,15 @@ struct Geo {                 // one frame of a batch
     int err;                 // geometry the kernels cannot handle
     float rstage;            // staging radius around a chunk (cutoff + margin), tiles family
     float rnear;             // near-cell radius around a solute atom (cutoff + radius + margin)
-    int kbits;               // bits per dimension of the Morton keys of the fine cells
+    int kbits;               // bits per dimension of the sort keys of the fine cells
     int ortho;               // diagonal cell matrix: cells are boxes (exact near-cell test)
     double guard;            // bound on |d2(FP32) - d2(FP64)| for pairs up to the cutoff
+    float guard_up;          // the same, rounded up
+    // tiles family: fixed-point fractional coordinates, 2^fix units per cell
+    int fix;
+    float Hfix[9];           // lattice vectors per unit (FP32)
+    float gd0, gd1, gd2;     // guard of a direct FP32 d2: gd0 + gd1 d + gd2 d2 (with the roundings of decide32)
+    float rho;               // |error| of an FP32 difference of two fixed-point positions, in 2^-24 of its length
     float guard32;           // guard + (cutoff^2 + guard + 1) 2^-21, rounded up: covers FP32 b -+ guard32 rounding
 };
 
@@ -109,13 +117,20 @@ struct KP {                  // job parameters, by value
     int cap;                 // cell slots per frame
     int F;                   // frames in the batch
     int64_t Nu, Nv;
-    int mpt;                 // molecules per chunk (tiles family)
-    int mol_lane;            // tiles family, 3-atom solvent molecules: one molecule per lane row
-    int tcap;                // staged solute atoms per round (tiles family)
+    int mpt;                 // molecules per chunk of the real pass (tiles family)
+    int mpt_r;               // the same of the random passes
+    int mol_lane;            // tiles family: 3-atom solvent molecules (their three atoms evaluated together)
     int glds;                // molecule-pair kernels: group counts privatised in LDS
     int gnu, gnv;            // group counts of the solute / solvent side
     int NP;                  // passes per frame, 1 + K (tiles family)
-    int kcap;                // molecule sort keys per (frame, pass): Morton codes of the fine cells
+    // The random passes of a frame place molecules around the same solute
+    // atoms and only their sums are kept, so they are sorted and evaluated
+    // together: NG groups of KM passes (the last one may hold fewer), each one
+    // row of slots (pass within the group times Mv plus the molecule).
+    int KM, NG;
+    int kcap;                // molecule sort keys of the real pass: Hilbert positions of the fine cells
+    int ksub;                // bits per dimension the random groups' keys have beyond them
+    int kcapr;               // sort keys of a random group: kcap << 3 ksub
     int place_all;           // molecule-pair family: place every slot of a random pass (verification)
 };
 
@@ -161,13 +176,17 @@ struct Bufs {
     unsigned char* near;     // [F][cap]
     unsigned* dfield;        // [2][F][cap] 0xffffffff - bits of the distances from a near cell's centre and
                              // lower corner to the nearest solute atom image nearby (0: none), b_dfield
-    int* mkey;               // [F][NP][Mv] Morton key of the centre's cell, -1 when far
+    // (rows of a frame: the real pass, then the NG random groups; row_base, key_row)
+    int* mkey;               // [F][NP][Mv] Hilbert key of the centre's cell, -1 when far
     int* mrank;              // [F][NP][Mv] rank of a near molecule among those of its key (count order)
-    int* mcnt;               // [F][NP][kcap+1]
-    int* mstart;             // [F][NP][kcap+1]
-    int* msorted;            // [F][NP][Mv]
-    int* nnear;              // [F][NP]
-    int* chunk_base;         // [F*npass + 2] chunk offsets of one launch, total, evaluation chunk counter
+    int* mcnt;               // [F][kcap | NG x kcapr] molecules per key
+    int* mstart;             // the same shape: first sorted position of a non-empty key
+    int* msum;               // [F][parts of kcap | NG x parts of kcapr] molecules per part of a row's keys
+    int* msorted;            // [F][NP][Mv] slots in key order
+    int* nnear;              // [F][1 + NG]
+    ull* resmask;            // one word per chunk of a launch: molecules left to the FP64 resolve (over mkey,
+                             // whose keys the scatter has read by then)
+    int* chunk_base;         // [F*rows + 2] chunk offsets of one launch, total, evaluation chunk counter
     // accumulators
     ull* cnt_md; ull* cnt_rdf; ull* cnt_md_r; ull* cnt_rdf_r;
     ull* cnt_gu; ull* cnt_gv; ull* cnt_gu_r; ull* cnt_gv_r;
@@ -184,6 +203,10 @@ template <class T>
 using gptr = __attribute__((address_space(1))) T*;
 typedef float f4v __attribute__((ext_vector_type(4)));
 
+// a frame's geometry in the constant address space (not written while the
+// reading kernel runs): fields read where they are used, by scalar loads
+using GeoC = __attribute__((address_space(4))) const Geo;
+
 template <class T>
 __device__ __forceinline__ T ldg(const T* p)
 {
@@ -199,6 +222,25 @@ __device__ __forceinline__ Geo ldc_geo(const Geo* p)
     Geo g;
     __builtin_memcpy(&g, (__attribute__((address_space(4))) const Geo*)p, sizeof(Geo));
     return g;
+}
+
+// first entry of a row of the sorted molecules: the real pass or random group grp of frame f
+__device__ __forceinline__ int64_t row_base(const KP& P, int f, bool random, int grp)
+{
+    return ((int64_t)f * P.NP + (random ? 1 + (int64_t)grp * P.KM : 0)) * P.Mv;
+}
+
+// slots of a random group (all its passes)
+__device__ __forceinline__ int group_slots(const KP& P, int grp)
+{
+    return min(P.KM, P.K - grp * P.KM) * P.Mv;
+}
+
+// first key count of row r of frame f (0: real pass, 1 + grp)
+__device__ __forceinline__ int64_t key_row(const KP& P, int f, int r)
+{
+    const int64_t per = (int64_t)P.kcap + (int64_t)P.NG * P.kcapr;
+    return f * per + (r > 0 ? P.kcap + (int64_t)(r - 1) * P.kcapr : 0);
 }
 
 struct Rec {
@@ -239,6 +281,25 @@ __device__ __forceinline__ void load3(const T* p, int64_t atom, double& x, doubl
 
 __device__ __forceinline__ float4 mk4(float x, float y, float z, float w) { return make_float4(x, y, z, w); }
 
+// a fixed-point position (tiles family), kept in the bits of a float4 with w
+__device__ __forceinline__ float4 fix4(int x, int y, int z, float w)
+{
+    return mk4(__int_as_float(x), __int_as_float(y), __int_as_float(z), w);
+}
+
+// fixed-point difference to FP32 lengths; general cells sum three products
+template <class GEO>
+__device__ __forceinline__ void fix_cart(const GEO& g, int dx, int dy, int dz, float& x, float& y, float& z)
+{
+    const float a = (float)dx, b = (float)dy, c = (float)dz;
+    x = g.Hfix[0] * a; y = g.Hfix[4] * b; z = g.Hfix[8] * c;
+    if (!g.ortho) {
+        x = fmaf(g.Hfix[3], b, fmaf(g.Hfix[6], c, x));
+        y = fmaf(g.Hfix[1], a, fmaf(g.Hfix[7], c, y));
+        z = fmaf(g.Hfix[2], a, fmaf(g.Hfix[5], b, z));
+    }
+}
+
 __device__ __forceinline__ void cell_of_frac(const Geo& g, double f0, double f1, double f2, int& cell, int& c0, int& c1,
                                              int& c2)
 {
@@ -254,17 +315,17 @@ __device__ __forceinline__ void cell_of_frac(const Geo& g, double f0, double f1,
     cell_of_frac(g, f0, f1, f2, cell, c0, c1, c2);
 }
 
-// cell_of_frac of the fractional coordinates u01(r0), u01(r1), u01(r2), in
-// integers: r 2^-32 is exact in FP64 and so is its product with nc (at most
-// 32 + 21 significant bits), so (int)(u01(r) nc) = floor(r nc / 2^32) =
-// (r nc) >> 32, always below nc
-__device__ __forceinline__ void cell_of_draws(const Geo& g, uint32_t r0, uint32_t r1, uint32_t r2, int& cell, int& c0,
+// Sub-cells (2^sub per cell and dimension) of the fractional coordinates
+// u01(r0), u01(r1), u01(r2), in integers: r 2^-32 is exact in FP64 and so is
+// its product with nc (at most 32 + 21 significant bits), so (int)(u01(r) nc) =
+// floor(r nc / 2^32) = (r nc) >> 32, always below nc; the cell of cell_of_frac
+// is the sub-cell shifted down by sub.
+__device__ __forceinline__ void cell_of_draws(const Geo& g, uint32_t r0, uint32_t r1, uint32_t r2, int sub, int& c0,
                                               int& c1, int& c2)
 {
-    c0 = (int)(((uint64_t)r0 * (uint64_t)g.nc[0]) >> 32);
-    c1 = (int)(((uint64_t)r1 * (uint64_t)g.nc[1]) >> 32);
-    c2 = (int)(((uint64_t)r2 * (uint64_t)g.nc[2]) >> 32);
-    cell = (c2 * g.nc[1] + c1) * g.nc[0] + c0;
+    c0 = (int)(((uint64_t)r0 * ((uint64_t)g.nc[0] << sub)) >> 32);
+    c1 = (int)(((uint64_t)r1 * ((uint64_t)g.nc[1] << sub)) >> 32);
+    c2 = (int)(((uint64_t)r2 * ((uint64_t)g.nc[2] << sub)) >> 32);
 }
 
 // fractional coordinates of a point, the lattice translation n = floor(f)
@@ -278,6 +339,15 @@ __device__ __forceinline__ void wrap_point(const Geo& g, double x, double y, dou
     n[0] = floor(f0); n[1] = floor(f1); n[2] = floor(f2);
     fr[0] = f0 - n[0]; fr[1] = f1 - n[1]; fr[2] = f2 - n[2];
     for (int k = 0; k < 3; k++) if (fr[k] >= 1.0) { fr[k] = 0.0; n[k] += 1.0; }
+}
+
+// fixed-point position of a point (FP64), not wrapped
+__device__ __forceinline__ float4 fix_point(const Geo& g, double x, double y, double z, float w)
+{
+    const double* Hi = g.cell.Hi;
+    const double sc = ldexp(1.0, g.fix);
+    return fix4((int)rint((Hi[0] * x + Hi[3] * y + Hi[6] * z) * sc), (int)rint((Hi[1] * x + Hi[4] * y + Hi[7] * z) * sc),
+                (int)rint((Hi[2] * x + Hi[5] * y + Hi[8] * z) * sc), w);
 }
 
 // Molecule made whole around its first atom (minimum image of every atom
@@ -421,13 +491,40 @@ __device__ __forceinline__ void b_grid(KP P, Bufs B, int mols_family, int bx_, i
         g.ncell = ncell;
     }
     const double* H = g.cell.H;
-    double xm = 0.0;
-    for (int r = 0; r < 3; r++) xm = fmax(xm, fabs(H[r]) + fabs(H[3 + r]) + fabs(H[6 + r]));
-    xm += fmax(ru, rv) + P.cutsys + 1.0;
-    double E = 10.0 * halfulp32(2.0 * xm) + 1e-7;
-    double dmax = P.cutsys + 0.5;
-    double G = E * (2.0 * 1.7320508075688772 * dmax + 3.0 * E) + 8.0 * 0x1p-24 * dmax * dmax;
+    double dmax = P.cutsys + 0.5, E, G;
+    if (mols_family) {
+        double xm = 0.0;
+        for (int r = 0; r < 3; r++) xm = fmax(xm, fabs(H[r]) + fabs(H[3 + r]) + fabs(H[6 + r]));
+        xm += fmax(ru, rv) + P.cutsys + 1.0;
+        E = 10.0 * halfulp32(2.0 * xm) + 1e-7;
+        G = E * (2.0 * 1.7320508075688772 * dmax + 3.0 * E) + 8.0 * 0x1p-24 * dmax * dmax;
+    } else {
+        // Fixed point: positions are fractions of the cell in units of 2^-fix,
+        // fix leaving room for atoms a molecule radius outside the cell and for
+        // differences of two of them.  A position is off by half a unit per
+        // fraction, a difference of two by E per coordinate; the difference is
+        // exact in integers, and turning it into a length rounds the
+        // conversion, the FP32 lattice vector and the product (a diagonal cell:
+        // 3 u), plus the additions over terms of at most kappa times the length
+        // in a general one.
+        const double smin = fmin(g.sp[0], fmin(g.sp[1], g.sp[2]));
+        g.fix = 29 - (int)ceil(log2(1.0 + (rv + P.cutsys) / smin));
+        double kappa = 0.0, hs = 0.0;
+        for (int r = 0; r < 3; r++) {
+            kappa = fmax(kappa, fabs(H[r]) / g.sp[0] + fabs(H[3 + r]) / g.sp[1] + fabs(H[6 + r]) / g.sp[2]);
+            hs = fmax(hs, fabs(H[r]) + fabs(H[3 + r]) + fabs(H[6 + r]));
+        }
+        for (int k = 0; k < 9; k++) g.Hfix[k] = (float)ldexp(H[k], -g.fix);
+        const double rho = g.ortho ? 3.0 : 5.0 * 1.7320508075688772 * kappa;
+        g.rho = (float)(rho * (1.0 + 1e-6));
+        E = ldexp(hs, -g.fix) + 1e-9;
+        G = E * (2.0 * 1.7320508075688772 * dmax + 3.0 * E) + (2.0 * rho + 4.0) * 0x1p-24 * dmax * dmax;
+        g.gd0 = (float)(3.0 * E * E + 1e-9) * (1.0f + 1e-6f);
+        g.gd1 = (float)(2.0 * 1.7320508075688772 * E) * (1.0f + 1e-5f);
+        g.gd2 = (float)(((2.0 * rho + 4.0) + 4.0) * 0x1p-24) * (1.0f + 1e-5f);
+    }
     g.guard = G;
+    g.guard_up = nextafterf((float)G, INFINITY);
     g.guard32 = nextafterf((float)(G + (P.cut2 + G + 1.0) * 0x1p-21), INFINITY);
     float hi = (float)(P.cut2 + G);
     g.cut2_hi = nextafterf(hi, INFINITY);
@@ -436,7 +533,7 @@ __device__ __forceinline__ void b_grid(KP P, Bufs B, int mols_family, int bx_, i
     float rp = (float)(P.cutsys + ru + rv + 1e-2);
     g.rpre2 = rp * rp;
     g.rstage = (float)(P.cutsys + 20.0 * E + 1e-3);
-    g.rnear = (float)(P.cutsys + rv + 20.0 * E + 1e-2);
+    g.rnear = (float)(P.cutsys + rv + 20.0 * E + 1e-2 + 1e-6 * (g.sp[0] + g.sp[1] + g.sp[2]));
 }
 
 __global__ void k_grid(KP P, Bufs B, int mols_family)
@@ -461,12 +558,9 @@ __device__ __forceinline__ void b_wrap_atoms(KP P, Bufs B, const T* xu, int bx_,
         wrap_point(g, x, y, z, fr, n);
         int cell;
         cell_of_frac(g, fr[0], fr[1], fr[2], cell);
-        const double* H = g.cell.H;
-        double wx = H[0] * fr[0] + H[3] * fr[1] + H[6] * fr[2];
-        double wy = H[1] * fr[0] + H[4] * fr[1] + H[7] * fr[2];
-        double wz = H[2] * fr[0] + H[5] * fr[1] + H[8] * fr[2];
         int64_t o = (int64_t)f * B.nitems + i;
-        B.tmp4[o] = mk4((float)wx, (float)wy, (float)wz, __int_as_float(i));
+        const double sc = ldexp(1.0, g.fix);
+        B.tmp4[o] = fix4((int)rint(fr[0] * sc), (int)rint(fr[1] * sc), (int)rint(fr[2] * sc), __int_as_float(i));
         B.tmpcell[o] = cell;
         atomicAdd(&B.cnt[(int64_t)f * (P.cap + 1) + cell], 1);
     }
@@ -623,6 +717,13 @@ __device__ __forceinline__ void group_hit(ull* gc, int nbins, int b, int64_t ato
     }
 }
 
+// group_hit where the molecule-local atom is known (no division)
+__device__ __forceinline__ void group_hit_local(ull* gc, int nbins, int b, int local, int64_t atom, const int* ptr, const int* idx)
+{
+    if (!ptr) atomicAdd(&gc[(int64_t)local * nbins + b], 1ull);
+    else for (int k = ptr[atom]; k < ptr[atom + 1]; k++) atomicAdd(&gc[(int64_t)idx[k] * nbins + b], 1ull);
+}
+
 // bins and the dbulk test of a record from its distances where the fast
 // decision did not set them (setbin, src/results.jl:28)
 __device__ __forceinline__ void rec_complete(const KP& P, Rec& r)
@@ -646,22 +747,6 @@ __device__ __forceinline__ void hist_record(const KP& P, unsigned* sh, ull* gu, 
     if (r.ref) {
         const int rb = r.rbin;
         if (rb < P.nbins) atomicAdd(&sh[P.nbins + rb], 1u);
-    }
-}
-
-// the same with the md/rdf counts straight into the global counters
-__device__ __forceinline__ void hist_record_global(const KP& P, ull* md, ull* rdf, ull* gu, ull* gv, const Rec& r)
-{
-    if (!r.within) return;
-    const int b = r.bin;
-    if (b >= P.nbins) return;   // unreachable: d <= cutoff (validated at job creation)
-    atomicAdd(&md[b], 1ull);
-    group_hit(gu, P.nbins, b, r.i, P.gu_ptr, P.gu_idx, P.nu);
-    if (P.self_) group_hit(gu, P.nbins, b, r.j, P.gv_ptr, P.gv_idx, P.nu);
-    else group_hit(gv, P.nbins, b, r.j, P.gv_ptr, P.gv_idx, P.nv);
-    if (r.ref) {
-        const int rb = r.rbin;
-        if (rb < P.nbins) atomicAdd(&rdf[rb], 1ull);
     }
 }
 
@@ -1630,7 +1715,21 @@ struct MolDst {
         p[3 * a] = x; p[3 * a + 1] = y; p[3 * a + 2] = z;
         w[a] = f4v{(float)x, (float)y, (float)z, 0.f};
     }
-    // the first atom's fourth FP32 component
+};
+
+// the same with fixed-point positions for the evaluation
+struct MolDstFix {
+    gptr<double> p;
+    gptr<f4v> w;
+    const Geo& g;
+    __device__ MolDstFix(double* q, float4* v, const Geo& geo) : p((gptr<double>)q), w((gptr<f4v>)v), g(geo) {}
+    __device__ void operator()(int a, double x, double y, double z) const
+    {
+        p[3 * a] = x; p[3 * a + 1] = y; p[3 * a + 2] = z;
+        const float4 u = fix_point(g, x, y, z, 0.f);
+        w[a] = f4v{u.x, u.y, u.z, 0.f};
+    }
+    // the first atom's fourth component
     __device__ void set_w0(float x) const { ((gptr<float>)w)[3] = x; }
 };
 
@@ -1675,9 +1774,7 @@ __global__ void k_place(KP P, Bufs B, const TV* xv)
 // ---------------------------------------------------------------------------
 // tiles family: one solute molecule, solvent molecules of up to 64 atoms
 // ---------------------------------------------------------------------------
-constexpr int TCAP_DEFAULT = 640;   // staged solute atoms per round (10 KiB of LDS)
 constexpr int RB_PIECES = 8;        // read-back pieces of cm_job_finish
-constexpr int TCAP_MOL = 512;       // the same with the squared norms (20 B each: 10 KiB)
 constexpr int CBCAP = 1024;         // chunk-table entries kept in LDS
 // The last DYN_PCT per cent of an evaluation launch's chunks are handed out
 // on request, in launches of at least DYN_MIN chunks per workgroup, in about
@@ -1689,8 +1786,6 @@ constexpr int CBCAP = 1024;         // chunk-table entries kept in LDS
 constexpr int DYN_PCT = 35;
 constexpr int DYN_MIN = 2;
 constexpr int DYN_GRABS = 8;
-constexpr int SU = 4;               // staging: atoms per lane per step
-constexpr int SEG = 8;              // staging: atoms of a row per lane (segment)
 
 __device__ __forceinline__ int wrap_index(int i, int n, int& m)
 {
@@ -1699,30 +1794,59 @@ __device__ __forceinline__ int wrap_index(int i, int n, int& m)
     return i - q * n;
 }
 
-// Morton code of a fine cell: chunks of consecutive molecules in this order
-// stay compact in space
-// bits 0..9 of x moved to bits 0, 3, 6, ..., 27
-__device__ __forceinline__ unsigned spread3(unsigned x)
+// Sort keys: the position of a fine cell (or half-cell) on the Hilbert curve of
+// its grid, so that consecutive molecules stay compact in space (a run of 64
+// near molecules of ten merged passes: boxes of 8.6 A a side and 166 staged
+// solute atoms, against 11.0 A and 288 along the Morton curve).  HILBERT[state][octant]: the
+// octant's place among the eight of its parent cube (bits 0..2) and the state
+// of its own eight (bits 3..7), the 24 orientations of the curve of Skilling,
+// "Programming the Hilbert curve" (AIP Conf. Proc. 707, 2004).
+__device__ const __align__(16) unsigned char HILBERT[24 * 8] = {
+    0x08, 0x3f, 0x23, 0x2c, 0x19, 0x36, 0x02, 0x05,
+    0x10, 0xab, 0x41, 0x0a, 0x57, 0x1c, 0x5e, 0x0d,
+    0x00, 0x29, 0x77, 0x6e, 0x63, 0x12, 0x44, 0x15,
+    0x28, 0x8b, 0x6f, 0x0c, 0x01, 0x1a, 0x76, 0x1d,
+    0x86, 0x47, 0x25, 0x4c, 0xb1, 0x58, 0x22, 0x03,
+    0x40, 0x11, 0x4b, 0x2a, 0x5f, 0x56, 0x04, 0x2d,
+    0x7c, 0x27, 0x3b, 0xa0, 0x35, 0x06, 0x32, 0x71,
+    0xbc, 0x87, 0x3d, 0x46, 0x33, 0xb0, 0x3a, 0x59,
+    0x18, 0x37, 0x09, 0x3e, 0x83, 0x14, 0x42, 0x45,
+    0xae, 0xb9, 0x4d, 0x4a, 0x0f, 0x38, 0x24, 0x2b,
+    0x94, 0x55, 0x5b, 0x52, 0x4f, 0x2e, 0x98, 0x69,
+    0xb4, 0x53, 0x5d, 0x5a, 0xaf, 0xb8, 0x0e, 0x39,
+    0x8e, 0x79, 0x1f, 0x30, 0x65, 0x62, 0x84, 0x13,
+    0x9c, 0x6d, 0x67, 0x16, 0x73, 0x6a, 0x90, 0x51,
+    0xa4, 0x6b, 0x8f, 0x78, 0x75, 0x72, 0x1e, 0x31,
+    0x7a, 0x61, 0xbb, 0x80, 0x7d, 0x96, 0x34, 0xb7,
+    0x26, 0x07, 0xa1, 0x70, 0x85, 0x64, 0x82, 0x43,
+    0x66, 0x8d, 0x17, 0xac, 0x91, 0x8a, 0x50, 0x1b,
+    0x92, 0x95, 0xb3, 0x54, 0x89, 0x7e, 0xa8, 0xbf,
+    0x9a, 0x9d, 0xa9, 0xbe, 0xa3, 0x6c, 0x88, 0x7f,
+    0xa2, 0x9b, 0x81, 0x60, 0xa5, 0x74, 0xb6, 0x97,
+    0x4e, 0xad, 0x99, 0xaa, 0x2f, 0x8c, 0x68, 0x0b,
+    0xb2, 0x93, 0xb5, 0x5c, 0x21, 0x48, 0xa6, 0x9f,
+    0xba, 0x49, 0xbd, 0x9e, 0x7b, 0x20, 0x3c, 0xa7,
+};
+
+// the table in LDS (48 words), for a kernel whose lanes walk it
+__device__ __forceinline__ void hilbert_load(unsigned* tab)
 {
-    x &= 0x3ffu;
-    x = (x | (x << 16)) & 0x030000ffu;
-    x = (x | (x << 8)) & 0x0300f00fu;
-    x = (x | (x << 4)) & 0x030c30c3u;
-    x = (x | (x << 2)) & 0x09249249u;
-    return x;
+    if (threadIdx.x < 48) tab[threadIdx.x] = ((const unsigned*)HILBERT)[threadIdx.x];
+    __syncthreads();
 }
 
-// Morton code of the fine cell (c0, c1, c2), each below 2^kbits
-__device__ __forceinline__ int morton_key3(const Geo& g, int c0, int c1, int c2)
+// key of the cell (c0, c1, c2), each below 2^bits; tab: hilbert_load's
+__device__ __forceinline__ int hilbert_key(const unsigned* tab, int bits, int c0, int c1, int c2)
 {
-    if (g.kbits <= 10) return (int)(spread3(c0) | (spread3(c1) << 1) | (spread3(c2) << 2));
-    unsigned k = 0;
-    for (int b = 0; b < g.kbits; b++) {
-        k |= (((unsigned)c0 >> b) & 1u) << (3 * b);
-        k |= (((unsigned)c1 >> b) & 1u) << (3 * b + 1);
-        k |= (((unsigned)c2 >> b) & 1u) << (3 * b + 2);
+    const unsigned char* t = (const unsigned char*)tab;
+    int key = 0, state = 0;
+    for (int b = bits - 1; b >= 0; b--) {
+        const int o = ((c0 >> b) & 1) | (((c1 >> b) & 1) << 1) | (((c2 >> b) & 1) << 2);
+        const int e = t[state * 8 + o];
+        key = (key << 3) | (e & 7);
+        state = e >> 3;
     }
-    return (int)k;
+    return key;
 }
 
 // Fine-grid index ranges covering the box [lo - r, hi + r] (fractional
@@ -1759,6 +1883,26 @@ __device__ __forceinline__ void cell_range(const Geo& g, float lx, float ly, flo
     }
 }
 
+
+// The same in FP32 for a box of half sides ex, ey, ez (radius included) about a
+// fixed-point centre, widened by more than its rounding (a few 1e-4 cells at
+// the largest grids), and kept to the images that an atom within a cell of the
+// home cell can reach
+template <class GEO>
+__device__ __forceinline__ void cell_range32(const GEO& g, int cx, int cy, int cz, float ex, float ey, float ez, int ilo[3],
+                                             int ihi[3])
+{
+    const int c[3] = {cx, cy, cz};
+    const float unit = ldexpf(1.0f, -g.fix);
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        const float m = (float)c[k] * unit;
+        const float e = fabsf(g.Hi32[k]) * ex + fabsf(g.Hi32[3 + k]) * ey + fabsf(g.Hi32[6 + k]) * ez;
+        const float n = (float)g.nc[k];
+        ilo[k] = max((int)floorf((m - e) * n - 2e-3f), -8 * g.nc[k]);
+        ihi[k] = min((int)floorf((m + e) * n + 2e-3f), 9 * g.nc[k]);
+    }
+}
 
 // cells near the solute: every cell within rnear of a solute atom (index
 // box).  A block takes 256 consecutive atoms of one frame (neighbours along
@@ -1798,7 +1942,9 @@ __device__ __forceinline__ void b_near_mark(KP P, Bufs B, int bx_, int nbx_, int
             }
         };
         for (int64_t at = bx_ * (int64_t)blockDim.x + threadIdx.x; at < P.nu; at += (int64_t)nbx_ * blockDim.x) {
-            const float4 s = B.tmp4[(int64_t)f * P.nu + at];
+            const float4 u = B.tmp4[(int64_t)f * P.nu + at];
+            float4 s;
+            fix_cart(g, __float_as_int(u.x), __float_as_int(u.y), __float_as_int(u.z), s.x, s.y, s.z);
             int ilo[3], ihi[3];
             cell_range(g, s.x, s.y, s.z, s.x, s.y, s.z, g.rnear, ilo, ihi);
             for (int iz = ilo[2]; iz <= ihi[2]; iz++) {
@@ -1903,21 +2049,20 @@ __device__ __forceinline__ void b_dfield(KP P, Bufs B, int bx_, int nbx_, int by
             const int c2 = (iz * g.nc[1] + iy) * g.nc[0] + ix;
             const int k0 = st[c2], k1 = st[c2 + 1];
             int k = k0;
+            auto dist = [&](const float4& a) {
+                float ex, ey, ez;
+                fix_cart(g, __float_as_int(a.x), __float_as_int(a.y), __float_as_int(a.z), ex, ey, ez);
+                ex -= rx; ey -= ry; ez -= rz;
+                best = fminf(best, ex * ex + ey * ey + ez * ez);
+            };
             for (; k + 3 < k1; k += 4) {
                 float4 a[4];
 #pragma unroll
                 for (int u = 0; u < 4; u++) a[u] = srt[k + u];
 #pragma unroll
-                for (int u = 0; u < 4; u++) {
-                    const float ex = a[u].x - rx, ey = a[u].y - ry, ez = a[u].z - rz;
-                    best = fminf(best, ex * ex + ey * ey + ez * ez);
-                }
+                for (int u = 0; u < 4; u++) dist(a[u]);
             }
-            for (; k < k1; k++) {
-                const float4 a = srt[k];
-                const float ex = a.x - rx, ey = a.y - ry, ez = a.z - rz;
-                best = fminf(best, ex * ex + ey * ey + ez * ez);
-            }
+            for (; k < k1; k++) dist(srt[k]);
         }
         // minimum over each eight-lane half (centre: lanes 0-6, corner: 8-15)
         best = fminf(best, __shfl_xor(best, 1, 64));
@@ -1999,9 +2144,9 @@ __device__ __forceinline__ float molecule_bound(const Geo& g, const BoundLoads& 
 }
 
 // real pass: centre of every solvent molecule (made whole around its first
-// atom) wrapped into the cell; near molecules get the Morton key of the cell
+// atom) wrapped into the cell; near molecules get the Hilbert key of the cell
 template <class T>
-__device__ __forceinline__ void b_prep_solvent_tiles(KP P, Bufs B, const T* xv, int bx_, int nbx_, int by_, int nby_)
+__device__ __forceinline__ void b_prep_solvent_tiles(KP P, Bufs B, const T* xv, const unsigned* tab, int bx_, int nbx_, int by_, int nby_)
 {
     int64_t total = (int64_t)P.F * P.Mv;
     for (int64_t it = bx_ * (int64_t)blockDim.x + threadIdx.x; it < total; it += (int64_t)nbx_ * blockDim.x) {
@@ -2016,16 +2161,18 @@ __device__ __forceinline__ void b_prep_solvent_tiles(KP P, Bufs B, const T* xv, 
         cell_of_frac(g, fr[0], fr[1], fr[2], cell, c0, c1, c2);
         int64_t kb = (int64_t)f * P.NP * P.Mv + v;
         if (!B.near[(int64_t)f * P.cap + cell]) { B.mkey[kb] = -1; continue; }
-        const int key = morton_key3(g, c0, c1, c2);
+        const int key = hilbert_key(tab, g.kbits, c0, c1, c2);
         B.mkey[kb] = key;
-        B.mrank[kb] = atomicAdd(&B.mcnt[(int64_t)f * P.NP * (P.kcap + 1) + key], 1);
+        B.mrank[kb] = atomicAdd(&B.mcnt[key_row(P, f, 0) + key], 1);
     }
 }
 
 template <class T>
 __global__ void k_prep_solvent_tiles(KP P, Bufs B, const T* xv)
 {
-    b_prep_solvent_tiles<T>(P, B, xv, blockIdx.x, gridDim.x, blockIdx.y, gridDim.y);
+    __shared__ unsigned tab[48];
+    hilbert_load(tab);
+    b_prep_solvent_tiles<T>(P, B, xv, tab, blockIdx.x, gridDim.x, blockIdx.y, gridDim.y);
 }
 
 // real pass: atoms of the near molecules in sorted order, FP32, in the frame of
@@ -2038,7 +2185,7 @@ __device__ __forceinline__ void b_fill_real(KP P, Bufs B, const T* xv, int bx_, 
         int f = (int)(it / P.Mv);
         int pos = (int)(it - (int64_t)f * P.Mv);
         const int64_t fp = (int64_t)f * P.NP;
-        if (pos >= B.nnear[fp]) continue;
+        if (pos >= B.nnear[(int64_t)f * (1 + P.NG)]) continue;
         const int v = B.msorted[fp * P.Mv + pos];
         const Geo g = ldc_geo(B.geo + f);
         const T* x = xv + (int64_t)f * P.Nv * 3;
@@ -2062,7 +2209,7 @@ __device__ __forceinline__ void b_fill_real(KP P, Bufs B, const T* xv, int bx_, 
             double xa, ya, za, ox, oy, oz;
             load3(x, a0 + a, xa, ya, za);
             cm::minimage(g.cell, xa - x0, ya - y0, za - z0, &ox, &oy, &oz);
-            dst[a] = mk4((float)(x0 + ox - tx), (float)(y0 + oy - ty), (float)(z0 + oz - tz), a == 0 ? ub : 0.f);
+            dst[a] = fix_point(g, x0 + ox - tx, y0 + oy - ty, z0 + oz - tz, a == 0 ? ub : 0.f);
         }
     }
 }
@@ -2073,28 +2220,80 @@ __global__ void k_fill_real(KP P, Bufs B, const T* xv)
     b_fill_real<T>(P, B, xv, blockIdx.x, gridDim.x, blockIdx.y, gridDim.y);
 }
 
-// exclusive scan of the cell counts of passes [p0, p0+np) of every frame (one
-// block per (frame, pass)); writes the number of near molecules of the pass
-// (the counts stay: the scatter counts them back down to zero)
-__device__ __forceinline__ void b_scan_rows(KP P, Bufs B, int p0, int np, int bx_, int nbx_, int by_, int nby_)
+// Keys per part of a row scan: a row is scanned by one block per part, at
+// most SCAN_PARTS of them, each part a multiple of 4096 keys (one step of the block).
+constexpr int SCAN_PARTS = 512;
+__host__ __device__ __forceinline__ int scan_part(int n)
+{
+    const int p = (n + SCAN_PARTS - 1) / SCAN_PARTS;
+    return p <= 8192 ? 8192 : (p + 4095) / 4096 * 4096;
+}
+__host__ __device__ __forceinline__ int scan_parts(int n) { return (n + scan_part(n) - 1) / scan_part(n); }
+
+// first part of row r of frame f in msum
+__device__ __forceinline__ int64_t part_row(const KP& P, int f, int r)
+{
+    const int p0 = scan_parts(P.kcap), pk = scan_parts(P.kcapr);
+    return (int64_t)f * (p0 + P.NG * pk) + (r > 0 ? p0 + (r - 1) * pk : 0);
+}
+
+// Molecules per part of the rows' key counts (rows of several parts): block
+// (part, row of the launch; the random groups of every frame, or the real pass)
+__device__ __forceinline__ void b_scan_sums(KP P, Bufs B, int random, int bx_, int nbx_, int by_, int nby_)
+{
+    __shared__ int wsum[16];
+    const int nr = random ? P.NG : 1, f = by_ / nr, r = random ? 1 + by_ - f * nr : 0;
+    const int n = random ? P.kcapr : P.kcap, sp = scan_part(n);
+    const int* c = B.mcnt + key_row(P, f, r);
+    const int lo = bx_ * sp, hi = min(n, lo + sp);
+    int t = 0;
+    for (int i = lo + threadIdx.x; i < hi; i += blockDim.x) t += c[i];
+    t = wave_incl_scan(t);
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    if (lane == 63) wsum[wid] = t;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int tot = 0;
+        for (int w = 0; w < nw; w++) tot += wsum[w];
+        B.msum[part_row(P, f, r) + bx_] = tot;
+    }
+}
+
+__global__ void __launch_bounds__(1024) k_scan_sums(KP P, Bufs B, int random)
+{
+    b_scan_sums(P, B, random, blockIdx.x, gridDim.x, blockIdx.y, gridDim.y);
+}
+
+// Exclusive scan of the key counts of the real pass or the random groups of
+// every frame (block (part, row)), each part starting from the molecules of
+// the parts before it; writes the number of near molecules of the row
+__device__ __forceinline__ void b_scan_rows(KP P, Bufs B, int random, int bx_, int nbx_, int by_, int nby_)
 {
     __shared__ int wsum[16];
     __shared__ int carry;
-    const int f = bx_ / np, pp = p0 + (int)(bx_ - (bx_ / np) * np);
-    const int64_t row = (int64_t)f * P.NP + pp;
-    int* c = B.mcnt + row * (P.kcap + 1);
-    int* st = B.mstart + row * (P.kcap + 1);
-    const int n = P.kcap;
+    const int nr = random ? P.NG : 1, f = by_ / nr, r = random ? 1 + by_ - f * nr : 0;
+    const int n = random ? P.kcapr : P.kcap, sp = scan_part(n);
+    const int64_t row = (int64_t)f * (1 + P.NG) + r;
+    const int* c = B.mcnt + key_row(P, f, r);
+    int* st = B.mstart + key_row(P, f, r);
     if (threadIdx.x == 0) carry = 0;
     __syncthreads();
     int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    if (bx_ > 0 && wid == 0) {
+        int t = 0;
+        for (int k = lane; k < bx_; k += 64) t += B.msum[part_row(P, f, r) + k];
+        t = wave_incl_scan(t);
+        if (lane == 63) carry = t;
+    }
+    __syncthreads();
     // four consecutive keys per thread, the threads' sums scanned over the
     // wavefront (DPP) and across the block's wavefronts
-    for (int base = 0; base < n; base += 4 * blockDim.x) {
+    const int lo = bx_ * sp, hi = min(n, lo + sp);
+    for (int base = lo; base < hi; base += 4 * blockDim.x) {
         const int i0 = base + 4 * threadIdx.x;
         int v[4];
 #pragma unroll
-        for (int u = 0; u < 4; u++) v[u] = i0 + u < n ? c[i0 + u] : 0;
+        for (int u = 0; u < 4; u++) v[u] = i0 + u < hi ? c[i0 + u] : 0;
         const int tsum = v[0] + v[1] + v[2] + v[3];
         const int incl = wave_incl_scan(tsum);
         if (lane == 63) wsum[wid] = incl;
@@ -2106,54 +2305,51 @@ __device__ __forceinline__ void b_scan_rows(KP P, Bufs B, int p0, int np, int bx
         // holds molecules of): most keys are empty, so only the others are written
 #pragma unroll
         for (int u = 0; u < 4; u++) {
-            if (i0 + u < n && v[u] != 0) st[i0 + u] = e;
+            if (i0 + u < hi && v[u] != 0) st[i0 + u] = e;
             e += v[u];
         }
         __syncthreads();
         if (threadIdx.x == 0) carry += tot;
         __syncthreads();
     }
-    if (threadIdx.x == 0) {
-        st[n] = carry;
-        B.nnear[row] = carry;
-    }
+    if (threadIdx.x == 0 && hi == n) B.nnear[row] = carry;
 }
 
-__global__ void __launch_bounds__(1024) k_scan_rows(KP P, Bufs B, int p0, int np)
+__global__ void __launch_bounds__(1024) k_scan_rows(KP P, Bufs B, int random)
 {
-    b_scan_rows(P, B, p0, np, blockIdx.x, gridDim.x, blockIdx.y, gridDim.y);
+    b_scan_rows(P, B, random, blockIdx.x, gridDim.x, blockIdx.y, gridDim.y);
 }
 
-// molecules of passes [p0, p0+np) sorted by cell
-__device__ __forceinline__ void b_mol_scatter(KP P, Bufs B, int p0, int np, int bx_, int nbx_, int by_, int nby_)
+// molecules of the real pass or of the random groups sorted by key
+__device__ __forceinline__ void b_mol_scatter(KP P, Bufs B, int random, int bx_, int nbx_, int by_, int nby_)
 {
-    // grid: x over the molecules, y over the (frame, pass) pairs
-    const int v = bx_ * blockDim.x + threadIdx.x;
-    if (v >= P.Mv) return;
-    for (int fq = by_; fq < P.F * np; fq += nby_) {
-        const int f = fq / np;
-        const int p = p0 + fq - f * np;
-        int64_t fp = (int64_t)f * P.NP + p;
-        int key = B.mkey[fp * P.Mv + v];
+    // grid: x over a row's slots, y over the rows
+    const int nr = random ? P.NG : 1;
+    const int s = bx_ * blockDim.x + threadIdx.x;
+    for (int fq = by_; fq < P.F * nr; fq += nby_) {
+        const int f = fq / nr, grp = fq - (fq / nr) * nr;
+        if (s >= (random ? group_slots(P, grp) : P.Mv)) continue;
+        const int64_t row = row_base(P, f, random, grp);
+        const int key = B.mkey[row + s];
         if (key < 0) continue;
         // the key's range starts where the scan put it; the molecule's rank
         // within the key was taken when the key was counted
-        const int pos = B.mstart[fp * (P.kcap + 1) + key] + B.mrank[fp * P.Mv + v];
-        B.msorted[fp * P.Mv + pos] = v;
+        const int pos = B.mstart[key_row(P, f, random ? 1 + grp : 0) + key] + B.mrank[row + s];
+        B.msorted[row + pos] = s;
     }
 }
 
-__global__ void k_mol_scatter(KP P, Bufs B, int p0, int np)
+__global__ void k_mol_scatter(KP P, Bufs B, int random)
 {
-    b_mol_scatter(P, B, p0, np, blockIdx.x, gridDim.x, blockIdx.y, gridDim.y);
+    b_mol_scatter(P, B, random, blockIdx.x, gridDim.x, blockIdx.y, gridDim.y);
 }
 
-// chunk offsets of the passes [p0, p0+np) of every frame (one block)
-__device__ __forceinline__ void b_chunk_table(KP P, Bufs B, int p0, int np, int bx_, int nbx_, int by_, int nby_)
+// chunk offsets of the real pass or the random groups of every frame (one block)
+__device__ __forceinline__ void b_chunk_table(KP P, Bufs B, int random, int bx_, int nbx_, int by_, int nby_)
 {
     __shared__ int wsum[16];
     __shared__ int carry;
-    int n = P.F * np;
+    const int nr = random ? P.NG : 1, n = P.F * nr, mpt = random ? P.mpt_r : P.mpt;
     if (threadIdx.x == 0) carry = 0;
     __syncthreads();
     int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
@@ -2161,15 +2357,10 @@ __device__ __forceinline__ void b_chunk_table(KP P, Bufs B, int p0, int np, int 
         int idx = base + threadIdx.x;
         int v = 0;
         if (idx < n) {
-            int f = idx / np, p = p0 + idx - f * np;
-            int nn = B.nnear[(int64_t)f * P.NP + p];
-            v = (nn + P.mpt - 1) / P.mpt;
+            const int f = idx / nr, r = random ? 1 + idx - f * nr : 0;
+            v = (B.nnear[(int64_t)f * (1 + P.NG) + r] + mpt - 1) / mpt;
         }
-        int incl = v;
-        for (int o = 1; o < 64; o <<= 1) {
-            int t = __shfl_up(incl, o, 64);
-            if (lane >= o) incl += t;
-        }
+        const int incl = wave_incl_scan(v);
         if (lane == 63) wsum[wid] = incl;
         __syncthreads();
         int woff = 0, tot = 0;
@@ -2185,15 +2376,15 @@ __device__ __forceinline__ void b_chunk_table(KP P, Bufs B, int p0, int np, int 
     }
 }
 
-__global__ void __launch_bounds__(1024) k_chunk_table(KP P, Bufs B, int p0, int np)
+__global__ void __launch_bounds__(1024) k_chunk_table(KP P, Bufs B, int random)
 {
-    b_chunk_table(P, B, p0, np, blockIdx.x, gridDim.x, blockIdx.y, gridDim.y);
+    b_chunk_table(P, B, random, blockIdx.x, gridDim.x, blockIdx.y, gridDim.y);
 }
 
 // randomize_solvent! (src/mddf.jl:65-88), first half: the new centre of every
-// slot; slots whose centre falls in a near cell get the Morton key of the cell
+// slot; slots whose centre falls in a near cell get the Hilbert key of the (half-)cell
 // (the others cannot have an atom within the cutoff of the solute)
-__device__ __forceinline__ void b_place_keys(KP P, Bufs B, int bx_, int nbx_, int by_, int nby_)
+__device__ __forceinline__ void b_place_keys(KP P, Bufs B, const unsigned* tab, int bx_, int nbx_, int by_, int nby_)
 {
     // grid: x over the slots, y over the (frame, pass) pairs
     const int v = bx_ * blockDim.x + threadIdx.x;
@@ -2202,20 +2393,24 @@ __device__ __forceinline__ void b_place_keys(KP P, Bufs B, int bx_, int nbx_, in
         const int f = fk / P.K;
         const int k = fk - f * P.K;
         const Geo g = ldc_geo(B.geo + f);
-        int64_t fp = (int64_t)f * P.NP + 1 + k;
+        const int grp = k / P.KM, sub = P.ksub;
+        const int64_t e = row_base(P, f, true, grp) + (int64_t)(k - grp * P.KM) * P.Mv + v;
         cm::u32x4 r = cm::philox4x32_10({(uint32_t)v, (uint32_t)k, g.frame, cm::TAG_SLOT}, P.key0, P.key1);
-        int cell, c0, c1, c2;
-        cell_of_draws(g, r.y, r.z, r.w, cell, c0, c1, c2);
-        if (!B.near[(int64_t)f * P.cap + cell]) { B.mkey[fp * P.Mv + v] = -1; continue; }
-        const int key = morton_key3(g, c0, c1, c2);
-        B.mkey[fp * P.Mv + v] = key;
-        B.mrank[fp * P.Mv + v] = atomicAdd(&B.mcnt[fp * (P.kcap + 1) + key], 1);
+        int c0, c1, c2;
+        cell_of_draws(g, r.y, r.z, r.w, sub, c0, c1, c2);
+        const int cell = ((c2 >> sub) * g.nc[1] + (c1 >> sub)) * g.nc[0] + (c0 >> sub);
+        if (!B.near[(int64_t)f * P.cap + cell]) { B.mkey[e] = -1; continue; }
+        const int key = hilbert_key(tab, g.kbits + sub, c0, c1, c2);
+        B.mkey[e] = key;
+        B.mrank[e] = atomicAdd(&B.mcnt[key_row(P, f, 1 + grp) + key], 1);
     }
 }
 
 __global__ void k_place_keys(KP P, Bufs B)
 {
-    b_place_keys(P, B, blockIdx.x, gridDim.x, blockIdx.y, gridDim.y);
+    __shared__ unsigned tab[48];
+    hilbert_load(tab);
+    b_place_keys(P, B, tab, blockIdx.x, gridDim.x, blockIdx.y, gridDim.y);
 }
 
 // second half: the placement of the near slots, written in sorted order (FP64
@@ -2223,15 +2418,15 @@ __global__ void k_place_keys(KP P, Bufs B)
 template <class TV>
 __device__ __forceinline__ void b_place_near(KP P, Bufs B, const TV* xv, int bx_, int nbx_, int by_, int nby_)
 {
-    // grid: x over the sorted positions, y over the (frame, pass) pairs
+    // grid: x over the sorted positions of a group, y over the (frame, group) rows
     const int pos = bx_ * blockDim.x + threadIdx.x;
-    if (pos >= P.Mv) return;
-    for (int fk = by_; fk < P.F * P.K; fk += nby_) {
-        const int f = fk / P.K;
-        const int k = fk - f * P.K;
-        int64_t fp = (int64_t)f * P.NP + 1 + k;
-        if (pos >= ldg(B.nnear + fp)) continue;
-        const int v = ldg(B.msorted + fp * P.Mv + pos);
+    for (int fg = by_; fg < P.F * P.NG; fg += nby_) {
+        const int f = fg / P.NG;
+        const int grp = fg - f * P.NG;
+        if (pos >= ldg(B.nnear + (int64_t)f * (1 + P.NG) + 1 + grp)) continue;
+        const int slot = ldg(B.msorted + row_base(P, f, true, grp) + pos);
+        const int kk = slot / P.Mv, v = slot - kk * P.Mv, k = grp * P.KM + kk;
+        const int64_t at = ((int64_t)f * P.K + (int64_t)grp * P.KM) * P.Nv + (int64_t)pos * P.nv;
         const Geo g = ldc_geo(B.geo + f);
         cm::u32x4 r = cm::philox4x32_10({(uint32_t)v, (uint32_t)k, g.frame, cm::TAG_SLOT}, P.key0, P.key1);
         cm::u32x4 r2 = cm::philox4x32_10({(uint32_t)v, (uint32_t)k, g.frame, cm::TAG_SLOT + 1u}, P.key0, P.key1);
@@ -2239,7 +2434,7 @@ __device__ __forceinline__ void b_place_near(KP P, Bufs B, const TV* xv, int bx_
         int nb = ldg(B.nbulk + lk);
         int64_t jmol = nb > 0 ? (int64_t)ldg(B.blist + lk * P.Mv + cm::draw_index(r.x, nb)) : cm::draw_index(r.x, P.Mv);
         MolSrc<TV> src(xv + (int64_t)f * P.Nv * 3 + jmol * P.nv * 3);
-        MolDst dst(B.P + (fk * P.Nv + (int64_t)pos * P.nv) * 3, B.vw_r + fk * P.Nv + (int64_t)pos * P.nv);
+        MolDstFix dst(B.P + 3 * at, B.vw_r + at, g);
         double uc[3] = {cm::u01(r.y), cm::u01(r.z), cm::u01(r.w)};
         double ua[3] = {cm::u01(r2.x), cm::u01(r2.y), cm::u01(r2.z)};
         // the placed centre is H uc (a rigid copy of a molecule of the frame):
@@ -2279,278 +2474,485 @@ __device__ __forceinline__ Rec rec_shfl_xor(const Rec& r, int o)
     return q;
 }
 
-// Column reduction of a running minimum over the C lanes of a row: DPP
-// quad permutations for the partners 1 and 2 lanes away (no LDS traffic),
-// a lane shuffle beyond.
-template <int O>
-__device__ __forceinline__ int xor_lane(int x)
+// Matrix-core distances.  A tile is 16 staged solute atoms (rows) against one
+// atom of 16 solvent molecules (columns): with s' = s - c and y' = y - c about
+// the chunk centre c, v_mfma_f32_16x16x4_f32 forms |s'|^2 - 2 y'.s' for the 256
+// pairs from the rows (s'x, s'y, s'z, |s'|^2) and the columns (-2 y', 1).  Lane
+// l gives the component l / 16 of row and column l % 16 and receives rows
+// 4 (l / 16) .. + 3 of its column.
+typedef float f4m __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ f4m pair_tile(float a, float b)
 {
-    if constexpr (O == 1) return __builtin_amdgcn_update_dpp(0, x, 0xB1, 0xf, 0xf, false);   // quad_perm 1,0,3,2
-    else if constexpr (O == 2) return __builtin_amdgcn_update_dpp(0, x, 0x4E, 0xf, 0xf, false);   // quad_perm 2,3,0,1
-    else return __shfl_xor(x, O, 64);
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, f4m{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
 }
 
-template <int O>
-__device__ __forceinline__ void col_merge(Best& b)
+// Running minimum b and second smallest s over four more values: the second
+// smallest of {b <= s} and {x, y} is min(s, med3(b, x, y)), so each pair of
+// values takes one three-input minimum and one median, and the medians go into
+// s two at a time: five instructions for four values.
+__device__ __forceinline__ void min2_4(float& b, float& s, const f4m& v)
 {
-    const float b2 = __int_as_float(xor_lane<O>(__float_as_int(b.best)));
-    const float s2 = __int_as_float(xor_lane<O>(__float_as_int(b.second)));
-    const int i2 = xor_lane<O>(b.bi);
-    const float ns = fminf(fmaxf(b.best, b2), fminf(b.second, s2));
-    if (b2 < b.best) b.bi = i2;
-    b.best = fminf(b.best, b2);
-    b.second = ns;
+    const float m = fminf(fminf(b, v[0]), v[1]), t0 = __builtin_amdgcn_fmed3f(b, v[0], v[1]);
+    const float t1 = __builtin_amdgcn_fmed3f(m, v[2], v[3]);
+    b = fminf(fminf(m, v[2]), v[3]);
+    s = fminf(fminf(s, t0), t1);
 }
 
-template <int C>
-__device__ __forceinline__ void col_reduce(Best& b)
-{
-    if constexpr (C >= 2) col_merge<1>(b);
-    if constexpr (C >= 4) col_merge<2>(b);
-    if constexpr (C >= 8) col_merge<4>(b);
-}
+// a minimum with its second smallest value and the code of its candidate
+struct Min2 {
+    float b, s;
+    int c;
+    __device__ __forceinline__ void init() { b = INFINITY; s = INFINITY; c = -1; }
+    __device__ __forceinline__ void merge(float b2, float s2, int c2)
+    {
+        s = fminf(fmaxf(b, b2), fminf(s, s2));
+        c = b2 < b ? c2 : c;
+        b = fminf(b, b2);
+    }
+};
 
-// Minimum distances of the solvent molecules of one chunk per wavefront
-// (64 threads).  Lane = (row, column); the C columns of a row split the
-// staged solute atoms between them.  NVM = 0: a row is one solvent atom and
-// the atoms of a molecule are combined across rows.  NVM > 0 (molecules of
-// NVM atoms, e.g. water): a row is one molecule, each lane evaluates every
-// staged atom against all NVM atoms it holds in registers (one LDS read per
-// NVM pairs) and combines them in the lane.
-template <class TU, class TV, bool RANDOM, int C, int NVM, bool VERIFY>
-__device__ __forceinline__ void eval_tiles_chunks(const KP& P, const Bufs& B, const TU* xu, const TV* xv, int ch0, int ch1,
-                                                  int chs, float4* stg, float* stw, const int* cbs, bool cb_lds,
-                                                  int* ctr)
+// The lanes 16 and 32 away hold the other rows of the same 16 molecules (per
+// group): merged over them, lane l ends with molecule (l / 32) 16 + l % 16 of two
+// groups or l % 16 of one.
+template <int GH>
+__device__ __forceinline__ Min2 gather_groups(const Min2 (&m)[GH], int lane)
 {
-    // chunks of one job below ch1: ch0, ch0 + chs, ... below tdyn, then
-    // (with a counter ctr, zero at the start of the launch) the chunks from
-    // tdyn on in the order the workgroups ask for them, so the ones that
-    // finish early take more of the last chunks.  The chunks' costs vary
-    // with their staged atoms, and a fixed stride alone leaves a tail of
-    // workgroups still busy; requests go to one device-wide counter, so
-    // only the last DYN_PCT per cent are handed out that way, a few
-    // consecutive chunks per request.
-    // LDS: the staging buffer stg (P.tcap float4: atom, index; relative to
-    // the chunk centre when NVM > 0), with NVM > 0 the squared norms stw of
-    // the staged atoms, and (cb_lds) the job's chunk table cbs
-    const int tcap = P.tcap;
-    // staging ranks per lane per step (fewer with a molecule per lane, whose
-    // evaluation holds more registers)
-    constexpr int SUk = NVM > 0 ? 2 : SU;
-    const int lane = threadIdx.x;
-    const int row = lane / C, col = lane - (lane / C) * C;
-    const int p0 = RANDOM ? 1 : 0;
-    const int npass = RANDOM ? P.K : 1;
-    const int nfp = P.F * npass;
-    ull* gu = RANDOM ? B.cnt_gu_r : B.cnt_gu;
-    ull* gv = RANDOM ? B.cnt_gv_r : B.cnt_gv;
-    ull* gmd = RANDOM ? B.cnt_md_r : B.cnt_md;
-    ull* grdf = RANDOM ? B.cnt_rdf_r : B.cnt_rdf;
-    const int ndyn = (int)((int64_t)ch1 * DYN_PCT / 100);
-    const int tdyn = ctr && ch1 >= DYN_MIN * chs ? ch1 - ndyn : ch1;
-    const int dgrab = max(1, ndyn / (chs * DYN_GRABS));   // chunks per request
-    int dnext = 0, dend = 0;
-    auto next_chunk = [&](int c) {
-        if (c < tdyn || tdyn == ch1) return c;
-        if (dnext < dend) return dnext++;
-        int g = 0;
-        if (lane == 0) g = atomicAdd(ctr, dgrab);
-        dnext = tdyn + __builtin_amdgcn_readlane(g, 0);
-        dend = dnext + dgrab;
-        return dnext++;
+    auto recv = [&](Min2& keep, const Min2& send, int o) {
+        keep.merge(__shfl_xor(send.b, o, 64), __shfl_xor(send.s, o, 64), __shfl_xor(send.c, o, 64));
     };
-    for (int ch = next_chunk(ch0); ch < ch1; ch = next_chunk(ch + chs)) {
-        int lo_ = 0, hi_ = nfp;
-        while (hi_ - lo_ > 1) {
-            int mid = (lo_ + hi_) >> 1;
-            if ((cb_lds ? cbs[mid] : B.chunk_base[mid]) <= ch) lo_ = mid; else hi_ = mid;
+    auto pick = [](bool hi, const Min2& x, const Min2& y) {
+        Min2 r;
+        r.b = hi ? y.b : x.b; r.s = hi ? y.s : x.s; r.c = hi ? y.c : x.c;
+        return r;
+    };
+    const bool h5 = (lane & 32) != 0;
+    Min2 k = GH == 2 ? pick(h5, m[0], m[GH - 1]) : m[0];
+    recv(k, GH == 2 ? pick(h5, m[GH - 1], m[0]) : m[0], 32);
+    recv(k, k, 16);
+    return k;
+}
+
+// LDS of the evaluation: the block's histograms, the launch's chunk table,
+// then one area per wavefront
+extern __shared__ float dyn[];
+
+// LDS writes of a wavefront before reads of its other lanes (its LDS
+// operations execute in order: only the compiler must keep them so)
+__device__ __forceinline__ void wave_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+constexpr int TQ_GEN = 4;           // solvent atoms per block of tiles (molecules of any size)
+constexpr int EV_ROWS = 32;         // staged atoms per step (two row tiles)
+constexpr int TCAP = 288;           // staged solute atoms per round (at least 256, a multiple of 32)
+constexpr int SEG = 4;              // staging: consecutive atoms per lane
+
+// words of a wavefront's area: staged components and indices, the columns of
+// one block of tiles (-2 y' and |y'|^2 per atom), the segments of one step
+__host__ __device__ constexpr int eval_wave_words(int G, int TQ) { return 5 * TCAP + 4 * TQ * 16 * G + 2 * 64; }
+
+// Block histograms.  Millions of records per launch go into a few hundred md
+// and rdf bins: as global atomics they bounded the launch (the random passes of
+// 40 frames of the globule job 1.65 ms with them, 1.05 ms with the same kernel
+// and no md/rdf updates), so every block counts in LDS and adds its non-zero
+// bins once at its end.  Word offsets into dyn; negative: straight to memory
+// (histograms beyond EV_HIST words).
+constexpr int EV_HIST = 8192;
+struct EvHist {
+    int md, rdf, gv;
+    __host__ __device__ static int words(const KP& P)
+    {
+        return (2 * P.nbins <= EV_HIST ? 2 * P.nbins : 0) + gvw(P);
+    }
+    __host__ __device__ static int gvw(const KP& P)
+    {
+        const int64_t n = (int64_t)P.gnv * P.nbins;
+        return 2 * P.nbins <= EV_HIST && n <= EV_HIST - 2 * P.nbins ? (int)n : 0;
+    }
+    __device__ explicit EvHist(const KP& P)
+    {
+        const bool in = 2 * P.nbins <= EV_HIST;
+        md = in ? 0 : -1;
+        rdf = in ? P.nbins : -1;
+        gv = gvw(P) > 0 ? 2 * P.nbins : -1;
+    }
+};
+
+__device__ __forceinline__ void ev_hist_clear(const KP& P)
+{
+    for (int k = threadIdx.x; k < EvHist::words(P); k += blockDim.x) ((unsigned*)dyn)[k] = 0u;
+}
+
+template <bool RANDOM>
+__device__ __forceinline__ void ev_hist_flush(const KP& P, const Bufs& B)
+{
+    const EvHist h(P);
+    const unsigned* sh = (const unsigned*)dyn;
+    ull* md = RANDOM ? B.cnt_md_r : B.cnt_md;
+    ull* rdf = RANDOM ? B.cnt_rdf_r : B.cnt_rdf;
+    ull* gv = RANDOM ? B.cnt_gv_r : B.cnt_gv;
+    if (h.md >= 0)
+        for (int k = threadIdx.x; k < P.nbins; k += blockDim.x) {
+            if (sh[k]) atomicAdd(&md[k], (ull)sh[k]);
+            if (sh[P.nbins + k]) atomicAdd(&rdf[k], (ull)sh[P.nbins + k]);
         }
-        const int fq = lo_;
-        const int f = fq / npass, pidx = fq - (fq / npass) * npass;
-        const int p = p0 + pidx;
-        const int64_t fp = (int64_t)f * P.NP + p;
-        const Geo& g = B.geo[f];
-        const int m0 = (ch - (cb_lds ? cbs[fq] : B.chunk_base[fq])) * P.mpt;
-        const int ml = NVM ? row : row / P.nv, a = NVM ? 0 : row - (row / P.nv) * P.nv;
-        // the molecule's loads are issued together with the near count that
-        // decides whether the lane has a molecule (positions past the count
-        // read a valid slot and are discarded)
-        const int mpos = min(m0 + ml, P.Mv - 1);
-        const int nm = min(P.mpt, B.nnear[fp] - m0);
-        const int vld = B.msorted[fp * P.Mv + mpos];
-        const float4* vwb = RANDOM ? B.vw_r + ((int64_t)f * P.K + pidx) * P.Nv : B.vw + (int64_t)f * P.Nv;
-        const int64_t pbase = (int64_t)mpos * P.nv;   // sorted position of the molecule
-        float4 y = mk4(0.f, 0.f, 0.f, 0.f);
-        float4 ym[NVM > 0 ? NVM : 1];   // molecule per lane: its atoms
-        if constexpr (NVM > 0) {
-#pragma unroll
-            for (int q = 0; q < NVM; q++) ym[q] = vwb[pbase + q];
-        } else {
-            y = vwb[pbase + a];
+    const int n = EvHist::gvw(P);
+    for (int k = threadIdx.x; k < n; k += blockDim.x)
+        if (sh[h.gv + k]) atomicAdd(&gv[k], (ull)sh[h.gv + k]);
+}
+
+// The counts of a complete record (update_counters!, src/update_counters.jl:43-88)
+// of solute atom i and atom `local` of the solvent molecule whose first atom is
+// jbase (one solute molecule: i is molecule-local).  With h null, straight to
+// memory.
+template <bool RANDOM>
+__device__ __forceinline__ void ev_hist_record(const KP& P, const Bufs& B, const EvHist* h, const Rec& r, int local, int64_t jbase)
+{
+    if (!r.within) return;
+    const int b = r.bin;
+    if (b >= P.nbins) return;   // unreachable: d <= cutoff (validated at job creation)
+    unsigned* sh = (unsigned*)dyn;
+    if (h && h->md >= 0) atomicAdd(&sh[h->md + b], 1u);
+    else atomicAdd(&(RANDOM ? B.cnt_md_r : B.cnt_md)[b], 1ull);
+    group_hit_local(RANDOM ? B.cnt_gu_r : B.cnt_gu, P.nbins, b, r.i, r.i, P.gu_ptr, P.gu_idx);
+    if (h && h->gv >= 0) {
+        if (!P.gv_ptr) atomicAdd(&sh[h->gv + local * P.nbins + b], 1u);
+        else
+            for (int k = P.gv_ptr[jbase + local]; k < P.gv_ptr[jbase + local + 1]; k++)
+                atomicAdd(&sh[h->gv + P.gv_idx[k] * P.nbins + b], 1u);
+    } else {
+        group_hit_local(RANDOM ? B.cnt_gv_r : B.cnt_gv, P.nbins, b, local, jbase + local, P.gv_ptr, P.gv_idx);
+    }
+    if (r.ref && r.rbin < P.nbins) {
+        if (h && h->rdf >= 0) atomicAdd(&sh[h->rdf + r.rbin], 1u);
+        else atomicAdd(&(RANDOM ? B.cnt_rdf_r : B.cnt_rdf)[r.rbin], 1ull);
+    }
+}
+
+// where a chunk of a launch lies: frame, random group, its row of the sorted
+// molecules, first molecule, molecules, first atom (B.vw / B.vw_r, B.P)
+struct ChunkAt {
+    int f, grp, m0, nm;
+    int64_t row, atom;
+    template <class CB>
+    __device__ ChunkAt(const KP& P, const Bufs& B, bool random, int ch, CB base)
+    {
+        const int nr = random ? P.NG : 1;
+        int lo = 0, hi = P.F * nr;
+        while (hi - lo > 1) {
+            const int mid = (lo + hi) >> 1;
+            if (base(mid) <= ch) lo = mid; else hi = mid;
         }
-        const bool active = ml < nm;
-        const int v = active ? vld : 0;
-        float alx, aly, alz, ahx, ahy, ahz;   // box of the lane's atoms
-        if constexpr (NVM > 0) {
+        const int fq = __builtin_amdgcn_readfirstlane(lo);
+        const int mpt = random ? P.mpt_r : P.mpt;
+        f = fq / nr;
+        grp = fq - f * nr;
+        m0 = __builtin_amdgcn_readfirstlane((ch - base(fq)) * mpt);
+        row = row_base(P, f, random, grp);
+        nm = min(mpt, ldg(B.nnear + (int64_t)f * (1 + P.NG) + (random ? 1 + grp : 0)) - m0);
+        atom = (random ? ((int64_t)f * P.K + (int64_t)grp * P.KM) * P.Nv : (int64_t)f * P.Nv) + (int64_t)m0 * P.nv;
+    }
+};
+
+// Minimum distances of the solvent molecules of one chunk, one wavefront.  The
+// chunk's molecules (at most 16 G) are consecutive in the sorted order, so their
+// atoms are contiguous; TQ solvent atoms of every molecule are evaluated
+// together (all three of 3-atom molecules, blocks of four otherwise).  Records
+// that FP32 decides are counted here; the molecules it cannot decide (a bin
+// edge, the cutoff or dbulk within the guard, or an argmin closer than the
+// guard) are left to k_resolve: one bit each in the chunk's word of resmask, and
+// the squared radii that hold every candidate in the w of the molecule's first
+// two atoms.
+//
+// What bounds it: per step of 32 staged atoms and 16 molecules a solvent atom
+// costs two matrix instructions (64 cycles) and 12 vector ones (48 cycles) that
+// keep the minimum, the second smallest and the step; they run side by side.
+// The rest is latency (segment loads, LDS), which the block's other wavefronts
+// fill: no FP64 here keeps the kernel at 128 registers, 16 wavefronts per CU.
+template <class TU, class TV, bool RANDOM, int G, int TQ, bool VERIFY>
+__device__ __forceinline__ void eval_chunk(const KP& P, const Bufs& B, const TU* xu, const TV* xv, int ch, const ChunkAt& at,
+                                           int wofs, const EvHist& hist)
+{
+    // wofs: the wavefront's LDS area.  Staged atoms relative to the chunk
+    // centre, atom n's component k (x, y, z, squared norm) at (n / 16) 64 + 16 k
+    // + n % 16 (the order in which the lanes of a row tile read them), their
+    // indices, the columns [atom of the block][-2 y'x, -2 y'y, -2 y'z, |y'|^2]
+    // [molecule], the segments of a staging step
+    constexpr int MC = 16 * G;
+    float* const lds = dyn + wofs;
+    int* const si = (int*)(lds + 4 * TCAP);
+    float* const yb = lds + 5 * TCAP;
+    int2* const sd = (int2*)(yb + 4 * TQ * MC);
+    // (opaque per chunk: what depends on the lane alone is formed where it is
+    // used, not held in registers over the whole launch)
+    int lane = threadIdx.x & 63;
+    asm volatile("" : "+v"(lane));
+    // groups are evaluated two at a time (half h of four groups: the lanes with
+    // bit 4 equal to h keep its molecules)
+    constexpr int GH = G == 1 ? 1 : 2;
+    // the molecule of the chunk this lane decides, and whether it is the one
+    // lane that does
+    const int ml = (G == 4 ? ((lane >> 4) & 1) << 5 : 0) + (G == 1 ? 0 : (lane >> 5) << 4) + (lane & 15);
+    const bool lead = G == 4 || (G == 2 ? (lane & 16) == 0 : lane < 16);
+    const int f = at.f, nm = at.nm;
+    const GeoC& g = *(const GeoC*)(B.geo + f);
+    float4* vwb = (RANDOM ? B.vw_r : B.vw) + at.atom;   // the chunk's atoms
+    const int na = nm * P.nv;
+    const bool active = lead && ml < nm;
+    const int slot = ldg(B.msorted + at.row + at.m0 + min(ml, nm - 1));
+    // box of the chunk's atoms about an atom in their middle; the first
+    // atom's w is the molecule's bound
+    const gptr<const f4v> vg = (gptr<const f4v>)vwb;
+    const f4v mid = vg[(nm >> 1) * P.nv];
+    int cix = __builtin_amdgcn_readfirstlane(__float_as_int(mid.x)), ciy = __builtin_amdgcn_readfirstlane(__float_as_int(mid.y)),
+        ciz = __builtin_amdgcn_readfirstlane(__float_as_int(mid.z));
+    // position relative to the chunk's (integer) centre
+    auto rel = [&](f4v y, float& x_, float& y_, float& z_) {
+        fix_cart(g, __float_as_int(y.x) - cix, __float_as_int(y.y) - ciy, __float_as_int(y.z) - ciz, x_, y_, z_);
+    };
+    float alx = INFINITY, aly = INFINITY, alz = INFINITY, ahx = -INFINITY, ahy = -INFINITY, ahz = -INFINITY, um = 0.f;
+    auto box = [&](const f4v& y) {
+        float x_, y_, z_;
+        rel(y, x_, y_, z_);
+        alx = fminf(alx, x_); aly = fminf(aly, y_); alz = fminf(alz, z_);
+        ahx = fmaxf(ahx, x_); ahy = fmaxf(ahy, y_); ahz = fmaxf(ahz, z_);
+        um = fmaxf(um, y.w);
+    };
+    if (TQ == 3) {
+        // 3-atom molecules: at most 3 G / 4 loads per lane, together
+        f4v y[(3 * G + 3) / 4];
 #pragma unroll
-            for (int q = 0; q < NVM; q++) if (!active) ym[q] = mk4(0.f, 0.f, 0.f, 0.f);
-            alx = ahx = ym[0].x; aly = ahy = ym[0].y; alz = ahz = ym[0].z;
+        for (int t = 0; t < (3 * G + 3) / 4; t++) y[t] = vg[min(64 * t + lane, na - 1)];
 #pragma unroll
-            for (int q = 1; q < NVM; q++) {
-                alx = fminf(alx, ym[q].x); aly = fminf(aly, ym[q].y); alz = fminf(alz, ym[q].z);
-                ahx = fmaxf(ahx, ym[q].x); ahy = fmaxf(ahy, ym[q].y); ahz = fmaxf(ahz, ym[q].z);
+        for (int t = 0; t < (3 * G + 3) / 4; t++) box(y[t]);
+    } else {
+        for (int e = lane; e < na; e += 256) {
+            f4v y[4];
+#pragma unroll
+            for (int t = 0; t < 4; t++) y[t] = vg[min(e + 64 * t, na - 1)];
+#pragma unroll
+            for (int t = 0; t < 4; t++) box(y[t]);
+        }
+    }
+    um = wave_max(um);
+    // the centre moves to the middle of the box (in whole units: exact), the
+    // box with it (to FP32 rounding, inside the staging radius' slack)
+    float bx, by, bz;   // half sides
+    {
+        const float lx = wave_min(alx), ly = wave_min(aly), lz = wave_min(alz);
+        const float hx = wave_max(ahx), hy = wave_max(ahy), hz = wave_max(ahz);
+        const float mx = 0.5f * (lx + hx), my = 0.5f * (ly + hy), mz = 0.5f * (lz + hz);
+        bx = sgpr_f(0.5f * (hx - lx) + 1e-4f); by = sgpr_f(0.5f * (hy - ly) + 1e-4f); bz = sgpr_f(0.5f * (hz - lz) + 1e-4f);
+        const float sc = ldexpf(1.0f, g.fix);
+        cix += __builtin_amdgcn_readfirstlane((int)rintf((g.Hi32[0] * mx + g.Hi32[3] * my + g.Hi32[6] * mz) * sc));
+        ciy += __builtin_amdgcn_readfirstlane((int)rintf((g.Hi32[1] * mx + g.Hi32[4] * my + g.Hi32[7] * mz) * sc));
+        ciz += __builtin_amdgcn_readfirstlane((int)rintf((g.Hi32[2] * mx + g.Hi32[5] * my + g.Hi32[8] * mz) * sc));
+    }
+    const float rs_full = g.rstage;
+    // Distances relative to the chunk centre c (a fixed-point position, no
+    // rounding of its own): |y' - s'|^2 = (|s'|^2 - 2 y'.s') + |y'|^2.  With u =
+    // 2^-24, Y >= |y'| and S >= |s'| for every staged atom, y' and s' are off by
+    // at most rho u Y and rho u S (fix_cart), which moves d^2 by at most
+    // 2 rho u (Y + S) d (d <= cutsys + 0.5 where it matters); the norms (3 u S^2,
+    // 3 u Y^2), the four products and three additions of a tile in whatever
+    // order (2 u Y S + 3 u (S^2 + 2 Y S)) and the last sum (u (Y + S)^2) add at
+    // most 7 u (Y + S)^2.  Both widen the frame's guard for this chunk (FP32
+    // here, every value rounded outward by the factors; S <= Y + the staging
+    // radius, which is at most um + 0.3).  The columns hold -2 y' (exact scaling).
+    float Gcf, cut2_hi_c, amb_c;
+    {
+        const float Yb = __builtin_amdgcn_sqrtf(bx * bx + by * by + bz * bz) * (1.0f + 4e-6f) + 1e-3f;
+        const float YS = 2.0f * Yb + fminf(rs_full, um + 0.3f) * (1.0f + 1e-5f) + 1e-3f;
+        const float gd = 0x1p-24f * YS * (2.0f * g.rho * ((float)P.cutsys + 0.5f) + 7.0f * YS) * (1.0f + 1e-5f) + 1e-8f;
+        Gcf = sgpr_f((g.guard_up + gd) * (1.0f + 1e-6f));
+        cut2_hi_c = sgpr_f((P.c2hi32 + Gcf) * (1.0f + 1e-6f));
+        amb_c = sgpr_f(2.0f * Gcf + cut2_hi_c * 0x1p-20f);
+    }
+    // Staging radius.  Each molecule carries an upper bound U on its
+    // atoms' nearest solute distance (molecule_bound).  A solute atom that
+    // can decide anything for an atom p of the chunk (its FP64 nearest,
+    // or within the FP32 decision band of it) is within
+    // sqrt(U^2 + 2 G + amb) of p, hence of the AABB; staging out to
+    // sqrt(U^2 + 2 amb + 4 G) plus a slack over FP32 rounding keeps every
+    // such atom, and the farther ones cannot change a decision.
+    float rs = rs_full;
+    if (um < rs_full)
+        rs = sgpr_f(fminf(rs_full, fminf(__builtin_amdgcn_sqrtf(fmaf(um, um, 2.0f * amb_c + 4.0f * Gcf)) * (1.0f + 1e-5f) + 1e-2f, um + 0.3f)));
+    const float rs2 = rs * rs;
+    int ilo[3], ihi[3];
+    cell_range32(g, cix, ciy, ciz, bx + rs, by + rs, bz + rs, ilo, ihi);
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        ilo[k] = __builtin_amdgcn_readfirstlane(ilo[k]);
+        ihi[k] = __builtin_amdgcn_readfirstlane(ihi[k]);
+    }
+    const int ny = ihi[1] - ilo[1] + 1, nz = ihi[2] - ilo[2] + 1;
+    const gptr<const int> st = (gptr<const int>)(B.start + (int64_t)f * (P.cap + 1));
+    const gptr<const f4v> srt = (gptr<const f4v>)(B.sorted + (int64_t)f * B.nitems);
+    // the lane's molecule over all rounds: minimum, second smallest and
+    // argmin pair, and the same for the reference atom
+    float mb = INFINITY, ms = INFINITY, rb = INFINITY, rsec = INFINITY;
+    float mdir = INFINITY, rdir = INFINITY;   // the argmin pairs' d^2 in the direct form
+    int mi = -1, ma = 0, ri = -1;
+    const unsigned long long lt_mask = (1ull << lane) - 1ull;
+    auto evaluate = [&](int n) {
+        // rows past n are far away and never the minimum
+        const int nsteps = (n + EV_ROWS - 1) / EV_ROWS;
+        if (lane < nsteps * EV_ROWS - n) {
+            const int q = n + lane, o = (q >> 4) * 64 + (q & 15);
+            lds[o] = 0.f; lds[o + 16] = 0.f; lds[o + 32] = 0.f; lds[o + 48] = 1e30f;
+            si[q] = -1;
+        }
+        Min2 wm, wr;
+        wm.init(); wr.init();
+        const int nvv = TQ == 3 ? 3 : P.nv;
+        for (int qb = 0; qb < nvv; qb += TQ) {
+            // columns of this block of atoms (zero where there is no molecule or atom)
+            for (int e = lane; e < MC * TQ; e += 64) {
+                const int m = e / TQ, qq = e - m * TQ;
+                float yx = 0.f, yy = 0.f, yz = 0.f;
+                if (m < nm && qb + qq < nvv) rel(vg[m * nvv + qb + qq], yx, yy, yz);
+                float* o = yb + qq * 4 * MC + m;
+                o[0] = -2.0f * yx; o[MC] = -2.0f * yy; o[2 * MC] = -2.0f * yz;
+                o[3 * MC] = fmaf(yx, yx, fmaf(yy, yy, yz * yz));
             }
-        } else {
-            if (!active) y = mk4(0.f, 0.f, 0.f, 0.f);
-            alx = ahx = y.x; aly = ahy = y.y; alz = ahz = y.z;
-        }
-        const float lx = wave_min(active ? alx : INFINITY), ly = wave_min(active ? aly : INFINITY),
-                    lz = wave_min(active ? alz : INFINITY);
-        const float hx = wave_max(active ? ahx : -INFINITY), hy = wave_max(active ? ahy : -INFINITY),
-                    hz = wave_max(active ? ahz : -INFINITY);
-        const float rs_full = g.rstage;
-        // NVM > 0: distances relative to the chunk centre c.  With y' = y - c
-        // and s' = s - c, |y' - s'|^2 = (|s'|^2 - 2 y'.s') + |y'|^2: three FMAs
-        // per pair against the staged (s', |s'|^2), |y'|^2 added once per atom.
-        // With u = 2^-24, Y >= |y'| and S >= |s'| for every staged atom, the
-        // rounding of the c subtractions moves y' - s' by at most u (Y + S),
-        // so d^2 by at most 2 u (Y + S) d (d <= cutsys + 0.5 where it
-        // matters); the norms (3 u S^2, 3 u Y^2), the FMA chain (3 u (S^2 +
-        // 2 Y S)) and the last sum (u (Y + S)^2) add at most 7 u (Y + S)^2.
-        // Both widen the frame's guard for this chunk.
-        // The molecule's atoms are kept as -2 y' (exact scaling of y').
-        // The per-chunk values are wave-uniform and held in scalar registers.
-        float ccx = 0.f, ccy = 0.f, ccz = 0.f;
-        float Gcf = (float)g.guard, cut2_hi_c = g.cut2_hi, amb_c = g.amb, G32c = g.guard32;
-        if constexpr (NVM > 0) {
-            ccx = sgpr_f(0.5f * (lx + hx)); ccy = sgpr_f(0.5f * (ly + hy)); ccz = sgpr_f(0.5f * (lz + hz));
-            const double ex = (double)hx - lx, ey = (double)hy - ly, ez = (double)hz - lz;
-            // (+ the rounding of c itself, at most 2^-24 |c| per component)
-            const double Yb = 0.5 * sqrt(ex * ex + ey * ey + ez * ez) * (1.0 + 1e-6) +
-                              1e-6 * ((double)fabsf(ccx) + fabsf(ccy) + fabsf(ccz)) + 1e-5;
-            const double Sb = Yb + (double)rs_full * (1.0 + 1e-5) + 1e-4;
-            const double Gc = g.guard + 0x1p-24 * (Yb + Sb) * (2.0 * (P.cutsys + 0.5) + 7.0 * (Yb + Sb)) + 1e-9;
-            Gcf = sgpr_f(nextafterf((float)Gc, INFINITY));
-            cut2_hi_c = sgpr_f(nextafterf((float)(P.cut2 + Gc), INFINITY));
-            amb_c = sgpr_f(nextafterf((float)(2.0 * Gc) + 8.0f * (float)(halfulp32((double)cut2_hi_c) * 2.0), INFINITY));
-            G32c = sgpr_f(nextafterf((float)(Gc + (P.cut2 + Gc + 1.0) * 0x1p-21), INFINITY));
+            wave_sync();
+#pragma unroll 1
+            for (int h = 0; h < G / GH; h++) {
+                const float* yh = yb + h * 16 * GH + (lane & 15);
+                float bc[GH][TQ], vb[GH][TQ], vs[GH][TQ];
+                int vc[GH][TQ];
 #pragma unroll
-            for (int q = 0; q < NVM; q++)
-                ym[q] = mk4(-2.0f * (ym[q].x - ccx), -2.0f * (ym[q].y - ccy), -2.0f * (ym[q].z - ccz), ym[q].w);
-        }
-        // Staging radius.  Each molecule carries an upper bound U on its
-        // atoms' nearest solute distance (molecule_bound).  A solute atom that
-        // can decide anything for an atom p of the chunk (its FP64 nearest,
-        // or within the FP32 decision band of it) is within
-        // sqrt(U^2 + 2 G + amb) of p, hence of the AABB; staging out to
-        // sqrt(U^2 + 2 amb + 4 G) plus a slack over FP32 rounding keeps every
-        // such atom, and the farther ones cannot change a decision.
-        float rs = rs_full;
-        {
-            const float um = wave_max(active ? (NVM > 0 ? ym[0].w : y.w) : 0.f);
-            if (um < rs_full)
-                rs = sgpr_f(fminf(rs_full, sqrtf(fmaf(um, um, 2.0f * amb_c + 4.0f * Gcf)) * (1.0f + 1e-5f) + 1e-2f));
-        }
-        const float rs2 = rs * rs;
-        int ilo[3], ihi[3];
-        cell_range(g, lx, ly, lz, hx, hy, hz, rs, ilo, ihi);
-        const int nx = ihi[0] - ilo[0] + 1, ny = ihi[1] - ilo[1] + 1, nz = ihi[2] - ilo[2] + 1;
-        const int ncl = nx * ny * nz;
-        const int* st = B.start + (int64_t)f * (P.cap + 1);
-        const float4* srt = B.sorted + (int64_t)f * B.nitems;
-        Best bb;
-        bb.init();
-        Best bq[NVM > 0 ? NVM : 1];   // molecule per lane: each atom's running minimum
+                for (int gg = 0; gg < GH; gg++)
 #pragma unroll
-        for (int q = 0; q < (NVM > 0 ? NVM : 1); q++) bq[q].init();
-        int rounds = 0;
-        int nst = 0;   // staged atoms (uniform)
-        const unsigned long long lt_mask = (1ull << lane) - 1ull;
-        auto evaluate = [&](int n) {
-            __syncthreads();
-            if constexpr (NVM > 0) {
-                // |s'|^2 - 2 y'.s' per atom of the molecule (|y'|^2 added after
-                // the last round); four staged atoms per step, loads first
-                int k = col;
-                for (; k + 3 * C < n; k += 4 * C) {
-                    float4 sv[4];
-                    float wv[4];
+                    for (int qq = 0; qq < TQ; qq++) {
+                        const float c = yh[(qq * 4 + (lane >> 4)) * MC + gg * 16];
+                        bc[gg][qq] = lane >= 48 ? 1.0f : c;
+                        vb[gg][qq] = INFINITY; vs[gg][qq] = INFINITY; vc[gg][qq] = 0;
+                    }
+#pragma unroll 1
+                for (int k = 0; k < nsteps; k++) {
+                    const float a0 = lds[k * 128 + lane], a1 = lds[k * 128 + 64 + lane];
 #pragma unroll
-                    for (int u = 0; u < 4; u++) { sv[u] = stg[k + u * C]; wv[u] = stw[k + u * C]; }
+                    for (int gg = 0; gg < GH; gg++)
 #pragma unroll
-                    for (int u = 0; u < 4; u++)
-#pragma unroll
-                        for (int q = 0; q < NVM; q++)
-                            bq[q].offer(fmaf(ym[q].x, sv[u].x, fmaf(ym[q].y, sv[u].y, fmaf(ym[q].z, sv[u].z, wv[u]))),
-                                        __float_as_int(sv[u].w), 0);
+                        for (int qq = 0; qq < TQ; qq++) {
+                            const f4m v0 = pair_tile(a0, bc[gg][qq]), v1 = pair_tile(a1, bc[gg][qq]);
+                            const float b0 = vb[gg][qq];
+                            min2_4(vb[gg][qq], vs[gg][qq], v0);
+                            min2_4(vb[gg][qq], vs[gg][qq], v1);
+                            vc[gg][qq] = vb[gg][qq] < b0 ? k : vc[gg][qq];
+                        }
                 }
-                for (; k < n; k += C) {
-                    const float4 s0 = stg[k];
-                    const float w0 = stw[k];
+                // + |y'|^2, the atoms of the block into the molecule; code: atom, step
+                Min2 mm[GH], mr[GH];
 #pragma unroll
-                    for (int q = 0; q < NVM; q++)
-                        bq[q].offer(fmaf(ym[q].x, s0.x, fmaf(ym[q].y, s0.y, fmaf(ym[q].z, s0.z, w0))), __float_as_int(s0.w), 0);
+                for (int gg = 0; gg < GH; gg++) {
+                    mm[gg].init(); mr[gg].init();
+#pragma unroll
+                    for (int qq = 0; qq < TQ; qq++) {
+                        if (qb + qq >= nvv) continue;
+                        const float y2 = yh[(qq * 4 + 3) * MC + gg * 16];
+                        const float b2 = vb[gg][qq] + y2, s2 = vs[gg][qq] + y2;
+                        const int code = ((qb + qq) << 16) | (vc[gg][qq] << 2) | (lane >> 4);
+                        mm[gg].merge(b2, s2, code);
+                        if (qb + qq == P.iref) { mr[gg].b = b2; mr[gg].s = s2; mr[gg].c = code; }
+                    }
                 }
-                __syncthreads();
-                return;
+                const Min2 gm = gather_groups<GH>(mm, lane), gr = gather_groups<GH>(mr, lane);
+                if (G < 4 || ((lane >> 4) & 1) == h) {
+                    wm.merge(gm.b, gm.s, gm.c);
+                    if (gr.b < INFINITY) wr = gr;   // (one block holds the reference atom)
+                }
             }
-            int k = col;
-            for (; k + 3 * C < n; k += 4 * C) {
-                float4 s0 = stg[k], s1 = stg[k + C], s2 = stg[k + 2 * C], s3 = stg[k + 3 * C];
-                float dx, dy, dz;
-                dx = y.x - s0.x; dy = y.y - s0.y; dz = y.z - s0.z;
-                bb.offer(fmaf(dx, dx, fmaf(dy, dy, dz * dz)), __float_as_int(s0.w), 0);
-                dx = y.x - s1.x; dy = y.y - s1.y; dz = y.z - s1.z;
-                bb.offer(fmaf(dx, dx, fmaf(dy, dy, dz * dz)), __float_as_int(s1.w), 0);
-                dx = y.x - s2.x; dy = y.y - s2.y; dz = y.z - s2.z;
-                bb.offer(fmaf(dx, dx, fmaf(dy, dy, dz * dz)), __float_as_int(s2.w), 0);
-                dx = y.x - s3.x; dy = y.y - s3.y; dz = y.z - s3.z;
-                bb.offer(fmaf(dx, dx, fmaf(dy, dy, dz * dz)), __float_as_int(s3.w), 0);
+            wave_sync();
+        }
+        // the candidate of a code: eight staged atoms of one step, the
+        // nearest of them (the tile's arithmetic is not repeated: when it
+        // matters the minimum is below every other value by more than the
+        // rounding of both forms, else the molecule is resolved in FP64)
+        auto candidate = [&](int code, float& best) {
+            const int q = code >> 16, k = (code >> 2) & 0x3fff, jl = code & 3;
+            float yx, yy, yz;
+            rel(vg[min(ml, nm - 1) * P.nv + q], yx, yy, yz);
+            best = INFINITY;
+            int bi = 0;
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                const float* o = lds + k * 128 + t * 64 + 4 * jl;
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const float dx = yx - o[i], dy = yy - o[16 + i], dz = yz - o[32 + i];
+                    const float d2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+                    // (padding rows sit at the centre and are no candidates)
+                    const bool lt = d2 < best && o[48 + i] < 1e29f;
+                    best = lt ? d2 : best;
+                    bi = lt ? k * EV_ROWS + t * 16 + 4 * jl + i : bi;
+                }
             }
-            for (; k < n; k += C) {
-                float4 s0 = stg[k];
-                float dx = y.x - s0.x, dy = y.y - s0.y, dz = y.z - s0.z;
-                bb.offer(fmaf(dx, dx, fmaf(dy, dy, dz * dz)), __float_as_int(s0.w), 0);
-            }
-            __syncthreads();
+            return si[bi];
         };
-        // Stage the solute atoms of the cells in range, 64 cells at a time: the
-        // atoms of those cells are ranked (wave scan of the counts), each lane
-        // loads the atoms of its ranks, and the ones within rs of the AABB are
-        // appended at ballot/popcount offsets.
-        // Staging walks rows of cells (x fastest in memory): a slot is the part
-        // of one (y, z) row of the index box that lies in one periodic image
-        // along x, so its atoms are one contiguous range of the sorted list.
-        // With a diagonal cell, rows farther than rs from the AABB are
-        // dropped and each row is trimmed to the x range within rs (plus a
-        // slack over FP32 rounding); the per-atom AABB test below is exact.
-        int q0;
-        wrap_index(ilo[0], g.nc[0], q0);
-        int q1;
-        wrap_index(ihi[0], g.nc[0], q1);
-        const int npc = q1 - q0 + 1;
-        const int nslots = ny * nz * npc;
-        const float rsl = rs + 1e-3f, rsl2 = rsl * rsl;
-        const float hcx = g.H32[0] / g.nc[0], hcy = g.H32[4] / g.nc[1], hcz = g.H32[8] / g.nc[2];
-        for (int sb = 0; sb < nslots; sb += 64) {
-            const int si = sb + lane;
-            int cstart = 0, cnt = 0;
-            float tx = 0.f, ty = 0.f, tz = 0.f;
-            if (si < nslots) {
-                const int r = si / npc, pc = si - r * npc;
+        if (wm.b < mb) { mi = candidate(wm.c, mdir); ma = wm.c >> 16; }
+        ms = fminf(fmaxf(mb, wm.b), fminf(ms, wm.s));
+        mb = fminf(mb, wm.b);
+        if (wr.b < rb) ri = candidate(wr.c, rdir);
+        rsec = fminf(fmaxf(rb, wr.b), fminf(rsec, wr.s));
+        rb = fminf(rb, wr.b);
+        wave_sync();
+    };
+    // Staging walks rows of cells (x fastest in memory): a slot is the part
+    // of one (y, z) row of the index box that lies in one periodic image
+    // along x, so its atoms are one contiguous range of the sorted list.
+    // With a diagonal cell, rows farther than rs from the AABB are
+    // dropped and each row is trimmed to the x range within rs (plus a
+    // slack over FP32 rounding); the per-atom AABB test below is exact.
+    // The rows are cut into segments of up to SEG consecutive atoms; in a step
+    // each lane takes one segment (listed in LDS by the rows' lanes), loads its
+    // atoms together and appends the ones within rs of the AABB at
+    // ballot/popcount offsets.  A step that would overflow the buffer evaluates
+    // what is staged first.  The staged set does not depend on the order (FP32
+    // ties between candidates go to the FP64 resolve).
+    int q0;
+    wrap_index(ilo[0], g.nc[0], q0);
+    int q1;
+    wrap_index(ihi[0], g.nc[0], q1);
+    const int npc = q1 - q0 + 1;
+    const int nslots = ny * nz * npc;
+    // (slack over the FP32 rounding of absolute coordinates)
+    const float slk = 1e-3f + 1e-6f * (fabsf(g.H32[0]) + fabsf(g.H32[4]) + fabsf(g.H32[8]));
+    const float rsl = rs + slk, rsl2 = rsl * rsl;
+    // (diagonal cells) the box's ends and the cells' sides
+    const float hcx = g.H32[0] * __builtin_amdgcn_rcpf((float)g.nc[0]), hcy = g.H32[4] * __builtin_amdgcn_rcpf((float)g.nc[1]),
+                hcz = g.H32[8] * __builtin_amdgcn_rcpf((float)g.nc[2]), icx = __builtin_amdgcn_rcpf(hcx);
+    const float ccx = g.Hfix[0] * (float)cix, ccy = g.Hfix[4] * (float)ciy, ccz = g.Hfix[8] * (float)ciz;
+    int nst = 0;            // staged atoms (uniform)
+    int sb = -64, s0 = 0, NS = 0;   // slots of the current 64, its next segment and number of segments
+    int cstart = 0, cnt = 0, nseg = 0, sexcl = 0, code = 0;   // the lane's row: atoms, segments, image
+    for (;;) {
+        while (s0 >= NS && sb + 64 < nslots) {
+            // the next 64 row slots
+            sb += 64;
+            s0 = 0;
+            const int sl = sb + lane;
+            cstart = 0; cnt = 0;
+            if (sl < nslots) {
+                const int r = sl / npc, pc = sl - r * npc;
                 const int iy = ilo[1] + r % ny, iz = ilo[2] + r / ny;
                 int x0 = ilo[0], x1 = ihi[0];
                 bool keep = true;
                 if (g.ortho) {
-                    const float dy = fmaxf(fmaxf(iy * hcy - hy, ly - (iy + 1) * hcy), 0.f);
-                    const float dz = fmaxf(fmaxf(iz * hcz - hz, lz - (iz + 1) * hcz), 0.f);
+                    const float dy = fmaxf(fabsf((iy + 0.5f) * hcy - ccy) - (by + 0.5f * hcy), 0.f);
+                    const float dz = fmaxf(fabsf((iz + 0.5f) * hcz - ccz) - (bz + 0.5f * hcz), 0.f);
                     const float r2 = rsl2 - dy * dy - dz * dz;
                     if (r2 < 0.f) {
                         keep = false;
                     } else {
-                        const float rx = sqrtf(r2) + 1e-3f;
-                        x0 = max(x0, (int)floorf((lx - rx) / hcx));
-                        x1 = min(x1, (int)floorf((hx + rx) / hcx));
+                        const float rx = __builtin_amdgcn_sqrtf(r2) * (1.0f + 1e-6f) + bx + slk;
+                        x0 = max(x0, (int)floorf((ccx - rx) * icx - 1e-3f));
+                        x1 = min(x1, (int)floorf((ccx + rx) * icx + 1e-3f));
                     }
                 }
                 const int mx = q0 + pc;
@@ -2562,279 +2964,344 @@ __device__ __forceinline__ void eval_tiles_chunks(const KP& P, const Bufs& B, co
                     const int crow = (cz * g.nc[1] + cy) * g.nc[0] - mx * g.nc[0];
                     cstart = st[crow + x0];
                     cnt = st[crow + x1 + 1] - cstart;
-                    shift_of(g, mx, my, mz, tx, ty, tz);
+                    code = ((mx + 16) << 8) | ((my + 16) << 16) | ((mz + 16) << 24);
                 }
             }
-            // The atoms of the rows are staged in segments of up to SEG
-            // consecutive atoms: each lane takes one segment per step (owner
-            // row found by a search over the wave's segment prefix, once per
-            // SEG atoms), loads its atoms SUk at a time with the loads in
-            // flight together, and appends the ones within rs of the AABB at
-            // ballot/popcount offsets.  The staged set does not depend on the
-            // order (FP32 ties between candidates go to the FP64 resolve).
-            const int nseg = (cnt + SEG - 1) / SEG;
+            nseg = (cnt + SEG - 1) / SEG;
             const int sincl = wave_incl_scan(nseg);
-            const int sexcl = sincl - nseg;
-            const int NS = __builtin_amdgcn_readlane(sincl, 63);
-            for (int s0 = 0; s0 < NS; s0 += 64) {
-                const int sg = s0 + lane;
-                int j = 0;
-#pragma unroll
-                for (int step = 32; step >= 1; step >>= 1) {
-                    const int e = __shfl(sexcl, (j + step) & 63, 64);
-                    j = (j + step < 64 && e <= sg) ? j + step : j;
-                }
-                const int sj = __shfl(cstart, j, 64), cj = __shfl(cnt, j, 64), ej = __shfl(sexcl, j, 64);
-                const float ox = __shfl(tx, j, 64), oy = __shfl(ty, j, 64), oz = __shfl(tz, j, 64);
-                const int k0 = (sg - ej) * SEG;
-                const int n = sg < NS ? min(SEG, cj - k0) : 0;
-                const int abase = sj + k0;
-                const int nmax = wave_max_i(n);
-                for (int kk = 0; kk < nmax; kk += SUk) {
-                    float4 q[SUk];
-#pragma unroll
-                    for (int u = 0; u < SUk; u++) q[u] = srt[kk + u < n ? abase + kk + u : 0];
-#pragma unroll
-                    for (int u = 0; u < SUk; u++) q[u] = mk4(q[u].x + ox, q[u].y + oy, q[u].z + oz, q[u].w);
-#pragma unroll
-                    for (int u = 0; u < SUk; u++) {
-                        if (kk + u >= nmax) break;
-                        if (nst + 64 > tcap) {
-                            evaluate(nst);
-                            rounds++;
-                            nst = 0;
-                        }
-                        const float dx = fmaxf(fmaxf(lx - q[u].x, q[u].x - hx), 0.f);
-                        const float dy = fmaxf(fmaxf(ly - q[u].y, q[u].y - hy), 0.f);
-                        const float dz = fmaxf(fmaxf(lz - q[u].z, q[u].z - hz), 0.f);
-                        const bool pass = kk + u < n && dx * dx + dy * dy + dz * dz <= rs2;
-                        const unsigned long long m = __ballot(pass);
-                        if (pass) {
-                            const int slot = nst + __popcll(m & lt_mask);
-                            if constexpr (NVM > 0) {
-                                const float sx_ = q[u].x - ccx, sy_ = q[u].y - ccy, sz_ = q[u].z - ccz;
-                                stg[slot] = mk4(sx_, sy_, sz_, q[u].w);
-                                stw[slot] = fmaf(sx_, sx_, fmaf(sy_, sy_, sz_ * sz_));
-                            } else {
-                                stg[slot] = q[u];
-                            }
-                        }
-                        nst += __popcll(m);
-                    }
-                }
-            }
+            sexcl = sincl - nseg;
+            NS = __builtin_amdgcn_readlane(sincl, 63);
         }
-        const bool one_round = rounds == 0;
-        const int last_n = nst;   // the last staged batch stays in LDS until the next chunk
-        if (last_n > 0) evaluate(last_n);
-        float mb, ms, rb, rsec;
-        int mi, ma, ri;
-        if constexpr (NVM > 0) {
-            // + |y'|^2; columns -> each atom's minimum; atoms -> the molecule, in the lane
+        const bool more = s0 < NS;
+        f4v q[SEG];
+        bool pass[SEG];
+        int total = 0;
+        if (more) {
+            // segments s0 .. s0 + 63: first atom, row lane and atoms
+            for (int t = max(0, s0 - sexcl); t < nseg && sexcl + t < s0 + 64; t++)
+                sd[sexcl + t - s0] = make_int2(cstart + SEG * t, code | min(SEG, cnt - SEG * t));
+            wave_sync();
+            int2 d = sd[lane];
+            wave_sync();
+            if (s0 + lane >= NS) d = make_int2(0, 0);
+            const int n = d.y & 255;
 #pragma unroll
-            for (int q = 0; q < NVM; q++) {
-                const float yy2 = 0.25f * fmaf(ym[q].x, ym[q].x, fmaf(ym[q].y, ym[q].y, ym[q].z * ym[q].z));
-                bq[q].best += yy2;
-                bq[q].second += yy2;
-            }
+            for (int u = 0; u < SEG; u++) q[u] = srt[u < n ? d.x + u : 0];
+            // the image's origin relative to the centre
+            const int ox = ((((d.y >> 8) & 255) - 16) << g.fix) - cix, oy = ((((d.y >> 16) & 255) - 16) << g.fix) - ciy,
+                      oz = ((((d.y >> 24) & 255) - 16) << g.fix) - ciz;
 #pragma unroll
-            for (int q = 0; q < NVM; q++) col_reduce<C>(bq[q]);
-            mb = bq[0].best; ms = bq[0].second; mi = bq[0].bi; ma = 0;
-            rb = bq[0].best; rsec = bq[0].second; ri = bq[0].bi;
-#pragma unroll
-            for (int q = 1; q < NVM; q++) {
-                const float ns = fminf(fmaxf(mb, bq[q].best), fminf(ms, bq[q].second));
-                if (bq[q].best < mb) { mi = bq[q].bi; ma = q; }
-                mb = fminf(mb, bq[q].best);
-                ms = ns;
-                if (q == P.iref) { rb = bq[q].best; rsec = bq[q].second; ri = bq[q].bi; }
+            for (int u = 0; u < SEG; u++) {
+                float x_, y_, z_;
+                fix_cart(g, __float_as_int(q[u].x) + ox, __float_as_int(q[u].y) + oy, __float_as_int(q[u].z) + oz, x_, y_, z_);
+                q[u].x = x_; q[u].y = y_; q[u].z = z_;
+                const float dx = fmaxf(fabsf(q[u].x) - bx, 0.f), dy = fmaxf(fabsf(q[u].y) - by, 0.f),
+                            dz = fmaxf(fabsf(q[u].z) - bz, 0.f);
+                pass[u] = u < n && dx * dx + dy * dy + dz * dz <= rs2;
+                total += __popcll(__ballot(pass[u]));
             }
-        } else {
-            // columns of a row -> the row's atom
-            col_reduce<C>(bb);
-            // atoms of a molecule -> the molecule (leader lane: atom 0, column 0)
-            const int mrow0 = ml * P.nv;
-            mb = bb.best; ms = bb.second;
-            mi = bb.bi; ma = 0;
-            for (int q = 1; q < P.nv; q++) {
-                const int src = ((mrow0 + q) * C) & 63;
-                float b2 = __shfl(bb.best, src, 64), s2 = __shfl(bb.second, src, 64);
-                int i2 = __shfl(bb.bi, src, 64);
-                float ns = fminf(fmaxf(mb, b2), fminf(ms, s2));
-                if (b2 < mb) { mi = i2; ma = q; }
-                mb = fminf(mb, b2);
-                ms = ns;
-            }
-            const int srcr = ((mrow0 + P.iref) * C) & 63;
-            rb = __shfl(bb.best, srcr, 64);
-            rsec = __shfl(bb.second, srcr, 64);
-            ri = __shfl(bb.bi, srcr, 64);
+            s0 += 64;
         }
-        const bool leader = active && a == 0 && col == 0;
-        const TU* xuf = xu + (int64_t)f * P.Nu * 3;
-        const int64_t jbase = (int64_t)v * P.nv;
-        auto ysrc = [&](int q, double& y0, double& y1, double& y2) {
-            if (RANDOM) {
-                const double* pp = B.P + (((int64_t)f * P.K + pidx) * P.Nv + pbase + q) * 3;
-                y0 = pp[0]; y1 = pp[1]; y2 = pp[2];
-            } else load3(xv + (int64_t)f * P.Nv * 3, jbase + q, y0, y1, y2);
+        const bool full = nst + total > TCAP;
+        if (nst > 0 && (!more || full)) {
+            evaluate(nst);
+            nst = 0;
+        }
+        if (!more) break;
+        if (full) {
+            // (loaded again, so that nothing is held across the evaluation)
+            s0 -= 64;
+            continue;
+        }
+#pragma unroll
+        for (int u = 0; u < SEG; u++) {
+            const unsigned long long m = __ballot(pass[u]);
+            if (pass[u]) {
+                const int a = nst + __popcll(m & lt_mask);
+                const int o = (a >> 4) * 64 + (a & 15);
+                lds[o] = q[u].x; lds[o + 16] = q[u].y; lds[o + 32] = q[u].z;
+                lds[o + 48] = fmaf(q[u].x, q[u].x, fmaf(q[u].y, q[u].y, q[u].z * q[u].z));
+                si[a] = __float_as_int(q[u].w);
+            }
+            nst += __popcll(m);
+        }
+    }
+    const int v = RANDOM ? slot - (slot / P.Mv) * P.Mv : slot;   // solvent molecule (random passes: slot)
+    const int64_t jbase = (int64_t)v * P.nv;
+    Rec r = rec_zero();
+    bool undec = false, amb = false;   // left to the FP64 resolve (amb: an argmin FP32 cannot separate)
+    if (active) {
+        // a separated argmin decides with its direct d^2, whose guard is
+        // relative to d^2 itself: fixed-point units (E) and fix_cart's rounding
+        // of an exact integer difference, 2 rho + 4 rounding units, plus the
+        // roundings of decide32's own sums
+        auto decide = [&](float d2, int& bn, int& bk) {
+            const float Gd = fmaf(g.gd2, d2, g.gd1 * __builtin_amdgcn_sqrtf(d2)) + g.gd0;
+            return decide32(P, Gd, d2, bn, bk);
         };
-        Rec r = rec_zero();
-        bool exh = false;
-        bool d32 = false, dref32 = false;   // r.d / r.dref hold FP32 squared distances (bins decided without them)
-        if (leader) {
-            if (mb <= cut2_hi_c) {
-                if (ms - mb > amb_c) {
-                    int bn, bk;
-                    const int dd = decide32(P, G32c, mb, bn, bk);
-                    if (dd != 0) {
-                        if (dd == 2) { r.within = 1; r.i = mi; r.j = jbase + ma; r.d = mb; r.bin = bn; r.bulk = bk; d32 = true; }
-                    } else {
-                        double x0, x1, x2, y0, y1, y2;
-                        load3(xuf, mi, x0, x1, x2);
-                        ysrc(ma, y0, y1, y2);
-                        double d2 = cm::canon_d2(g.cell, x0, x1, x2, y0, y1, y2);
-                        if (d2 <= P.cut2) { r.within = 1; r.i = mi; r.j = jbase + ma; r.d = sqrt(d2); }
-                    }
-                } else exh = true;
-            }
-            if (rb <= cut2_hi_c) {
-                if (rsec - rb > amb_c) {
-                    int bn, bk;
-                    const int dd = decide32(P, G32c, rb, bn, bk);
-                    if (dd != 0) {
-                        if (dd == 2) { r.ref = 1; r.dref = rb; r.rbin = bn; dref32 = true; }
-                    } else {
-                        double x0, x1, x2, y0, y1, y2;
-                        load3(xuf, ri, x0, x1, x2);
-                        ysrc(P.iref, y0, y1, y2);
-                        double d2 = cm::canon_d2(g.cell, x0, x1, x2, y0, y1, y2);
-                        if (d2 <= P.cut2) { r.ref = 1; r.dref = sqrt(d2); }
-                    }
-                } else exh = true;
-            }
+        int bn, bk;
+        if (mb <= cut2_hi_c) {
+            amb = !(ms - mb > amb_c);
+            const int dd = decide(mdir, bn, bk);
+            if (dd == 2) { r.within = 1; r.i = mi; r.j = jbase + ma; r.bin = bn; r.bulk = bk; }
+            undec = dd == 0;
         }
-        // ambiguous molecules: every staged pair within the band, in FP64
-        unsigned long long amask = __ballot(exh);
-        if (amask && lane == 0) atomicAdd(&B.stats[0], (ull)__popcll(amask));
-        while (amask) {
-            const int L = __ffsll((long long)amask) - 1;
-            amask &= amask - 1ull;
-            const float bandm = __shfl(mb, L, 64) + amb_c, bandr = __shfl(rb, L, 64) + amb_c;
-            const int mlL = NVM ? L / C : (L / C) / P.nv;
-            const int vL = __shfl(v, L, 64);
-            const int64_t jb = (int64_t)vL * P.nv;
-            const int64_t pb = (int64_t)(m0 + mlL) * P.nv;
-            Rec loc = rec_zero();
-            for (int q = 0; q < P.nv; q++) {
-                const int sl = NVM ? (mlL * C) & 63 : ((mlL * P.nv + q) * C) & 63;
-                float4 yq = y;
-                if constexpr (NVM > 0) {
-#pragma unroll
-                    for (int t = 0; t < NVM; t++)
-                        if (t == q) yq = ym[t];
-                }
-                float yx = __shfl(yq.x, sl, 64), yy = __shfl(yq.y, sl, 64), yz = __shfl(yq.z, sl, 64);
-                // NVM > 0: back from -2 y' (relative, exact) ...
-                if constexpr (NVM > 0) { yx *= -0.5f; yy *= -0.5f; yz *= -0.5f; }
-                double Y0, Y1, Y2;
-                if (RANDOM) {
-                    const double* pp = B.P + (((int64_t)f * P.K + pidx) * P.Nv + pb + q) * 3;
-                    Y0 = pp[0]; Y1 = pp[1]; Y2 = pp[2];
-                } else load3(xv + (int64_t)f * P.Nv * 3, jb + q, Y0, Y1, Y2);
-                const bool isref = q == P.iref;
-                if (one_round) {
-                    // NVM > 0: y' against the staged atoms relative to the chunk centre
-                    for (int k = lane; k < last_n; k += 64) {
-                        float4 s = stg[k];
-                        float dx = yx - s.x, dy = yy - s.y, dz = yz - s.z;
-                        float d2f = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-                        if (d2f <= bandm || (isref && d2f <= bandr)) {
-                            int i = __float_as_int(s.w);
-                            double x0, x1, x2;
-                            load3(xuf, i, x0, x1, x2);
-                            double d2 = cm::canon_d2(g.cell, x0, x1, x2, Y0, Y1, Y2);
-                            if (d2 <= P.cut2) rec_offer(loc, i, jb + q, sqrt(d2), isref);
-                        }
-                    }
-                } else {
-                    // staged buffer recycled: scan the cells around the atom out
-                    // to the band (an FP32 d2 within the band means an FP64 d2
-                    // within band + guard), every pair there in FP64
-                    int jlo[3], jhi[3];
-                    const float band = isref ? fmaxf(bandm, bandr) : bandm;
-                    const float rband = fminf(sqrtf(band + Gcf) + 1e-3f, rs);
-                    // ... and to absolute coordinates (rounding within the 1e-3 slack)
-                    const float yax = NVM > 0 ? yx + ccx : yx, yay = NVM > 0 ? yy + ccy : yy, yaz = NVM > 0 ? yz + ccz : yz;
-                    cell_range(g, yax, yay, yaz, yax, yay, yaz, rband, jlo, jhi);
-                    const int mxn = jhi[0] - jlo[0] + 1, myn = jhi[1] - jlo[1] + 1, mzn = jhi[2] - jlo[2] + 1;
-                    const int ncq = mxn * myn * mzn;
-                    for (int ci = lane; ci < ncq; ci += 64) {
-                        int ix = jlo[0] + ci % mxn, iy = jlo[1] + (ci / mxn) % myn, iz = jlo[2] + ci / (mxn * myn);
-                        int mx, my, mz;
-                        int cx = wrap_index(ix, g.nc[0], mx), cy = wrap_index(iy, g.nc[1], my), cz = wrap_index(iz, g.nc[2], mz);
-                        int cell = (cz * g.nc[1] + cy) * g.nc[0] + cx;
-                        for (int pq = st[cell]; pq < st[cell + 1]; pq++) {
-                            int i = __float_as_int(srt[pq].w);
-                            double x0, x1, x2;
-                            load3(xuf, i, x0, x1, x2);
-                            double d2 = cm::canon_d2(g.cell, x0, x1, x2, Y0, Y1, Y2);
-                            if (d2 <= P.cut2) rec_offer(loc, i, jb + q, sqrt(d2), isref);
-                        }
-                    }
-                }
-            }
-            for (int o = 32; o >= 1; o >>= 1) rec_merge(loc, rec_shfl_xor(loc, o));
-            if (lane == L) { r = loc; d32 = dref32 = false; }
+        if (rb <= cut2_hi_c) {
+            amb = amb || !(rsec - rb > amb_c);
+            const int dd = decide(rdir, bn, bk);
+            if (dd == 2) { r.ref = 1; r.rbin = bn; }
+            undec = undec || dd == 0;
         }
-        if (leader) {
-            rec_complete(P, r);
-            hist_record_global(P, gmd, grdf, gu, gv, r);
+        undec = undec || amb;
+        if (undec) {
+            // every candidate of the record: d^2 (FP32) within these of the
+            // molecule's atoms, the reference atom's own beyond
+            const float band = amb_c + 2.0f * Gcf;
+            const float w0 = fminf(mb + band, cut2_hi_c), w1 = fminf(fmaxf(rb, mb) + band, cut2_hi_c);
+            const int o = ml * P.nv;
+            ((float*)(vwb + o))[3] = w0;
+            if (P.nv > 1) ((float*)(vwb + o + 1))[3] = w1;
+        } else {
+            ev_hist_record<RANDOM>(P, B, &hist, r, ma, jbase);
             if (!RANDOM && P.K > 0) B.bflag[(int64_t)f * P.kb * P.Mv + v] = inbulk(P, r) ? 1 : 0;
             if constexpr (VERIFY) {
-                // verification: the record with its FP64 distances (the
-                // argmin pairs are exact; the distances of records decided
-                // from FP32 bounds are formed here)
+                // verification: the record with its FP64 distances
+                auto dist = [&](int i, int a) {
+                    double x0, x1, x2, y0, y1, y2;
+                    load3(xu + (int64_t)f * P.Nu * 3, i, x0, x1, x2);
+                    if (RANDOM) load3(B.P + 3 * at.atom, (int64_t)ml * P.nv + a, y0, y1, y2);
+                    else load3(xv + (int64_t)f * P.Nv * 3, jbase + a, y0, y1, y2);
+                    return sqrt(cm::canon_d2(B.geo[f].cell, x0, x1, x2, y0, y1, y2));
+                };
                 VRec o;
-                o.within = r.within; o.i = r.within ? r.i : -1; o.j = r.within ? r.j : -1;
-                o.d = r.within ? r.d : INFINITY;
-                o.ref = r.ref; o.pad = 0; o.dref = r.ref ? r.dref : INFINITY;
-                double x0, x1, x2, y0, y1, y2;
-                if (r.within && d32) {
-                    load3(xuf, r.i, x0, x1, x2);
-                    ysrc((int)(r.j - jbase), y0, y1, y2);
-                    o.d = sqrt(cm::canon_d2(g.cell, x0, x1, x2, y0, y1, y2));
-                }
-                if (r.ref && dref32) {
-                    load3(xuf, ri, x0, x1, x2);
-                    ysrc(P.iref, y0, y1, y2);
-                    o.dref = sqrt(cm::canon_d2(g.cell, x0, x1, x2, y0, y1, y2));
-                }
-                B.vrec[fp * P.Mv + v] = o;
+                o.within = r.within; o.i = r.i; o.j = r.j; o.ref = r.ref; o.pad = 0;
+                o.d = r.within ? dist(r.i, ma) : INFINITY;
+                o.dref = r.ref ? dist(ri, P.iref) : INFINITY;
+                // slot: pass within the group times Mv plus the molecule
+                B.vrec[at.row + slot] = o;
             }
         }
-        __syncthreads();
+    }
+    // one bit per molecule, in molecule order
+    unsigned long long um_ = __ballot(undec);
+    if (G == 2) um_ = (um_ & 0xffffull) | ((um_ >> 16) & 0xffff0000ull);
+    if (G == 4) um_ = (um_ & 0xffff00000000ffffull) | ((um_ & 0xffff0000ull) << 16) | ((um_ >> 16) & 0xffff0000ull);
+    if (lane == 0) {
+        B.resmask[ch] = um_;
+        if (um_) atomicAdd(&B.stats[0], (ull)__popcll(um_));
     }
 }
 
-// Minimum distances of the solvent molecules of one chunk per wavefront
-// (64 threads), over every chunk of one job's launch (persistent grid).
-template <class TU, class TV, bool RANDOM, int C, int NVM, bool VERIFY>
-__global__ void __launch_bounds__(64, 3) k_eval_tiles(KP P, Bufs B, const TU* xu, const TV* xv)
+// Chunks of one job's launch, handed to the wavefronts (w of the launch's W):
+// w, w + W, ... below tdyn, then (with a counter ctr, zero at the start of the
+// launch) the chunks from tdyn on in the order the wavefronts ask for them, so
+// the ones that finish early take more of the last chunks.  The chunks' costs
+// vary with their staged atoms, and a fixed stride alone leaves a tail of
+// wavefronts still busy; requests go to one device-wide counter, so only the
+// last DYN_PCT per cent are handed out that way, a few consecutive chunks per
+// request.
+struct ChunkFeed {
+    int total, W, tdyn, dgrab, dnext, dend;
+    int* ctr;
+    __device__ ChunkFeed(int total_, int W_, int* ctr_) : total(total_), W(W_), dnext(0), dend(0), ctr(ctr_)
+    {
+        const int ndyn = (int)((int64_t)total * DYN_PCT / 100);
+        tdyn = total >= DYN_MIN * W ? total - ndyn : total;
+        dgrab = max(1, ndyn / (W * DYN_GRABS));
+    }
+    // the chunk to run given the next one of the stride
+    __device__ int next(int c)
+    {
+        if (c < tdyn || tdyn == total) return c;
+        if (dnext < dend) return dnext++;
+        int g = 0;
+        if ((threadIdx.x & 63) == 0) g = atomicAdd(ctr, dgrab);
+        dnext = tdyn + __builtin_amdgcn_readfirstlane(g);
+        dend = dnext + dgrab;
+        return dnext++;
+    }
+};
+
+// A kernel's first two arguments (KP, Bufs) read again from the kernel argument
+// segment: called per chunk, so that the compiler loads a field where it is
+// used (a scalar cache hit) instead of holding them all in scalar registers
+// over the whole launch (about a hundred spilled to vector registers otherwise).
+struct JobArgs {
+    const KP& P;
+    const Bufs& B;
+};
+__device__ __forceinline__ JobArgs job_args()
 {
-    // dynamic LDS: staging buffer, squared norms (NVM > 0), then the chunk
-    // table of this launch when it has at most CBCAP entries
-    extern __shared__ float4 dyn[];
-    float4* stg = dyn;
-    float* stw = (float*)(dyn + P.tcap);
-    int* cbs = (int*)(stw + (NVM > 0 ? P.tcap : 0));
-    const int nfp = P.F * (RANDOM ? P.K : 1);
+    using cptr = __attribute__((address_space(4))) const char*;
+    cptr k = (cptr)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(k));
+    constexpr size_t off = (sizeof(KP) + alignof(Bufs) - 1) / alignof(Bufs) * alignof(Bufs);
+    return {*(const KP*)k, *(const Bufs*)(k + off)};
+}
+
+// Evaluation of one job's launch (persistent grid, blocks of independent
+// wavefronts that share the LDS histograms and the chunk table)
+template <class TU, class TV, bool RANDOM, int G, int TQ, bool VERIFY>
+__global__ void __launch_bounds__(1024) k_eval_tiles(KP P, Bufs B, const TU* xu, const TV* xv)
+{
+    const int nfp = P.F * (RANDOM ? P.NG : 1);
     const bool cb_lds = nfp + 1 <= CBCAP;
+    int* cbs = (int*)dyn + EvHist::words(P);
+    const int wbase = (EvHist::words(P) + (cb_lds ? nfp + 1 : 0) + 3) & ~3;
     if (cb_lds)
-        for (int k = threadIdx.x; k <= nfp; k += 64) cbs[k] = B.chunk_base[k];
+        for (int k = threadIdx.x; k <= nfp; k += blockDim.x) cbs[k] = B.chunk_base[k];
+    ev_hist_clear(P);
     __syncthreads();
-    eval_tiles_chunks<TU, TV, RANDOM, C, NVM, VERIFY>(P, B, xu, xv, blockIdx.x, B.chunk_base[nfp], gridDim.x, stg, stw,
-                                                     cbs, cb_lds, B.chunk_base + nfp + 1);
+    const EvHist hist(P);
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
+    const int total = B.chunk_base[nfp];
+    ChunkFeed feed(total, gridDim.x * nw, B.chunk_base + nfp + 1);
+    auto base = [&](int k) { return cb_lds ? cbs[k] : B.chunk_base[k]; };
+    for (int ch = feed.next(blockIdx.x + wid * gridDim.x); ch < total; ch = feed.next(ch + feed.W)) {
+        const JobArgs a = job_args();
+        const ChunkAt at(a.P, a.B, RANDOM, ch, base);
+        eval_chunk<TU, TV, RANDOM, G, TQ, VERIFY>(a.P, a.B, xu, xv, ch, at, wbase + wid * eval_wave_words(G, TQ), hist);
+    }
+    __syncthreads();
+    ev_hist_flush<RANDOM>(P, B);
+}
+
+// FP64 records of the molecules FP32 left undecided (one or two per cent): a
+// block takes 64 consecutive chunks of a row, lists their marked molecules in
+// LDS and gives each 16 lanes (four solvent atoms times four rows of cells).
+// Every solute atom within the molecule's radii (FP32, wider than the guard) is
+// evaluated exactly, ties to the smallest (i, j).  Kept out of the evaluation,
+// whose registers and code it would double.
+constexpr int RES_CHUNKS = 64;
+
+template <class TU, class TV, bool RANDOM, bool VERIFY>
+__device__ __forceinline__ void resolve_one(const KP& P, const Bufs& B, const TU* xu, const TV* xv, int f, int64_t row,
+                                            int64_t atom, int pos)
+{
+    // pos: sorted position in the row (the same in the 16 lanes), -1: none
+    const int lane = threadIdx.x & 63, sub = lane & 15;
+    const GeoC& g = *(const GeoC*)(B.geo + f);
+    Rec r = rec_zero();
+    int64_t v = 0, jbase = 0;
+    int slot = 0;
+    if (pos >= 0) {
+        const gptr<const f4v> vg = (gptr<const f4v>)((RANDOM ? B.vw_r : B.vw) + atom + (int64_t)pos * P.nv);
+        const gptr<const int> st = (gptr<const int>)(B.start + (int64_t)f * (P.cap + 1));
+        const gptr<const f4v> srt = (gptr<const f4v>)(B.sorted + (int64_t)f * B.nitems);
+        const TU* xuf = xu + (int64_t)f * P.Nu * 3;
+        slot = ldg(B.msorted + row + pos);
+        v = RANDOM ? slot - (slot / P.Mv) * P.Mv : slot;
+        jbase = v * P.nv;
+        const float w0 = vg[0].w, w1 = P.nv > 1 ? vg[1].w : w0;
+        for (int a = sub >> 2; a < P.nv; a += 4) {
+            const f4v y = vg[a];
+            const bool isref = a == P.iref;
+            const float R2 = isref ? fmaxf(w0, w1) : w0;
+            double y0, y1, y2;
+            if (RANDOM) load3(B.P + 3 * (atom + (int64_t)pos * P.nv), a, y0, y1, y2);
+            else load3(xv + (int64_t)f * P.Nv * 3, jbase + a, y0, y1, y2);
+            const int ux = __float_as_int(y.x), uy = __float_as_int(y.y), uz = __float_as_int(y.z);
+            const float rr_ = __builtin_amdgcn_sqrtf(R2) * (1.0f + 1e-5f) + 1e-3f;
+            int jlo[3], jhi[3];
+            cell_range32(g, ux, uy, uz, rr_, rr_, rr_, jlo, jhi);
+            const int nyr = jhi[1] - jlo[1] + 1, rows = nyr * (jhi[2] - jlo[2] + 1);
+            for (int rr = sub & 3; rr < rows; rr += 4) {
+                int my, mz;
+                const int cy = wrap_index(jlo[1] + rr % nyr, g.nc[1], my), cz = wrap_index(jlo[2] + rr / nyr, g.nc[2], mz);
+                const int crow = (cz * g.nc[1] + cy) * g.nc[0];
+                for (int x0 = jlo[0]; x0 <= jhi[0];) {
+                    // the part of the row in one periodic image
+                    int mx;
+                    const int cx = wrap_index(x0, g.nc[0], mx);
+                    const int nx = min(jhi[0] - x0 + 1, g.nc[0] - cx);
+                    const int qx = ux - (mx << g.fix), qy = uy - (my << g.fix), qz = uz - (mz << g.fix);
+                    const int k1 = st[crow + cx + nx];
+                    for (int k = st[crow + cx]; k < k1; k += 8) {
+                        f4v s[8];
+#pragma unroll
+                        for (int u = 0; u < 8; u++) s[u] = srt[min(k + u, k1 - 1)];
+#pragma unroll
+                        for (int u = 0; u < 8; u++) {
+                            float dx, dy, dz;
+                            fix_cart(g, __float_as_int(s[u].x) - qx, __float_as_int(s[u].y) - qy, __float_as_int(s[u].z) - qz,
+                                     dx, dy, dz);
+                            if (k + u < k1 && fmaf(dx, dx, fmaf(dy, dy, dz * dz)) <= R2) {
+                                const int i = __float_as_int(s[u].w);
+                                double p0, p1, p2;
+                                load3(xuf, i, p0, p1, p2);
+                                const double d2 = cm::canon_d2(B.geo[f].cell, p0, p1, p2, y0, y1, y2);
+                                if (d2 <= P.cut2) rec_offer(r, i, jbase + a, sqrt(d2), isref);
+                            }
+                        }
+                    }
+                    x0 += nx;
+                }
+            }
+        }
+    }
+    for (int o = 8; o >= 1; o >>= 1) rec_merge(r, rec_shfl_xor(r, o));
+    if (pos >= 0 && sub == 0) {
+        rec_complete(P, r);
+        ev_hist_record<RANDOM>(P, B, nullptr, r, (int)(r.j - jbase), jbase);
+        if (!RANDOM && P.K > 0) B.bflag[(int64_t)f * P.kb * P.Mv + v] = inbulk(P, r) ? 1 : 0;
+        if constexpr (VERIFY) {
+            VRec o;
+            o.within = r.within; o.i = r.i; o.j = r.j; o.d = r.d; o.ref = r.ref; o.pad = 0; o.dref = r.dref;
+            B.vrec[row + slot] = o;
+        }
+    }
+}
+
+// grid: x over the parts of a row (RES_CHUNKS chunks each), y over the rows
+template <class TU, class TV, bool RANDOM, bool VERIFY>
+__device__ __forceinline__ void b_resolve(const KP& P, const Bufs& B, const TU* xu, const TV* xv, int bx_, int nbx_, int by_,
+                                          int nby_)
+{
+    __shared__ int list[RES_CHUNKS * 64];
+    __shared__ int nlist;
+    const int nr = RANDOM ? P.NG : 1, mpt = RANDOM ? P.mpt_r : P.mpt;
+    for (int fq = by_; fq < P.F * nr; fq += nby_) {
+        const int f = fq / nr, grp = fq - f * nr;
+        const int c0 = ldg(B.chunk_base + fq), c1 = ldg(B.chunk_base + fq + 1);
+        const int64_t row = row_base(P, f, RANDOM, grp);
+        const int64_t atom = RANDOM ? ((int64_t)f * P.K + (int64_t)grp * P.KM) * P.Nv : (int64_t)f * P.Nv;
+        for (int cb = c0 + bx_ * RES_CHUNKS; cb < c1; cb += nbx_ * RES_CHUNKS) {
+            // one wavefront lists the marked molecules' positions
+            if (threadIdx.x < 64) {
+                const int ch = cb + threadIdx.x;
+                ull m = ch < c1 ? B.resmask[ch] : 0ull;
+                const int n = __popcll(m), incl = wave_incl_scan(n);
+                int o = incl - n;
+                while (m) {
+                    list[o++] = (ch - c0) * mpt + __ffsll((long long)m) - 1;
+                    m &= m - 1ull;
+                }
+                if (threadIdx.x == 63) nlist = incl;
+            }
+            __syncthreads();
+            const int n = nlist;
+            for (int k = 0; k < n; k += BLOCK / 16) {
+                const int q = k + (threadIdx.x >> 4);
+                resolve_one<TU, TV, RANDOM, VERIFY>(P, B, xu, xv, f, row, atom, q < n ? list[q] : -1);
+            }
+            __syncthreads();
+        }
+    }
+}
+
+template <class TU, class TV, bool RANDOM, bool VERIFY>
+__global__ void __launch_bounds__(BLOCK, 3) k_resolve(KP P, Bufs B, const TU* xu, const TV* xv)
+{
+    b_resolve<TU, TV, RANDOM, VERIFY>(P, B, xu, xv, blockIdx.x, gridDim.x, blockIdx.y, gridDim.y);
+}
+
+// parts of the resolve's grid along a row: about 2048 blocks in all, at most
+// one per RES_CHUNKS chunks
+int64_t resolve_parts(const KP& P, bool random)
+{
+    const int64_t rows = (int64_t)P.F * (random ? P.NG : 1), mpt = random ? P.mpt_r : P.mpt;
+    const int64_t chunks = ((random ? (int64_t)P.KM : 1) * P.Mv + mpt - 1) / mpt;
+    return std::max<int64_t>(1, std::min<int64_t>((chunks + RES_CHUNKS - 1) / RES_CHUNKS, 2048 / rows + 1));
 }
 
 // Fills n16 16-byte words and then ntail single bytes with zeros (a kernel,
@@ -2916,9 +3383,9 @@ __global__ void k_pack16(const ull* cnt, uint16_t* out, ull* hits, int64_t n, in
 // ---------------------------------------------------------------------------
 constexpr int MS_MAX = 128;   // jobs per round
 enum MStage {
-    MS_ZERO, MS_RADII, MS_GRID, MS_WRAP, MS_SCAN_CELLS, MS_SCATTER, MS_NEAR, MS_DFIELD, MS_PREP, MS_SCAN_ROWS0,
-    MS_MOL_SCATTER0, MS_FILL, MS_CHUNK0, MS_BULK_INIT, MS_BULK_COMPACT, MS_PLACE_KEYS, MS_SCAN_ROWSK,
-    MS_MOL_SCATTERK, MS_PLACE_NEAR, MS_CHUNKK, MS_GEO_FLAGS, MS_N
+    MS_ZERO, MS_RADII, MS_GRID, MS_WRAP, MS_SCAN_CELLS, MS_SCATTER, MS_NEAR, MS_DFIELD, MS_PREP, MS_SCAN_SUMS0,
+    MS_SCAN_ROWS0, MS_MOL_SCATTER0, MS_FILL, MS_CHUNK0, MS_BULK_INIT, MS_BULK_COMPACT, MS_PLACE_KEYS, MS_SCAN_SUMSK,
+    MS_SCAN_ROWSK, MS_MOL_SCATTERK, MS_PLACE_NEAR, MS_CHUNKK, MS_RESOLVE0, MS_RESOLVEK, MS_GEO_FLAGS, MS_N
 };
 
 struct SysDev {
@@ -3033,8 +3500,10 @@ __global__ void km_dfield(const MultiTab* __restrict__ MT)
 template <class T>
 __global__ void km_prep_solvent_tiles(const MultiTab* __restrict__ MT)
 {
+    __shared__ unsigned tab[48];
+    hilbert_load(tab);
     multi_blocks<MS_PREP, false>(MT, [&](const SysDev& S, int bx, int nbx, int by, int nby) {
-        b_prep_solvent_tiles<T>(S.P, S.B, (const T*)S.xv, bx, nbx, by, nby);
+        b_prep_solvent_tiles<T>(S.P, S.B, (const T*)S.xv, tab, bx, nbx, by, nby);
     });
 }
 
@@ -3042,7 +3511,15 @@ template <bool RANDOM>
 __global__ void __launch_bounds__(1024) km_scan_rows(const MultiTab* __restrict__ MT)
 {
     multi_blocks<RANDOM ? MS_SCAN_ROWSK : MS_SCAN_ROWS0, true>(MT, [&](const SysDev& S, int bx, int nbx, int by, int nby) {
-        b_scan_rows(S.P, S.B, RANDOM ? 1 : 0, RANDOM ? S.P.K : 1, bx, nbx, by, nby);
+        b_scan_rows(S.P, S.B, RANDOM ? 1 : 0, bx, nbx, by, nby);
+    });
+}
+
+template <bool RANDOM>
+__global__ void __launch_bounds__(1024) km_scan_sums(const MultiTab* __restrict__ MT)
+{
+    multi_blocks<RANDOM ? MS_SCAN_SUMSK : MS_SCAN_SUMS0, true>(MT, [&](const SysDev& S, int bx, int nbx, int by, int nby) {
+        b_scan_sums(S.P, S.B, RANDOM ? 1 : 0, bx, nbx, by, nby);
     });
 }
 
@@ -3051,7 +3528,7 @@ __global__ void km_mol_scatter(const MultiTab* __restrict__ MT)
 {
     multi_blocks<RANDOM ? MS_MOL_SCATTERK : MS_MOL_SCATTER0, false>(MT, [&](const SysDev& S, int bx, int nbx, int by,
                                                                             int nby) {
-        b_mol_scatter(S.P, S.B, RANDOM ? 1 : 0, RANDOM ? S.P.K : 1, bx, nbx, by, nby);
+        b_mol_scatter(S.P, S.B, RANDOM ? 1 : 0, bx, nbx, by, nby);
     });
 }
 
@@ -3067,7 +3544,7 @@ template <bool RANDOM>
 __global__ void __launch_bounds__(1024) km_chunk_table(const MultiTab* __restrict__ MT)
 {
     multi_blocks<RANDOM ? MS_CHUNKK : MS_CHUNK0, true>(MT, [&](const SysDev& S, int bx, int nbx, int by, int nby) {
-        b_chunk_table(S.P, S.B, RANDOM ? 1 : 0, RANDOM ? S.P.K : 1, bx, nbx, by, nby);
+        b_chunk_table(S.P, S.B, RANDOM ? 1 : 0, bx, nbx, by, nby);
     });
 }
 
@@ -3087,8 +3564,10 @@ __global__ void __launch_bounds__(1024) km_bulk_compact(const MultiTab* __restri
 
 __global__ void km_place_keys(const MultiTab* __restrict__ MT)
 {
+    __shared__ unsigned tab[48];
+    hilbert_load(tab);
     multi_blocks<MS_PLACE_KEYS, false>(MT, [&](const SysDev& S, int bx, int nbx, int by, int nby) {
-        b_place_keys(S.P, S.B, bx, nbx, by, nby);
+        b_place_keys(S.P, S.B, tab, bx, nbx, by, nby);
     });
 }
 
@@ -3107,56 +3586,80 @@ __global__ void km_geo_flags(const MultiTab* __restrict__ MT)
     });
 }
 
-// The evaluation over the chunks of every job of the round: chunk g of the
-// launch is chunk g - cb[j] of job j, cb the prefix of the jobs' chunk counts
-// (read from their chunk tables at the start of the launch; jobs without
-// random passes have none in the random launch).
-template <class TU, class TV, bool RANDOM, int C, int NVM>
-__global__ void __launch_bounds__(64, 3) km_eval_tiles(const MultiTab* __restrict__ MT, int* ctr)
+// The chunks of every job of a round in tickets of about `per` chunks of one
+// job, taken by blocks from the counter ctr (zero at the start of the launch):
+// a ticket's chunks lie at a stride over its job, so the tickets of a job cost
+// about the same.  The LDS histograms belong to one job: a block flushes them
+// when its next ticket is another job's.  body(job, hist, chunk) runs per
+// wavefront; tab: words of the chunk tables' place in LDS, 3 (MS_MAX + 1).
+template <bool RANDOM, class Fn>
+__device__ __forceinline__ void multi_tickets(const MultiTab* __restrict__ MT, int* ctr, Fn body)
 {
-    extern __shared__ float4 dyn[];
-    __shared__ int cb[MS_MAX + 1];
+    __shared__ int nch[MS_MAX], tk[MS_MAX + 1], s_t;
     const int n = MT->nsys;
-    if (threadIdx.x == 0) {
-        int acc = 0;
-        for (int j = 0; j < n; j++) {
-            cb[j] = acc;
-            const KP& Pj = MT->sys[j].P;
-            const int nfp = Pj.F * (RANDOM ? Pj.K : 1);
-            acc += (RANDOM && Pj.K == 0) ? 0 : MT->sys[j].B.chunk_base[nfp];
-        }
-        cb[n] = acc;
+    for (int j = threadIdx.x; j < n; j += blockDim.x) {
+        const KP& Pj = MT->sys[j].P;
+        nch[j] = (RANDOM && Pj.K == 0) ? 0 : MT->sys[j].B.chunk_base[Pj.F * (RANDOM ? Pj.NG : 1)];
     }
     __syncthreads();
-    const int total = __builtin_amdgcn_readfirstlane(cb[n]);
-    // a fixed stride, then the last DYN_PCT per cent of the chunks on request
-    // from the counter ctr (zero at the start of the launch), as in the
-    // single-job evaluation; either way a block's chunks increase
-    const int ndyn = (int)((int64_t)total * DYN_PCT / 100);
-    const int tdyn = total >= DYN_MIN * (int)gridDim.x ? total - ndyn : total;
-    const int dgrab = max(1, ndyn / ((int)gridDim.x * DYN_GRABS));
-    int dnext = 0, dend = 0;
-    auto next_chunk = [&](int g) {
-        if (g < tdyn || tdyn == total) return g;
-        if (dnext < dend) return dnext++;
-        int v = 0;
-        if (threadIdx.x == 0) v = atomicAdd(ctr, dgrab);
-        dnext = tdyn + __builtin_amdgcn_readlane(v, 0);
-        dend = dnext + dgrab;
-        return dnext++;
-    };
-    int lo = 0;
-    for (int g = next_chunk(blockIdx.x); g < total; g = next_chunk(g + gridDim.x)) {
-        while (cb[lo + 1] <= g) lo++;
-        // uniform (the same in every lane): the job's parameters are scalar loads
-        lo = __builtin_amdgcn_readfirstlane(lo);
-        const SysDev& S = MT->sys[lo];
-        const int ch = g - __builtin_amdgcn_readfirstlane(cb[lo]);
-        float4* stg = dyn;
-        float* stw = (float*)(dyn + S.P.tcap);
-        eval_tiles_chunks<TU, TV, RANDOM, C, NVM, false>(S.P, S.B, (const TU*)S.xu, (const TV*)S.xv, ch, ch + 1, 1, stg,
-                                                         stw, nullptr, false, nullptr);
+    const int nw = blockDim.x >> 6;
+    if (threadIdx.x == 0) {
+        int64_t total = 0;
+        for (int j = 0; j < n; j++) total += nch[j];
+        const int per = (int)max((int64_t)nw, min((int64_t)16 * nw, total / ((int64_t)gridDim.x * 8)));
+        int acc = 0;
+        for (int j = 0; j < n; j++) {
+            tk[j] = acc;
+            acc += (nch[j] + per - 1) / per;
+        }
+        tk[n] = acc;
     }
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int cur = -1;
+    for (;;) {
+        __syncthreads();
+        if (threadIdx.x == 0) s_t = atomicAdd(ctr, 1);
+        __syncthreads();
+        const int t = __builtin_amdgcn_readfirstlane(s_t);
+        if (t >= tk[n]) break;
+        int lo = 0, hi = n;
+        while (hi - lo > 1) {
+            const int mid = (lo + hi) >> 1;
+            if (tk[mid] <= t) lo = mid; else hi = mid;
+        }
+        lo = __builtin_amdgcn_readfirstlane(lo);
+        if (lo != cur) {
+            if (cur >= 0) ev_hist_flush<RANDOM>(MT->sys[cur].P, MT->sys[cur].B);
+            __syncthreads();
+            ev_hist_clear(MT->sys[lo].P);
+            __syncthreads();
+            cur = lo;
+        }
+        const int nt = tk[lo + 1] - tk[lo], nc = nch[lo];
+        for (int ch = t - tk[lo] + wid * nt; ch < nc; ch += nw * nt) body(MT->sys[lo], ch);
+    }
+    if (cur >= 0) ev_hist_flush<RANDOM>(MT->sys[cur].P, MT->sys[cur].B);
+}
+
+template <class TU, class TV, bool RANDOM, int G, int TQ>
+__global__ void __launch_bounds__(1024) km_eval_tiles(const MultiTab* __restrict__ MT, int* ctr)
+{
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    multi_tickets<RANDOM>(MT, ctr, [&](const SysDev& S, int ch) {
+        const EvHist hist(S.P);
+        auto base = [&](int k) { return ldg(S.B.chunk_base + k); };
+        const ChunkAt at(S.P, S.B, RANDOM, ch, base);
+        eval_chunk<TU, TV, RANDOM, G, TQ, false>(S.P, S.B, (const TU*)S.xu, (const TV*)S.xv, ch, at,
+                                                ((EvHist::words(S.P) + 3) & ~3) + wid * eval_wave_words(G, TQ), hist);
+    });
+}
+
+template <class TU, class TV, bool RANDOM>
+__global__ void __launch_bounds__(BLOCK, 3) km_resolve(const MultiTab* __restrict__ MT)
+{
+    multi_blocks<RANDOM ? MS_RESOLVEK : MS_RESOLVE0, true>(MT, [&](const SysDev& S, int bx, int nbx, int by, int nby) {
+        b_resolve<TU, TV, RANDOM, false>(S.P, S.B, (const TU*)S.xu, (const TV*)S.xv, bx, nbx, by, nby);
+    });
 }
 
 // ---------------------------------------------------------------------------
@@ -3443,12 +3946,13 @@ struct cm_job {
     // batch buffers
     DevBuf geo, cells_cnt, cells_start, tmp4, tmpcell, sorted, solw, ucen, vw, vcell, vcen;
     DevBuf P, vw_r, vcen_r, bflag, blist, nbulk, uk, drawn_ptr, drawn_idx;
-    DevBuf near, mkey, mrank, mcnt, mstart, msorted, nnear, chunk_base;
+    DevBuf near, mkey, mrank, mcnt, mstart, msum, msorted, nnear, chunk_base;
     DevBuf xin_u, xin_v;
     double cell_frac = 0.5;   // tiles family: fine cell side as a fraction of the cutoff
-    int tile_c = 1;           // tiles family: columns per atom row (1, 2, 4 or 8)
+    int tile_c = 4;           // tiles family: 64 / (solvent molecules per chunk of the real pass): 1, 2, 4 or 8
     int eval_grid = 0;        // tiles family: workgroups of the persistent evaluation kernel (0: fill the device)
     int cus = 256;            // compute units of the device
+    int lds_max = 65536;      // LDS bytes one block may use
     int Fcap = 0;
     int cap_cells = 0;
     bool finished = false;
@@ -3555,46 +4059,74 @@ int64_t cells_for(const cm_job* J, const double* cell9, int64_t* keys)
     return n;
 }
 
-// grid 0: as many workgroups as the device holds at once (persistent kernel)
-template <class TU, class TV, bool RANDOM, int C>
-void launch_tiles_one(hipStream_t s, int grid, int cus, const KP& P, const Bufs& B, const void* xu, const void* xv)
+// groups of 16 molecules an evaluating wavefront holds for mpt molecules per chunk
+int chunk_groups(int mpt) { return mpt > 32 ? 4 : (mpt > 16 ? 2 : 1); }
+
+// Wavefronts per block of an evaluation and its LDS: as many (up to 16) as fit
+// one CU's LDS together with the histograms and the chunk table
+struct EvShape {
+    int waves;
+    size_t lds;
+    EvShape(const KP& P, int G, int TQ, int table, int lds_max)
+    {
+        const size_t head = 4 * (((size_t)EvHist::words(P) + table + 3) & ~(size_t)3), per = 4 * (size_t)eval_wave_words(G, TQ);
+        waves = (int)std::max<int64_t>(1, std::min<int64_t>(16, ((int64_t)lds_max - (int64_t)head) / (int64_t)per));
+        lds = head + per * waves;
+    }
+};
+
+int lds_per_block(int dev)
 {
-    const int nfp = P.F * (RANDOM ? P.K : 1);
-    const size_t shm = (sizeof(float4) + (P.mol_lane ? sizeof(float) : 0)) * (size_t)P.tcap +
-                       sizeof(int) * (size_t)std::min(nfp + 1, CBCAP);
-    // 3-atom solvent molecules: one molecule per lane
+    int v = 0;
+    if (hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess || v < 65536) v = 65536;
+    return v;
+}
+
+// grid 0: as many workgroups as the device holds at once (persistent kernel)
+template <class TU, class TV, bool RANDOM, int G, int TQ>
+void launch_tiles_one(hipStream_t s, int grid, const cm_job* J, const KP& P, const Bufs& B, const void* xu, const void* xv)
+{
+    const int nfp = P.F * (RANDOM ? P.NG : 1);
+    const EvShape sh(P, G, TQ, nfp + 1 <= CBCAP ? nfp + 1 : 0, J->lds_max);
     // verification (records kept) in its own instantiations, so that the
     // ordinary kernels carry none of its registers
-    auto kern = B.vrec ? (P.mol_lane ? k_eval_tiles<TU, TV, RANDOM, C, 3, true> : k_eval_tiles<TU, TV, RANDOM, C, 0, true>)
-                       : (P.mol_lane ? k_eval_tiles<TU, TV, RANDOM, C, 3, false> : k_eval_tiles<TU, TV, RANDOM, C, 0, false>);
+    auto kern = B.vrec ? k_eval_tiles<TU, TV, RANDOM, G, TQ, true> : k_eval_tiles<TU, TV, RANDOM, G, TQ, false>;
     if (grid <= 0) {
         int nb = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kern, 64, shm) != hipSuccess || nb < 1) nb = 1;
-        grid = nb * cus;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kern, 64 * sh.waves, sh.lds) != hipSuccess || nb < 1) nb = 1;
+        grid = nb * J->cus;
     }
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(64), shm, s, P, B, (const TU*)xu, (const TV*)xv);
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * sh.waves), sh.lds, s, P, B, (const TU*)xu, (const TV*)xv);
+    auto res = B.vrec ? k_resolve<TU, TV, RANDOM, true> : k_resolve<TU, TV, RANDOM, false>;
+    hipLaunchKernelGGL(res, dim3((unsigned)resolve_parts(P, RANDOM), (unsigned)std::min(nfp, 65535)), dim3(BLOCK), 0, s, P, B,
+                       (const TU*)xu, (const TV*)xv);
 }
 
-template <int C>
-void launch_tiles(bool f32, bool random, hipStream_t s, int grid, int cus, const KP& P, const Bufs& B, const void* xu,
-                  const void* xv)
+template <class TU, class TV, bool RANDOM>
+void launch_tiles(hipStream_t s, int grid, const cm_job* J, const KP& P, const Bufs& B, const void* xu, const void* xv)
+{
+    const int g = chunk_groups(RANDOM ? P.mpt_r : P.mpt);
+    if (P.mol_lane) {
+        if (g == 4) launch_tiles_one<TU, TV, RANDOM, 4, 3>(s, grid, J, P, B, xu, xv);
+        else if (g == 2) launch_tiles_one<TU, TV, RANDOM, 2, 3>(s, grid, J, P, B, xu, xv);
+        else launch_tiles_one<TU, TV, RANDOM, 1, 3>(s, grid, J, P, B, xu, xv);
+    } else {
+        if (g == 4) launch_tiles_one<TU, TV, RANDOM, 4, TQ_GEN>(s, grid, J, P, B, xu, xv);
+        else if (g == 2) launch_tiles_one<TU, TV, RANDOM, 2, TQ_GEN>(s, grid, J, P, B, xu, xv);
+        else launch_tiles_one<TU, TV, RANDOM, 1, TQ_GEN>(s, grid, J, P, B, xu, xv);
+    }
+}
+
+void launch_tiles_any(bool f32, bool random, hipStream_t s, int grid, const cm_job* J, const KP& P, const Bufs& B,
+                      const void* xu, const void* xv)
 {
     if (f32) {
-        if (random) launch_tiles_one<float, double, true, C>(s, grid, cus, P, B, xu, nullptr);
-        else launch_tiles_one<float, float, false, C>(s, grid, cus, P, B, xu, xv);
+        if (random) launch_tiles<float, double, true>(s, grid, J, P, B, xu, nullptr);
+        else launch_tiles<float, float, false>(s, grid, J, P, B, xu, xv);
     } else {
-        if (random) launch_tiles_one<double, double, true, C>(s, grid, cus, P, B, xu, nullptr);
-        else launch_tiles_one<double, double, false, C>(s, grid, cus, P, B, xu, xv);
+        if (random) launch_tiles<double, double, true>(s, grid, J, P, B, xu, nullptr);
+        else launch_tiles<double, double, false>(s, grid, J, P, B, xu, xv);
     }
-}
-
-void launch_tiles_c(int c, bool f32, bool random, hipStream_t s, int grid, int cus, const KP& P, const Bufs& B,
-                    const void* xu, const void* xv)
-{
-    if (c == 8) launch_tiles<8>(f32, random, s, grid, cus, P, B, xu, xv);
-    else if (c == 4) launch_tiles<4>(f32, random, s, grid, cus, P, B, xu, xv);
-    else if (c == 2) launch_tiles<2>(f32, random, s, grid, cus, P, B, xu, xv);
-    else launch_tiles<1>(f32, random, s, grid, cus, P, B, xu, xv);
 }
 
 // Verification mode: waits for the batch and keeps, per frame, the records
@@ -3616,7 +4148,7 @@ int verify_collect(cm_job* J, int F, const int64_t* frame_index)
         HIPCHK(hipMemcpy(P.data(), J->P.p, sizeof(double) * P.size(), hipMemcpyDeviceToHost));
         if (J->atoms_family) {
             msorted.resize((size_t)F * NP * Mv);
-            nnear.resize((size_t)F * NP);
+            nnear.resize((size_t)F * (1 + J->kp.NG));
             HIPCHK(hipMemcpy(msorted.data(), J->msorted.p, sizeof(int) * msorted.size(), hipMemcpyDeviceToHost));
             HIPCHK(hipMemcpy(nnear.data(), J->nnear.p, sizeof(int) * nnear.size(), hipMemcpyDeviceToHost));
         }
@@ -3627,22 +4159,24 @@ int verify_collect(cm_job* J, int F, const int64_t* frame_index)
         vf.placed.assign((size_t)K * Nv * 3, NAN);
         vf.placed_flag.assign((size_t)K * Mv, 0);
         vf.draws.assign((size_t)K, 0);
-        for (int64_t k = 0; k < K; k++) {
-            const double* src = P.data() + ((size_t)f * K + k) * Nv * 3;
-            double* dst = vf.placed.data() + (size_t)k * Nv * 3;
-            if (J->atoms_family) {
-                // near slots only, stored at their sorted positions
-                const int64_t fp = (int64_t)f * NP + 1 + k;
-                for (int64_t pos = 0; pos < nnear[fp]; pos++) {
-                    const int64_t v = msorted[fp * Mv + pos];
-                    std::memcpy(dst + v * nv * 3, src + pos * nv * 3, sizeof(double) * 3 * nv);
-                    vf.placed_flag[k * Mv + v] = 1;
+        if (J->atoms_family) {
+            // near slots only, stored at their sorted positions within their group
+            const int64_t KM = J->kp.KM, NG = J->kp.NG;
+            for (int64_t grp = 0; grp < (K > 0 ? NG : 0); grp++) {
+                const double* src = P.data() + ((size_t)f * K + grp * KM) * Nv * 3;
+                const int* ms = msorted.data() + ((size_t)f * NP + 1 + grp * KM) * Mv;
+                for (int64_t pos = 0; pos < nnear[f * (1 + NG) + 1 + grp]; pos++) {
+                    const int64_t slot = grp * KM * Mv + ms[pos];   // pass times Mv plus the molecule
+                    std::memcpy(vf.placed.data() + slot * nv * 3, src + pos * nv * 3, sizeof(double) * 3 * nv);
+                    vf.placed_flag[slot] = 1;
                 }
-            } else {
-                std::memcpy(dst, src, sizeof(double) * 3 * Nv);
-                std::fill(vf.placed_flag.begin() + k * Mv, vf.placed_flag.begin() + (k + 1) * Mv, (uint8_t)1);
-                vf.draws[k] = J->huk[(size_t)f * K + k];
             }
+            continue;
+        }
+        for (int64_t k = 0; k < K; k++) {
+            std::memcpy(vf.placed.data() + (size_t)k * Nv * 3, P.data() + ((size_t)f * K + k) * Nv * 3, sizeof(double) * 3 * Nv);
+            std::fill(vf.placed_flag.begin() + k * Mv, vf.placed_flag.begin() + (k + 1) * Mv, (uint8_t)1);
+            vf.draws[k] = J->huk[(size_t)f * K + k];
         }
     }
     return CM_OK;
@@ -3722,6 +4256,8 @@ Bufs batch_bufs(const cm_job* J, Geo* geo)
     B.mrank = (int*)J->mrank.p;
     B.mcnt = (int*)J->mcnt.p;
     B.mstart = (int*)J->mstart.p;
+    B.msum = (int*)J->msum.p;
+    B.resmask = (ull*)J->mkey.p;
     B.msorted = (int*)J->msorted.p;
     B.nnear = (int*)J->nnear.p;
     B.chunk_base = (int*)J->chunk_base.p;
@@ -3733,6 +4269,18 @@ Bufs batch_bufs(const cm_job* J, Geo* geo)
     return B;
 }
 
+// bytes of the key counts of a batch (and of the keys' starts)
+size_t key_bytes(const KP& P, int F) { return sizeof(int) * (size_t)F * ((size_t)P.kcap + (size_t)P.NG * P.kcapr); }
+
+// scan of the key counts of the real pass (random 0) or the random groups of a batch
+void launch_scan(hipStream_t s, const KP& P, const Bufs& B, int random)
+{
+    const int parts = scan_parts(random ? P.kcapr : P.kcap);
+    const dim3 gr((unsigned)parts, (unsigned)(P.F * (random ? P.NG : 1)));
+    if (parts > 1) hipLaunchKernelGGL(k_scan_sums, gr, dim3(1024), 0, s, P, B, random);
+    hipLaunchKernelGGL(k_scan_rows, gr, dim3(1024), 0, s, P, B, random);
+}
+
 int run_batch(cm_job* J, int F, const int64_t* frame_index, const void* xu_dev, const void* xv_dev, int dtype,
               const double* cells, int64_t cap, int64_t kcap)
 {
@@ -3740,6 +4288,7 @@ int run_batch(cm_job* J, int F, const int64_t* frame_index, const void* xu_dev, 
     P.F = F;
     P.cap = (int)cap;
     P.kcap = (int)kcap;
+    P.kcapr = (int)(kcap << (3 * P.ksub));
     const bool tiles = J->atoms_family;
     // geometry on the host: cells, inverse, spacings (and the fine grid of the tiles family)
     J->hgeo.assign(F, Geo());
@@ -3784,7 +4333,7 @@ int run_batch(cm_job* J, int F, const int64_t* frame_index, const void* xu_dev, 
     if (int r = zero_async(J->cells_cnt.p, sizeof(int) * (size_t)F * (cap + 1), s)) return r;
     if (tiles) {
         if (int r = zero_async(J->near.p, near_bytes(F, cap), s)) return r;
-        if (int r = zero_async(J->mcnt.p, sizeof(int) * (size_t)F * P.NP * (kcap + 1), s)) return r;
+        if (int r = zero_async(J->mcnt.p, key_bytes(P, F), s)) return r;
     }
 
     const bool f32 = dtype == CM_F32;
@@ -3833,11 +4382,11 @@ int run_batch(cm_job* J, int F, const int64_t* frame_index, const void* xu_dev, 
         int64_t n = (int64_t)F * P.Mv;
         if (f32) hipLaunchKernelGGL(k_prep_solvent_tiles<float>, dim3(grid_for(n)), dim3(BLOCK), 0, s, P, B, vf);
         else hipLaunchKernelGGL(k_prep_solvent_tiles<double>, dim3(grid_for(n)), dim3(BLOCK), 0, s, P, B, vd);
-        hipLaunchKernelGGL(k_scan_rows, dim3(F), dim3(1024), 0, s, P, B, 0, 1);
-        hipLaunchKernelGGL(k_mol_scatter, grid_slots(P.Mv, F), dim3(BLOCK), 0, s, P, B, 0, 1);
+        launch_scan(s, P, B, 0);
+        hipLaunchKernelGGL(k_mol_scatter, grid_slots(P.Mv, F), dim3(BLOCK), 0, s, P, B, 0);
         if (f32) hipLaunchKernelGGL(k_fill_real<float>, dim3(grid_for(n)), dim3(BLOCK), 0, s, P, B, vf);
         else hipLaunchKernelGGL(k_fill_real<double>, dim3(grid_for(n)), dim3(BLOCK), 0, s, P, B, vd);
-        hipLaunchKernelGGL(k_chunk_table, dim3(1), dim3(1024), 0, s, P, B, 0, 1);
+        hipLaunchKernelGGL(k_chunk_table, dim3(1), dim3(1024), 0, s, P, B, 0);
     } else {
         int64_t n = (int64_t)F * P.Mv;
         if (f32) hipLaunchKernelGGL(k_prep_solvent<float>, dim3(grid_for(n)), dim3(BLOCK), 0, s, P, B, vf);
@@ -3848,7 +4397,7 @@ int run_batch(cm_job* J, int F, const int64_t* frame_index, const void* xu_dev, 
     // real pass
     if (J->profiling) HIPCHK(hipEventRecord(ev[0], s));
     if (tiles) {
-        launch_tiles_c(J->tile_c, f32, false, s, J->eval_grid, J->cus, P, B, xu_dev, xv_dev);
+        launch_tiles_any(f32, false, s, J->eval_grid, J, P, B, xu_dev, xv_dev);
     } else {
         int64_t n = (int64_t)F * P.Mv;
         const int gwords = P.glds ? P.nbins * (P.gnu + (P.self_ ? 0 : P.gnv)) : 0;
@@ -3880,11 +4429,12 @@ int run_batch(cm_job* J, int F, const int64_t* frame_index, const void* xu_dev, 
         hipLaunchKernelGGL(k_bulk_compact, dim3(F * P.kb), dim3(1024), 0, s, P, B);
         if (tiles) {
             hipLaunchKernelGGL(k_place_keys, grid_slots(P.Mv, F * P.K), dim3(BLOCK), 0, s, P, B);
-            hipLaunchKernelGGL(k_scan_rows, dim3(F * P.K), dim3(1024), 0, s, P, B, 1, P.K);
-            hipLaunchKernelGGL(k_mol_scatter, grid_slots(P.Mv, F * P.K), dim3(BLOCK), 0, s, P, B, 1, P.K);
-            if (f32) hipLaunchKernelGGL(k_place_near<float>, grid_slots(P.Mv, F * P.K), dim3(BLOCK), 0, s, P, B, vf);
-            else hipLaunchKernelGGL(k_place_near<double>, grid_slots(P.Mv, F * P.K), dim3(BLOCK), 0, s, P, B, vd);
-            hipLaunchKernelGGL(k_chunk_table, dim3(1), dim3(1024), 0, s, P, B, 1, P.K);
+            launch_scan(s, P, B, 1);
+            const dim3 gs = grid_slots(P.KM * P.Mv, F * P.NG);
+            hipLaunchKernelGGL(k_mol_scatter, gs, dim3(BLOCK), 0, s, P, B, 1);
+            if (f32) hipLaunchKernelGGL(k_place_near<float>, gs, dim3(BLOCK), 0, s, P, B, vf);
+            else hipLaunchKernelGGL(k_place_near<double>, gs, dim3(BLOCK), 0, s, P, B, vd);
+            hipLaunchKernelGGL(k_chunk_table, dim3(1), dim3(1024), 0, s, P, B, 1);
         } else {
             if (f32) hipLaunchKernelGGL(k_place<float>, grid_slots(P.Mv, F * P.K), dim3(BLOCK), 0, s, P, B, vf);
             else hipLaunchKernelGGL(k_place<double>, grid_slots(P.Mv, F * P.K), dim3(BLOCK), 0, s, P, B, vd);
@@ -3892,7 +4442,7 @@ int run_batch(cm_job* J, int F, const int64_t* frame_index, const void* xu_dev, 
         HIPCHK(hipGetLastError());
         if (J->profiling) HIPCHK(hipEventRecord(ev[2], s));
         if (tiles) {
-            launch_tiles_c(J->tile_c, f32, true, s, J->eval_grid, J->cus, P, B, xu_dev, nullptr);
+            launch_tiles_any(f32, true, s, J->eval_grid, J, P, B, xu_dev, nullptr);
         } else {
             const int gwords = P.glds ? P.nbins * (P.gnu + (P.self_ ? 0 : P.gnv)) : 0;
             const size_t shr = sizeof(unsigned) * (2 * P.nbins + gwords);
@@ -3937,12 +4487,18 @@ int alloc_batch(cm_job* J, int F, int64_t cap, int64_t kcap, int dtype_size, boo
         if ((r = ensure(J, J->vcen, 16 * F * Mv))) return r;
     } else {
         if ((r = ensure(J, J->near, near_bytes(F, cap)))) return r;
-        if ((r = ensure(J, J->mkey, (size_t)4 * F * NP * Mv))) return r;
+        // (also one 8-byte word per chunk of a launch: chunks hold 8 molecules
+        // or more, or are the only one of their row)
+        if ((r = ensure(J, J->mkey, (size_t)4 * F * NP * Mv + (size_t)8 * F * (1 + J->kp.NG)))) return r;
         if ((r = ensure(J, J->mrank, (size_t)4 * F * NP * Mv))) return r;
-        if ((r = ensure(J, J->mcnt, round16((size_t)4 * F * NP * (kcap + 1))))) return r;
-        if ((r = ensure(J, J->mstart, (size_t)4 * F * NP * (kcap + 1)))) return r;
+        KP P = J->kp;
+        P.kcap = (int)kcap;
+        P.kcapr = (int)(kcap << (3 * P.ksub));
+        if ((r = ensure(J, J->mcnt, round16(key_bytes(P, F))))) return r;
+        if ((r = ensure(J, J->mstart, key_bytes(P, F)))) return r;
+        if ((r = ensure(J, J->msum, (size_t)4 * F * (scan_parts(P.kcap) + P.NG * scan_parts(P.kcapr))))) return r;
         if ((r = ensure(J, J->msorted, (size_t)4 * F * NP * Mv))) return r;
-        if ((r = ensure(J, J->nnear, (size_t)4 * F * NP))) return r;
+        if ((r = ensure(J, J->nnear, (size_t)4 * F * (1 + P.NG)))) return r;
         if ((r = ensure(J, J->chunk_base, (size_t)4 * (F * std::max(J->K, 1) + 2)))) return r;
     }
     if (J->K > 0) {
@@ -4126,6 +4682,16 @@ int validate_desc(const cm_job_desc& d)
     return CM_OK;
 }
 
+// Molecules per chunk (one wavefront each): 64 / tile_c in the real pass.  KM
+// random passes place KM times the molecules in the same space, so their
+// chunks hold up to four times as many in no more space.
+void set_chunks(cm_job* J)
+{
+    KP& P = J->kp;
+    P.mpt = 64 / J->tile_c;
+    P.mpt_r = std::min(64, P.mpt * (P.KM >= 8 ? 4 : (P.KM >= 3 ? 2 : 1)));
+}
+
 // (re)initialises a job on its stream for a validated description; device
 // buffers already held by J are kept and grown as needed
 // host-side fields of a job for a validated description (no device work)
@@ -4184,16 +4750,18 @@ void job_params(cm_job* J, const cm_job_desc& d)
     P.Nu = Nu;
     P.Nv = Nv;
     P.NP = 1 + J->K;
-    // 3-atom solvent molecules: one molecule per lane row, 4 columns (16
-    // molecules per chunk); otherwise one column, every lane a solvent atom
-    // (the per-chunk costs of smaller chunks outweigh their shorter staged
-    // lists)
     P.mol_lane = P.nv == 3 ? 1 : 0;
-    J->tile_c = P.mol_lane ? 4 : 1;
-    P.mpt = P.mol_lane ? 64 / J->tile_c : 64 / P.nv;
-    // molecule per lane stages |s'|^2 beside each atom: fewer per round so
-    // that 12 one-wavefront blocks per CU still fit
-    P.tcap = P.mol_lane ? TCAP_MOL : TCAP_DEFAULT;
+    // random passes merged into groups of at most 16 (and of fewer than 2^31
+    // slots); eight or more passes per group get keys of half-cells
+    {
+        const int64_t most = std::max<int64_t>(1, std::min<int64_t>(16, (INT32_MAX - BLOCK) / std::max<int64_t>(P.Mv, 1)));
+        P.NG = J->K > 0 ? (int)((J->K + most - 1) / most) : 0;
+        P.KM = J->K > 0 ? (J->K + P.NG - 1) / P.NG : 1;
+        P.NG = J->K > 0 ? (J->K + P.KM - 1) / P.KM : 0;
+        P.ksub = J->K >= 8 * std::max(P.NG, 1) ? 1 : 0;
+    }
+    J->tile_c = 4;
+    set_chunks(J);
     P.gnu = d.n_groups_u;
     P.gnv = d.n_groups_v;
     // molecule-pair kernels keep the group counts in LDS when they fit
@@ -4203,6 +4771,7 @@ void job_params(cm_job* J, const cm_job_desc& d)
         if (hipGetDevice(&dev) == hipSuccess)
             if (hipDeviceGetAttribute(&J->cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || J->cus < 1)
                 J->cus = 256;
+        J->lds_max = lds_per_block(dev);
     }
     J->acc_len = 4 * (int64_t)d.nbins + 2 * (int64_t)d.n_groups_u * d.nbins + 2 * (int64_t)d.n_groups_v * d.nbins;
 }
@@ -4624,12 +5193,11 @@ int cm_job_set_tuning(cm_job* J, double cell_fraction, int32_t columns, int32_t 
     if (!(cell_fraction >= 0.2 && cell_fraction <= 1.0)) return fail(CM_EINVAL, "cell_fraction must be in [0.2, 1]");
     if (columns != 0 && columns != 1 && columns != 2 && columns != 4 && columns != 8)
         return fail(CM_EINVAL, "columns must be 0 (default), 1, 2, 4 or 8");
-    if (columns == 0) columns = J->tile_c;
-    if (!J->kp.mol_lane && (64 / columns) / J->kp.nv < 1) return fail(CM_EINVAL, "too many columns for the solvent molecule size");
+    if (!J->kp.mol_lane && columns > 0 && (64 / columns) / J->kp.nv < 1) return fail(CM_EINVAL, "too many columns for the solvent molecule size");
     if (eval_workgroups < 0) return fail(CM_EINVAL, "eval_workgroups must be >= 0");
     J->cell_frac = cell_fraction;
-    J->tile_c = columns;
-    J->kp.mpt = J->kp.mol_lane ? 64 / columns : (64 / columns) / J->kp.nv;
+    if (columns > 0) J->tile_c = columns;
+    set_chunks(J);
     J->eval_grid = eval_workgroups;
     return CM_OK;
 }
@@ -4717,7 +5285,7 @@ void cm_job_destroy(cm_job* J)
     DevBuf* bufs[] = {&J->cnt, &J->acc, &J->hits, &J->stats, &J->gmap, &J->geo, &J->cells_cnt, &J->cells_start,
                       &J->tmp4, &J->tmpcell, &J->sorted, &J->solw, &J->ucen, &J->vw, &J->vcell, &J->vcen, &J->P,
                       &J->vw_r, &J->vcen_r, &J->bflag, &J->blist, &J->nbulk, &J->uk, &J->drawn_ptr,
-                      &J->drawn_idx, &J->xin_u, &J->xin_v, &J->near, &J->mkey, &J->mrank, &J->mcnt, &J->mstart,
+                      &J->drawn_idx, &J->xin_u, &J->xin_v, &J->near, &J->mkey, &J->mrank, &J->mcnt, &J->mstart, &J->msum,
                       &J->msorted, &J->nnear, &J->chunk_base, &J->vrec};
     for (DevBuf* b : bufs) dev_put(*b);
     pin_put(J->hres);
@@ -5054,6 +5622,7 @@ constexpr int MS_FMAX = 48;        // frames of one job per round (the single-jo
 constexpr int MG_256 = 32768;      // blocks of the 256-thread stage launches
 constexpr int MG_1024 = 4096;      // blocks of the 1024-thread stage launches
 constexpr int MG_64 = 1024;        // blocks of the 64-thread stage launches
+constexpr int MG_RES = 4096;       // blocks of the resolve launches
 constexpr int64_t MULTI_BUDGET = (int64_t)64 << 30;   // batch buffers of one submission's jobs together
 
 struct MultiRunner {
@@ -5102,25 +5671,38 @@ int multi_init(MultiRunner& R)
 }
 
 template <class KERN>
-int persistent_grid(KERN kern, size_t shm, int cus)
+int persistent_grid(KERN kern, int threads, size_t shm, int cus)
 {
     int nb = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kern, 64, shm) != hipSuccess || nb < 1) nb = 1;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kern, threads, shm) != hipSuccess || nb < 1) nb = 1;
     return nb * cus;
+}
+
+// LDS words of the histograms of a group of jobs (their largest): part of the
+// kernel variant, as the launches' LDS is fixed when a round is captured
+int multi_hist_words(const KP& P)
+{
+    const int w = (EvHist::words(P) + 3) & ~3;
+    return (w + 1023) / 1024 * 1024;
 }
 
 // the stage launches of one round (every argument but the table address is
 // fixed per kernel variant, so the sequence can be captured and replayed)
-template <class T, int C, int NVM>
-void multi_launch(hipStream_t s, const MultiTab* tab, int tcap, int cus)
+template <class T, int TQ, int G, int GR>
+void multi_launch(hipStream_t s, const MultiTab* tab, int hist, int lds_max, int cus)
 {
-    const size_t shm = (sizeof(float4) + (NVM > 0 ? sizeof(float) : 0)) * (size_t)tcap;
-    auto ev_real = km_eval_tiles<T, T, false, C, NVM>;
-    auto ev_rand = km_eval_tiles<T, double, true, C, NVM>;
-    // persistent grids of the two evaluations (occupancy queried once per
-    // variant, before any capture)
-    static const int g_real = persistent_grid(ev_real, shm, cus);
-    static const int g_rand = persistent_grid(ev_rand, shm, cus);
+    auto ev_real = km_eval_tiles<T, T, false, G, TQ>;
+    auto ev_rand = km_eval_tiles<T, double, true, GR, TQ>;
+    // (the chunk tables of multi_tickets are static LDS)
+    auto waves = [&](int g) {
+        return (int)std::max<int64_t>(1, std::min<int64_t>(16, (lds_max - 2048 - 4 * (int64_t)hist) / (4 * (int64_t)eval_wave_words(g, TQ))));
+    };
+    const int w_real = waves(G), w_rand = waves(GR);
+    const size_t shm = 4 * ((size_t)hist + (size_t)w_real * eval_wave_words(G, TQ));
+    const size_t shm_r = 4 * ((size_t)hist + (size_t)w_rand * eval_wave_words(GR, TQ));
+    // persistent grids of the two evaluations
+    const int g_real = persistent_grid(ev_real, 64 * w_real, shm, cus);
+    const int g_rand = persistent_grid(ev_rand, 64 * w_rand, shm_r, cus);
     hipLaunchKernelGGL(km_zero, dim3(MG_256), dim3(BLOCK), 0, s, tab);
     hipLaunchKernelGGL(km_radii<T>, dim3(MG_256), dim3(BLOCK), 0, s, tab);
     hipLaunchKernelGGL(km_grid, dim3(MG_64), dim3(64), 0, s, tab);
@@ -5130,41 +5712,57 @@ void multi_launch(hipStream_t s, const MultiTab* tab, int tcap, int cus)
     hipLaunchKernelGGL(km_near_mark, dim3(MG_256), dim3(BLOCK), 0, s, tab);
     hipLaunchKernelGGL(km_dfield, dim3(MG_256), dim3(BLOCK), 0, s, tab);
     hipLaunchKernelGGL(km_prep_solvent_tiles<T>, dim3(MG_256), dim3(BLOCK), 0, s, tab);
+    hipLaunchKernelGGL(km_scan_sums<false>, dim3(MG_1024), dim3(1024), 0, s, tab);
     hipLaunchKernelGGL(km_scan_rows<false>, dim3(MG_1024), dim3(1024), 0, s, tab);
     hipLaunchKernelGGL(km_mol_scatter<false>, dim3(MG_256), dim3(BLOCK), 0, s, tab);
     hipLaunchKernelGGL(km_fill_real<T>, dim3(MG_256), dim3(BLOCK), 0, s, tab);
     hipLaunchKernelGGL(km_chunk_table<false>, dim3(MG_1024), dim3(1024), 0, s, tab);
     hipLaunchKernelGGL(km_bulk_init, dim3(MG_256), dim3(BLOCK), 0, s, tab);
     int* ctr = (int*)((char*)tab + MT_CTR_OFF);
-    hipLaunchKernelGGL(ev_real, dim3(g_real), dim3(64), shm, s, tab, ctr);
+    hipLaunchKernelGGL(ev_real, dim3(g_real), dim3(64 * w_real), shm, s, tab, ctr);
+    hipLaunchKernelGGL((km_resolve<T, T, false>), dim3(MG_RES), dim3(BLOCK), 0, s, tab);
     hipLaunchKernelGGL(km_bulk_compact, dim3(MG_1024), dim3(1024), 0, s, tab);
     hipLaunchKernelGGL(km_place_keys, dim3(MG_256), dim3(BLOCK), 0, s, tab);
+    hipLaunchKernelGGL(km_scan_sums<true>, dim3(MG_1024), dim3(1024), 0, s, tab);
     hipLaunchKernelGGL(km_scan_rows<true>, dim3(MG_1024), dim3(1024), 0, s, tab);
     hipLaunchKernelGGL(km_mol_scatter<true>, dim3(MG_256), dim3(BLOCK), 0, s, tab);
     hipLaunchKernelGGL(km_place_near<T>, dim3(MG_256), dim3(BLOCK), 0, s, tab);
     hipLaunchKernelGGL(km_chunk_table<true>, dim3(MG_1024), dim3(1024), 0, s, tab);
-    hipLaunchKernelGGL(ev_rand, dim3(g_rand), dim3(64), shm, s, tab, ctr + 1);
+    hipLaunchKernelGGL(ev_rand, dim3(g_rand), dim3(64 * w_rand), shm_r, s, tab, ctr + 1);
+    hipLaunchKernelGGL((km_resolve<T, double, true>), dim3(MG_RES), dim3(BLOCK), 0, s, tab);
     hipLaunchKernelGGL(km_geo_flags, dim3(MG_64), dim3(64), 0, s, tab);
 }
 
-template <class T, int NVM>
-void multi_launch_c(int c, hipStream_t s, const MultiTab* tab, int tcap, int cus)
+// groups of molecules per wavefront of the jobs of a variant (multi_variant)
+template <class T, int TQ>
+void multi_launch_g(int g, int gr, hipStream_t s, const MultiTab* tab, int hist, int lds_max, int cus)
 {
-    if (c == 8) multi_launch<T, 8, NVM>(s, tab, tcap, cus);
-    else if (c == 4) multi_launch<T, 4, NVM>(s, tab, tcap, cus);
-    else if (c == 2) multi_launch<T, 2, NVM>(s, tab, tcap, cus);
-    else multi_launch<T, 1, NVM>(s, tab, tcap, cus);
+    if (g == 4) multi_launch<T, TQ, 4, 4>(s, tab, hist, lds_max, cus);
+    else if (g == 2 && gr == 4) multi_launch<T, TQ, 2, 4>(s, tab, hist, lds_max, cus);
+    else if (g == 2) multi_launch<T, TQ, 2, 2>(s, tab, hist, lds_max, cus);
+    else if (gr == 4) multi_launch<T, TQ, 1, 4>(s, tab, hist, lds_max, cus);
+    else if (gr == 2) multi_launch<T, TQ, 1, 2>(s, tab, hist, lds_max, cus);
+    else multi_launch<T, TQ, 1, 1>(s, tab, hist, lds_max, cus);
 }
 
-void multi_launch_any(bool f32, int mol_lane, int c, hipStream_t s, const MultiTab* tab, int tcap, int cus)
+void multi_launch_any(int dtype, const cm_job* J, hipStream_t s, const MultiTab* tab, int cus)
 {
-    if (f32) {
-        if (mol_lane) multi_launch_c<float, 3>(c, s, tab, tcap, cus);
-        else multi_launch_c<float, 0>(c, s, tab, tcap, cus);
+    const int g = chunk_groups(J->kp.mpt), gr = chunk_groups(J->kp.mpt_r);
+    const int hist = multi_hist_words(J->kp), lds_max = J->lds_max;
+    if (dtype == CM_F32) {
+        if (J->kp.mol_lane) multi_launch_g<float, 3>(g, gr, s, tab, hist, lds_max, cus);
+        else multi_launch_g<float, TQ_GEN>(g, gr, s, tab, hist, lds_max, cus);
     } else {
-        if (mol_lane) multi_launch_c<double, 3>(c, s, tab, tcap, cus);
-        else multi_launch_c<double, 0>(c, s, tab, tcap, cus);
+        if (J->kp.mol_lane) multi_launch_g<double, 3>(g, gr, s, tab, hist, lds_max, cus);
+        else multi_launch_g<double, TQ_GEN>(g, gr, s, tab, hist, lds_max, cus);
     }
+}
+
+// jobs that share the kernels of a round's launches
+int multi_variant(int dtype, const cm_job* J)
+{
+    return (dtype == CM_F32 ? 1 : 0) | (J->kp.mol_lane ? 2 : 0) | (chunk_groups(J->kp.mpt) << 2) | (chunk_groups(J->kp.mpt_r) << 5) |
+           (multi_hist_words(J->kp) << 8);
 }
 
 // one job's part of a multi-job submission
@@ -5195,17 +5793,23 @@ void stage_blocks(const KP& P, int F, const int64_t z16[3], int nbx[MS_N], int c
     set(MS_NEAR, (P.nu + BLOCK - 1) / BLOCK, std::min(F, 65535));
     set(MS_DFIELD, grid_for((int64_t)F * P.cap * 16), 1);
     set(MS_PREP, grid_for((int64_t)F * P.Mv), 1);
-    set(MS_SCAN_ROWS0, F, 1);
+    const int p0 = scan_parts(P.kcap), pk = scan_parts(P.kcapr);
+    set(MS_SCAN_SUMS0, p0, p0 > 1 ? F : 0);
+    set(MS_SCAN_ROWS0, p0, F);
     set(MS_MOL_SCATTER0, mvb, std::min(F, 65535));
     set(MS_FILL, grid_for((int64_t)F * P.Mv), 1);
     set(MS_CHUNK0, 1, 1);
     set(MS_BULK_INIT, grid_for((int64_t)F * P.kb * P.Mv), K > 0 ? 1 : 0);
     set(MS_BULK_COMPACT, (int64_t)F * P.kb, K > 0 ? 1 : 0);
     set(MS_PLACE_KEYS, mvb, K > 0 ? std::min(F * K, 65535) : 0);
-    set(MS_SCAN_ROWSK, (int64_t)F * K, K > 0 ? 1 : 0);
-    set(MS_MOL_SCATTERK, mvb, K > 0 ? std::min(F * K, 65535) : 0);
-    set(MS_PLACE_NEAR, mvb, K > 0 ? std::min(F * K, 65535) : 0);
+    set(MS_SCAN_SUMSK, pk, K > 0 && pk > 1 ? F * P.NG : 0);
+    set(MS_SCAN_ROWSK, pk, K > 0 ? F * P.NG : 0);
+    const int64_t gvb = ((int64_t)P.KM * P.Mv + BLOCK - 1) / BLOCK;
+    set(MS_MOL_SCATTERK, gvb, K > 0 ? std::min(F * P.NG, 65535) : 0);
+    set(MS_PLACE_NEAR, gvb, K > 0 ? std::min(F * P.NG, 65535) : 0);
     set(MS_CHUNKK, 1, K > 0 ? 1 : 0);
+    set(MS_RESOLVE0, resolve_parts(P, false), F);
+    set(MS_RESOLVEK, K > 0 ? resolve_parts(P, true) : 1, K > 0 ? F * P.NG : 0);
     set(MS_GEO_FLAGS, 1, 1);
 }
 
@@ -5214,7 +5818,7 @@ int multi_run_group(MultiRunner& R, std::vector<MJob>& grp, int dtype)
 {
     const int ds = dtype == CM_F32 ? 4 : 8;
     const cm_job* J0 = grp[0].J;
-    const int variant = (dtype == CM_F32 ? 1 : 0) | (J0->kp.mol_lane ? 2 : 0) | (J0->tile_c << 2);
+    const int variant = multi_variant(dtype, J0);
     size_t maxr = 0;
     for (auto& m : grp) maxr = std::max(maxr, m.batches.size());
     for (size_t r = 0; r < maxr; r++) {
@@ -5256,6 +5860,7 @@ int multi_run_group(MultiRunner& R, std::vector<MJob>& grp, int dtype)
                 S.P.F = F;
                 S.P.cap = (int)m.cap;
                 S.P.kcap = (int)m.kcap;
+                S.P.kcapr = (int)(m.kcap << (3 * S.P.ksub));
                 S.B = batch_bufs(J, gd + goff);
                 S.B.dfield = (unsigned*)((char*)J->near.p + near_flags_bytes(F, m.cap));
                 S.xu = (const char*)fr.d_x_solute + (size_t)f0 * J->Nu * 3 * ds;
@@ -5265,7 +5870,7 @@ int multi_run_group(MultiRunner& R, std::vector<MJob>& grp, int dtype)
                 S.zp[2] = (uint4*)J->mcnt.p;
                 S.z16[0] = (int64_t)(round16(sizeof(int) * (size_t)F * (m.cap + 1)) / 16);
                 S.z16[1] = (int64_t)(near_bytes(F, m.cap) / 16);
-                S.z16[2] = (int64_t)(round16((size_t)4 * F * S.P.NP * (m.kcap + 1)) / 16);
+                S.z16[2] = (int64_t)(round16(key_bytes(S.P, F)) / 16);
                 stage_blocks(S.P, F, S.z16, S.nbx, cnt);
                 for (int st = 0; st < MS_N; st++) T->base[st][i + 1] = T->base[st][i] + cnt[st];
                 goff += F;
@@ -5275,14 +5880,12 @@ int multi_run_group(MultiRunner& R, std::vector<MJob>& grp, int dtype)
                                   R.stream));
             HIPCHK(hipEventRecord(R.up[R.cur], R.stream));
             R.cur ^= 1;
-            const bool f32 = dtype == CM_F32;
             if (R.graphs) {
                 auto it = R.exec.find(variant);
                 if (it == R.exec.end()) {
                     // first round of this variant: launched directly (which also
                     // settles the occupancy queries), captured from the next one
-                    multi_launch_any(f32, J0->kp.mol_lane, J0->tile_c, R.stream, (const MultiTab*)R.tab, J0->kp.tcap,
-                                     R.cus);
+                    multi_launch_any(dtype, J0, R.stream, (const MultiTab*)R.tab, R.cus);
                     HIPCHK(hipGetLastError());
                     R.exec.emplace(variant, nullptr);
                     R.rounds++;
@@ -5293,7 +5896,7 @@ int multi_run_group(MultiRunner& R, std::vector<MJob>& grp, int dtype)
                     hipGraph_t g = nullptr;
                     hipGraphExec_t x = nullptr;
                     HIPCHK(hipStreamBeginCapture(R.stream, hipStreamCaptureModeThreadLocal));
-                    multi_launch_any(f32, J0->kp.mol_lane, J0->tile_c, R.stream, (const MultiTab*)R.tab, J0->kp.tcap, R.cus);
+                    multi_launch_any(dtype, J0, R.stream, (const MultiTab*)R.tab, R.cus);
                     HIPCHK(hipStreamEndCapture(R.stream, &g));
                     HIPCHK(hipGraphInstantiate(&x, g, nullptr, nullptr, 0));
                     HIPCHK(hipGraphDestroy(g));
@@ -5301,7 +5904,7 @@ int multi_run_group(MultiRunner& R, std::vector<MJob>& grp, int dtype)
                 }
                 HIPCHK(hipGraphLaunch(it->second, R.stream));
             } else {
-                multi_launch_any(f32, J0->kp.mol_lane, J0->tile_c, R.stream, (const MultiTab*)R.tab, J0->kp.tcap, R.cus);
+                multi_launch_any(dtype, J0, R.stream, (const MultiTab*)R.tab, R.cus);
                 HIPCHK(hipGetLastError());
             }
             R.rounds++;
@@ -5386,7 +5989,7 @@ int cm_jobs_submit_device(int32_t njobs, cm_job* const* jobs, const cm_frames* f
         // the job's own stream may still run earlier work on these buffers
         HIPCHK(hipStreamSynchronize(J->stream));
         if (int r = alloc_batch(J, Fbig, m.cap, m.kcap, ds, false)) return r;
-        const int key = (fr.dtype == CM_F32 ? 1 : 0) | (J->kp.mol_lane ? 2 : 0) | (J->tile_c << 2);
+        const int key = multi_variant(fr.dtype, J);
         groups[key].push_back(m);
         group_dtype[key] = fr.dtype;
     }
@@ -5518,7 +6121,7 @@ int cm_mddf_noalloc(const cm_job_desc* desc, int32_t nframes, const int64_t* fra
     DevBuf* bufs[] = {&J->cnt, &J->acc, &J->hits, &J->stats, &J->gmap, &J->geo, &J->cells_cnt, &J->cells_start,
                       &J->tmp4, &J->tmpcell, &J->sorted, &J->solw, &J->ucen, &J->vw, &J->vcell, &J->vcen, &J->P,
                       &J->vw_r, &J->vcen_r, &J->bflag, &J->blist, &J->nbulk, &J->uk, &J->drawn_ptr,
-                      &J->drawn_idx, &J->xin_u, &J->xin_v, &J->near, &J->mkey, &J->mrank, &J->mcnt, &J->mstart,
+                      &J->drawn_idx, &J->xin_u, &J->xin_v, &J->near, &J->mkey, &J->mrank, &J->mcnt, &J->mstart, &J->msum,
                       &J->msorted, &J->nnear, &J->chunk_base};
     for (DevBuf* b : bufs) *b = DevBuf{};
     J->arena = (char*)D.ptr;

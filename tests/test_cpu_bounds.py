@@ -88,3 +88,63 @@ def test_direct_form_error_is_smaller_near_contact():
     v = fma32(dx[:, 0], dx[:, 0], fma32(dx[:, 1], dx[:, 1], f32(dx[:, 2] * dx[:, 2]))).astype(np.float64)
     d2 = np.sum((y.astype(np.float64) - s.astype(np.float64)) ** 2, axis=1)
     assert (np.abs(v - d2) <= 5.0 * U * d2 + 1e-12).all()
+
+
+def _hilbert_table():
+    """The kernel's state table, read from its source."""
+    import os
+    import re
+    src = open(os.path.join(os.path.dirname(__file__), "..", "complexmixtures.jl_amd", "csrc", "cmgpu.hip")).read()
+    body = re.search(r"HILBERT\[24 \* 8\] = \{(.*?)\};", src, re.S).group(1)
+    t = np.array([int(x, 16) for x in re.findall(r"0x[0-9a-f]+", body)])
+    return t.reshape(24, 8)
+
+
+def test_hilbert_keys_walk_the_grid():
+    """Every cell of a 2^b grid gets its own key and consecutive keys are face
+    neighbours (the property that keeps chunks of consecutive keys compact)."""
+    t = _hilbert_table()
+    for bits in (1, 2, 3, 5):
+        m = 1 << bits
+        g = np.stack(np.meshgrid(*[np.arange(m)] * 3, indexing="ij"), -1).reshape(-1, 3)
+        key, state = np.zeros(len(g), int), np.zeros(len(g), int)
+        for b in range(bits - 1, -1, -1):
+            o = ((g[:, 0] >> b) & 1) | (((g[:, 1] >> b) & 1) << 1) | (((g[:, 2] >> b) & 1) << 2)
+            e = t[state, o]
+            key, state = key * 8 + (e & 7), e >> 3
+        assert np.array_equal(np.sort(key), np.arange(m ** 3))
+        assert (np.abs(np.diff(g[np.argsort(key)], axis=0)).sum(1) == 1).all()
+
+
+def test_fixed_point_tile_distance_within_guard():
+    """The tile kernel's distance from fixed-point positions (integer difference
+    to the chunk centre, FP32 length, expanded form by an FMA chain) and the
+    direct form of a single pair against the exact d^2, on 200,000 pairs of a
+    110 A box: within the chunk's and the pair's claimed guards."""
+    rng = np.random.default_rng(2029)
+    L, fix, n = 110.0, 28, 200_000
+    E = L * 2.0 ** -fix + 1e-9
+    y = rng.uniform(0.0, L, (n, 3))
+    c = y + rng.uniform(-5.0, 5.0, (n, 3))
+    v = rng.normal(size=(n, 3))
+    d = rng.uniform(0.0, 10.5, n)
+    s = y + d[:, None] * v / np.linalg.norm(v, axis=1)[:, None]
+    q = [np.rint(a / L * 2.0 ** fix).astype(np.int64) for a in (y, s, c)]
+    h = np.float32(L * 2.0 ** -fix)
+    rel = lambda a: f32(f32(a) * np.float64(h))          # int -> float, times the FP32 unit
+    yp, sp = rel(q[0] - q[2]), rel(q[1] - q[2])
+    w = fma32(sp[:, 0], sp[:, 0], fma32(sp[:, 1], sp[:, 1], f32(sp[:, 2] * sp[:, 2])))
+    t = f32(np.zeros(n))
+    for a, b in ((sp[:, 0], -2 * yp[:, 0]), (sp[:, 1], -2 * yp[:, 1]), (sp[:, 2], -2 * yp[:, 2]), (w, np.ones(n, np.float32))):
+        t = fma32(a, f32(b), t)
+    got = f32(t + fma32(yp[:, 0], yp[:, 0], fma32(yp[:, 1], yp[:, 1], f32(yp[:, 2] * yp[:, 2])))).astype(np.float64)
+    d2 = ((y - s) ** 2).sum(1)
+    fixed = E * (2.0 * np.sqrt(3.0) * np.sqrt(d2) + 3.0 * E)
+    YS = np.linalg.norm(y - c, axis=1) + np.linalg.norm(s - c, axis=1)
+    bound = fixed + U * YS * (2.0 * 3.0 * np.sqrt(d2) + 7.0 * YS) + 1e-9
+    ratio = np.abs(got - d2) / bound
+    assert 0.05 < ratio.max() <= 1.0, ratio.max()
+    e = rel(q[0] - q[1])
+    direct = fma32(e[:, 0], e[:, 0], fma32(e[:, 1], e[:, 1], f32(e[:, 2] * e[:, 2]))).astype(np.float64)
+    ratio = np.abs(direct - d2) / (fixed + 10.0 * U * d2 + 1e-9)
+    assert 0.05 < ratio.max() <= 1.0, ratio.max()
