@@ -28,10 +28,19 @@
 //                       centre is near the solute, in sorted order
 //   then sort, chunk, k_eval_tiles and k_resolve again for the random passes.
 //
-// "mols" -- many solute molecules (self MDDF, small solutes): molecule
-// centres in a cell list, one thread per solvent molecule evaluating all atom
-// pairs of close molecule pairs (k_prep_solute_mols, k_prep_solvent,
-// k_eval_mols_real, k_place, k_eval_mols_rand).
+// "mols" -- many solute molecules (self MDDF, small solutes), molecules of up
+// to 16 atoms:
+//   k_cl_keys, k_grid, k_cl_scan, k_cl_order
+//                       molecule radii, molecules in Hilbert order
+//   k_cl_build          tiles of 16 solute rows, clusters of 16 solvent
+//                       molecules, their boxes
+//   k_cl_eval           per cluster: every tile whose box is within the cutoff,
+//                       distances on the matrix cores, pairs within the cutoff
+//                       queued and counted, what FP32 leaves open in FP64
+// Larger molecules, and jobs on a caller's scratch: molecule centres in a cell
+// list, one thread per solvent molecule evaluating all atom pairs of close
+// molecule pairs (k_radii, k_prep_solute_mols, k_prep_solvent,
+// k_eval_mols_real).  Both: k_place, k_eval_mols_rand for the random passes.
 //
 // k_flush turns integer hits into FP64 accumulators times the frame weight.
 //
@@ -94,7 +103,8 @@ struct Geo {                 // one frame of a batch
     int ortho;               // diagonal cell matrix: cells are boxes (exact near-cell test)
     double guard;            // bound on |d2(FP32) - d2(FP64)| for pairs up to the cutoff
     float guard_up;          // the same, rounded up
-    // tiles family: fixed-point fractional coordinates, 2^fix units per cell
+    unsigned rs_bits;        // molecule pairs on the matrix cores: largest radius of an A tile about its centre
+    // fixed-point fractional coordinates, 2^fix units per cell
     int fix;
     float Hfix[9];           // lattice vectors per unit (FP32)
     float gd0, gd1, gd2;     // guard of a direct FP32 d2: gd0 + gd1 d + gd2 d2 (with the roundings of decide32)
@@ -131,6 +141,9 @@ struct KP {                  // job parameters, by value
     int kcap;                // molecule sort keys of the real pass: Hilbert positions of the fine cells
     int ksub;                // bits per dimension the random groups' keys have beyond them
     int kcapr;               // sort keys of a random group: kcap << 3 ksub
+    // molecule pairs on the matrix cores: rows per solute molecule in an A
+    // tile (0: not used); A tiles, super tiles and B clusters per frame
+    int rpm, nT, nS, nB;
     int place_all;           // molecule-pair family: place every slot of a random pass (verification)
 };
 
@@ -144,6 +157,16 @@ struct VRec {
     int ref;
     int pad;
     double dref;
+};
+
+// one side (0: solute, 1: solvent) of the molecule pairs on the matrix cores:
+// M molecules of n atoms in the order of their keys (2^bits cells per dimension)
+struct ClSide {
+    int M, n, bits;
+    int *key, *rank;         // [F][M]
+    int* ord;                // [F][M] input index; bit 31: drawn by a random pass
+    int *cnt, *start;        // [F][8^bits]
+    double* cen;             // [F][M][3] centres as k_cl_keys forms them
 };
 
 struct Bufs {
@@ -187,6 +210,13 @@ struct Bufs {
     ull* resmask;            // one word per chunk of a launch: molecules left to the FP64 resolve (over mkey,
                              // whose keys the scatter has read by then)
     int* chunk_base;         // [F*rows + 2] chunk offsets of one launch, total, evaluation chunk counter
+    // molecule pairs on the matrix cores (self: one side)
+    ClSide cl[2];
+    float* clA;              // [F][nT][4][16] rows of the A tiles: x, y, z, squared norm
+    float* clB;              // [F][nB][nv][4][16] columns of the B clusters, per atom
+    float4* tinfo;           // [F][nT][3] fixed-point centre and radius, box middle, box half sides
+    float4* binfo;           // [F][nB][3] the same of the clusters
+    float4* sinfo;           // [F][nS][2] box middle and half sides of the super tiles
     // accumulators
     ull* cnt_md; ull* cnt_rdf; ull* cnt_md_r; ull* cnt_rdf_r;
     ull* cnt_gu; ull* cnt_gv; ull* cnt_gu_r; ull* cnt_gv_r;
@@ -241,6 +271,14 @@ __device__ __forceinline__ int64_t key_row(const KP& P, int f, int r)
 {
     const int64_t per = (int64_t)P.kcap + (int64_t)P.NG * P.kcapr;
     return f * per + (r > 0 ? P.kcap + (int64_t)(r - 1) * P.kcapr : 0);
+}
+
+// the fixed-point centre of a tile's or cluster's info (uniform: scalar loads)
+struct GeoI3 { int x, y, z; };
+__device__ __forceinline__ GeoI3 fix_info(const float4* p)
+{
+    const auto* q = (__attribute__((address_space(4))) const int*)p;
+    return {q[0], q[1], q[2]};
 }
 
 struct Rec {
@@ -491,32 +529,30 @@ __device__ __forceinline__ void b_grid(KP P, Bufs B, int mols_family, int bx_, i
         g.ncell = ncell;
     }
     const double* H = g.cell.H;
-    double dmax = P.cutsys + 0.5, E, G;
+    // Fixed point: positions are fractions of the cell in units of 2^-fix, fix
+    // leaving room for atoms a molecule radius outside the cell and for
+    // differences of two of them.  A position is off by half a unit per
+    // fraction, a difference of two by E per coordinate; the difference is
+    // exact in integers, and turning it into a length rounds the conversion,
+    // the FP32 lattice vector and the product (a diagonal cell: 3 u), plus the
+    // additions over terms of at most kappa times the length in a general one.
+    const double smin = fmin(g.sp[0], fmin(g.sp[1], g.sp[2]));
+    g.fix = 29 - (int)ceil(log2(1.0 + (fmax(ru, rv) + P.cutsys) / smin));
+    double kappa = 0.0, hs = 0.0;
+    for (int r = 0; r < 3; r++) {
+        kappa = fmax(kappa, fabs(H[r]) / g.sp[0] + fabs(H[3 + r]) / g.sp[1] + fabs(H[6 + r]) / g.sp[2]);
+        hs = fmax(hs, fabs(H[r]) + fabs(H[3 + r]) + fabs(H[6 + r]));
+    }
+    for (int k = 0; k < 9; k++) g.Hfix[k] = (float)ldexp(H[k], -g.fix);
+    const double rho = g.ortho ? 3.0 : 5.0 * 1.7320508075688772 * kappa;
+    g.rho = (float)(rho * (1.0 + 1e-6));
+    const double dmax = P.cutsys + 0.5;
+    double E, G;
     if (mols_family) {
-        double xm = 0.0;
-        for (int r = 0; r < 3; r++) xm = fmax(xm, fabs(H[r]) + fabs(H[3 + r]) + fabs(H[6 + r]));
-        xm += fmax(ru, rv) + P.cutsys + 1.0;
+        const double xm = hs + fmax(ru, rv) + P.cutsys + 1.0;
         E = 10.0 * halfulp32(2.0 * xm) + 1e-7;
         G = E * (2.0 * 1.7320508075688772 * dmax + 3.0 * E) + 8.0 * 0x1p-24 * dmax * dmax;
     } else {
-        // Fixed point: positions are fractions of the cell in units of 2^-fix,
-        // fix leaving room for atoms a molecule radius outside the cell and for
-        // differences of two of them.  A position is off by half a unit per
-        // fraction, a difference of two by E per coordinate; the difference is
-        // exact in integers, and turning it into a length rounds the
-        // conversion, the FP32 lattice vector and the product (a diagonal cell:
-        // 3 u), plus the additions over terms of at most kappa times the length
-        // in a general one.
-        const double smin = fmin(g.sp[0], fmin(g.sp[1], g.sp[2]));
-        g.fix = 29 - (int)ceil(log2(1.0 + (rv + P.cutsys) / smin));
-        double kappa = 0.0, hs = 0.0;
-        for (int r = 0; r < 3; r++) {
-            kappa = fmax(kappa, fabs(H[r]) / g.sp[0] + fabs(H[3 + r]) / g.sp[1] + fabs(H[6 + r]) / g.sp[2]);
-            hs = fmax(hs, fabs(H[r]) + fabs(H[3 + r]) + fabs(H[6 + r]));
-        }
-        for (int k = 0; k < 9; k++) g.Hfix[k] = (float)ldexp(H[k], -g.fix);
-        const double rho = g.ortho ? 3.0 : 5.0 * 1.7320508075688772 * kappa;
-        g.rho = (float)(rho * (1.0 + 1e-6));
         E = ldexp(hs, -g.fix) + 1e-9;
         G = E * (2.0 * 1.7320508075688772 * dmax + 3.0 * E) + (2.0 * rho + 4.0) * 0x1p-24 * dmax * dmax;
         g.gd0 = (float)(3.0 * E * E + 1e-9) * (1.0f + 1e-6f);
@@ -1150,6 +1186,52 @@ struct PairCtx {
         }
     }
 
+    // the same of solute molecule u and solvent molecule v (cross)
+    __device__ void cross_main(int u, int v, int i, int a, int mbin, int mbulk) const
+    {
+        if (mbin >= P.nbins) return;   // unreachable: d <= cutoff
+        atomicAdd(&sh[mbin], 1u);
+        const int64_t j = (int64_t)v * P.nv + a;
+        if (shg) {
+            unsigned* shv = shg + (int64_t)P.nbins * P.gnu;
+            if (!P.gu_ptr) atomicAdd(&shg[(int64_t)i * P.nbins + mbin], 1u);
+            else group_hit_lds(shg, P.nbins, mbin, i, P.gu_ptr, P.gu_idx, P.nu);
+            if (!P.gv_ptr) atomicAdd(&shv[(int64_t)a * P.nbins + mbin], 1u);
+            else group_hit_lds(shv, P.nbins, mbin, j, P.gv_ptr, P.gv_idx, P.nv);
+        } else {
+            group_hit_local(B.cnt_gu, P.nbins, mbin, i, i, P.gu_ptr, P.gu_idx);
+            group_hit_local(B.cnt_gv, P.nbins, mbin, a, j, P.gv_ptr, P.gv_idx);
+        }
+        if (P.K > 0) {
+            const int bulk = P.usecutoff ? mbulk : 0;
+            for (int qq = dp[u]; qq < dp[u + 1]; qq++) B.bflag[((int64_t)f * P.kb + di[qq]) * P.Mv + v] = bulk;
+        }
+    }
+
+    // the record of a cross pair from FP64 distances alone (not counted here)
+    __device__ void cross_exhaustive(int u, int v) const
+    {
+        Rec r = rec_zero();
+        const int64_t ub = (int64_t)u * P.nu, vb = (int64_t)v * P.nv;
+#pragma unroll 1
+        for (int a = 0; a < P.nv; a++) {
+            double y0, y1, y2;
+            load3(xvf, vb + a, y0, y1, y2);
+#pragma unroll 1
+            for (int i = 0; i < P.nu; i++) {
+                double x0, x1, x2;
+                load3(xuf, ub + i, x0, x1, x2);
+                const double d2 = cm::canon_d2(g.cell, x0, x1, x2, y0, y1, y2);
+                if (d2 <= P.cut2) rec_offer(r, i, vb + a, sqrt(d2), a == P.iref);
+            }
+        }
+        rec_complete(P, r);
+        hist_record_mols(P, sh, shg, B.cnt_gu, B.cnt_gv, r);
+        if (P.K > 0 && r.within)
+            for (int qq = dp[u]; qq < dp[u + 1]; qq++)
+                B.bflag[((int64_t)f * P.kb + di[qq]) * P.Mv + v] = inbulk(P, r) ? 1 : 0;
+    }
+
     __device__ void rdf_hit(int bin) const
     {
         if (bin < P.nbins) atomicAdd(&sh[P.nbins + bin], 1u);
@@ -1190,6 +1272,7 @@ struct PairCtx {
     {
         const int u = d0.x, v = d0.y;
         if (mask & 8) {
+            atomicAdd(&B.stats[0], 2ull);
             self_exhaustive(u, v);
             return;
         }
@@ -1217,7 +1300,6 @@ struct PairCtx {
     // src/minimum_distances.jl:30-39) and reference atoms
     __device__ void self_exhaustive(int u, int v) const
     {
-        atomicAdd(&B.stats[0], 2ull);
         Rec r1 = rec_zero(), r2 = rec_zero();
         const int64_t ub = (int64_t)u * P.nu, vb = (int64_t)v * P.nv;
         const int n = NU > 0 ? NU : P.nu;
@@ -3304,6 +3386,675 @@ int64_t resolve_parts(const KP& P, bool random)
     return std::max<int64_t>(1, std::min<int64_t>((chunks + RES_CHUNKS - 1) / RES_CHUNKS, 2048 / rows + 1));
 }
 
+// ---------------------------------------------------------------------------
+// molecule pairs on the matrix cores (molecules of up to CL_ATOMS atoms)
+// ---------------------------------------------------------------------------
+// Solute molecules, sorted along a Hilbert curve, fill the 16 rows of A tiles:
+// RPM rows per molecule (4, 8 or 16), 16 / RPM molecules per tile; solvent
+// molecules in the same kind of order fill the 16 columns of B clusters, one
+// column tile per atom.  Positions are FP32 relative to the tile's (cluster's)
+// fixed-point centre.  A wavefront takes one B cluster and every A tile whose box
+// is within the cutoff of its box: one matrix instruction per solvent atom q
+// gives 256 distances, four per lane, so a lane holds one molecule pair (RPM 4)
+// or a part of one, and keeps its minimum, second smallest value and the minima
+// over the reference atoms.  The pairs within the cutoff (about one in six) go
+// to an LDS queue and are counted 64 at a time; the ones FP32 cannot decide go
+// on to a second queue and are formed again in FP64, 64 at a time.
+//
+// The cell walk evaluates a pair in one thread, some 25 vector instructions per
+// distance with the tests of its neighbourhood; here a distance costs 2.25 (its
+// code, minimum and second smallest), and everything per tile or per pair
+// within the cutoff is shared by 64 lanes.  Measured, real pass: 33,400 waters
+// in a 100 A box, 24 frames, 3.66 -> 2.60 ms; 12,000 ureas in a triclinic 90 A
+// cell, 20 frames, 3.45 -> 2.63 ms; 901 waters, 40 frames, 0.76 -> 0.19 ms.
+// Bound by vector issue (busy 64 % of the time on the first, the matrix cores
+// 21 %, four wavefronts per SIMD at 128 registers).  Tiles hold few molecules
+// and the clusters 16 because the pairs of two boxes in reach, but not of
+// their molecules, are the waste: five of six here.
+constexpr int CL_ATOMS = 16;     // largest molecules of these kernels
+constexpr int CL_SUP = 16;       // A tiles per super tile (the unit of the first box test)
+constexpr int CL_Q = 128;        // queue entries per wavefront
+constexpr int CL_WORDS = 5 * CL_Q + 2 * CL_Q + 256;   // LDS words per wavefront: pair queue, deferred pairs, tile centres
+constexpr unsigned CL_DRAWN = 0x80000000u;            // (molecule indices are below 2^31)
+
+// k_cl_eval's arguments as they lie in the kernel argument segment
+template <class TU, class TV>
+struct ClArgs {
+    KP P;
+    Bufs B;
+    const TU* xu;
+    const TV* xv;
+    int S;
+};
+
+// Sort key of a molecule, the 2^bits grid cell of its centre, and the largest
+// molecule radius of a frame (blockIdx.y: frame, blockIdx.z: side).  The centre
+// is kept for k_cl_build: a molecule sorted by one periodic image and built at
+// another would span its tile across the cell.
+template <class T>
+__global__ void __launch_bounds__(BLOCK) k_cl_keys(KP P, Bufs B, const T* xu, const T* xv)
+{
+    __shared__ unsigned tab[48];
+    hilbert_load(tab);
+    const int side = blockIdx.z, f = blockIdx.y;
+    const ClSide s = B.cl[side];
+    Geo& g = B.geo[f];
+    const T* x = (side ? xv : xu) + (int64_t)f * s.M * s.n * 3;
+    float r2 = 0.f;
+    for (int m = blockIdx.x * blockDim.x + threadIdx.x; m < s.M; m += gridDim.x * blockDim.x) {
+        const int64_t a0 = (int64_t)m * s.n;
+        double c[3], fr[3], n[3], x0, y0, z0;
+        mol_centre(g, x, a0, s.n, c);
+        wrap_point(g, c[0], c[1], c[2], fr, n);
+        const int top = (1 << s.bits) - 1;
+        int ck[3];
+        for (int k = 0; k < 3; k++) ck[k] = min(top, max(0, (int)(fr[k] * (top + 1))));
+        const int key = hilbert_key(tab, s.bits, ck[0], ck[1], ck[2]);
+        const int64_t it = (int64_t)f * s.M + m;
+        for (int k = 0; k < 3; k++) s.cen[3 * it + k] = c[k];
+        s.key[it] = key;
+        s.rank[it] = atomicAdd(&s.cnt[((int64_t)f << (3 * s.bits)) + key], 1);
+        load3(x, a0, x0, y0, z0);
+        for (int a = 0; a < s.n; a++) {
+            double xa, ya, za;
+            load3(x, a0 + a, xa, ya, za);
+            float ox, oy, oz;
+            minimage32(g, (float)(xa - x0), (float)(ya - y0), (float)(za - z0), ox, oy, oz);
+            const float dx = ox - (float)(c[0] - x0), dy = oy - (float)(c[1] - y0), dz = oz - (float)(c[2] - z0);
+            r2 = fmaxf(r2, dx * dx + dy * dy + dz * dz);
+        }
+    }
+    const float r = block_max(r2 > 0.f || blockIdx.x * blockDim.x + threadIdx.x < s.M ? sqrtf(r2) * 1.0001f + 1e-3f : 0.f);
+    if (threadIdx.x == 0 && r > 0.f) {
+        // (self: both radii)
+        if (side == 1 || P.self_) atomicMax(&g.rv_bits, __float_as_uint(r));
+        if (side == 0) atomicMax(&g.ru_bits, __float_as_uint(r));
+    }
+}
+
+// exclusive scan of the key counts, one block per frame and side
+__global__ void __launch_bounds__(1024) k_cl_scan(KP P, Bufs B)
+{
+    __shared__ int wsum[16];
+    __shared__ int carry;
+    const ClSide s = B.cl[blockIdx.y];
+    const int n = 1 << (3 * s.bits);
+    const int* c = s.cnt + (int64_t)blockIdx.x * n;
+    int* st = s.start + (int64_t)blockIdx.x * n;
+    if (threadIdx.x == 0) carry = 0;
+    __syncthreads();
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    for (int base = 0; base < n; base += 4 * blockDim.x) {
+        const int i0 = base + 4 * threadIdx.x;
+        int v[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) v[u] = i0 + u < n ? c[i0 + u] : 0;
+        const int tsum = v[0] + v[1] + v[2] + v[3];
+        const int incl = wave_incl_scan(tsum);
+        if (lane == 63) wsum[wid] = incl;
+        __syncthreads();
+        int woff = 0, tot = 0;
+        for (int w = 0; w < nw; w++) { if (w < wid) woff += wsum[w]; tot += wsum[w]; }
+        int e = carry + woff + incl - tsum;
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            if (i0 + u < n && v[u] != 0) st[i0 + u] = e;
+            e += v[u];
+        }
+        __syncthreads();
+        if (threadIdx.x == 0) carry += tot;
+        __syncthreads();
+    }
+}
+
+__global__ void k_cl_order(KP P, Bufs B)
+{
+    const ClSide s = B.cl[blockIdx.y];
+    const int64_t total = (int64_t)P.F * s.M;
+    for (int64_t it = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; it < total; it += (int64_t)gridDim.x * blockDim.x) {
+        const int f = (int)(it / s.M);
+        const int m = (int)(it - (int64_t)f * s.M);
+        unsigned v = (unsigned)m;
+        if (P.K > 0 && blockIdx.y == 0) {
+            const int* dp = B.drawn_ptr + (int64_t)f * (P.Mu + 1) + m;
+            if (dp[0] < dp[1]) v |= CL_DRAWN;
+        }
+        s.ord[(int64_t)f * s.M + s.start[((int64_t)f << (3 * s.bits)) + s.key[it]] + s.rank[it]] = (int)v;
+    }
+}
+
+// atom of row (column) k: the reference atom is the first, so that the loops
+// know where its distances are
+__device__ __forceinline__ int cl_atom(int k, int iref) { return k == 0 ? iref : (k == iref ? 0 : k); }
+
+// minimum / maximum over groups of `width` consecutive lanes
+__device__ __forceinline__ float grp_min(float x, int width)
+{
+    for (int o = 1; o < width; o <<= 1) x = fminf(x, __shfl_xor(x, o, 64));
+    return x;
+}
+__device__ __forceinline__ float grp_max(float x, int width)
+{
+    for (int o = 1; o < width; o <<= 1) x = fmaxf(x, __shfl_xor(x, o, 64));
+    return x;
+}
+
+// The operands, one thread per atom.  blockIdx.z 0: the A tiles, a block per
+// super tile, a lane per row; blockIdx.z 1: the B clusters, a wavefront each,
+// the lane groups taking the atoms in turn.  blockIdx.y: frame.  Also the boxes
+// of tiles, super tiles and clusters, and for the random passes the solute atoms
+// and centres (frame of the centre's cell) in the input order.  Padding rows
+// and columns are so far away (1e30) that they never pass a test.
+template <class T>
+__global__ void __launch_bounds__(BLOCK) k_cl_build(KP P, Bufs B, const T* xu, const T* xv)
+{
+    __shared__ float box[6][CL_SUP], rad[CL_SUP];
+    const bool rows = blockIdx.z == 0;
+    const int f = blockIdx.y, lane = threadIdx.x & 63, l16 = threadIdx.x & 15;
+    const ClSide s = B.cl[rows || P.self_ ? 0 : 1];
+    Geo& g = B.geo[f];
+    const T* x = (rows || P.self_ ? xu : xv) + (int64_t)f * s.M * s.n * 3;
+    const int rpm = P.rpm, mp = 16 / rpm;
+    // the tile or cluster, the molecule, its first atom here and the stride
+    const int unit = rows ? blockIdx.x * CL_SUP + (threadIdx.x >> 4) : blockIdx.x * (BLOCK / 64) + (threadIdx.x >> 6);
+    const bool in = unit < (rows ? P.nT : P.nB);
+    const int pos = rows ? unit * mp + l16 / rpm : unit * 16 + l16;
+    const int a1 = rows ? l16 & (rpm - 1) : lane >> 4;
+    const bool on = in && pos < s.M;
+    const double* H = g.cell.H;
+    double n[3], fr[3], c[3], x0 = 0.0, y0 = 0.0, z0 = 0.0, tx = 0.0, ty = 0.0, tz = 0.0;
+    int m = 0, lo3[3], hi3[3];
+    for (int k = 0; k < 3; k++) { lo3[k] = 0x7fffffff; hi3[k] = (int)0x80000000; }
+    if (on) {
+        m = (int)((unsigned)s.ord[(int64_t)f * s.M + pos] & ~CL_DRAWN);
+        for (int k = 0; k < 3; k++) c[k] = s.cen[3 * ((int64_t)f * s.M + m) + k];
+        load3(x, (int64_t)m * s.n, x0, y0, z0);
+        wrap_point(g, c[0], c[1], c[2], fr, n);
+        const double sc = ldexp(1.0, g.fix);
+        for (int k = 0; k < 3; k++) lo3[k] = hi3[k] = (int)rint(fr[k] * sc);
+        tx = H[0] * n[0] + H[3] * n[1] + H[6] * n[2];
+        ty = H[1] * n[0] + H[4] * n[1] + H[7] * n[2];
+        tz = H[2] * n[0] + H[5] * n[1] + H[8] * n[2];
+        if (rows && P.K > 0 && a1 == 0)
+            B.ucen[(int64_t)f * P.Mu + m] = mk4((float)(c[0] - tx), (float)(c[1] - ty), (float)(c[2] - tz), __int_as_float(m));
+    }
+    // fixed-point centre of the tile (cluster): the middle of its molecules' centres
+    int ct[3];
+    double cx[3];
+    for (int k = 0; k < 3; k++) {
+        for (int o = 1; o < 16; o <<= 1) {
+            lo3[k] = min(lo3[k], __shfl_xor(lo3[k], o, 64));
+            hi3[k] = max(hi3[k], __shfl_xor(hi3[k], o, 64));
+        }
+        ct[k] = lo3[k] <= hi3[k] ? lo3[k] + (hi3[k] - lo3[k]) / 2 : 0;
+    }
+    const double un = ldexp(1.0, -g.fix);
+    for (int k = 0; k < 3; k++) cx[k] = (H[k] * ct[0] + H[3 + k] * ct[1] + H[6 + k] * ct[2]) * un;
+    float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY}, r2 = 0.f;
+    if (in)
+        for (int q = a1; q < (rows ? rpm : s.n); q += rows ? rpm : 4) {
+            const int a = rows && !P.self_ ? q : cl_atom(q, P.iref);
+            float e0 = 0.f, e1 = 0.f, e2 = 0.f, w = 1e30f;
+            if (on && q < s.n) {
+                double xa, ya, za, ox, oy, oz;
+                load3(x, (int64_t)m * s.n + a, xa, ya, za);
+                cm::minimage(g.cell, xa - x0, ya - y0, za - z0, &ox, &oy, &oz);
+                const double px = x0 + ox - tx, py = y0 + oy - ty, pz = z0 + oz - tz;
+                e0 = (float)(px - cx[0]); e1 = (float)(py - cx[1]); e2 = (float)(pz - cx[2]);
+                w = fmaf(e0, e0, fmaf(e1, e1, e2 * e2));
+                lo[0] = fminf(lo[0], e0); lo[1] = fminf(lo[1], e1); lo[2] = fminf(lo[2], e2);
+                hi[0] = fmaxf(hi[0], e0); hi[1] = fmaxf(hi[1], e1); hi[2] = fmaxf(hi[2], e2);
+                r2 = fmaxf(r2, w);
+                if (rows && P.K > 0)
+                    B.solw[(int64_t)f * P.Nu + (int64_t)m * s.n + a] = mk4((float)px, (float)py, (float)pz, 0.f);
+            }
+            float* o = rows ? B.clA + ((int64_t)f * P.nT + unit) * 64 + l16 : B.clB + (((int64_t)f * P.nB + unit) * s.n + q) * 64 + l16;
+            o[0] = e0; o[16] = e1; o[32] = e2; o[48] = w;
+        }
+    const int width = rows ? 16 : 64;
+    float l[3], h[3];
+    for (int k = 0; k < 3; k++) { l[k] = grp_min(lo[k], width); h[k] = grp_max(hi[k], width); }
+    const float r = sqrtf(grp_max(r2, width)) * (1.0f + 1e-6f);
+    // (nothing but padding or undefined positions: a box that nothing reaches)
+    const bool any = l[0] <= h[0];
+    float mid[3], half[3];
+    for (int k = 0; k < 3; k++) {
+        mid[k] = any ? (float)cx[k] + 0.5f * (l[k] + h[k]) : 0.f;
+        half[k] = any ? 0.5f * (h[k] - l[k]) : -1e30f;
+    }
+    if (in && (lane & (width - 1)) == 0) {
+        float4* info = (rows ? B.tinfo + 3 * ((int64_t)f * P.nT + unit) : B.binfo + 3 * ((int64_t)f * P.nB + unit));
+        info[0] = fix4(ct[0], ct[1], ct[2], r);
+        info[1] = mk4(mid[0], mid[1], mid[2], 0.f);
+        info[2] = mk4(half[0], half[1], half[2], 0.f);
+    }
+    if (!rows || (int)blockIdx.x >= P.nS) return;
+    if (l16 == 0) {
+        rad[threadIdx.x >> 4] = in ? r : 0.f;
+        for (int k = 0; k < 3; k++) {
+            box[k][threadIdx.x >> 4] = any ? mid[k] - half[k] : INFINITY;
+            box[3 + k][threadIdx.x >> 4] = any ? mid[k] + half[k] : -INFINITY;
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < CL_SUP) {
+        float sl[3], sg[3];
+        for (int k = 0; k < 3; k++) {
+            sl[k] = grp_min(box[k][threadIdx.x], CL_SUP);
+            sg[k] = grp_max(box[3 + k][threadIdx.x], CL_SUP);
+        }
+        // (the maximum rarely grows after the first blocks: a look before the
+        // atomic, which the blocks of a frame queue for)
+        const float rmax = grp_max(rad[threadIdx.x], CL_SUP);
+        if (threadIdx.x == 0) {
+            if (rmax > __uint_as_float(__hip_atomic_load(&g.rs_bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)))
+                atomicMax(&g.rs_bits, __float_as_uint(rmax));
+            float4* si = B.sinfo + 2 * ((int64_t)f * P.nS + blockIdx.x);
+            const bool sany = sl[0] <= sg[0];
+            si[0] = sany ? mk4(0.5f * (sl[0] + sg[0]), 0.5f * (sl[1] + sg[1]), 0.5f * (sl[2] + sg[2]), 0.f) : mk4(0.f, 0.f, 0.f, 0.f);
+            si[1] = sany ? mk4(0.5f * (sg[0] - sl[0]), 0.5f * (sg[1] - sl[1]), 0.5f * (sg[2] - sl[2]), 0.f) : mk4(-1e30f, -1e30f, -1e30f, 0.f);
+        }
+    }
+}
+
+// Whether a box (mid, half) can come within rc of the wavefront's box (bm, bh)
+// under some lattice shift of it by -1, 0 or 1 cells per dimension (all that
+// molecules with their centres in the cell can need), and which: bits 0..2,
+// 3..5, 6..8 of `sets` for shifts -1, 0, 1 along the three cell vectors.
+// Along cell vector k two boxes m cells apart are at least (|f_k + m| - e_k) sp_k
+// apart, f the fractions of mid - bm and e those of the half sides.
+__device__ __forceinline__ bool cl_reach(const GeoC& g, float rc, float4 mid, float4 half, const float bm[3],
+                                         const float bh[3], int& sets)
+{
+    const float dx = mid.x - bm[0], dy = mid.y - bm[1], dz = mid.z - bm[2];
+    const float hx = half.x + bh[0], hy = half.y + bh[1], hz = half.z + bh[2];
+    float sum = 0.f;
+    bool ok = true;
+    sets = 0;
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        const float f = g.Hi32[k] * dx + g.Hi32[3 + k] * dy + g.Hi32[6 + k] * dz;
+        const float e = fabsf(g.Hi32[k]) * hx + fabsf(g.Hi32[3 + k]) * hy + fabsf(g.Hi32[6 + k]) * hz;
+        float best = INFINITY;
+        int set = 0;
+#pragma unroll
+        for (int m = -1; m <= 1; m++) {
+            const float p = fmaxf(fabsf(f + (float)m) - e, 0.f) * (float)g.sp[k];
+            set |= p <= rc ? 1 << (m + 1) : 0;
+            best = fminf(best, p);
+        }
+        ok = ok && set != 0;
+        sum = fmaf(best, best, sum);
+        sets |= set << (3 * k);
+    }
+    // diagonal cells: the three distances are perpendicular; general ones with
+    // a single shift: the boxes' distance along the axes
+    if (!ok) return false;
+    if (g.ortho) return sum <= rc * rc;
+    const int sx = sets & 7, sy = (sets >> 3) & 7, sz = sets >> 6;
+    if ((sx & (sx - 1)) | (sy & (sy - 1)) | (sz & (sz - 1))) return true;
+    const float m0 = (float)(sx >> 1) - 1.0f, m1 = (float)(sy >> 1) - 1.0f, m2 = (float)(sz >> 1) - 1.0f;
+    const float gx = fmaxf(fabsf(dx + (g.H32[0] * m0 + g.H32[3] * m1 + g.H32[6] * m2)) - hx, 0.f);
+    const float gy = fmaxf(fabsf(dy + (g.H32[1] * m0 + g.H32[4] * m1 + g.H32[7] * m2)) - hy, 0.f);
+    const float gz = fmaxf(fabsf(dz + (g.H32[2] * m0 + g.H32[5] * m1 + g.H32[8] * m2)) - hz, 0.f);
+    return fmaf(gx, gx, fmaf(gy, gy, gz * gz)) <= rc * rc;
+}
+
+// a value of this lane's row of 16 and of row ^ 1 (O 16) or of row ^ 2 (O 32),
+// the lower row's in .x
+template <int O>
+__device__ __forceinline__ float2 row_pair(float x)
+{
+    const unsigned u = __float_as_uint(x);
+    const auto r = O == 16 ? __builtin_amdgcn_permlane16_swap(u, u, false, false) : __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    return make_float2(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
+// Out of line, with the kernel's arguments read where they are used and the
+// histograms by their LDS address (flat atomics took five times as long; glds:
+// words before the group histograms, 0: none): the FP64 record of a deferred
+// pair (input indices) ...
+using CArgs = __attribute__((address_space(4))) const char*;
+using LdsU = __attribute__((address_space(3))) unsigned*;
+template <class TU, class TV, bool SELF>
+__device__ __attribute__((noinline)) void cl_exact(CArgs k, int f, int u, int v, LdsU sh_, int glds)
+{
+    unsigned *const sh = (unsigned*)sh_, *const shg = glds ? sh + glds : nullptr;
+    const ClArgs<TU, TV>& a = *(const ClArgs<TU, TV>*)k;
+    const PairCtx<TU, TV, 0> ctx(a.P, a.B, f, a.xu, a.xv, sh, shg);
+    if (SELF) ctx.self_exhaustive(u, v);
+    else ctx.cross_exhaustive(u, v);
+}
+
+// ... and the updates of a decided pair where there is more than the plain
+// LDS histograms (custom or large groups, dbulk flags)
+template <class TU, class TV, bool SELF>
+__device__ __attribute__((noinline)) void cl_main(CArgs k, int f, int u, int v, int i, int q, int bin, int bulk, LdsU sh_, int glds)
+{
+    unsigned *const sh = (unsigned*)sh_, *const shg = glds ? sh + glds : nullptr;
+    const ClArgs<TU, TV>& a = *(const ClArgs<TU, TV>*)k;
+    const PairCtx<TU, TV, 0> ctx(a.P, a.B, f, a.xu, a.xv, sh, shg);
+    if (SELF) ctx.self_main(u, v, i, q, bin, bulk);
+    else ctx.cross_main(u, v, i, q, bin, bulk);
+}
+
+// Blocks of independent wavefronts that share the LDS histograms; XCD k takes
+// the k-th eighth of the (frame, cluster) items in frame-major order, so its L2
+// holds one or two frames at a time.
+template <class TU, class TV, int RPM, int NVT, bool SELF>
+__global__ void __launch_bounds__(NVT > 8 ? 512 : 1024) k_cl_eval(KP P_, Bufs B_, const TU* xu_, const TV* xv_, int S)
+{
+    constexpr int mp = 16 / RPM, RL = RPM / 4;   // molecules per tile, lane groups per molecule
+    constexpr int QB = NVT <= 4 ? 2 : (NVT <= 8 ? 3 : 4);
+    constexpr int CBITS = 2 + QB + (RPM == 4 ? 0 : (RPM == 8 ? 1 : 2));   // code: row of the lane, solvent atom, lane group
+    constexpr int CMASK = (1 << CBITS) - 1;
+    CArgs k0 = (CArgs)__builtin_amdgcn_kernarg_segment_ptr();
+    const KP& P = *(const KP*)k0;
+    const int gwords = P.glds ? P.nbins * (P.gnu + (SELF ? 0 : P.gnv)) : 0;
+    unsigned* const sh = (unsigned*)dyn;
+    unsigned* const shg = P.glds ? sh + 2 * P.nbins : nullptr;
+    hist_clear(sh, 2 * P.nbins + gwords);
+    const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
+    // the wavefront's queues: pairs within the cutoff (values, position of the
+    // solute molecule, column and doubt), deferred pairs (input indices)
+    float* const qv = dyn + ((2 * P.nbins + gwords + 3) & ~3) + wid * CL_WORDS;
+    int* const qi = (int*)qv;
+    int* const dq = (int*)(qv + 5 * CL_Q);
+    float* const tt = qv + 7 * CL_Q;   // centres of the 64 tiles of a turn at their first shift: x, y, z, squared norm
+    int qn = 0, dn = 0, fcur = -1, nexact = 0;
+    const unsigned long long lt = (1ull << lane) - 1ull;
+    const int col = lane & 15, kk = lane >> 4;   // operand component, and the lane group of the results
+    const int64_t items = (int64_t)P.F * P.nB * S;
+    const int xcd = blockIdx.x & 7, nblk = gridDim.x >> 3;
+    const int64_t ihi = items * (xcd + 1) / 8;
+    const float pk = ldexpf(1.0f, CBITS - 23);
+
+    auto deferred = [&](int n) {
+        wave_sync();
+        if (lane < n) {
+            CArgs ka = k0;
+            asm volatile("" : "+s"(ka));
+            cl_exact<TU, TV, SELF>(ka, fcur, dq[2 * (dn - n + lane)], dq[2 * (dn - n + lane) + 1], (LdsU)sh, shg ? 2 * P.nbins : 0);
+        }
+        wave_sync();
+        dn -= n;
+        nexact += n;
+    };
+
+    for (int64_t it = items * xcd / 8 + (int64_t)(blockIdx.x >> 3) * nw + wid; it < ihi; it += (int64_t)nblk * nw) {
+        CArgs ki = k0;
+        asm volatile("" : "+s"(ki));   // fields are read again where they are used (job_args)
+        const ClArgs<TU, TV>& A = *(const ClArgs<TU, TV>*)ki;
+        // (divisions run on the vector units: their results are scalars again)
+        const int64_t fbv = it / S;
+        const int f = __builtin_amdgcn_readfirstlane((int)(fbv / A.P.nB));
+        const int b = __builtin_amdgcn_readfirstlane((int)(fbv - (int64_t)f * A.P.nB));
+        const int64_t fb = (int64_t)f * A.P.nB + b;
+        const int s = (int)(it - fb * S);
+        if (f != fcur) {
+            while (dn > 0) deferred(min(dn, 64));
+            fcur = f;
+        }
+        const GeoC& g = *(const GeoC*)(A.B.geo + f);
+        // the wavefront's cluster: columns (-2 y', |y'|^2) and (-2 y', 1), box
+        const int nv = NVT > 4 ? A.P.nv : NVT;
+        // (the squares as the products' start, four registers an atom, where
+        // there is room, else as the operand's last component: 5 % of the time)
+        constexpr bool QUAD = NVT <= 4;
+        float Y[NVT], Z[NVT];
+        {
+            const gptr<const float> cb = (gptr<const float>)(A.B.clB + fb * 64 * A.P.nv);
+#pragma unroll
+            for (int q = 0; q < NVT; q++) {
+                const bool has = q < A.P.nv;
+                const float v = has ? cb[q * 64 + lane] : 0.f;
+                Y[q] = kk == 3 ? (has ? v : 1e30f) : -2.0f * v;
+                Z[q] = kk == 3 ? 1.0f : Y[q];
+                if (QUAD) Y[q] = has ? cb[q * 64 + 48 + col] : 1e30f;
+            }
+        }
+        const GeoI3 bc = fix_info(A.B.binfo + 3 * fb);
+        const float4 bmid = A.B.binfo[3 * fb + 1], bhalf = A.B.binfo[3 * fb + 2];
+        const float bm[3] = {sgpr_f(bmid.x), sgpr_f(bmid.y), sgpr_f(bmid.z)}, bh[3] = {sgpr_f(bhalf.x), sgpr_f(bhalf.y), sgpr_f(bhalf.z)};
+        // Guard of the values of pairs within the cutoff (u = 2^-24, S and Y the
+        // radii of tile and cluster, t between their centres: |t| <= cutoff + S
+        // + Y = W).  s' and y' are rounded by u S and u Y, t by rho u |t| (an
+        // exact integer difference): 2 sqrt(3) d times that.  |t - y'|^2, itself
+        // at most (d + S)^2: its norms, 3 u each, their sum and four additions to partial
+        // sums below Y^2 + 2 Y W + W^2.  The tile: 3 u S^2, the rounding of its
+        // columns, 2 u S (d + S), and four additions to sums below (d + 2 S)^2.
+        // The low CBITS bits of a value carry its code: below pk of it.
+        float Gx, thr;
+        {
+            const float Sx = __uint_as_float(g.rs_bits), Yx = A.B.binfo[3 * fb].w, cutf = (float)A.P.cutsys + 0.5f;
+            const float W = cutf + Sx + Yx, E2 = cutf + 2.0f * Sx;
+            const float gx = (0x1p-24f * (4.0f * fmaxf(Yx * (Yx + 2.0f * W), (cutf + Sx) * (cutf + Sx)) + 4.0f * (Yx * Yx + W * W) +
+                                          4.0f * E2 * E2 + Sx * (3.0f * Sx + 2.0f * (cutf + Sx)) +
+                                          3.5f * cutf * (Sx + Yx + g.rho * W)) + 1e-7f) * (1.0f + 1e-4f);
+            Gx = sgpr_f(gx);
+            thr = sgpr_f((A.P.c2hi32 + gx) * (1.0f + 1e-6f));
+        }
+        const float ambx = sgpr_f(2.0f * Gx + (thr + 1.0f) * (pk + 0x1p-21f));
+
+        // counts of up to 64 queued pairs
+        auto count = [&](int n) {
+            wave_sync();
+            const int k = qn - n + lane;
+            CArgs kc = k0;
+            asm volatile("" : "+s"(kc));
+            const ClArgs<TU, TV>& Q = *(const ClArgs<TU, TV>*)kc;
+            bool def = false;
+            int u = 0, v = 0;
+            if (lane < n) {
+                const float bv = qv[k], rv = qv[CL_Q + k], ru = SELF ? qv[2 * CL_Q + k] : INFINITY;
+                const int info = qi[4 * CL_Q + k];
+                const int code = __float_as_int(bv) & CMASK;
+                auto decide = [&](float x, int& bin, int& bulk) {
+                    const float c = __int_as_float(__float_as_int(x) & ~CMASK) * (1.0f + 0.5f * pk);
+                    return decide32(Q.P, Gx + c * (0.5f * pk + 0x1p-21f) + 1e-7f, c, bin, bulk);
+                };
+                int mbin, mbulk, vbin, ubin = 0, dummy;
+                const int dm = decide(bv, mbin, mbulk);
+                const int dv = decide(rv, vbin, dummy);
+                const int du = SELF ? decide(ru, ubin, dummy) : 1;
+                def = dm != 1 && (info >= 256 || dm == 0 || dv == 0 || du == 0);
+                const bool plain = shg && !Q.P.gu_ptr && !Q.P.gv_ptr;
+                bool drawn = false;
+                if (def || !plain || Q.P.K > 0) {
+                    const unsigned ou = (unsigned)ldg(Q.B.cl[0].ord + (int64_t)f * Q.P.Mu + qi[3 * CL_Q + k]);
+                    const unsigned ov = (unsigned)ldg(Q.B.cl[SELF ? 0 : 1].ord + (int64_t)f * Q.P.Mv + b * 16 + (info & 15));
+                    drawn = ((ou | ov) & CL_DRAWN) != 0;
+                    u = (int)(ou & ~CL_DRAWN);
+                    v = (int)(ov & ~CL_DRAWN);
+                }
+                if (dm == 2 && !def) {
+                    const int row = (code & 3) + (RPM == 4 ? 0 : 4 * (code >> (2 + QB)));
+                    const int q = cl_atom((code >> 2) & ((1 << QB) - 1), Q.P.iref), i = SELF ? cl_atom(row, Q.P.iref) : row;
+                    const int nb = Q.P.nbins;
+                    if (plain && !drawn) {
+                        if (mbin < nb) {
+                            atomicAdd(&sh[mbin], SELF ? 2u : 1u);
+                            atomicAdd(&sh[(2 + i) * nb + mbin], SELF ? 2u : 1u);
+                            atomicAdd(&sh[(2 + (SELF ? 0 : Q.P.gnu) + q) * nb + mbin], SELF ? 2u : 1u);
+                        }
+                    } else cl_main<TU, TV, SELF>(kc, f, u, v, i, q, mbin, mbulk, (LdsU)sh, shg ? 2 * nb : 0);
+                    if (dv == 2 && vbin < nb) atomicAdd(&sh[nb + vbin], 1u);
+                    if (SELF && du == 2 && ubin < nb) atomicAdd(&sh[nb + ubin], 1u);
+                }
+            }
+            const unsigned long long m = __ballot(def);
+            if (def) {
+                const int o = 2 * (dn + __popcll(m & lt));
+                dq[o] = u;
+                dq[o + 1] = v;
+            }
+            wave_sync();
+            qn -= n;
+            dn += __popcll(m);
+            if (dn >= 64) deferred(64);
+        };
+
+        // Tiles in reach: super tiles (a lane each), then the tiles of four of
+        // them (a lane each), then one after the other; the next tile's rows
+        // are loaded while one is evaluated.  After the last tile the queue is
+        // emptied.
+        const float rc = (float)A.P.cutsys + 2e-3f + 1e-6f * ((float)g.sp[0] + (float)g.sp[1] + (float)g.sp[2]);
+        const gptr<const float> ca = (gptr<const float>)(A.B.clA + (int64_t)f * A.P.nT * 64);
+        const int nS = A.P.nS;
+        int turn = 0;   // tiles in reach so far: split items (S > 1) take every S-th
+        int sb = -64;
+        unsigned long long smask = 0, tm = 0;
+        int tile = 0, sets = 0, tn = -1;
+        float an = 0.f;
+        // a lane's tile: its centre from the cluster's in fixed point; of the next
+        // tile that and its operand component
+        int ci[3] = {0, 0, 0}, sn = 0, nx[3] = {0, 0, 0};
+        float nt = 0.f;
+        bool more = true;
+        for (;;) {
+            const float a = an;
+            const int t = tn, st = sn, dx = nx[0], dy = nx[1], dz = nx[2];
+            float nt0 = nt;
+            tn = -1;
+            while (tm == 0 && more) {
+                CArgs kr = k0;
+                asm volatile("" : "+s"(kr));
+                const ClArgs<TU, TV>& R = *(const ClArgs<TU, TV>*)kr;
+                const GeoC& gr = *(const GeoC*)(R.B.geo + f);
+                if (smask == 0) {
+                    sb += 64;
+                    if (sb >= nS) { more = false; break; }
+                    bool in = false;
+                    if (sb + lane < nS) {
+                        const float4* si = R.B.sinfo + 2 * ((int64_t)f * nS + sb + lane);
+                        in = cl_reach(gr, rc, si[0], si[1], bm, bh, sets);
+                    }
+                    smask = __ballot(in);
+                    continue;
+                }
+                int mine = -1;
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const int bit = smask ? __ffsll((long long)smask) - 1 : -1;
+                    if (smask) smask &= smask - 1ull;
+                    mine = kk == j ? bit : mine;
+                }
+                tile = (sb + mine) * CL_SUP + col;
+                bool ok = false;
+                sets = 0;
+                // Self mode: a cluster's own molecules pair once; two blocks of 16
+                // molecules meet in the cluster that the parity of their sum
+                // names, which shares the work evenly (upper ones alone leave
+                // the first clusters twice the mean and the last ones nothing).
+                const int ub = tile * mp / 16;
+                if (mine >= 0 && tile < R.P.nT && (!SELF || ub == b || ((ub + b) & 1) == (ub > b ? 1 : 0))) {
+                    const float4* ti = R.B.tinfo + 3 * ((int64_t)f * R.P.nT + tile);
+                    ok = cl_reach(gr, rc, ti[1], ti[2], bm, bh, sets);
+                    const float4 t0 = ti[0];
+                    ci[0] = __float_as_int(t0.x) - bc.x; ci[1] = __float_as_int(t0.y) - bc.y; ci[2] = __float_as_int(t0.z) - bc.z;
+                    const int one = 1 << gr.fix;
+                    float tx, ty, tz;
+                    fix_cart(gr, ci[0] + (__builtin_ctz(sets | 8) - 1) * one, ci[1] + (__builtin_ctz((sets >> 3) | 8) - 1) * one,
+                             ci[2] + (__builtin_ctz((sets >> 6) | 8) - 1) * one, tx, ty, tz);
+                    *(float4*)&tt[4 * lane] = mk4(tx, ty, tz, fmaf(tx, tx, fmaf(ty, ty, tz * tz)));
+                }
+                wave_sync();
+                tm = __ballot(ok);
+                if (S > 1) {
+                    const int rank = turn + __popcll(tm & lt);
+                    turn = __builtin_amdgcn_readfirstlane((turn + __popcll(tm)) % S);
+                    tm = __ballot(ok && rank % S == s);
+                }
+            }
+            if (tm) {
+                const int bit = __ffsll((long long)tm) - 1;
+                tm &= tm - 1ull;
+                tn = __builtin_amdgcn_readlane(tile, bit);
+                sn = __builtin_amdgcn_readlane(sets, bit);
+#pragma unroll
+                for (int k = 0; k < 3; k++) nx[k] = __builtin_amdgcn_readlane(ci[k], bit);
+                nt = tt[4 * bit + kk];
+                an = ca[(int64_t)tn * 64 + lane];
+            }
+            if (t >= 0) {
+                float bb = INFINITY, ms = INFINITY, rv = INFINITY, ru = INFINITY;
+                int xs = st & 7, ys = (st >> 3) & 7, zs = st >> 6;
+                for (;;) {
+                    const float at = kk == 3 ? 1.0f : nt0, ct = kk == 3 ? nt0 : 0.f, bt = kk == 3 ? 0.f : 2.0f * nt0;
+#pragma unroll
+                    for (int q = 0; q < NVT; q++) {
+                        if (NVT > 4 && (q & 1) == 0 && q >= nv) break;   // (by twos: independent chains)
+                        // |t - y'|^2 in every row, then the distances
+                        const f4m c = QUAD ? __builtin_amdgcn_mfma_f32_16x16x4f32(nt0, Z[q], f4m{Y[q], Y[q], Y[q], Y[q]}, 0, 0, 0)
+                                           : __builtin_amdgcn_mfma_f32_16x16x4f32(at, Y[q] + ct, f4m{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                        f4m d = __builtin_amdgcn_mfma_f32_16x16x4f32(a, Z[q] + bt, c, 0, 0, 0);
+#pragma unroll
+                        for (int r = 0; r < 4; r++) d[r] = __int_as_float((__float_as_int(d[r]) & ~CMASK) | (r | (q << 2)));
+                        min2_4(bb, ms, d);
+                        if (q == 0) {
+                            rv = fminf(fminf(rv, d[0]), d[1]);
+                            rv = fminf(fminf(rv, d[2]), d[3]);
+                        }
+                        if (SELF) ru = fminf(ru, d[0]);
+                    }
+                    // further shifts in reach (boxes that two images of a tile reach)
+                    xs &= xs - 1;
+                    if (!xs) { xs = st & 7; ys &= ys - 1; }
+                    if (!ys) { ys = (st >> 3) & 7; zs &= zs - 1; }
+                    if (!zs) break;
+                    float tx, ty, tz;
+                    fix_cart(g, dx + (__builtin_ctz(xs) - 1) * (1 << g.fix), dy + (__builtin_ctz(ys) - 1) * (1 << g.fix),
+                             dz + (__builtin_ctz(zs) - 1) * (1 << g.fix), tx, ty, tz);
+                    nt0 = kk == 0 ? tx : (kk == 1 ? ty : (kk == 2 ? tz : fmaf(tx, tx, fmaf(ty, ty, tz * tz))));
+                }
+                // lane groups holding the other rows of the molecule
+                if constexpr (RPM > 4) {
+                    bb = __int_as_float(__float_as_int(bb) | ((kk & (RL - 1)) << (2 + QB)));
+                    if (SELF) ru = (kk & (RL - 1)) == 0 ? ru : INFINITY;
+                    auto merge = [&](auto pair) {
+                        const float2 b2 = pair(bb), s2 = pair(ms), v2 = pair(rv);
+                        ms = fminf(fminf(fmaxf(b2.x, b2.y), s2.x), s2.y);
+                        bb = fminf(b2.x, b2.y);
+                        rv = fminf(v2.x, v2.y);
+                        if (SELF) {
+                            const float2 u2 = pair(ru);
+                            ru = fminf(u2.x, u2.y);
+                        }
+                    };
+                    merge([](float x) { return row_pair<16>(x); });
+                    if constexpr (RPM > 8) merge([](float x) { return row_pair<32>(x); });
+                }
+                const int up = t * mp + (RPM == 4 ? kk : (RPM == 8 ? kk >> 1 : 0));
+                unsigned long long m = __ballot((RPM == 4 || (kk & (RL - 1)) == 0) && bb <= thr);
+                if (SELF && t * mp / 16 == b) m &= __ballot((up & 15) > col);
+                const bool hit = __builtin_amdgcn_inverse_ballot_w64(m);
+                if (hit) {
+                    const int k = qn + __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0));
+                    qv[k] = bb; qv[CL_Q + k] = rv;
+                    if (SELF) qv[2 * CL_Q + k] = ru;
+                    qi[3 * CL_Q + k] = up;
+                    qi[4 * CL_Q + k] = col | (ms - bb > ambx ? 0 : 256);
+                }
+                qn += __popcll(m);
+            }
+            const bool last = tn < 0 && t < 0 && !more;
+            if (qn >= 64 || last) count(min(qn, 64));
+            if (last) break;
+        }
+    }
+    while (dn > 0) deferred(min(dn, 64));
+    // (one atomic a block: on a single address they take about 10 ns each)
+    if (lane == 0) qi[0] = nexact;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        ull n = 0;
+        for (int w = 0; w < nw; w++) n += (ull)qi[w * CL_WORDS];
+        if (n) atomicAdd(&B_.stats[0], SELF ? 2 * n : n);
+    }
+    hist_flush(sh, P.nbins, B_.cnt_md, B_.cnt_rdf);
+    if (shg) groups_flush(P, shg, B_.cnt_gu, B_.cnt_gv);
+}
+
 // Fills n16 16-byte words and then ntail single bytes with zeros (a kernel,
 // not hipMemsetAsync: memset nodes captured in HIP graphs have given wrong
 // results on replays here, and a caller may capture these launches).
@@ -3946,6 +4697,7 @@ struct cm_job {
     // batch buffers
     DevBuf geo, cells_cnt, cells_start, tmp4, tmpcell, sorted, solw, ucen, vw, vcell, vcen;
     DevBuf P, vw_r, vcen_r, bflag, blist, nbulk, uk, drawn_ptr, drawn_idx;
+    DevBuf clmem;             // molecule pairs on the matrix cores: one block for all their buffers
     DevBuf near, mkey, mrank, mcnt, mstart, msum, msorted, nnear, chunk_base;
     DevBuf xin_u, xin_v;
     double cell_frac = 0.5;   // tiles family: fine cell side as a fraction of the cutoff
@@ -4021,16 +4773,55 @@ int ensure(cm_job* J, DevBuf& b, size_t bytes)
     return dev_take(b, bytes);
 }
 
+// Layout of the buffers of the molecule pairs on the matrix cores for F
+// frames; with base, their pointers.  Returns the bytes.
+size_t cl_layout(const KP& P, int64_t F, char* base, Bufs* B)
+{
+    size_t o = 0;
+    auto take = [&](size_t bytes) {
+        char* p = base ? base + o : nullptr;
+        o += (bytes + 255) & ~(size_t)255;
+        return p;
+    };
+    // the key counts first: cleared together per batch
+    ClSide cl[2] = {};
+    const int sides = P.self_ ? 1 : 2;
+    for (int k = 0; k < sides; k++) {
+        cl[k].M = k ? P.Mv : P.Mu;
+        cl[k].n = k ? P.nv : P.nu;
+        while (((int64_t)4 << (3 * cl[k].bits)) < cl[k].M && cl[k].bits < 9) cl[k].bits++;
+        cl[k].cnt = (int*)take((size_t)F << (3 * cl[k].bits) << 2);
+    }
+    const size_t zero = o;
+    for (int k = 0; k < sides; k++) {
+        cl[k].start = (int*)take((size_t)F << (3 * cl[k].bits) << 2);
+        cl[k].key = (int*)take((size_t)4 * F * cl[k].M);
+        cl[k].rank = (int*)take((size_t)4 * F * cl[k].M);
+        cl[k].ord = (int*)take((size_t)4 * F * cl[k].M);
+        cl[k].cen = (double*)take((size_t)24 * F * cl[k].M);
+    }
+    float* a = (float*)take((size_t)256 * F * P.nT);
+    float* b = (float*)take((size_t)256 * F * P.nB * P.nv);
+    float4* ti = (float4*)take((size_t)48 * F * P.nT);
+    float4* bi = (float4*)take((size_t)48 * F * P.nB);
+    float4* si = (float4*)take((size_t)32 * F * P.nS);
+    if (B) {
+        B->cl[0] = cl[0]; B->cl[1] = cl[1];
+        B->clA = a; B->clB = b; B->tinfo = ti; B->binfo = bi; B->sinfo = si;
+    }
+    return base ? zero : o;
+}
+
 int64_t per_frame_bytes(const cm_job* J, int dtype_size, bool host_input, int64_t cap, int64_t kcap)
 {
     int64_t Mu = J->d.nmols_u, Mv = J->d.nmols_v, NP = 1 + J->K;
     int64_t b = sizeof(Geo) + 64;
     if (host_input) b += (J->Nu + J->Nv) * 3 * dtype_size;
     int64_t items = J->atoms_family ? J->d.natoms_per_mol_u : Mu;
-    b += items * (16 + 16 + 4) + (cap + 1) * 8;
+    if (!J->kp.rpm) b += items * (16 + 16 + 4) + (cap + 1) * 8;
     if (!J->atoms_family) {
         b += J->Nu * 16 + Mu * 16 + (Mu + 1) * 4 + J->K * 8;
-        b += J->Nv * 16 + Mv * 20;
+        b += J->kp.rpm ? (int64_t)cl_layout(J->kp, 1, nullptr, nullptr) : J->Nv * 16 + Mv * 20;
         b += (int64_t)J->K * (J->Nv * (24 + 16) + Mv * 16);
     } else {
         b += cap * 9 + NP * ((kcap + 1) * 8 + Mv * 12 + 4) + 8;
@@ -4281,6 +5072,69 @@ void launch_scan(hipStream_t s, const KP& P, const Bufs& B, int random)
     hipLaunchKernelGGL(k_scan_rows, gr, dim3(1024), 0, s, P, B, random);
 }
 
+// molecule pairs on the matrix cores: order, operands and boxes of a batch
+template <class T>
+void launch_cl_prep(hipStream_t s, const KP& P, const Bufs& B, const void* xu, const void* xv)
+{
+    const unsigned sides = P.self_ ? 1 : 2, F = (unsigned)P.F;
+    const int64_t M = P.self_ ? P.Mu : std::max(P.Mu, P.Mv);
+    const unsigned gm = (unsigned)((M + BLOCK - 1) / BLOCK);
+    hipLaunchKernelGGL(k_cl_keys<T>, dim3(std::min(gm, 64u), F, sides), dim3(BLOCK), 0, s, P, B, (const T*)xu, (const T*)xv);
+    hipLaunchKernelGGL(k_grid, dim3(1), dim3(64), 0, s, P, B, 1);
+    hipLaunchKernelGGL(k_cl_scan, dim3(F, sides), dim3(1024), 0, s, P, B);
+    hipLaunchKernelGGL(k_cl_order, dim3(grid_for(M * F), sides), dim3(BLOCK), 0, s, P, B);
+    const unsigned gb = (unsigned)std::max(P.nS, (P.nB + BLOCK / 64 - 1) / (BLOCK / 64));
+    hipLaunchKernelGGL(k_cl_build<T>, dim3(gb, F, 2), dim3(BLOCK), 0, s, P, B,
+                       (const T*)xu, (const T*)xv);
+}
+
+template <class T, int RPM, int NVT, bool SELF>
+void launch_cl_one(hipStream_t s, const cm_job* J, const KP& P, const Bufs& B, const void* xu, const void* xv)
+{
+    auto kern = k_cl_eval<T, T, RPM, NVT, SELF>;
+    const int gwords = P.glds ? P.nbins * (P.gnu + (P.self_ ? 0 : P.gnv)) : 0;
+    const int64_t head = 4 * (int64_t)((2 * P.nbins + gwords + 3) & ~3);
+    const int waves = (int)std::max<int64_t>(1, std::min<int64_t>(NVT > 8 ? 8 : 16, (J->lds_max - head) / (4 * CL_WORDS)));
+    const size_t lds = (size_t)(head + 4 * (int64_t)CL_WORDS * waves);
+    int nb = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kern, 64 * waves, lds) != hipSuccess || nb < 1) nb = 1;
+    // small systems: S wavefronts split a cluster's tiles, so that every
+    // wavefront of the device has about two items
+    const int64_t items = (int64_t)P.F * P.nB, want = 2 * (int64_t)nb * J->cus * waves;
+    const int S = (int)std::min<int64_t>(16, std::max<int64_t>(1, want / std::max<int64_t>(items, 1)));
+    const int64_t blocks = std::min<int64_t>((int64_t)nb * J->cus, (items * S + waves - 1) / waves);
+    hipLaunchKernelGGL(kern, dim3((unsigned)((blocks + 7) / 8 * 8)), dim3(64 * waves), lds, s, P, B, (const T*)xu, (const T*)xv, S);
+}
+
+template <class T, int RPM>
+void launch_cl_rpm(hipStream_t s, const cm_job* J, const KP& P, const Bufs& B, const void* xu, const void* xv)
+{
+    if (P.self_) {
+        // the same molecules on both sides
+        if (RPM == 4 && P.nv == 3) launch_cl_one<T, RPM, RPM == 4 ? 3 : RPM, true>(s, J, P, B, xu, xv);
+        else launch_cl_one<T, RPM, RPM, true>(s, J, P, B, xu, xv);
+    } else {
+        if (P.nv == 3) launch_cl_one<T, RPM, 3, false>(s, J, P, B, xu, xv);
+        else if (P.nv <= 4) launch_cl_one<T, RPM, 4, false>(s, J, P, B, xu, xv);
+        else if (P.nv <= 8) launch_cl_one<T, RPM, 8, false>(s, J, P, B, xu, xv);
+        else launch_cl_one<T, RPM, 16, false>(s, J, P, B, xu, xv);
+    }
+}
+
+template <class T>
+void launch_cl(hipStream_t s, const cm_job* J, const KP& P, const Bufs& B, const void* xu, const void* xv)
+{
+    if (P.rpm == 4) launch_cl_rpm<T, 4>(s, J, P, B, xu, xv);
+    else if (P.rpm == 8) launch_cl_rpm<T, 8>(s, J, P, B, xu, xv);
+    else launch_cl_rpm<T, 16>(s, J, P, B, xu, xv);
+}
+
+void launch_cl_any(hipStream_t s, const cm_job* J, const KP& P, const Bufs& B, bool f32, const void* xu, const void* xv)
+{
+    if (f32) launch_cl<float>(s, J, P, B, xu, xv);
+    else launch_cl<double>(s, J, P, B, xu, xv);
+}
+
 int run_batch(cm_job* J, int F, const int64_t* frame_index, const void* xu_dev, const void* xv_dev, int dtype,
               const double* cells, int64_t cap, int64_t kcap)
 {
@@ -4330,7 +5184,10 @@ int run_batch(cm_job* J, int F, const int64_t* frame_index, const void* xu_dev, 
     } else if (J->K > 0) {
         if (int r = zero_async(J->uk.p, sizeof(int) * (size_t)F * J->K, s)) return r;
     }
-    if (int r = zero_async(J->cells_cnt.p, sizeof(int) * (size_t)F * (cap + 1), s)) return r;
+    if (P.rpm) {
+        const size_t zero = cl_layout(P, F, (char*)J->clmem.p, &B);
+        if (int r = zero_async(J->clmem.p, zero, s)) return r;
+    } else if (int r = zero_async(J->cells_cnt.p, sizeof(int) * (size_t)F * (cap + 1), s)) return r;
     if (tiles) {
         if (int r = zero_async(J->near.p, near_bytes(F, cap), s)) return r;
         if (int r = zero_async(J->mcnt.p, key_bytes(P, F), s)) return r;
@@ -4355,8 +5212,7 @@ int run_batch(cm_job* J, int F, const int64_t* frame_index, const void* xu_dev, 
         J->prof_random.push_back(P.K > 0 ? 1 : 0);
     }
     const int mols = tiles ? 0 : 1;
-    {
-        int64_t n = (int64_t)F * (P.Mv + (mols ? P.Mu : 0));
+    if (!P.rpm) {
         {
             const int64_t nm = (int64_t)P.Mv + (mols ? P.Mu : 0);
             const dim3 gr((unsigned)std::min<int64_t>((nm + BLOCK - 1) / BLOCK, 64), (unsigned)F);
@@ -4364,33 +5220,38 @@ int run_batch(cm_job* J, int F, const int64_t* frame_index, const void* xu_dev, 
             else hipLaunchKernelGGL(k_radii<double>, gr, dim3(BLOCK), 0, s, P, B, ud, vd, mols);
         }
     }
-    hipLaunchKernelGGL(k_grid, dim3(1), dim3(64), 0, s, P, B, mols);
-    if (tiles) {
-        int64_t n = (int64_t)F * P.nu;
-        if (f32) hipLaunchKernelGGL(k_wrap_atoms<float>, dim3(grid_for(n)), dim3(BLOCK), 0, s, P, B, uf);
-        else hipLaunchKernelGGL(k_wrap_atoms<double>, dim3(grid_for(n)), dim3(BLOCK), 0, s, P, B, ud);
+    if (!P.rpm) hipLaunchKernelGGL(k_grid, dim3(1), dim3(64), 0, s, P, B, mols);
+    if (P.rpm) {
+        if (f32) launch_cl_prep<float>(s, P, B, xu_dev, xv_dev);
+        else launch_cl_prep<double>(s, P, B, xu_dev, xv_dev);
     } else {
-        int64_t n = (int64_t)F * P.Mu;
-        if (f32) hipLaunchKernelGGL(k_prep_solute_mols<float>, dim3(grid_for(n)), dim3(BLOCK), 0, s, P, B, uf);
-        else hipLaunchKernelGGL(k_prep_solute_mols<double>, dim3(grid_for(n)), dim3(BLOCK), 0, s, P, B, ud);
-    }
-    hipLaunchKernelGGL(k_scan_cells, dim3(F), dim3(1024), 0, s, P, B);
-    hipLaunchKernelGGL(k_scatter, dim3(grid_for((int64_t)F * B.nitems)), dim3(BLOCK), 0, s, P, B, B.nitems);
-    if (tiles) {
-        hipLaunchKernelGGL(k_near_mark, dim3((P.nu + BLOCK - 1) / BLOCK, std::min(F, 65535)), dim3(BLOCK), 0, s, P, B);
-        hipLaunchKernelGGL(k_dfield, dim3(grid_for((int64_t)F * cap * 16)), dim3(BLOCK), 0, s, P, B);
-        int64_t n = (int64_t)F * P.Mv;
-        if (f32) hipLaunchKernelGGL(k_prep_solvent_tiles<float>, dim3(grid_for(n)), dim3(BLOCK), 0, s, P, B, vf);
-        else hipLaunchKernelGGL(k_prep_solvent_tiles<double>, dim3(grid_for(n)), dim3(BLOCK), 0, s, P, B, vd);
-        launch_scan(s, P, B, 0);
-        hipLaunchKernelGGL(k_mol_scatter, grid_slots(P.Mv, F), dim3(BLOCK), 0, s, P, B, 0);
-        if (f32) hipLaunchKernelGGL(k_fill_real<float>, dim3(grid_for(n)), dim3(BLOCK), 0, s, P, B, vf);
-        else hipLaunchKernelGGL(k_fill_real<double>, dim3(grid_for(n)), dim3(BLOCK), 0, s, P, B, vd);
-        hipLaunchKernelGGL(k_chunk_table, dim3(1), dim3(1024), 0, s, P, B, 0);
-    } else {
-        int64_t n = (int64_t)F * P.Mv;
-        if (f32) hipLaunchKernelGGL(k_prep_solvent<float>, dim3(grid_for(n)), dim3(BLOCK), 0, s, P, B, vf);
-        else hipLaunchKernelGGL(k_prep_solvent<double>, dim3(grid_for(n)), dim3(BLOCK), 0, s, P, B, vd);
+        if (tiles) {
+            int64_t n = (int64_t)F * P.nu;
+            if (f32) hipLaunchKernelGGL(k_wrap_atoms<float>, dim3(grid_for(n)), dim3(BLOCK), 0, s, P, B, uf);
+            else hipLaunchKernelGGL(k_wrap_atoms<double>, dim3(grid_for(n)), dim3(BLOCK), 0, s, P, B, ud);
+        } else {
+            int64_t n = (int64_t)F * P.Mu;
+            if (f32) hipLaunchKernelGGL(k_prep_solute_mols<float>, dim3(grid_for(n)), dim3(BLOCK), 0, s, P, B, uf);
+            else hipLaunchKernelGGL(k_prep_solute_mols<double>, dim3(grid_for(n)), dim3(BLOCK), 0, s, P, B, ud);
+        }
+        hipLaunchKernelGGL(k_scan_cells, dim3(F), dim3(1024), 0, s, P, B);
+        hipLaunchKernelGGL(k_scatter, dim3(grid_for((int64_t)F * B.nitems)), dim3(BLOCK), 0, s, P, B, B.nitems);
+        if (tiles) {
+            hipLaunchKernelGGL(k_near_mark, dim3((P.nu + BLOCK - 1) / BLOCK, std::min(F, 65535)), dim3(BLOCK), 0, s, P, B);
+            hipLaunchKernelGGL(k_dfield, dim3(grid_for((int64_t)F * cap * 16)), dim3(BLOCK), 0, s, P, B);
+            int64_t n = (int64_t)F * P.Mv;
+            if (f32) hipLaunchKernelGGL(k_prep_solvent_tiles<float>, dim3(grid_for(n)), dim3(BLOCK), 0, s, P, B, vf);
+            else hipLaunchKernelGGL(k_prep_solvent_tiles<double>, dim3(grid_for(n)), dim3(BLOCK), 0, s, P, B, vd);
+            launch_scan(s, P, B, 0);
+            hipLaunchKernelGGL(k_mol_scatter, grid_slots(P.Mv, F), dim3(BLOCK), 0, s, P, B, 0);
+            if (f32) hipLaunchKernelGGL(k_fill_real<float>, dim3(grid_for(n)), dim3(BLOCK), 0, s, P, B, vf);
+            else hipLaunchKernelGGL(k_fill_real<double>, dim3(grid_for(n)), dim3(BLOCK), 0, s, P, B, vd);
+            hipLaunchKernelGGL(k_chunk_table, dim3(1), dim3(1024), 0, s, P, B, 0);
+        } else {
+            int64_t n = (int64_t)F * P.Mv;
+            if (f32) hipLaunchKernelGGL(k_prep_solvent<float>, dim3(grid_for(n)), dim3(BLOCK), 0, s, P, B, vf);
+            else hipLaunchKernelGGL(k_prep_solvent<double>, dim3(grid_for(n)), dim3(BLOCK), 0, s, P, B, vd);
+        }
     }
     if (P.K > 0) hipLaunchKernelGGL(k_bulk_init, dim3(grid_for((int64_t)F * P.kb * P.Mv)), dim3(BLOCK), 0, s, P, B);
     HIPCHK(hipGetLastError());
@@ -4398,6 +5259,8 @@ int run_batch(cm_job* J, int F, const int64_t* frame_index, const void* xu_dev, 
     if (J->profiling) HIPCHK(hipEventRecord(ev[0], s));
     if (tiles) {
         launch_tiles_any(f32, false, s, J->eval_grid, J, P, B, xu_dev, xv_dev);
+    } else if (P.rpm) {
+        launch_cl_any(s, J, P, B, f32, xu_dev, xv_dev);
     } else {
         int64_t n = (int64_t)F * P.Mv;
         const int gwords = P.glds ? P.nbins * (P.gnu + (P.self_ ? 0 : P.gnv)) : 0;
@@ -4472,19 +5335,26 @@ int alloc_batch(cm_job* J, int F, int64_t cap, int64_t kcap, int dtype_size, boo
     int64_t Mu = J->d.nmols_u, Mv = J->d.nmols_v, NP = 1 + J->K;
     int64_t items = J->atoms_family ? J->d.natoms_per_mol_u : Mu;
     if ((r = ensure(J, J->geo, sizeof(Geo) * F))) return r;
-    if ((r = ensure(J, J->cells_cnt, round16(sizeof(int) * F * (cap + 1))))) return r;
-    if ((r = ensure(J, J->cells_start, sizeof(int) * F * (cap + 1)))) return r;
-    if ((r = ensure(J, J->tmp4, 16 * F * items))) return r;
-    if ((r = ensure(J, J->tmpcell, 4 * F * items))) return r;
-    if ((r = ensure(J, J->sorted, 16 * F * items))) return r;
-    if ((r = ensure(J, J->vw, 16 * F * J->Nv))) return r;
+    const bool cl = J->kp.rpm > 0;
+    if (cl) {
+        if ((r = ensure(J, J->clmem, cl_layout(J->kp, F, nullptr, nullptr)))) return r;
+    } else {
+        if ((r = ensure(J, J->cells_cnt, round16(sizeof(int) * F * (cap + 1))))) return r;
+        if ((r = ensure(J, J->cells_start, sizeof(int) * F * (cap + 1)))) return r;
+        if ((r = ensure(J, J->tmp4, 16 * F * items))) return r;
+        if ((r = ensure(J, J->tmpcell, 4 * F * items))) return r;
+        if ((r = ensure(J, J->sorted, 16 * F * items))) return r;
+        if ((r = ensure(J, J->vw, 16 * F * J->Nv))) return r;
+    }
     if (!J->atoms_family) {
         if ((r = ensure(J, J->solw, 16 * F * J->Nu))) return r;
         if ((r = ensure(J, J->ucen, 16 * F * Mu))) return r;
         if ((r = ensure(J, J->drawn_ptr, 4 * F * (Mu + 1)))) return r;
         if ((r = ensure(J, J->drawn_idx, 4 * F * std::max(J->K, 1)))) return r;
-        if ((r = ensure(J, J->vcell, 4 * F * Mv))) return r;
-        if ((r = ensure(J, J->vcen, 16 * F * Mv))) return r;
+        if (!cl) {
+            if ((r = ensure(J, J->vcell, 4 * F * Mv))) return r;
+            if ((r = ensure(J, J->vcen, 16 * F * Mv))) return r;
+        }
     } else {
         if ((r = ensure(J, J->near, near_bytes(F, cap)))) return r;
         // (also one 8-byte word per chunk of a launch: chunks hold 8 molecules
@@ -4762,6 +5632,17 @@ void job_params(cm_job* J, const cm_job_desc& d)
     }
     J->tile_c = 4;
     set_chunks(J);
+    // Molecule pairs on the matrix cores: molecules of up to CL_ATOMS atoms
+    // on both sides, the rows of one tile.  Larger ones would need minima over
+    // several tiles; their walk already spends its time on distances (one
+    // thread, 289 of them or more a pair).  The no-allocation entry point keeps
+    // the walk as well: its admission rule counts the walk's buffers.
+    if (!J->atoms_family && !J->arena && P.nu <= CL_ATOMS && P.nv <= CL_ATOMS) {
+        P.rpm = P.nu <= 4 ? 4 : (P.nu <= 8 ? 8 : 16);
+        P.nT = (int)(((int64_t)P.Mu * P.rpm + 15) / 16);
+        P.nS = (P.nT + CL_SUP - 1) / CL_SUP;
+        P.nB = (P.Mv + 15) / 16;
+    }
     P.gnu = d.n_groups_u;
     P.gnv = d.n_groups_v;
     // molecule-pair kernels keep the group counts in LDS when they fit
@@ -5286,7 +6167,7 @@ void cm_job_destroy(cm_job* J)
                       &J->tmp4, &J->tmpcell, &J->sorted, &J->solw, &J->ucen, &J->vw, &J->vcell, &J->vcen, &J->P,
                       &J->vw_r, &J->vcen_r, &J->bflag, &J->blist, &J->nbulk, &J->uk, &J->drawn_ptr,
                       &J->drawn_idx, &J->xin_u, &J->xin_v, &J->near, &J->mkey, &J->mrank, &J->mcnt, &J->mstart, &J->msum,
-                      &J->msorted, &J->nnear, &J->chunk_base, &J->vrec};
+                      &J->clmem, &J->msorted, &J->nnear, &J->chunk_base, &J->vrec};
     for (DevBuf* b : bufs) dev_put(*b);
     pin_put(J->hres);
     for (auto& a : J->prof_ev)
@@ -6091,6 +6972,7 @@ int cm_mddf_noalloc(const cm_job_desc* desc, int32_t nframes, const int64_t* fra
     int64_t need_fixed, capmax, kcapmax, Fmax, pfb;
     {
         cm_job plan;
+        plan.arena = (char*)1;   // (sized as the call below runs: from the scratch)
         job_params(&plan, *desc);
         need_fixed = noalloc_fixed_bytes(&plan);
         plan.d.memory_budget = (int64_t)SCRATCH_BYTES;
@@ -6122,7 +7004,7 @@ int cm_mddf_noalloc(const cm_job_desc* desc, int32_t nframes, const int64_t* fra
                       &J->tmp4, &J->tmpcell, &J->sorted, &J->solw, &J->ucen, &J->vw, &J->vcell, &J->vcen, &J->P,
                       &J->vw_r, &J->vcen_r, &J->bflag, &J->blist, &J->nbulk, &J->uk, &J->drawn_ptr,
                       &J->drawn_idx, &J->xin_u, &J->xin_v, &J->near, &J->mkey, &J->mrank, &J->mcnt, &J->mstart, &J->msum,
-                      &J->msorted, &J->nnear, &J->chunk_base};
+                      &J->clmem, &J->msorted, &J->nnear, &J->chunk_base};
     for (DevBuf* b : bufs) *b = DevBuf{};
     J->arena = (char*)D.ptr;
     J->arena_cap = SCRATCH_BYTES;
