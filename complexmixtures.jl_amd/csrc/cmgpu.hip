@@ -40,7 +40,8 @@
 // Larger molecules, and jobs on a caller's scratch: molecule centres in a cell
 // list, one thread per solvent molecule evaluating all atom pairs of close
 // molecule pairs (k_radii, k_prep_solute_mols, k_prep_solvent,
-// k_eval_mols_real).  Both: k_place, k_eval_mols_rand for the random passes.
+// k_eval_mols_real).  Both, for the random passes: k_mols_near (slots near their
+// drawn solute molecule), k_eval_mols_rand (their placement and records).
 //
 // k_flush turns integer hits into FP64 accumulators times the frame weight.
 //
@@ -188,7 +189,7 @@ struct Bufs {
     // random passes
     double* P;               // [F][K][Nv][3]
     float4* vw_r;            // [F][K][Nv]
-    float4* vcen_r;          // [F][K][Mv]
+    float4* vcen_r;          // mols, [F*K][Mv]: slots to evaluate, their centres and numbers (count: slot_counts)          // [F][K][Mv]
     unsigned char* bflag;    // [F][kb][Mv]
     int* blist;              // [F][kb][Mv]
     int* nbulk;              // [F][kb]
@@ -1650,74 +1651,6 @@ __global__ void __launch_bounds__(BLOCK, 3) k_eval_mols_real(KP P, Bufs B, const
     if (shg) groups_flush(P, shg, B.cnt_gu, B.cnt_gv);
 }
 
-// Whether placed slot v (centre cv) can have an atom pair with the drawn
-// solute molecule (centre cu) within the cutoff under some lattice shift:
-// the centre pre-check of the random passes of the molecule-pair family.
-// k_place and k_eval_mols_rand evaluate it with the same FP32 operations on
-// the same values, so a slot skipped by the placement is one the evaluation
-// skips.
-__device__ __forceinline__ bool mol_pair_near(const Geo& g, float4 cv, float4 cu)
-{
-    bool any = false;
-    for (int mz = -1; mz <= 1; mz++)
-    for (int my = -1; my <= 1; my++)
-    for (int mx = -1; mx <= 1; mx++) {
-        float fx = (float)mx, fy = (float)my, fz = (float)mz;
-        float tx = g.H32[0] * fx + g.H32[3] * fy + g.H32[6] * fz;
-        float ty = g.H32[1] * fx + g.H32[4] * fy + g.H32[7] * fz;
-        float tz = g.H32[2] * fx + g.H32[5] * fy + g.H32[8] * fz;
-        float dx = cv.x - (cu.x + tx), dy = cv.y - (cu.y + ty), dz = cv.z - (cu.z + tz);
-        any |= !(dx * dx + dy * dy + dz * dz > g.rpre2);
-    }
-    return any;
-}
-
-template <class TU>
-__global__ void __launch_bounds__(BLOCK) k_eval_mols_rand(KP P, Bufs B, const TU* xu)
-{
-    extern __shared__ unsigned sh[];
-    const int gwords = P.glds ? P.nbins * (P.gnu + (P.self_ ? 0 : P.gnv)) : 0;
-    hist_clear(sh, 2 * P.nbins + gwords);
-    unsigned* shg = P.glds ? sh + 2 * P.nbins : nullptr;
-    int64_t total = (int64_t)P.F * P.K * P.Mv;
-    for (int64_t it = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; it < total; it += (int64_t)gridDim.x * blockDim.x) {
-        int64_t fk = it / P.Mv;
-        int v = (int)(it - fk * P.Mv);
-        int f = (int)(fk / P.K);
-        int u = B.uk[fk];
-        if (P.self_ && u == v) continue;
-        const Geo& g = B.geo[f];
-        const float4* yw = B.vw_r + fk * P.Nv + (int64_t)v * P.nv;
-        float4 cv = B.vcen_r[fk * P.Mv + v];
-        float4 cu = B.ucen[(int64_t)f * P.Mu + u];
-        const float4* xs = B.solw + (int64_t)f * P.Nu + (int64_t)u * P.nu;
-        Best bm, br;
-        bm.init(); br.init();
-        // the slots k_place skipped fail this test (the same one)
-        if (!mol_pair_near(g, cv, cu)) continue;
-        for (int mz = -1; mz <= 1; mz++)
-        for (int my = -1; my <= 1; my++)
-        for (int mx = -1; mx <= 1; mx++) {
-            float fx = (float)mx, fy = (float)my, fz = (float)mz;
-            float tx = g.H32[0] * fx + g.H32[3] * fy + g.H32[6] * fz;
-            float ty = g.H32[1] * fx + g.H32[4] * fy + g.H32[7] * fz;
-            float tz = g.H32[2] * fx + g.H32[5] * fy + g.H32[8] * fz;
-            float dx = cv.x - (cu.x + tx), dy = cv.y - (cu.y + ty), dz = cv.z - (cu.z + tz);
-            if (dx * dx + dy * dy + dz * dz > g.rpre2) continue;
-            pairs_mol(P, xs, yw, tx, ty, tz, bm, br);
-        }
-        const TU* xuf = xu + (int64_t)f * P.Nu * 3;
-        int64_t jbase = (int64_t)v * P.nv;
-        auto ysrc = [&](int a, double& y0, double& y1, double& y2) {
-            const double* pp = B.P + (fk * P.Nv + jbase + a) * 3; y0 = pp[0]; y1 = pp[1]; y2 = pp[2];
-        };
-        Rec r = resolve_mols(P, g, xuf, u, v, ysrc, bm, br, &B.stats[0]);
-        hist_record_mols(P, sh, shg, B.cnt_gu_r, B.cnt_gv_r, r);
-    }
-    hist_flush(sh, P.nbins, B.cnt_md_r, B.cnt_rdf_r);
-    if (shg) groups_flush(P, shg, B.cnt_gu_r, B.cnt_gv_r);
-}
-
 // ---------------------------------------------------------------------------
 // bulk lists and random placement
 // ---------------------------------------------------------------------------
@@ -1739,8 +1672,14 @@ __global__ void k_bulk_init(KP P, Bufs B)
 }
 
 // ordered compaction of the bulk flags, one block per (frame, list)
-__device__ __forceinline__ void b_bulk_compact(KP P, Bufs B, int bx_, int nbx_, int by_, int nby_)
+// Slots listed per (frame, pass) of the molecule-pair family.  The counts take the
+// place of drawn_idx, which the real pass was the last to read.
+__device__ __forceinline__ int* slot_counts(const Bufs& B) { return B.drawn_idx; }
+
+__device__ __forceinline__ void b_bulk_compact(KP P, Bufs B, int bx_, int nbx_, int by_, int nby_, bool mols = false)
 {
+    if (mols)
+        for (int k = bx_ * blockDim.x + threadIdx.x; k < P.F * P.K; k += nbx_ * blockDim.x) slot_counts(B)[k] = 0;
     __shared__ int wsum[16];
     __shared__ int carry;
     int64_t fk = bx_;
@@ -1773,9 +1712,9 @@ __device__ __forceinline__ void b_bulk_compact(KP P, Bufs B, int bx_, int nbx_, 
     if (threadIdx.x == 0) B.nbulk[fk] = carry;
 }
 
-__global__ void __launch_bounds__(1024) k_bulk_compact(KP P, Bufs B)
+__global__ void __launch_bounds__(1024) k_bulk_compact(KP P, Bufs B, int mols)
 {
-    b_bulk_compact(P, B, blockIdx.x, gridDim.x, blockIdx.y, gridDim.y);
+    b_bulk_compact(P, B, blockIdx.x, gridDim.x, blockIdx.y, gridDim.y, mols != 0);
 }
 
 // The atoms of one source molecule (xyz interleaved) and the placed atoms
@@ -1790,12 +1729,12 @@ struct MolSrc {
 
 struct MolDst {
     gptr<double> p;
-    gptr<f4v> w;
-    __device__ MolDst(double* q, float4* v) : p((gptr<double>)q), w((gptr<f4v>)v) {}
+    float4* w;   // (k_eval_mols_rand reads these in the same thread)
+    __device__ MolDst(double* q, float4* v) : p((gptr<double>)q), w(v) {}
     __device__ void operator()(int a, double x, double y, double z) const
     {
         p[3 * a] = x; p[3 * a + 1] = y; p[3 * a + 2] = z;
-        w[a] = f4v{(float)x, (float)y, (float)z, 0.f};
+        w[a] = mk4((float)x, (float)y, (float)z, 0.f);
     }
 };
 
@@ -1815,42 +1754,142 @@ struct MolDstFix {
     __device__ void set_w0(float x) const { ((gptr<float>)w)[3] = x; }
 };
 
-// randomize_solvent!, src/mddf.jl:65-88, for every slot of every random pass
-template <class TV>
-__global__ void k_place(KP P, Bufs B, const TV* xv)
+// Whether placed slot v (centre cv) can have an atom pair with the drawn
+// solute molecule (centre cu) within the cutoff under some lattice shift: the
+// centre pre-check of the random passes of the molecule-pair family.  In a
+// diagonal cell the nearest image decides (rounding: rpre2's margin of 1e-2 A).
+__device__ __forceinline__ bool mol_pair_near(const Geo& g, float4 cv, float4 cu)
+{
+    const float dx = cv.x - cu.x, dy = cv.y - cu.y, dz = cv.z - cu.z;
+    if (g.ortho) {
+        float ox, oy, oz;
+        minimage32(g, dx, dy, dz, ox, oy, oz);
+        return !(ox * ox + oy * oy + oz * oz > g.rpre2);
+    }
+    bool any = false;
+    for (int mz = -1; mz <= 1; mz++)
+    for (int my = -1; my <= 1; my++)
+    for (int mx = -1; mx <= 1; mx++) {
+        const float fx = (float)mx, fy = (float)my, fz = (float)mz;
+        const float ex = dx - (g.H32[0] * fx + g.H32[3] * fy + g.H32[6] * fz);
+        const float ey = dy - (g.H32[1] * fx + g.H32[4] * fy + g.H32[7] * fz);
+        const float ez = dz - (g.H32[2] * fx + g.H32[5] * fy + g.H32[8] * fz);
+        any |= !(ex * ex + ey * ey + ez * ez > g.rpre2);
+    }
+    return any;
+}
+
+// The slots of the random passes that can be within the cutoff of their drawn
+// solute molecule (all of them when the placements are kept for verification),
+// listed per (frame, pass).  A few per cent are; placed and evaluated where
+// they lie, one or two lanes of a wavefront would work at a time.  16,667 waters
+// about 181 osmolytes, 20 frames of 10 passes: placement 125 and evaluation
+// 229 us so, 25 us for the list (random numbers and the test) and 68 us for
+// both now; with an atomic per wavefront the list alone took 217 us.
+constexpr int NEAR_SLOTS = 4;   // slots per thread: one atomic a block (each takes about 10 ns of its line's time)
+__global__ void __launch_bounds__(BLOCK) k_mols_near(KP P, Bufs B)
 {
     // grid: x over the slots, y over the (frame, pass) pairs
-    const int v = blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= P.Mv) return;
+    __shared__ float4 list[NEAR_SLOTS * BLOCK];
+    __shared__ int n, base;
+    const int v0 = blockIdx.x * NEAR_SLOTS * BLOCK, lane = threadIdx.x & 63;
     for (int fk = blockIdx.y; fk < P.F * P.K; fk += gridDim.y) {
         const int f = fk / P.K;
         const int k = fk - f * P.K;
         const Geo& g = B.geo[f];
-        cm::u32x4 r = cm::philox4x32_10({(uint32_t)v, (uint32_t)k, g.frame, cm::TAG_SLOT}, P.key0, P.key1);
-        double uc[3] = {cm::u01(r.y), cm::u01(r.z), cm::u01(r.w)};
-        // the new centre H*uc (inside the cell)
+        const int u = B.uk[fk];
+        const float4 cu = B.ucen[(int64_t)f * P.Mu + u];
         const double* H = g.cell.H;
-        double c0 = H[0] * uc[0] + H[3] * uc[1] + H[6] * uc[2];
-        double c1 = H[1] * uc[0] + H[4] * uc[1] + H[7] * uc[2];
-        double c2 = H[2] * uc[0] + H[5] * uc[1] + H[8] * uc[2];
-        const float4 cv = mk4((float)c0, (float)c1, (float)c2, 0.f);
-        B.vcen_r[(int64_t)fk * P.Mv + v] = cv;
-        // only slots the evaluation can reach are placed (all of them when
-        // the placements are kept for verification)
-        if (!P.place_all) {
-            const int u = B.uk[fk];
-            if (P.self_ && u == v) continue;
-            if (!mol_pair_near(g, cv, B.ucen[(int64_t)f * P.Mu + u])) continue;
+        if (threadIdx.x == 0) n = 0;
+        __syncthreads();
+        for (int v = v0 + threadIdx.x; v < v0 + NEAR_SLOTS * BLOCK; v += BLOCK) {
+            const cm::u32x4 r = cm::philox4x32_10({(uint32_t)v, (uint32_t)k, g.frame, cm::TAG_SLOT}, P.key0, P.key1);
+            const double uc[3] = {cm::u01(r.y), cm::u01(r.z), cm::u01(r.w)};
+            // the new centre H*uc (inside the cell)
+            const double c0 = H[0] * uc[0] + H[3] * uc[1] + H[6] * uc[2];
+            const double c1 = H[1] * uc[0] + H[4] * uc[1] + H[7] * uc[2];
+            const double c2 = H[2] * uc[0] + H[5] * uc[1] + H[8] * uc[2];
+            const float4 cv = mk4((float)c0, (float)c1, (float)c2, __int_as_float(v));
+            const bool take = v < P.Mv && (P.place_all || (!(P.self_ && u == v) && mol_pair_near(g, cv, cu)));
+            const unsigned long long m = __ballot(take);
+            if (!m) continue;
+            int o = 0;
+            if (lane == 0) o = atomicAdd(&n, __popcll(m));
+            o = __builtin_amdgcn_readfirstlane(o);
+            if (take) list[o + __popcll(m & ((1ull << lane) - 1ull))] = cv;
         }
-        cm::u32x4 r2 = cm::philox4x32_10({(uint32_t)v, (uint32_t)k, g.frame, cm::TAG_SLOT + 1u}, P.key0, P.key1);
-        int64_t lk = (int64_t)f * P.kb + (P.kb == 1 ? 0 : k);
-        int nb = B.nbulk[lk];
-        int64_t jmol = nb > 0 ? (int64_t)B.blist[lk * P.Mv + cm::draw_index(r.x, nb)] : cm::draw_index(r.x, P.Mv);
-        MolSrc<TV> src(xv + (int64_t)f * P.Nv * 3 + jmol * P.nv * 3);
-        MolDst dst(B.P + (fk * P.Nv + (int64_t)v * P.nv) * 3, B.vw_r + fk * P.Nv + (int64_t)v * P.nv);
-        double ua[3] = {cm::u01(r2.x), cm::u01(r2.y), cm::u01(r2.z)};
-        cm::random_move(src, dst, P.nv, P.iref, g.cell, uc, ua);
+        __syncthreads();
+        if (threadIdx.x == 0) base = n ? atomicAdd(&slot_counts(B)[fk], n) : 0;
+        __syncthreads();
+        for (int e = threadIdx.x; e < n; e += BLOCK) B.vcen_r[(int64_t)fk * P.Mv + base + e] = list[e];
+        __syncthreads();
     }
+}
+
+// The listed slots, one thread each: placement (randomize_solvent!,
+// src/mddf.jl:65-88) and the record of the drawn solute molecule with the
+// placed one.  blockIdx.y: (frame, pass) pairs; the wavefronts of the blocks of
+// a pair take 64 slots in turn.  A launch has one or two turns: bound by the
+// latency of one (FP64 rotation, minima, records) and the flush of the blocks'
+// few counts.
+template <class TU, class TV>
+__global__ void __launch_bounds__(BLOCK) k_eval_mols_rand(KP P, Bufs B, const TU* xu, const TV* xv)
+{
+    extern __shared__ unsigned sh[];
+    const int gwords = P.glds ? P.nbins * (P.gnu + (P.self_ ? 0 : P.gnv)) : 0;
+    hist_clear(sh, 2 * P.nbins + gwords);
+    unsigned* shg = P.glds ? sh + 2 * P.nbins : nullptr;
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    for (int fk = blockIdx.y; fk < P.F * P.K; fk += gridDim.y) {
+        const int f = fk / P.K;
+        const int k = fk - f * P.K;
+        const Geo& g = B.geo[f];
+        const int u = B.uk[fk], count = slot_counts(B)[fk];
+        const int64_t lk = (int64_t)f * P.kb + (P.kb == 1 ? 0 : k);
+        const int nb = B.nbulk[lk];
+        const float4 cu = B.ucen[(int64_t)f * P.Mu + u];
+        const float4* xs = B.solw + (int64_t)f * P.Nu + (int64_t)u * P.nu;
+        for (int n = (wid * gridDim.x + blockIdx.x) * 64 + lane; n < count; n += nw * gridDim.x * 64) {
+            const float4 cv = B.vcen_r[(int64_t)fk * P.Mv + n];
+            const int v = __float_as_int(cv.w);
+            const cm::u32x4 r = cm::philox4x32_10({(uint32_t)v, (uint32_t)k, g.frame, cm::TAG_SLOT}, P.key0, P.key1);
+            const cm::u32x4 r2 = cm::philox4x32_10({(uint32_t)v, (uint32_t)k, g.frame, cm::TAG_SLOT + 1u}, P.key0, P.key1);
+            const double uc[3] = {cm::u01(r.y), cm::u01(r.z), cm::u01(r.w)};
+            const double ua[3] = {cm::u01(r2.x), cm::u01(r2.y), cm::u01(r2.z)};
+            const int64_t jmol = nb > 0 ? (int64_t)B.blist[lk * P.Mv + cm::draw_index(r.x, nb)] : cm::draw_index(r.x, P.Mv);
+            MolSrc<TV> src(xv + (int64_t)f * P.Nv * 3 + jmol * P.nv * 3);
+            const int64_t jbase = (int64_t)v * P.nv;
+            MolDst dst(B.P + (fk * (int64_t)P.Nv + jbase) * 3, B.vw_r + fk * (int64_t)P.Nv + jbase);
+            cm::random_move(src, dst, P.nv, P.iref, g.cell, uc, ua);
+            if ((P.self_ && u == v) || (P.place_all && !mol_pair_near(g, cv, cu))) continue;
+            const float4* yw = B.vw_r + fk * (int64_t)P.Nv + jbase;
+            Best bm, br;
+            bm.init(); br.init();
+            // the lattice shifts in reach, then a shift of its own per lane and turn
+            unsigned near = 0;
+            for (int q = 0; q < 27; q++) {
+                const float fx = (float)(q % 3 - 1), fy = (float)(q / 3 % 3 - 1), fz = (float)(q / 9 - 1);
+                const float dx = cv.x - (cu.x + (g.H32[0] * fx + g.H32[3] * fy + g.H32[6] * fz));
+                const float dy = cv.y - (cu.y + (g.H32[1] * fx + g.H32[4] * fy + g.H32[7] * fz));
+                const float dz = cv.z - (cu.z + (g.H32[2] * fx + g.H32[5] * fy + g.H32[8] * fz));
+                near |= dx * dx + dy * dy + dz * dz > g.rpre2 ? 0u : 1u << q;
+            }
+            for (; near; near &= near - 1) {
+                const int q = __builtin_ctz(near);
+                const float fx = (float)(q % 3 - 1), fy = (float)(q / 3 % 3 - 1), fz = (float)(q / 9 - 1);
+                pairs_mol(P, xs, yw, g.H32[0] * fx + g.H32[3] * fy + g.H32[6] * fz, g.H32[1] * fx + g.H32[4] * fy + g.H32[7] * fz,
+                          g.H32[2] * fx + g.H32[5] * fy + g.H32[8] * fz, bm, br);
+            }
+            const TU* xuf = xu + (int64_t)f * P.Nu * 3;
+            auto ysrc = [&](int a, double& y0, double& y1, double& y2) {
+                const double* pp = B.P + (fk * (int64_t)P.Nv + jbase + a) * 3; y0 = pp[0]; y1 = pp[1]; y2 = pp[2];
+            };
+            Rec rec = resolve_mols(P, g, xuf, u, v, ysrc, bm, br, &B.stats[0]);
+            hist_record_mols(P, sh, shg, B.cnt_gu_r, B.cnt_gv_r, rec);
+        }
+    }
+    hist_flush(sh, P.nbins, B.cnt_md_r, B.cnt_rdf_r);
+    if (shg) groups_flush(P, shg, B.cnt_gu_r, B.cnt_gv_r);
 }
 
 // ---------------------------------------------------------------------------
@@ -5289,7 +5328,7 @@ int run_batch(cm_job* J, int F, const int64_t* frame_index, const void* xu_dev, 
     HIPCHK(hipGetLastError());
     // random passes
     if (P.K > 0) {
-        hipLaunchKernelGGL(k_bulk_compact, dim3(F * P.kb), dim3(1024), 0, s, P, B);
+        hipLaunchKernelGGL(k_bulk_compact, dim3(F * P.kb), dim3(1024), 0, s, P, B, tiles ? 0 : 1);
         if (tiles) {
             hipLaunchKernelGGL(k_place_keys, grid_slots(P.Mv, F * P.K), dim3(BLOCK), 0, s, P, B);
             launch_scan(s, P, B, 1);
@@ -5299,8 +5338,7 @@ int run_batch(cm_job* J, int F, const int64_t* frame_index, const void* xu_dev, 
             else hipLaunchKernelGGL(k_place_near<double>, gs, dim3(BLOCK), 0, s, P, B, vd);
             hipLaunchKernelGGL(k_chunk_table, dim3(1), dim3(1024), 0, s, P, B, 1);
         } else {
-            if (f32) hipLaunchKernelGGL(k_place<float>, grid_slots(P.Mv, F * P.K), dim3(BLOCK), 0, s, P, B, vf);
-            else hipLaunchKernelGGL(k_place<double>, grid_slots(P.Mv, F * P.K), dim3(BLOCK), 0, s, P, B, vd);
+            hipLaunchKernelGGL(k_mols_near, grid_slots((P.Mv + NEAR_SLOTS - 1) / NEAR_SLOTS, F * P.K), dim3(BLOCK), 0, s, P, B);
         }
         HIPCHK(hipGetLastError());
         if (J->profiling) HIPCHK(hipEventRecord(ev[2], s));
@@ -5309,9 +5347,12 @@ int run_batch(cm_job* J, int F, const int64_t* frame_index, const void* xu_dev, 
         } else {
             const int gwords = P.glds ? P.nbins * (P.gnu + (P.self_ ? 0 : P.gnv)) : 0;
             const size_t shr = sizeof(unsigned) * (2 * P.nbins + gwords);
-            const int64_t n = (int64_t)F * P.K * P.Mv;
-            if (f32) hipLaunchKernelGGL(k_eval_mols_rand<float>, dim3(grid_for(n)), dim3(BLOCK), shr, s, P, B, uf);
-            else hipLaunchKernelGGL(k_eval_mols_rand<double>, dim3(grid_for(n)), dim3(BLOCK), shr, s, P, B, ud);
+            // about four blocks per CU; pairs of their own where there are enough
+            const int64_t fk = (int64_t)F * P.K, want = 4 * (int64_t)J->cus;
+            const unsigned gy = (unsigned)std::min<int64_t>(fk, want);
+            const unsigned gx = (unsigned)std::max<int64_t>(1, std::min<int64_t>((P.Mv + BLOCK - 1) / BLOCK, want / gy));
+            if (f32) hipLaunchKernelGGL((k_eval_mols_rand<float, float>), dim3(gx, gy), dim3(BLOCK), shr, s, P, B, uf, vf);
+            else hipLaunchKernelGGL((k_eval_mols_rand<double, double>), dim3(gx, gy), dim3(BLOCK), shr, s, P, B, ud, vd);
         }
         if (J->profiling) HIPCHK(hipEventRecord(ev[3], s));
     }
