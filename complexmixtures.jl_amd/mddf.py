@@ -71,15 +71,15 @@ def _job_for(R, options, tmeta, coordination_number_only, **kw):
 
 
 def _store_raw(R, raw):
-    R.md_count[:] = raw["md_count"]
-    R.md_count_random[:] = raw["md_count_random"]
-    R.rdf_count[:] = raw["rdf_count"]
-    R.rdf_count_random[:] = raw["rdf_count_random"]
-    R.solute_group_count[:] = raw["solute_group_count"]
-    R.solute_group_count_random[:] = raw["solute_group_count_random"]
+    """The job's sums become the result's arrays (the job is done with them: no
+    copy, and the zeros they replace are never touched)."""
+    names = ["md_count", "md_count_random", "rdf_count", "rdf_count_random", "solute_group_count",
+             "solute_group_count_random"]
     if not R.autocorrelation:
-        R.solvent_group_count[:] = raw["solvent_group_count"]
-        R.solvent_group_count_random[:] = raw["solvent_group_count_random"]
+        names += ["solvent_group_count", "solvent_group_count_random"]
+    for k in names:
+        assert raw[k].shape == getattr(R, k).shape, k
+        setattr(R, k, raw[k])
     R.volume.total = raw["volume_total"]
 
 

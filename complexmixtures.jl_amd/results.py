@@ -38,6 +38,14 @@ def shellradius(i, step):
     return (0.5 * (_cube(rmin + step) + _cube(rmin))) ** (1 / 3)
 
 
+def _shellradii(nbins, step):
+    """shellradius of every bin: the same operations on arrays, but for the
+    power, which stays the scalar one to the last bit"""
+    rmin = np.arange(nbins, dtype=np.float64) * step
+    e = 1 / 3
+    return [x ** e for x in (0.5 * (_cube(rmin + step) + _cube(rmin))).tolist()]
+
+
 @dataclass
 class Density:
     solute: float = 0.0
@@ -121,7 +129,8 @@ def make_result(trajectory, options, trajectory_data, frame_weights=None):
 
 def isautocorrelation(trajectory):
     """src/results.jl:240-243"""
-    return list(trajectory.solute.indices) == list(trajectory.solvent.indices)
+    u, v = trajectory.solute.indices, trajectory.solvent.indices
+    return u is v or (len(u) == len(v) and list(u) == list(v))
 
 
 def set_samples(R):
@@ -152,22 +161,22 @@ def finalresults(R, options, coordination_number_only):
 
 def _mddf_final_results(R, options):
     """src/results.jl:320-376"""
-    R.d[:] = [shellradius(i, options.binstep) for i in range(1, R.nbins + 1)]
+    R.d[:] = _shellradii(R.nbins, options.binstep)
     solvent_nmols, nrandom = set_samples(R)
     Q = sum_frame_weights(R)
     nu = R.solute.nmols
-    R.md_count[:] = R.md_count / (nu * Q)
-    R.solute_group_count[:] = R.solute_group_count / (nu * Q)
-    R.solute_group_count_random[:] = R.solute_group_count_random / (nrandom * Q)
+    R.md_count /= nu * Q
+    R.solute_group_count /= nu * Q
+    R.solute_group_count_random /= nrandom * Q
     if R.autocorrelation:
         R.solvent_group_count[:] = R.solute_group_count
         R.solvent_group_count_random[:] = R.solute_group_count_random
     else:
-        R.solvent_group_count[:] = R.solvent_group_count / (nu * Q)
-        R.solvent_group_count_random[:] = R.solvent_group_count_random / (nrandom * Q)
-    R.md_count_random[:] = R.md_count_random / (nrandom * Q)
-    R.rdf_count[:] = R.rdf_count / (nu * Q)
-    R.rdf_count_random[:] = R.rdf_count_random / (nrandom * Q)
+        R.solvent_group_count /= nu * Q
+        R.solvent_group_count_random /= nrandom * Q
+    R.md_count_random /= nrandom * Q
+    R.rdf_count /= nu * Q
+    R.rdf_count_random /= nrandom * Q
     R.volume.total = R.volume.total / Q
     R.volume.shell[:] = R.volume.total * (R.rdf_count_random / solvent_nmols)
     step = R.files[0].options.binstep
@@ -216,16 +225,16 @@ def _coordination_number_final_results(R, options):
         import warnings
         warnings.warn("\ncoordination_number_only was set to true, so the MDDF and KB integrals were not computed. \n"
                       "(to remove this warning use `Options(silent=true)`)\n")
-    R.d[:] = [shellradius(i, options.binstep) for i in range(1, R.nbins + 1)]
+    R.d[:] = _shellradii(R.nbins, options.binstep)
     Q = sum_frame_weights(R)
     nu = R.solute.nmols
-    R.md_count[:] = R.md_count / (nu * Q)
-    R.solute_group_count[:] = R.solute_group_count / (nu * Q)
+    R.md_count /= nu * Q
+    R.solute_group_count /= nu * Q
     if R.autocorrelation:
         R.solvent_group_count[:] = R.solute_group_count
     else:
-        R.solvent_group_count[:] = R.solvent_group_count / (nu * Q)
-    R.rdf_count[:] = R.rdf_count / (nu * Q)
+        R.solvent_group_count /= nu * Q
+    R.rdf_count /= nu * Q
     R.volume.total = R.volume.total / Q
     R.density.solvent = R.solvent.nmols / R.volume.total
     R.density.solute = R.solute.nmols / R.volume.total

@@ -108,14 +108,17 @@ def group_csr(sel, atom_positions, groups_of):
     Returns (None, None) without custom groups."""
     if not groups_of.custom_groups:
         return None, None
-    where = {}
-    for g, inds in enumerate(groups_of.group_atom_indices):
-        for a in inds:
-            where.setdefault(a, []).append(g)
-    ptr = np.zeros(len(atom_positions) + 1, dtype=np.int32)
-    idx = []
-    for k, p in enumerate(atom_positions):
-        gs = where.get(sel.indices[p], [])
-        idx.extend(gs)
-        ptr[k + 1] = ptr[k] + len(gs)
-    return ptr, np.array(idx if idx else [0], dtype=np.int32)
+    # the groups' atoms sorted (stably: an atom's groups stay in order), then the
+    # run of each position's atom; array operations, since there is one position
+    # per solvent atom
+    groups = [np.asarray(g, dtype=np.int64) for g in groups_of.group_atom_indices]
+    atoms = np.concatenate(groups) if groups else np.zeros(0, dtype=np.int64)
+    order = np.argsort(atoms, kind="stable")
+    atoms = atoms[order]
+    ids = np.repeat(np.arange(len(groups), dtype=np.int32), [len(g) for g in groups])[order]
+    at = np.asarray(sel.indices, dtype=np.int64)[np.asarray(atom_positions, dtype=np.int64)]
+    lo, hi = np.searchsorted(atoms, at, "left"), np.searchsorted(atoms, at, "right")
+    ptr = np.zeros(len(at) + 1, dtype=np.int32)
+    np.cumsum(hi - lo, out=ptr[1:])
+    idx = ids[np.arange(ptr[-1]) + np.repeat(lo - ptr[:-1], hi - lo)]
+    return ptr, idx if idx.size else np.zeros(1, dtype=np.int32)
