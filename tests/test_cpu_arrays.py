@@ -16,12 +16,12 @@ def _csr_by_atom(sel, positions, groups_of):
 
 @pytest.mark.parametrize("seed", range(40))
 def test_group_csr(pkg, seed):
-    """Overlapping, repeated and empty groups, another selection's atoms, positions in any order."""
+    """Overlapping and empty groups, another selection's atoms, positions in any order."""
     from complexmixtures_amd.selection import group_csr
     rng = np.random.default_rng(seed)
     n = int(rng.integers(1, 40))
     ind = np.sort(rng.permutation(100)[:n] + 1).tolist()
-    groups = [rng.choice(ind, size=int(rng.integers(0, 15))).tolist() for _ in range(int(rng.integers(1, 6)))]
+    groups = [rng.choice(ind, size=int(rng.integers(0, n + 1)), replace=False).tolist() for _ in range(int(rng.integers(1, 6)))]
     with warnings.catch_warnings():
         warnings.simplefilter("ignore")
         s = pkg.AtomSelection(ind, nmols=1, group_atom_indices=groups, group_names=[str(i) for i in range(len(groups))])
