@@ -5,8 +5,8 @@
 //
 // "tiles" -- one solute molecule of any size (proteins, polymers), solvent
 // molecules of up to 64 atoms.  Per batch of frames, on the job's stream:
-//   k_radii             solvent molecule radius about its centre
-//   k_grid              per-frame FP32 thresholds (guard band)
+//   k_radii             solvent molecule radius about its centre, then per-frame
+//                       FP32 thresholds (guard band)
 //   k_wrap_atoms, k_scan_cells, k_scatter
 //                       solute atoms in a fine cell grid (counting sort + scan)
 //   k_near_mark         cells within cutoff + radius of some solute atom
@@ -30,7 +30,7 @@
 //
 // "mols" -- many solute molecules (self MDDF, small solutes), molecules of up
 // to 16 atoms:
-//   k_cl_keys, k_grid, k_cl_scan, k_cl_order
+//   k_cl_keys, k_cl_scan, k_cl_order
 //                       molecule radii, molecules in Hilbert order
 //   k_cl_build          tiles of 16 solute rows, clusters of 16 solvent
 //                       molecules, their boxes
@@ -98,6 +98,7 @@ struct Geo {                 // one frame of a batch
     float rpre2;             // molecule-centre pre-check radius^2 (mols family)
     unsigned ru_bits, rv_bits;   // molecule radii (float bits, atomicMax)
     int err;                 // geometry the kernels cannot handle
+    unsigned radii_done;     // blocks of the radii launch that have reported (the last one runs frame_grid)
     float rstage;            // staging radius around a chunk (cutoff + margin), tiles family
     float rnear;             // near-cell radius around a solute atom (cutoff + radius + margin)
     int kbits;               // bits per dimension of the sort keys of the fine cells
@@ -437,86 +438,18 @@ __device__ __forceinline__ float block_max(float x)
     return r;
 }
 
-// molecule radii (bound on the distance of an atom from the centre of its
-// molecule, with a margin over FP32 rounding); blockIdx.y = frame
-template <class T>
-__device__ __forceinline__ void b_radii(KP P, Bufs B, const T* xu, const T* xv, int do_solute, int bx_, int nbx_, int by_, int nby_)
-{
-    const int f = by_;
-    Geo& g = B.geo[f];
-    const int64_t nmol = (int64_t)P.Mv + (do_solute ? P.Mu : 0);
-    float rv = 0.f, ru = 0.f;
-    for (int64_t m = bx_ * (int64_t)blockDim.x + threadIdx.x; m < nmol; m += (int64_t)nbx_ * blockDim.x) {
-        const bool solv = m < P.Mv;
-        const T* x = solv ? xv + (int64_t)f * P.Nv * 3 : xu + (int64_t)f * P.Nu * 3;
-        const int n = solv ? P.nv : P.nu;
-        const int64_t a0 = solv ? m * P.nv : (m - P.Mv) * P.nu;
-        double x0, y0, z0;
-        load3(x, a0, x0, y0, z0);
-        float sx = 0.f, sy = 0.f, sz = 0.f;
-        for (int a = 0; a < n; a++) {
-            double xa, ya, za;
-            load3(x, a0 + a, xa, ya, za);
-            float ox, oy, oz;
-            minimage32(g, (float)(xa - x0), (float)(ya - y0), (float)(za - z0), ox, oy, oz);
-            sx += ox; sy += oy; sz += oz;
-        }
-        sx /= n; sy /= n; sz /= n;
-        float r2 = 0.f;
-        for (int a = 0; a < n; a++) {
-            double xa, ya, za;
-            load3(x, a0 + a, xa, ya, za);
-            float ox, oy, oz;
-            minimage32(g, (float)(xa - x0), (float)(ya - y0), (float)(za - z0), ox, oy, oz);
-            float dx = ox - sx, dy = oy - sy, dz = oz - sz;
-            r2 = fmaxf(r2, dx * dx + dy * dy + dz * dz);
-        }
-        const float r = sqrtf(r2) * 1.0001f + 1e-3f;
-        if (solv) rv = fmaxf(rv, r); else ru = fmaxf(ru, r);
-    }
-    rv = block_max(rv);
-    ru = block_max(ru);
-    if (threadIdx.x == 0) {
-        if (rv > 0.f) atomicMax(&g.rv_bits, __float_as_uint(rv));
-        if (ru > 0.f) atomicMax(&g.ru_bits, __float_as_uint(ru));
-    }
-}
-
-template <class T>
-__global__ void k_radii(KP P, Bufs B, const T* xu, const T* xv, int do_solute)
-{
-    b_radii<T>(P, B, xu, xv, do_solute, blockIdx.x, gridDim.x, blockIdx.y, gridDim.y);
-}
-
 __device__ __forceinline__ double halfulp32(double x)
 {
     if (!(x > 1e-30)) return 0x1p-150;
     return ldexp(1.0, ilogb(x) - 24);
 }
 
-// geometry errors of a batch's frames into the job's error bits (bit 0:
-// molecules too large for the cell, bit 1: grid larger than its allocation),
-// read with the accumulators at the end of the job
-__device__ __forceinline__ void b_geo_flags(KP P, Bufs B, int bx_, int nbx_, int by_, int nby_)
-{
-    for (int f = threadIdx.x; f < P.F; f += blockDim.x) {
-        const int e = B.geo[f].err;
-        if (e) atomicOr(&B.stats[2], e == 2 ? 1ull : 2ull);
-    }
-}
 
-__global__ void k_geo_flags(KP P, Bufs B)
+__device__ void frame_grid(const KP& P, const Bufs& B, int mols_family, int f)
 {
-    b_geo_flags(P, B, blockIdx.x, gridDim.x, blockIdx.y, gridDim.y);
-}
-
-__device__ __forceinline__ void b_grid(KP P, Bufs B, int mols_family, int bx_, int nbx_, int by_, int nby_)
-{
-    int f = bx_ * blockDim.x + threadIdx.x;
-    if (f >= P.F) return;
     Geo& g = B.geo[f];
-    double ru = mols_family ? (double)__uint_as_float(g.ru_bits) : 0.0;
-    double rv = (double)__uint_as_float(g.rv_bits);
+    auto radius = [](unsigned* p) { return (double)__uint_as_float(__hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)); };
+    const double ru = mols_family ? radius(&g.ru_bits) : 0.0, rv = radius(&g.rv_bits);
     if (mols_family) {
         double side = P.cutsys + ru + rv + 1e-3 + 1e-7 * (g.sp[0] + g.sp[1] + g.sp[2]);
         int ncell = 1;
@@ -528,6 +461,9 @@ __device__ __forceinline__ void b_grid(KP P, Bufs B, int mols_family, int bx_, i
         }
         if (ncell > P.cap) g.err = 3;
         g.ncell = ncell;
+        // the job's error bits (bit 0: molecules too large for the cell, bit 1: grid
+        // larger than its allocation), read with the accumulators at the end
+        if (g.err) atomicOr(&B.stats[2], g.err == 2 ? 1ull : 2ull);
     }
     const double* H = g.cell.H;
     // Fixed point: positions are fractions of the cell in units of 2^-fix, fix
@@ -573,9 +509,69 @@ __device__ __forceinline__ void b_grid(KP P, Bufs B, int mols_family, int bx_, i
     g.rnear = (float)(P.cutsys + rv + 20.0 * E + 1e-2 + 1e-6 * (g.sp[0] + g.sp[1] + g.sp[2]));
 }
 
-__global__ void k_grid(KP P, Bufs B, int mols_family)
+// The end of a block of a radii launch: `blocks` of them report per frame, and
+// the last one derives the frame's thresholds (a launch of its own took 3 to 5 us
+// of every call).  The blocks run on different XCDs: agent-scope atomics, each
+// waited for before the report counts.  (A fence would write the L2 back: with
+// one per block the radii of 40,000 molecules, 40 frames took 124 us, not 30.)
+__device__ __forceinline__ void radii_report(const KP& P, const Bufs& B, int mols_family, int f, float ru, float rv, int blocks)
 {
-    b_grid(P, B, mols_family, blockIdx.x, gridDim.x, blockIdx.y, gridDim.y);
+    if (threadIdx.x != 0) return;
+    Geo& g = B.geo[f];
+    // (with their results used, the maxima are performed before the count)
+    unsigned old = 0;
+    if (rv > 0.f) old |= atomicMax(&g.rv_bits, __float_as_uint(rv));
+    if (ru > 0.f) old |= atomicMax(&g.ru_bits, __float_as_uint(ru));
+    asm volatile("s_waitcnt vmcnt(0)" ::"v"(old) : "memory");
+    if (atomicAdd(&g.radii_done, 1u) == (unsigned)blocks - 1u) frame_grid(P, B, mols_family, f);
+}
+
+// molecule radii (bound on the distance of an atom from the centre of its
+// molecule, with a margin over FP32 rounding); blockIdx.y = frame
+template <class T>
+__device__ __forceinline__ void b_radii(KP P, Bufs B, const T* xu, const T* xv, int do_solute, int bx_, int nbx_, int by_, int nby_)
+{
+    const int f = by_;
+    Geo& g = B.geo[f];
+    const int64_t nmol = (int64_t)P.Mv + (do_solute ? P.Mu : 0);
+    float rv = 0.f, ru = 0.f;
+    for (int64_t m = bx_ * (int64_t)blockDim.x + threadIdx.x; m < nmol; m += (int64_t)nbx_ * blockDim.x) {
+        const bool solv = m < P.Mv;
+        const T* x = solv ? xv + (int64_t)f * P.Nv * 3 : xu + (int64_t)f * P.Nu * 3;
+        const int n = solv ? P.nv : P.nu;
+        const int64_t a0 = solv ? m * P.nv : (m - P.Mv) * P.nu;
+        double x0, y0, z0;
+        load3(x, a0, x0, y0, z0);
+        float sx = 0.f, sy = 0.f, sz = 0.f;
+        for (int a = 0; a < n; a++) {
+            double xa, ya, za;
+            load3(x, a0 + a, xa, ya, za);
+            float ox, oy, oz;
+            minimage32(g, (float)(xa - x0), (float)(ya - y0), (float)(za - z0), ox, oy, oz);
+            sx += ox; sy += oy; sz += oz;
+        }
+        sx /= n; sy /= n; sz /= n;
+        float r2 = 0.f;
+        for (int a = 0; a < n; a++) {
+            double xa, ya, za;
+            load3(x, a0 + a, xa, ya, za);
+            float ox, oy, oz;
+            minimage32(g, (float)(xa - x0), (float)(ya - y0), (float)(za - z0), ox, oy, oz);
+            float dx = ox - sx, dy = oy - sy, dz = oz - sz;
+            r2 = fmaxf(r2, dx * dx + dy * dy + dz * dz);
+        }
+        const float r = sqrtf(r2) * 1.0001f + 1e-3f;
+        if (solv) rv = fmaxf(rv, r); else ru = fmaxf(ru, r);
+    }
+    rv = block_max(rv);
+    ru = block_max(ru);
+    radii_report(P, B, do_solute, f, ru, rv, nbx_);
+}
+
+template <class T>
+__global__ void k_radii(KP P, Bufs B, const T* xu, const T* xv, int do_solute)
+{
+    b_radii<T>(P, B, xu, xv, do_solute, blockIdx.x, gridDim.x, blockIdx.y, gridDim.y);
 }
 
 // ---------------------------------------------------------------------------
@@ -2029,6 +2025,11 @@ __device__ __forceinline__ void cell_range32(const GEO& g, int cx, int cy, int c
 // box).  A block takes 256 consecutive atoms of one frame (neighbours along
 // the chain, whose cell ranges overlap): the marks go into a bitmap of the
 // frame's cells in LDS first, and the block writes each marked cell once.
+// Lanes an atom in k_near_mark.  Few atoms: eight, each with an eighth of the
+// serial walk over the atom's cells (30 atoms: 25 -> 11 us).  From a block's worth
+// on, one: the cell ranges that every lane forms are extra (1,000 atoms: 36 us,
+// 45 with eight; 5,000: 47 and 65).
+__host__ __device__ __forceinline__ int near_lanes(int nu) { return nu < 256 ? 8 : 1; }
 constexpr int NEAR_WORDS = 8192;   // LDS bitmap words (frames of up to 262,144 cells; larger: direct stores)
 
 __device__ __forceinline__ void b_near_mark(KP P, Bufs B, int bx_, int nbx_, int by_, int nby_)
@@ -2062,13 +2063,16 @@ __device__ __forceinline__ void b_near_mark(KP P, Bufs B, int bx_, int nbx_, int
                 for (int c = c0; c <= c1; c++) nr[c] = 1;
             }
         };
-        for (int64_t at = bx_ * (int64_t)blockDim.x + threadIdx.x; at < P.nu; at += (int64_t)nbx_ * blockDim.x) {
+        // a few lanes an atom take its layers of cells in turn
+        const int lanes = near_lanes(P.nu);
+        for (int64_t e = bx_ * (int64_t)blockDim.x + threadIdx.x; e < (int64_t)P.nu * lanes; e += (int64_t)nbx_ * blockDim.x) {
+            const int64_t at = e / lanes;
             const float4 u = B.tmp4[(int64_t)f * P.nu + at];
             float4 s;
             fix_cart(g, __float_as_int(u.x), __float_as_int(u.y), __float_as_int(u.z), s.x, s.y, s.z);
             int ilo[3], ihi[3];
             cell_range(g, s.x, s.y, s.z, s.x, s.y, s.z, g.rnear, ilo, ihi);
-            for (int iz = ilo[2]; iz <= ihi[2]; iz++) {
+            for (int iz = ilo[2] + (int)(e % lanes); iz <= ihi[2]; iz += lanes) {
                 int mz; int cz = wrap_index(iz, g.nc[2], mz);
                 const float dz = g.ortho ? gap(s.z, iz * hz, (iz + 1) * hz) : 0.f;
                 for (int iy = ilo[1]; iy <= ihi[1]; iy++) {
@@ -3504,11 +3508,8 @@ __global__ void __launch_bounds__(BLOCK) k_cl_keys(KP P, Bufs B, const T* xu, co
         }
     }
     const float r = block_max(r2 > 0.f || blockIdx.x * blockDim.x + threadIdx.x < s.M ? sqrtf(r2) * 1.0001f + 1e-3f : 0.f);
-    if (threadIdx.x == 0 && r > 0.f) {
-        // (self: both radii)
-        if (side == 1 || P.self_) atomicMax(&g.rv_bits, __float_as_uint(r));
-        if (side == 0) atomicMax(&g.ru_bits, __float_as_uint(r));
-    }
+    // (self: both radii)
+    radii_report(P, B, 1, f, side == 0 ? r : 0.f, side == 1 || P.self_ ? r : 0.f, gridDim.x * gridDim.z);
 }
 
 // exclusive scan of the key counts, one block per frame and side
@@ -4097,11 +4098,32 @@ __global__ void __launch_bounds__(NVT > 8 ? 512 : 1024) k_cl_eval(KP P_, Bufs B_
 // Fills n16 16-byte words and then ntail single bytes with zeros (a kernel,
 // not hipMemsetAsync: memset nodes captured in HIP graphs have given wrong
 // results on replays here, and a caller may capture these launches).
-__global__ void k_zero(uint4* p, int64_t n16, unsigned char* tail, int ntail)
+// Several ranges in one launch (each its own word): nine of a small call's
+// thirty launches were fills, some 4 us each.
+struct FillList {
+    static constexpr int MAX = 6;
+    int n = 0;
+    unsigned char* p[MAX];   // 16-byte aligned
+    int64_t bytes[MAX];
+    unsigned word[MAX];
+    void add(void* q, size_t b, unsigned w = 0)
+    {
+        if (!b) return;
+        p[n] = (unsigned char*)q;
+        bytes[n] = (int64_t)b;
+        word[n++] = w;
+    }
+};
+__global__ void k_fill(FillList L)
 {
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; k < n16; k += stride) p[k] = make_uint4(0u, 0u, 0u, 0u);
-    if (blockIdx.x == 0 && (int)threadIdx.x < ntail) tail[threadIdx.x] = 0;
+    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, stride = (int64_t)gridDim.x * blockDim.x;
+    for (int r = 0; r < L.n; r++) {
+        uint4* p = (uint4*)L.p[r];
+        const unsigned w = L.word[r];
+        const int64_t n16 = L.bytes[r] >> 4;
+        for (int64_t k = t; k < n16; k += stride) p[k] = make_uint4(w, w, w, w);
+        if (t < (L.bytes[r] & 15)) L.p[r][16 * n16 + t] = (unsigned char)(w >> (8 * (t & 3)));
+    }
 }
 
 // verification records of molecules no chunk evaluates: not within the
@@ -4173,9 +4195,9 @@ __global__ void k_pack16(const ull* cnt, uint16_t* out, ull* hits, int64_t n, in
 // ---------------------------------------------------------------------------
 constexpr int MS_MAX = 128;   // jobs per round
 enum MStage {
-    MS_ZERO, MS_RADII, MS_GRID, MS_WRAP, MS_SCAN_CELLS, MS_SCATTER, MS_NEAR, MS_DFIELD, MS_PREP, MS_SCAN_SUMS0,
+    MS_ZERO, MS_RADII, MS_WRAP, MS_SCAN_CELLS, MS_SCATTER, MS_NEAR, MS_DFIELD, MS_PREP, MS_SCAN_SUMS0,
     MS_SCAN_ROWS0, MS_MOL_SCATTER0, MS_FILL, MS_CHUNK0, MS_BULK_INIT, MS_BULK_COMPACT, MS_PLACE_KEYS, MS_SCAN_SUMSK,
-    MS_SCAN_ROWSK, MS_MOL_SCATTERK, MS_PLACE_NEAR, MS_CHUNKK, MS_RESOLVE0, MS_RESOLVEK, MS_GEO_FLAGS, MS_N
+    MS_SCAN_ROWSK, MS_MOL_SCATTERK, MS_PLACE_NEAR, MS_CHUNKK, MS_RESOLVE0, MS_RESOLVEK, MS_N
 };
 
 struct SysDev {
@@ -4241,13 +4263,6 @@ __global__ void __launch_bounds__(BLOCK) km_radii(const MultiTab* __restrict__ M
 {
     multi_blocks<MS_RADII, true>(MT, [&](const SysDev& S, int bx, int nbx, int by, int nby) {
         b_radii<T>(S.P, S.B, (const T*)S.xu, (const T*)S.xv, 0, bx, nbx, by, nby);
-    });
-}
-
-__global__ void km_grid(const MultiTab* __restrict__ MT)
-{
-    multi_blocks<MS_GRID, false>(MT, [&](const SysDev& S, int bx, int nbx, int by, int nby) {
-        b_grid(S.P, S.B, 0, bx, nbx, by, nby);
     });
 }
 
@@ -4369,13 +4384,6 @@ __global__ void km_place_near(const MultiTab* __restrict__ MT)
     });
 }
 
-__global__ void km_geo_flags(const MultiTab* __restrict__ MT)
-{
-    multi_blocks<MS_GEO_FLAGS, false>(MT, [&](const SysDev& S, int bx, int nbx, int by, int nby) {
-        b_geo_flags(S.P, S.B, bx, nbx, by, nby);
-    });
-}
-
 // The chunks of every job of a round in tickets of about `per` chunks of one
 // job, taken by blocks from the counter ctr (zero at the start of the launch):
 // a ticket's chunks lie at a stride over its job, so the tickets of a job cost
@@ -4471,6 +4479,14 @@ int fail(int code, const std::string& msg)
 
 // x: blocks over n molecules or slots; y: one per (frame, pass) pair, up to
 // the grid limit (the kernels stride over y beyond it)
+// blocks per frame of k_near_mark: every lane an item while that is few blocks
+// (each clears and writes out its bitmap), then as many as there are atoms for
+int near_blocks(int nu)
+{
+    const int all = (int)(((int64_t)nu * near_lanes(nu) + BLOCK - 1) / BLOCK);
+    return std::max(1, std::min(all, std::max(4, (nu + BLOCK - 1) / BLOCK)));
+}
+
 dim3 grid_slots(int n, int pairs)
 {
     return dim3((unsigned)std::max(1, (n + BLOCK - 1) / BLOCK), (unsigned)std::max(1, std::min(pairs, 65535)));
@@ -4486,13 +4502,12 @@ int grid_for(int64_t n)
 
 // zeroes `bytes` bytes at p (16-byte aligned: every buffer here starts on a
 // 256-byte boundary) on stream s
-int zero_async(void* p, size_t bytes, hipStream_t s)
+int fill_async(const FillList& L, hipStream_t s)
 {
-    if (!bytes) return CM_OK;
-    const int64_t n16 = (int64_t)(bytes / 16);
-    const int ntail = (int)(bytes - 16 * (size_t)n16);
-    hipLaunchKernelGGL(k_zero, dim3((unsigned)std::max<int64_t>(1, std::min<int64_t>((n16 + BLOCK - 1) / BLOCK, 2048))),
-                       dim3(BLOCK), 0, s, (uint4*)p, n16, (unsigned char*)p + 16 * n16, ntail);
+    if (!L.n) return CM_OK;
+    int64_t n16 = 1;
+    for (int r = 0; r < L.n; r++) n16 = std::max(n16, L.bytes[r] >> 4);
+    hipLaunchKernelGGL(k_fill, dim3((unsigned)std::min<int64_t>((n16 + BLOCK - 1) / BLOCK, 2048)), dim3(BLOCK), 0, s, L);
     HIPCHK(hipGetLastError());
     return CM_OK;
 }
@@ -5119,7 +5134,6 @@ void launch_cl_prep(hipStream_t s, const KP& P, const Bufs& B, const void* xu, c
     const int64_t M = P.self_ ? P.Mu : std::max(P.Mu, P.Mv);
     const unsigned gm = (unsigned)((M + BLOCK - 1) / BLOCK);
     hipLaunchKernelGGL(k_cl_keys<T>, dim3(std::min(gm, 64u), F, sides), dim3(BLOCK), 0, s, P, B, (const T*)xu, (const T*)xv);
-    hipLaunchKernelGGL(k_grid, dim3(1), dim3(64), 0, s, P, B, 1);
     hipLaunchKernelGGL(k_cl_scan, dim3(F, sides), dim3(1024), 0, s, P, B);
     hipLaunchKernelGGL(k_cl_order, dim3(grid_for(M * F), sides), dim3(BLOCK), 0, s, P, B);
     const unsigned gb = (unsigned)std::max(P.nS, (P.nB + BLOCK / 64 - 1) / (BLOCK / 64));
@@ -5196,6 +5210,7 @@ int run_batch(cm_job* J, int F, const int64_t* frame_index, const void* xu_dev, 
         hipLaunchKernelGGL(k_vrec_init, dim3(grid_for(nrec)), dim3(BLOCK), 0, s, B.vrec, nrec);
     }
 
+    FillList fills;
     // random draws of the reference solute molecules (mddf_frame!, src/mddf.jl:374-376);
     // with one solute molecule every draw is molecule 0
     if (!tiles && J->K > 0) {
@@ -5221,16 +5236,19 @@ int run_batch(cm_job* J, int F, const int64_t* frame_index, const void* xu_dev, 
         HIPCHK(hipMemcpyAsync(J->drawn_ptr.p, J->hdp.data(), sizeof(int) * J->hdp.size(), hipMemcpyHostToDevice, s));
         HIPCHK(hipMemcpyAsync(J->drawn_idx.p, J->hdi.data(), sizeof(int) * J->hdi.size(), hipMemcpyHostToDevice, s));
     } else if (J->K > 0) {
-        if (int r = zero_async(J->uk.p, sizeof(int) * (size_t)F * J->K, s)) return r;
+        fills.add(J->uk.p, sizeof(int) * (size_t)F * J->K);
     }
     if (P.rpm) {
         const size_t zero = cl_layout(P, F, (char*)J->clmem.p, &B);
-        if (int r = zero_async(J->clmem.p, zero, s)) return r;
-    } else if (int r = zero_async(J->cells_cnt.p, sizeof(int) * (size_t)F * (cap + 1), s)) return r;
+        fills.add(J->clmem.p, zero);
+    } else fills.add(J->cells_cnt.p, sizeof(int) * (size_t)F * (cap + 1));
     if (tiles) {
-        if (int r = zero_async(J->near.p, near_bytes(F, cap), s)) return r;
-        if (int r = zero_async(J->mcnt.p, key_bytes(P, F), s)) return r;
+        fills.add(J->near.p, near_bytes(F, cap));
+        fills.add(J->mcnt.p, key_bytes(P, F));
+        // the bulk flags' start (k_bulk_init without a molecule to leave out)
+        if (P.K > 0) fills.add(J->bflag.p, (size_t)F * P.kb * P.Mv, P.usecutoff ? 0u : 0x01010101u);
     }
+    if (int r = fill_async(fills, s)) return r;
 
     const bool f32 = dtype == CM_F32;
     const float* uf = (const float*)xu_dev;
@@ -5259,7 +5277,6 @@ int run_batch(cm_job* J, int F, const int64_t* frame_index, const void* xu_dev, 
             else hipLaunchKernelGGL(k_radii<double>, gr, dim3(BLOCK), 0, s, P, B, ud, vd, mols);
         }
     }
-    if (!P.rpm) hipLaunchKernelGGL(k_grid, dim3(1), dim3(64), 0, s, P, B, mols);
     if (P.rpm) {
         if (f32) launch_cl_prep<float>(s, P, B, xu_dev, xv_dev);
         else launch_cl_prep<double>(s, P, B, xu_dev, xv_dev);
@@ -5276,7 +5293,7 @@ int run_batch(cm_job* J, int F, const int64_t* frame_index, const void* xu_dev, 
         hipLaunchKernelGGL(k_scan_cells, dim3(F), dim3(1024), 0, s, P, B);
         hipLaunchKernelGGL(k_scatter, dim3(grid_for((int64_t)F * B.nitems)), dim3(BLOCK), 0, s, P, B, B.nitems);
         if (tiles) {
-            hipLaunchKernelGGL(k_near_mark, dim3((P.nu + BLOCK - 1) / BLOCK, std::min(F, 65535)), dim3(BLOCK), 0, s, P, B);
+            hipLaunchKernelGGL(k_near_mark, dim3(near_blocks(P.nu), std::min(F, 65535)), dim3(BLOCK), 0, s, P, B);
             hipLaunchKernelGGL(k_dfield, dim3(grid_for((int64_t)F * cap * 16)), dim3(BLOCK), 0, s, P, B);
             int64_t n = (int64_t)F * P.Mv;
             if (f32) hipLaunchKernelGGL(k_prep_solvent_tiles<float>, dim3(grid_for(n)), dim3(BLOCK), 0, s, P, B, vf);
@@ -5292,7 +5309,7 @@ int run_batch(cm_job* J, int F, const int64_t* frame_index, const void* xu_dev, 
             else hipLaunchKernelGGL(k_prep_solvent<double>, dim3(grid_for(n)), dim3(BLOCK), 0, s, P, B, vd);
         }
     }
-    if (P.K > 0) hipLaunchKernelGGL(k_bulk_init, dim3(grid_for((int64_t)F * P.kb * P.Mv)), dim3(BLOCK), 0, s, P, B);
+    if (P.K > 0 && !tiles) hipLaunchKernelGGL(k_bulk_init, dim3(grid_for((int64_t)F * P.kb * P.Mv)), dim3(BLOCK), 0, s, P, B);
     HIPCHK(hipGetLastError());
     // real pass
     if (J->profiling) HIPCHK(hipEventRecord(ev[0], s));
@@ -5356,10 +5373,9 @@ int run_batch(cm_job* J, int F, const int64_t* frame_index, const void* xu_dev, 
         }
         if (J->profiling) HIPCHK(hipEventRecord(ev[3], s));
     }
-    // geometry errors detected on the device: kept in the job's error bits and
-    // reported when the job is collected, so the host does not wait for the
-    // batch here and prepares the next one while it runs
-    hipLaunchKernelGGL(k_geo_flags, dim3(1), dim3(64), 0, s, P, B);
+    // (geometry errors detected on the device are in the job's error bits and
+    // reported when the job is collected: the host does not wait for the batch
+    // here and prepares the next one while it runs)
     HIPCHK(hipGetLastError());
     J->frames += F;
     if (J->verify) return verify_collect(J, F, frame_index);
@@ -5709,10 +5725,12 @@ int job_setup(cm_job* J, const cm_job_desc& d)
     if ((r = ensure(J, J->acc, 8 * J->acc_len))) return r;
     if ((r = ensure(J, J->hits, 8 * 4 * nb))) return r;
     if ((r = ensure(J, J->stats, 64))) return r;
-    if ((r = zero_async(J->cnt.p, 8 * J->acc_len, J->stream))) return r;
-    if ((r = zero_async(J->acc.p, 8 * J->acc_len, J->stream))) return r;
-    if ((r = zero_async(J->hits.p, 8 * 4 * nb, J->stream))) return r;
-    if ((r = zero_async(J->stats.p, 64, J->stream))) return r;
+    FillList fills;
+    fills.add(J->cnt.p, 8 * J->acc_len);
+    fills.add(J->acc.p, 8 * J->acc_len);
+    fills.add(J->hits.p, 8 * 4 * nb);
+    fills.add(J->stats.p, 64);
+    if ((r = fill_async(fills, J->stream))) return r;
     // The page-locked read-back buffer is taken now, while the device is idle
     // for this job: page-locking tens of MB (hipHostMalloc) while the job's
     // kernels run stalled one of them about fourfold (a 2.4 ms evaluation took
@@ -5750,7 +5768,7 @@ int job_setup(cm_job* J, const cm_job_desc& d)
     return CM_OK;
 }
 
-// The geometry error bits a job's batches left on the device (k_geo_flags):
+// The geometry error bits a job's batches left on the device (frame_grid):
 // bit 0 molecules too large for the cell of the molecule-pair kernels, bit 1
 // a cell grid larger than its allocation.  The same decoding for cm_job_finish
 // and for the request server.
@@ -6543,7 +6561,6 @@ constexpr int MS_FMAX = 48;        // frames of one job per round (the single-jo
 // of 2048 took 1.8x the single-job launches' time in the near placement).
 constexpr int MG_256 = 32768;      // blocks of the 256-thread stage launches
 constexpr int MG_1024 = 4096;      // blocks of the 1024-thread stage launches
-constexpr int MG_64 = 1024;        // blocks of the 64-thread stage launches
 constexpr int MG_RES = 4096;       // blocks of the resolve launches
 constexpr int64_t MULTI_BUDGET = (int64_t)64 << 30;   // batch buffers of one submission's jobs together
 
@@ -6627,7 +6644,6 @@ void multi_launch(hipStream_t s, const MultiTab* tab, int hist, int lds_max, int
     const int g_rand = persistent_grid(ev_rand, 64 * w_rand, shm_r, cus);
     hipLaunchKernelGGL(km_zero, dim3(MG_256), dim3(BLOCK), 0, s, tab);
     hipLaunchKernelGGL(km_radii<T>, dim3(MG_256), dim3(BLOCK), 0, s, tab);
-    hipLaunchKernelGGL(km_grid, dim3(MG_64), dim3(64), 0, s, tab);
     hipLaunchKernelGGL(km_wrap_atoms<T>, dim3(MG_256), dim3(BLOCK), 0, s, tab);
     hipLaunchKernelGGL(km_scan_cells, dim3(MG_1024), dim3(1024), 0, s, tab);
     hipLaunchKernelGGL(km_scatter, dim3(MG_256), dim3(BLOCK), 0, s, tab);
@@ -6652,7 +6668,6 @@ void multi_launch(hipStream_t s, const MultiTab* tab, int hist, int lds_max, int
     hipLaunchKernelGGL(km_chunk_table<true>, dim3(MG_1024), dim3(1024), 0, s, tab);
     hipLaunchKernelGGL(ev_rand, dim3(g_rand), dim3(64 * w_rand), shm_r, s, tab, ctr + 1);
     hipLaunchKernelGGL((km_resolve<T, double, true>), dim3(MG_RES), dim3(BLOCK), 0, s, tab);
-    hipLaunchKernelGGL(km_geo_flags, dim3(MG_64), dim3(64), 0, s, tab);
 }
 
 // groups of molecules per wavefront of the jobs of a variant (multi_variant)
@@ -6708,11 +6723,10 @@ void stage_blocks(const KP& P, int F, const int64_t z16[3], int nbx[MS_N], int c
     const int K = P.K;
     set(MS_ZERO, std::min<int64_t>(1024, std::max<int64_t>(1, (z16[0] + z16[1] + z16[2] + BLOCK - 1) / BLOCK)), 1);
     set(MS_RADII, std::min<int64_t>(mvb, 64), F);
-    set(MS_GRID, (F + 63) / 64, 1);
     set(MS_WRAP, grid_for((int64_t)F * P.nu), 1);
     set(MS_SCAN_CELLS, F, 1);
     set(MS_SCATTER, grid_for((int64_t)F * P.nu), 1);
-    set(MS_NEAR, (P.nu + BLOCK - 1) / BLOCK, std::min(F, 65535));
+    set(MS_NEAR, near_blocks(P.nu), std::min(F, 65535));
     set(MS_DFIELD, grid_for((int64_t)F * P.cap * 16), 1);
     set(MS_PREP, grid_for((int64_t)F * P.Mv), 1);
     const int p0 = scan_parts(P.kcap), pk = scan_parts(P.kcapr);
@@ -6732,7 +6746,6 @@ void stage_blocks(const KP& P, int F, const int64_t z16[3], int nbx[MS_N], int c
     set(MS_CHUNKK, 1, K > 0 ? 1 : 0);
     set(MS_RESOLVE0, resolve_parts(P, false), F);
     set(MS_RESOLVEK, K > 0 ? resolve_parts(P, true) : 1, K > 0 ? F * P.NG : 0);
-    set(MS_GEO_FLAGS, 1, 1);
 }
 
 // the rounds of one group of jobs that share the kernel variant
