@@ -146,7 +146,7 @@ struct KP {                  // job parameters, by value
     // molecule pairs on the matrix cores: rows per solute molecule in an A
     // tile (0: not used); A tiles, super tiles and B clusters per frame
     int rpm, nT, nS, nB;
-    int place_all;           // molecule-pair family: place every slot of a random pass (verification)
+    int place_all;           // verification: every slot of a random pass placed (molecule pairs), FP64 positions kept (tiles)
 };
 
 // MinimumDistance record as the verification getters return it
@@ -1723,6 +1723,20 @@ struct MolSrc {
     __device__ double operator()(int a, int k) const { return (double)p[3 * a + k]; }
 };
 
+// the same of three atoms, read once (with a constant count random_move's loops
+// unroll, and the wrapped positions that it forms twice are formed once)
+template <class TV>
+struct MolSrc3 {
+    TV x[9];
+    __device__ MolSrc3(const TV* q)
+    {
+        const gptr<const TV> p = (gptr<const TV>)q;
+#pragma unroll
+        for (int k = 0; k < 9; k++) x[k] = p[k];
+    }
+    __device__ double operator()(int a, int k) const { return (double)(a == 0 ? x[k] : (a == 1 ? x[3 + k] : x[6 + k])); }
+};
+
 struct MolDst {
     gptr<double> p;
     float4* w;   // (k_eval_mols_rand reads these in the same thread)
@@ -1739,15 +1753,23 @@ struct MolDstFix {
     gptr<double> p;
     gptr<f4v> w;
     const Geo& g;
-    __device__ MolDstFix(double* q, float4* v, const Geo& geo) : p((gptr<double>)q), w((gptr<f4v>)v), g(geo) {}
+    bool keep;   // the FP64 positions too
+    __device__ MolDstFix(double* q, float4* v, const Geo& geo, bool k) : p((gptr<double>)q), w((gptr<f4v>)v), g(geo), keep(k) {}
     __device__ void operator()(int a, double x, double y, double z) const
     {
-        p[3 * a] = x; p[3 * a + 1] = y; p[3 * a + 2] = z;
+        if (keep) { p[3 * a] = x; p[3 * a + 1] = y; p[3 * a + 2] = z; }
         const float4 u = fix_point(g, x, y, z, 0.f);
         w[a] = f4v{u.x, u.y, u.z, 0.f};
     }
     // the first atom's fourth component
     __device__ void set_w0(float x) const { ((gptr<float>)w)[3] = x; }
+};
+
+// the FP64 positions alone
+struct MolDst64 {
+    gptr<double> p;
+    __device__ MolDst64(double* q) : p((gptr<double>)q) {}
+    __device__ void operator()(int a, double x, double y, double z) const { p[3 * a] = x; p[3 * a + 1] = y; p[3 * a + 2] = z; }
 };
 
 // Whether placed slot v (centre cv) can have an atom pair with the drawn
@@ -2538,8 +2560,31 @@ __global__ void k_place_keys(KP P, Bufs B)
     b_place_keys(P, B, tab, blockIdx.x, gridDim.x, blockIdx.y, gridDim.y);
 }
 
-// second half: the placement of the near slots, written in sorted order (FP64
-// for the exact resolve, FP32 for the evaluation)
+// The random move of slot v of pass k (randomize_solvent!, src/mddf.jl:65-88):
+// source molecule, new centre and turns
+template <class TV>
+struct SlotMove {
+    const TV* x;
+    double uc[3], ua[3];
+    template <class GEO>
+    __device__ SlotMove(const KP& P, const Bufs& B, const GEO& g, const TV* xv, int f, int k, int v)
+    {
+        const cm::u32x4 r = cm::philox4x32_10({(uint32_t)v, (uint32_t)k, g.frame, cm::TAG_SLOT}, P.key0, P.key1);
+        const cm::u32x4 r2 = cm::philox4x32_10({(uint32_t)v, (uint32_t)k, g.frame, cm::TAG_SLOT + 1u}, P.key0, P.key1);
+        const int64_t lk = (int64_t)f * P.kb;
+        const int nb = ldg(B.nbulk + lk);
+        const int64_t jmol = nb > 0 ? (int64_t)ldg(B.blist + lk * P.Mv + cm::draw_index(r.x, nb)) : cm::draw_index(r.x, P.Mv);
+        x = xv + (int64_t)f * P.Nv * 3 + jmol * P.nv * 3;
+        uc[0] = cm::u01(r.y); uc[1] = cm::u01(r.z); uc[2] = cm::u01(r.w);
+        ua[0] = cm::u01(r2.x); ua[1] = cm::u01(r2.y); ua[2] = cm::u01(r2.z);
+    }
+};
+
+// second half: the placement of the near slots, written in sorted order in
+// fixed point.  Their FP64 positions are kept for verification only: k_resolve
+// forms them again for the few molecules it looks at (72 of 120 bytes a water,
+// in strided stores: 40,000 waters, 40 frames of 10 passes 282 us -> 171 us with
+// the atoms of three-atom molecules read once; 8-atom molecules 601 -> 294 us).
 template <class TV>
 __device__ __forceinline__ void b_place_near(KP P, Bufs B, const TV* xv, int bx_, int nbx_, int by_, int nby_)
 {
@@ -2553,27 +2598,24 @@ __device__ __forceinline__ void b_place_near(KP P, Bufs B, const TV* xv, int bx_
         const int kk = slot / P.Mv, v = slot - kk * P.Mv, k = grp * P.KM + kk;
         const int64_t at = ((int64_t)f * P.K + (int64_t)grp * P.KM) * P.Nv + (int64_t)pos * P.nv;
         const Geo g = ldc_geo(B.geo + f);
-        cm::u32x4 r = cm::philox4x32_10({(uint32_t)v, (uint32_t)k, g.frame, cm::TAG_SLOT}, P.key0, P.key1);
-        cm::u32x4 r2 = cm::philox4x32_10({(uint32_t)v, (uint32_t)k, g.frame, cm::TAG_SLOT + 1u}, P.key0, P.key1);
-        int64_t lk = (int64_t)f * P.kb;
-        int nb = ldg(B.nbulk + lk);
-        int64_t jmol = nb > 0 ? (int64_t)ldg(B.blist + lk * P.Mv + cm::draw_index(r.x, nb)) : cm::draw_index(r.x, P.Mv);
-        MolSrc<TV> src(xv + (int64_t)f * P.Nv * 3 + jmol * P.nv * 3);
-        MolDstFix dst(B.P + 3 * at, B.vw_r + at, g);
-        double uc[3] = {cm::u01(r.y), cm::u01(r.z), cm::u01(r.w)};
-        double ua[3] = {cm::u01(r2.x), cm::u01(r2.y), cm::u01(r2.z)};
+        const SlotMove<TV> mv(P, B, g, xv, f, k, v);
+        MolDstFix dst(B.P + 3 * at, B.vw_r + at, g, P.place_all != 0);
         // the placed centre is H uc (a rigid copy of a molecule of the frame):
         // the first atom's w carries the molecule's nearest-solute bound
         int cell, c0, c1, c2;
-        cell_of_frac(g, uc[0], uc[1], uc[2], cell, c0, c1, c2);
-        const float ub = molecule_bound(g, bound_loads(P, B, g, f, cell, c0, c1, c2), c0, c1, c2, uc);
-        cm::random_move(src, dst, P.nv, P.iref, g.cell, uc, ua);
+        cell_of_frac(g, mv.uc[0], mv.uc[1], mv.uc[2], cell, c0, c1, c2);
+        const float ub = molecule_bound(g, bound_loads(P, B, g, f, cell, c0, c1, c2), c0, c1, c2, mv.uc);
+        if (P.nv == 3) {
+            cm::random_move(MolSrc3<TV>(mv.x), dst, 3, P.iref, g.cell, mv.uc, mv.ua);
+        } else {
+            cm::random_move(MolSrc<TV>(mv.x), dst, P.nv, P.iref, g.cell, mv.uc, mv.ua);
+        }
         dst.set_w0(ub);
     }
 }
 
 template <class TV>
-__global__ void k_place_near(KP P, Bufs B, const TV* xv)
+__global__ void __launch_bounds__(BLOCK) k_place_near(KP P, Bufs B, const TV* xv)
 {
     b_place_near<TV>(P, B, xv, blockIdx.x, gridDim.x, blockIdx.y, gridDim.y);
 }
@@ -3300,7 +3342,7 @@ __global__ void __launch_bounds__(1024) k_eval_tiles(KP P, Bufs B, const TU* xu,
 constexpr int RES_CHUNKS = 64;
 
 template <class TU, class TV, bool RANDOM, bool VERIFY>
-__device__ __forceinline__ void resolve_one(const KP& P, const Bufs& B, const TU* xu, const TV* xv, int f, int64_t row,
+__device__ __forceinline__ void resolve_one(const KP& P, const Bufs& B, const TU* xu, const TV* xv, int f, int grp, int64_t row,
                                             int64_t atom, int pos)
 {
     // pos: sorted position in the row (the same in the 16 lanes), -1: none
@@ -3317,13 +3359,24 @@ __device__ __forceinline__ void resolve_one(const KP& P, const Bufs& B, const TU
         slot = ldg(B.msorted + row + pos);
         v = RANDOM ? slot - (slot / P.Mv) * P.Mv : slot;
         jbase = v * P.nv;
+        double* const yp = B.P + 3 * (atom + (int64_t)pos * P.nv);
+        if (RANDOM && !P.place_all) {
+            // the molecule's FP64 positions, by one lane (k_place_near's move)
+            if (sub == 0) {
+                MolDst64 dst(yp);
+                const SlotMove<TV> mv(P, B, B.geo[f], xv, f, grp * P.KM + slot / P.Mv, (int)v);
+                cm::random_move(MolSrc<TV>(mv.x), dst, P.nv, P.iref, B.geo[f].cell, mv.uc, mv.ua);
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+            __builtin_amdgcn_wave_barrier();
+        }
         const float w0 = vg[0].w, w1 = P.nv > 1 ? vg[1].w : w0;
         for (int a = sub >> 2; a < P.nv; a += 4) {
             const f4v y = vg[a];
             const bool isref = a == P.iref;
             const float R2 = isref ? fmaxf(w0, w1) : w0;
             double y0, y1, y2;
-            if (RANDOM) load3(B.P + 3 * (atom + (int64_t)pos * P.nv), a, y0, y1, y2);
+            if (RANDOM) load3((const double*)yp, a, y0, y1, y2);
             else load3(xv + (int64_t)f * P.Nv * 3, jbase + a, y0, y1, y2);
             const int ux = __float_as_int(y.x), uy = __float_as_int(y.y), uz = __float_as_int(y.z);
             const float rr_ = __builtin_amdgcn_sqrtf(R2) * (1.0f + 1e-5f) + 1e-3f;
@@ -3407,7 +3460,7 @@ __device__ __forceinline__ void b_resolve(const KP& P, const Bufs& B, const TU* 
             const int n = nlist;
             for (int k = 0; k < n; k += BLOCK / 16) {
                 const int q = k + (threadIdx.x >> 4);
-                resolve_one<TU, TV, RANDOM, VERIFY>(P, B, xu, xv, f, row, atom, q < n ? list[q] : -1);
+                resolve_one<TU, TV, RANDOM, VERIFY>(P, B, xu, xv, f, grp, row, atom, q < n ? list[q] : -1);
             }
             __syncthreads();
         }
@@ -4966,10 +5019,10 @@ void launch_tiles_any(bool f32, bool random, hipStream_t s, int grid, const cm_j
                       const void* xu, const void* xv)
 {
     if (f32) {
-        if (random) launch_tiles<float, double, true>(s, grid, J, P, B, xu, nullptr);
+        if (random) launch_tiles<float, float, true>(s, grid, J, P, B, xu, xv);
         else launch_tiles<float, float, false>(s, grid, J, P, B, xu, xv);
     } else {
-        if (random) launch_tiles<double, double, true>(s, grid, J, P, B, xu, nullptr);
+        if (random) launch_tiles<double, double, true>(s, grid, J, P, B, xu, xv);
         else launch_tiles<double, double, false>(s, grid, J, P, B, xu, xv);
     }
 }
@@ -5360,7 +5413,7 @@ int run_batch(cm_job* J, int F, const int64_t* frame_index, const void* xu_dev, 
         HIPCHK(hipGetLastError());
         if (J->profiling) HIPCHK(hipEventRecord(ev[2], s));
         if (tiles) {
-            launch_tiles_any(f32, true, s, J->eval_grid, J, P, B, xu_dev, nullptr);
+            launch_tiles_any(f32, true, s, J->eval_grid, J, P, B, xu_dev, xv_dev);
         } else {
             const int gwords = P.glds ? P.nbins * (P.gnu + (P.self_ ? 0 : P.gnv)) : 0;
             const size_t shr = sizeof(unsigned) * (2 * P.nbins + gwords);
@@ -6631,7 +6684,7 @@ template <class T, int TQ, int G, int GR>
 void multi_launch(hipStream_t s, const MultiTab* tab, int hist, int lds_max, int cus)
 {
     auto ev_real = km_eval_tiles<T, T, false, G, TQ>;
-    auto ev_rand = km_eval_tiles<T, double, true, GR, TQ>;
+    auto ev_rand = km_eval_tiles<T, T, true, GR, TQ>;
     // (the chunk tables of multi_tickets are static LDS)
     auto waves = [&](int g) {
         return (int)std::max<int64_t>(1, std::min<int64_t>(16, (lds_max - 2048 - 4 * (int64_t)hist) / (4 * (int64_t)eval_wave_words(g, TQ))));
@@ -6667,7 +6720,7 @@ void multi_launch(hipStream_t s, const MultiTab* tab, int hist, int lds_max, int
     hipLaunchKernelGGL(km_place_near<T>, dim3(MG_256), dim3(BLOCK), 0, s, tab);
     hipLaunchKernelGGL(km_chunk_table<true>, dim3(MG_1024), dim3(1024), 0, s, tab);
     hipLaunchKernelGGL(ev_rand, dim3(g_rand), dim3(64 * w_rand), shm_r, s, tab, ctr + 1);
-    hipLaunchKernelGGL((km_resolve<T, double, true>), dim3(MG_RES), dim3(BLOCK), 0, s, tab);
+    hipLaunchKernelGGL((km_resolve<T, T, true>), dim3(MG_RES), dim3(BLOCK), 0, s, tab);
 }
 
 // groups of molecules per wavefront of the jobs of a variant (multi_variant)
