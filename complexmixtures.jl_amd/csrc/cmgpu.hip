@@ -1066,6 +1066,7 @@ __device__ Rec resolve_mols(const KP& P, const Geo& g, const TU* xuf, int u, int
 constexpr int QCAP = 128;
 constexpr int DCAP = 128;   // deferred FP64 entries per wavefront (self)
 constexpr int GLDS_MAX = 32 * 1024;   // bytes of LDS group counts per block
+constexpr int GLDS_MAX_CL = 64 << 10;   // the same of the molecule pairs on the matrix cores
 
 __device__ __forceinline__ int wave_max_i(int x)
 {
@@ -5756,7 +5757,11 @@ void job_params(cm_job* J, const cm_job_desc& d)
     P.gnu = d.n_groups_u;
     P.gnv = d.n_groups_v;
     // molecule-pair kernels keep the group counts in LDS when they fit
-    P.glds = (int64_t)d.nbins * (d.n_groups_u + (d.autocorrelation ? 0 : d.n_groups_v)) * 4 <= GLDS_MAX ? 1 : 0;
+    // (on the matrix cores the blocks are 16 wavefronts, one a CU, with 74 KB of
+    // queues, so the groups may take more than in the walk's small blocks; out
+    // of line, straight into the global counters, the groups of 14 + 3 atoms took
+    // 118 of 312 us: 181 osmolytes in 16,667 waters, 20 frames)
+    P.glds = (int64_t)d.nbins * (d.n_groups_u + (d.autocorrelation ? 0 : d.n_groups_v)) * 4 <= (P.rpm ? GLDS_MAX_CL : GLDS_MAX) ? 1 : 0;
     {
         int dev = 0;
         if (hipGetDevice(&dev) == hipSuccess)

@@ -89,3 +89,10 @@ def test_exact_ties(pkg, oracle):
     s = pkg.AtomSelection(list(range(1, 121)), nmols=40)
     traj = pkg.MemoryTrajectory(x, x, np.eye(3)[None] * 27.0, s, s)
     _check(pkg, oracle, traj, dbulk=8.0, n_random_samples=2, irefatom=2)
+
+
+@pytest.mark.parametrize("binstep", [0.02, 0.01, 0.005])
+def test_group_histograms_in_and_beyond_lds(pkg, oracle, binstep):
+    """17 groups of 400, 800 and 1,600 bins: 27, 54 and 109 kB, of which 64 kB may lie in LDS."""
+    traj = _traj(pkg, 14, 12, 3, 150, seed=8)
+    _check(pkg, oracle, traj, dbulk=8.0, binstep=binstep, n_random_samples=3)
