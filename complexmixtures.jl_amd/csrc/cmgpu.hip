@@ -109,7 +109,7 @@ struct Geo {                 // one frame of a batch
     // fixed-point fractional coordinates, 2^fix units per cell
     int fix;
     float Hfix[9];           // lattice vectors per unit (FP32)
-    float gd0, gd1, gd2;     // guard of a direct FP32 d2: gd0 + gd1 d + gd2 d2 (with the roundings of decide32)
+    float gd0, gd1, gd2;     // guard of a direct FP32 d2 but for the coordinates' rounding: gd0 + gd1 d + gd2 d2 (with decide32's)
     float rho;               // |error| of an FP32 difference of two fixed-point positions, in 2^-24 of its length
     float guard32;           // guard + (cutoff^2 + guard + 1) 2^-21, rounded up: covers FP32 b -+ guard32 rounding
 };
@@ -2930,11 +2930,12 @@ __device__ __forceinline__ void eval_chunk(const KP& P, const Bufs& B, const TU*
     // most 7 u (Y + S)^2.  Both widen the frame's guard for this chunk (FP32
     // here, every value rounded outward by the factors; S <= Y + the staging
     // radius, which is at most um + 0.3).  The columns hold -2 y' (exact scaling).
-    float Gcf, cut2_hi_c, amb_c;
+    float Gcf, cut2_hi_c, amb_c, gdir;   // gdir: the coordinates' rounding in a direct d^2, per d
     {
         const float Yb = __builtin_amdgcn_sqrtf(bx * bx + by * by + bz * bz) * (1.0f + 4e-6f) + 1e-3f;
         const float YS = 2.0f * Yb + fminf(rs_full, um + 0.3f) * (1.0f + 1e-5f) + 1e-3f;
         const float gd = 0x1p-24f * YS * (2.0f * g.rho * ((float)P.cutsys + 0.5f) + 7.0f * YS) * (1.0f + 1e-5f) + 1e-8f;
+        gdir = sgpr_f((g.gd1 + 0x1p-23f * g.rho * YS) * (1.0f + 1e-5f));
         Gcf = sgpr_f((g.guard_up + gd) * (1.0f + 1e-6f));
         cut2_hi_c = sgpr_f((P.c2hi32 + Gcf) * (1.0f + 1e-6f));
         amb_c = sgpr_f(2.0f * Gcf + cut2_hi_c * 0x1p-20f);
@@ -3199,12 +3200,12 @@ __device__ __forceinline__ void eval_chunk(const KP& P, const Bufs& B, const TU*
     Rec r = rec_zero();
     bool undec = false, amb = false;   // left to the FP64 resolve (amb: an argmin FP32 cannot separate)
     if (active) {
-        // a separated argmin decides with its direct d^2, whose guard is
-        // relative to d^2 itself: fixed-point units (E) and fix_cart's rounding
-        // of an exact integer difference, 2 rho + 4 rounding units, plus the
-        // roundings of decide32's own sums
+        // a separated argmin decides with its direct d^2, whose guard shrinks
+        // with d: fixed-point units (E) and the rounding of both positions
+        // about the chunk centre, 2 rho u (Y + S) (gdir), times d, plus 2 rho + 4
+        // units of d^2 and the roundings of decide32's own sums
         auto decide = [&](float d2, int& bn, int& bk) {
-            const float Gd = fmaf(g.gd2, d2, g.gd1 * __builtin_amdgcn_sqrtf(d2)) + g.gd0;
+            const float Gd = fmaf(g.gd2, d2, gdir * (__builtin_amdgcn_sqrtf(d2) * (1.0f + 1e-6f))) + g.gd0;
             return decide32(P, Gd, d2, bn, bk);
         };
         int bn, bk;

@@ -13,8 +13,8 @@ systems whose solute size is log-uniform over 200-20,000 atoms in cubic water
 boxes of 30-150 A, 10-200 frames per request, 30% with the ideal-gas reference
 passes (n_random_samples 10; the others are coordination-number requests) and
 20% self-MDDF (water vs water).  The autotuner picks the cell size and the
-tile (columns per row) of the single-solute kernels per system by timing
-them on a few frames.
+molecules per wavefront (columns) of the single-solute kernels per system by
+timing them on a few frames.
 """
 import hashlib
 import queue

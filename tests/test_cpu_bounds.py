@@ -148,3 +148,28 @@ def test_fixed_point_tile_distance_within_guard():
     direct = fma32(e[:, 0], e[:, 0], fma32(e[:, 1], e[:, 1], f32(e[:, 2] * e[:, 2]))).astype(np.float64)
     ratio = np.abs(direct - d2) / (fixed + 10.0 * U * d2 + 1e-9)
     assert 0.05 < ratio.max() <= 1.0, ratio.max()
+
+
+def test_direct_distance_guard_about_a_centre():
+    """The guard of a direct FP32 d^2 between two positions held relative to a
+    third one (each rounded once): fixed-point units and the coordinates'
+    rounding times d, rounding units times d^2; the fixed-point terms alone do
+    not cover short distances between positions far from the centre."""
+    import numpy as np
+    rng = np.random.default_rng(3)
+    box, fix, n = 48.0, 28, 200000
+    unit, u, rho = box * 2.0 ** -fix, 2.0 ** -24, 3.0
+    ctr = rng.integers(0, 1 << fix, size=(n, 3))
+    s = ctr + np.rint(rng.uniform(-14, 14, size=(n, 3)) / unit).astype(np.int64)
+    y = s + np.rint(rng.normal(size=(n, 3)) * rng.choice([0.05, 0.5, 4.0], size=(n, 1)) / unit).astype(np.int64)
+    h = np.float32(unit)
+    rel = [h * (p - ctr).astype(np.float32) for p in (s, y)]
+    d = (rel[1] - rel[0]).astype(np.float32)
+    d2 = (d[:, 0] * d[:, 0] + d[:, 1] * d[:, 1] + d[:, 2] * d[:, 2]).astype(np.float32)
+    exact = (((y - s) * unit) ** 2).sum(axis=1)
+    err = np.abs(d2.astype(np.float64) - exact)
+    S, Y = (np.linalg.norm((p - ctr) * unit, axis=1) for p in (s, y))
+    E, r = unit + 1e-9, np.sqrt(exact)
+    fixed = 3 * E * E + 1e-9 + 2 * np.sqrt(3) * E * r + (2 * rho + 4) * u * exact
+    assert (err <= fixed + 2 * rho * u * (S + Y) * r).all()
+    assert (err > fixed).any()
