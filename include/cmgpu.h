@@ -102,7 +102,7 @@ typedef struct cm_kernel_stats {
     int64_t total_launches;
     int64_t frames;             /* frames processed */
     int64_t candidate_pairs;    /* FP32 pair evaluations (when counting is on) */
-    int64_t fp64_rechecks;      /* molecules resolved with the exhaustive FP64 pass */
+    int64_t fp64_rechecks;      /* molecules (pairs) that FP32 left to the FP64 pass */
 } cm_kernel_stats;
 
 /* MinimumDistance record (src/minimum_distances.jl:12-19), as the
@@ -189,11 +189,11 @@ int cm_multi_stats(int64_t *rounds, int64_t *launches);
 
 /* Tuning of the single-solute kernels (no counterpart in the reference; the
  * reference's Options.lcell plays this role for CellListMap): fine cell side
- * as a fraction of the cutoff (0.2-1.0), columns per row of a wavefront (1, 2,
- * 4 or 8; a row is one solvent atom, or one whole molecule for 3-atom solvent
- * molecules; 0 keeps the default: 4 for 3-atom molecules, else 1) and
- * workgroups of the persistent evaluation kernel (0 = as many as the device
- * holds at once).  Results do not depend on these. */
+ * as a fraction of the cutoff (0.2-1.0), columns (1, 2, 4 or 8: 64 / columns
+ * solvent molecules per wavefront of the real pass, up to four times as many
+ * in the random passes; 0 keeps the default, 4) and workgroups of the
+ * persistent evaluation kernel (0 = as many as the device holds at once).
+ * Results do not depend on these. */
 int cm_job_set_tuning(cm_job *job, double cell_fraction, int32_t columns, int32_t eval_workgroups);
 
 /* Kernel timing of the job (HIP events on the job's stream, recorded around
