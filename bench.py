@@ -510,7 +510,7 @@ def main():
                      "traffic_note": f"HBM bytes per {frames_per_launch}-frame launch pair (real + random "
                                      "evaluation), from the counter summary in profiles/",
                      "algorithmic_bytes_per_launch": round(bpf * frames_per_launch),
-                     "kernel": "k_eval_tiles (real + random passes)", "pairs_per_frame": round(W),
+                     "kernel": "k_eval_tiles + k_resolve (real + random passes)", "pairs_per_frame": round(W),
                      "eval_ms_per_frame": round(st["eval_ms"] / nf, 5),
                      "eval_ms_job": round(st["eval_ms"], 3), "eval_launches_job": st["eval_launches"],
                      "timing": f"HIP events around every evaluation launch of the {args.steps} timed jobs",
