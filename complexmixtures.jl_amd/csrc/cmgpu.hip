@@ -3343,6 +3343,20 @@ __global__ void __launch_bounds__(1024) k_eval_tiles(KP P, Bufs B, const TU* xu,
 // whose registers and code it would double.
 constexpr int RES_CHUNKS = 64;
 
+// chunks a block of the resolve takes at a time: 64, in small launches as few
+// as give about a thousand blocks (34 frames of 50 chunks of ureas: 67 us a launch
+// with a block a frame, 55 so)
+__host__ __device__ __forceinline__ int64_t resolve_row_chunks(const KP& P, bool random)
+{
+    const int64_t mpt = random ? P.mpt_r : P.mpt;
+    return ((random ? (int64_t)P.KM : 1) * P.Mv + mpt - 1) / mpt;
+}
+__host__ __device__ __forceinline__ int resolve_step(const KP& P, bool random)
+{
+    const int64_t n = resolve_row_chunks(P, random) * P.F * (random ? P.NG : 1) / 1024;
+    return n < 2 ? 2 : (n > RES_CHUNKS ? RES_CHUNKS : (int)n);
+}
+
 template <class TU, class TV, bool RANDOM, bool VERIFY>
 __device__ __forceinline__ void resolve_one(const KP& P, const Bufs& B, const TU* xu, const TV* xv, int f, int grp, int64_t row,
                                             int64_t atom, int pos)
@@ -3432,24 +3446,24 @@ __device__ __forceinline__ void resolve_one(const KP& P, const Bufs& B, const TU
     }
 }
 
-// grid: x over the parts of a row (RES_CHUNKS chunks each), y over the rows
+// grid: x over the parts of a row (resolve_step chunks each), y over the rows
 template <class TU, class TV, bool RANDOM, bool VERIFY>
 __device__ __forceinline__ void b_resolve(const KP& P, const Bufs& B, const TU* xu, const TV* xv, int bx_, int nbx_, int by_,
                                           int nby_)
 {
     __shared__ int list[RES_CHUNKS * 64];
     __shared__ int nlist;
-    const int nr = RANDOM ? P.NG : 1, mpt = RANDOM ? P.mpt_r : P.mpt;
+    const int nr = RANDOM ? P.NG : 1, mpt = RANDOM ? P.mpt_r : P.mpt, step = resolve_step(P, RANDOM);
     for (int fq = by_; fq < P.F * nr; fq += nby_) {
         const int f = fq / nr, grp = fq - f * nr;
         const int c0 = ldg(B.chunk_base + fq), c1 = ldg(B.chunk_base + fq + 1);
         const int64_t row = row_base(P, f, RANDOM, grp);
         const int64_t atom = RANDOM ? ((int64_t)f * P.K + (int64_t)grp * P.KM) * P.Nv : (int64_t)f * P.Nv;
-        for (int cb = c0 + bx_ * RES_CHUNKS; cb < c1; cb += nbx_ * RES_CHUNKS) {
+        for (int cb = c0 + bx_ * step; cb < c1; cb += nbx_ * step) {
             // one wavefront lists the marked molecules' positions
             if (threadIdx.x < 64) {
                 const int ch = cb + threadIdx.x;
-                ull m = ch < c1 ? B.resmask[ch] : 0ull;
+                ull m = (int)threadIdx.x < step && ch < c1 ? B.resmask[ch] : 0ull;
                 const int n = __popcll(m), incl = wave_incl_scan(n);
                 int o = incl - n;
                 while (m) {
@@ -3476,12 +3490,11 @@ __global__ void __launch_bounds__(BLOCK, 3) k_resolve(KP P, Bufs B, const TU* xu
 }
 
 // parts of the resolve's grid along a row: about 2048 blocks in all, at most
-// one per RES_CHUNKS chunks
+// one per step of chunks
 int64_t resolve_parts(const KP& P, bool random)
 {
-    const int64_t rows = (int64_t)P.F * (random ? P.NG : 1), mpt = random ? P.mpt_r : P.mpt;
-    const int64_t chunks = ((random ? (int64_t)P.KM : 1) * P.Mv + mpt - 1) / mpt;
-    return std::max<int64_t>(1, std::min<int64_t>((chunks + RES_CHUNKS - 1) / RES_CHUNKS, 2048 / rows + 1));
+    const int64_t rows = (int64_t)P.F * (random ? P.NG : 1), step = resolve_step(P, random);
+    return std::max<int64_t>(1, std::min<int64_t>((resolve_row_chunks(P, random) + step - 1) / step, 2048 / rows + 1));
 }
 
 // ---------------------------------------------------------------------------
