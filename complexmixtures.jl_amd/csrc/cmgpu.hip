@@ -98,6 +98,7 @@ struct Geo {                 // one frame of a batch
     float rpre2;             // molecule-centre pre-check radius^2 (mols family)
     unsigned ru_bits, rv_bits;   // molecule radii (float bits, atomicMax)
     int err;                 // geometry the kernels cannot handle
+    unsigned voids;          // tiles family: solvent molecules without a position (b_prep_solvent_tiles)
     unsigned radii_done;     // blocks of the radii launch that have reported (the last one runs frame_grid)
     float rstage;            // staging radius around a chunk (cutoff + margin), tiles family
     float rnear;             // near-cell radius around a solute atom (cutoff + radius + margin)
@@ -381,6 +382,10 @@ __device__ __forceinline__ void wrap_point(const Geo& g, double x, double y, dou
     for (int k = 0; k < 3; k++) if (fr[k] >= 1.0) { fr[k] = 0.0; n[k] += 1.0; }
 }
 
+// whether wrapped coordinates are not numbers (NaN or infinite coordinates
+// make them NaN)
+__device__ __forceinline__ bool undefined3(const double fr[3]) { return fr[0] != fr[0] || fr[1] != fr[1] || fr[2] != fr[2]; }
+
 // fixed-point position of a point (FP64), not wrapped
 __device__ __forceinline__ float4 fix_point(const Geo& g, double x, double y, double z, float w)
 {
@@ -592,6 +597,13 @@ __device__ __forceinline__ void b_wrap_atoms(KP P, Bufs B, const T* xu, int bx_,
         int cell;
         cell_of_frac(g, fr[0], fr[1], fr[2], cell);
         int64_t o = (int64_t)f * B.nitems + i;
+        // (an atom with a coordinate that is no number has no fixed-point
+        // position and no distance: it stays out of the cells)
+        if (undefined3(fr)) {
+            B.tmp4[o] = fix4(0, 0, 0, __int_as_float(-1));
+            B.tmpcell[o] = -1;
+            continue;
+        }
         const double sc = ldexp(1.0, g.fix);
         B.tmp4[o] = fix4((int)rint(fr[0] * sc), (int)rint(fr[1] * sc), (int)rint(fr[2] * sc), __int_as_float(i));
         B.tmpcell[o] = cell;
@@ -691,6 +703,7 @@ __device__ __forceinline__ void b_scatter(KP P, Bufs B, int nper, int bx_, int n
         int e = (int)(it - (int64_t)f * nper);
         int64_t o = (int64_t)f * B.nitems + e;
         int cell = B.tmpcell[o];
+        if (cell < 0) continue;   // no position (b_wrap_atoms)
         int64_t cb = (int64_t)f * (P.cap + 1);
         int pos = B.start[cb + cell] + atomicAdd(&B.cnt[cb + cell], 1);
         B.sorted[(int64_t)f * B.nitems + pos] = B.tmp4[o];
@@ -1651,6 +1664,9 @@ __global__ void __launch_bounds__(BLOCK, 3) k_eval_mols_real(KP P, Bufs B, const
 // ---------------------------------------------------------------------------
 // bulk lists and random placement
 // ---------------------------------------------------------------------------
+// bulk flags: bit 0, in the bulk; bit 1 (tiles family), without a position
+constexpr unsigned char BULK_VOID = 2;
+
 __device__ __forceinline__ void b_bulk_init(KP P, Bufs B, int bx_, int nbx_, int by_, int nby_)
 {
     int64_t total = (int64_t)P.F * P.kb * P.Mv;
@@ -1691,7 +1707,7 @@ __device__ __forceinline__ void b_bulk_compact(KP P, Bufs B, int bx_, int nbx_, 
         const int v0 = base + 4 * threadIdx.x;
         int fl4[4];
 #pragma unroll
-        for (int u = 0; u < 4; u++) fl4[u] = v0 + u < P.Mv ? fl[v0 + u] : 0;
+        for (int u = 0; u < 4; u++) fl4[u] = v0 + u < P.Mv ? fl[v0 + u] & 1 : 0;
         const int cnt = fl4[0] + fl4[1] + fl4[2] + fl4[3];
         const int incl = wave_incl_scan(cnt);
         if (lane == 63) wsum[wid] = incl;
@@ -2091,6 +2107,7 @@ __device__ __forceinline__ void b_near_mark(KP P, Bufs B, int bx_, int nbx_, int
         for (int64_t e = bx_ * (int64_t)blockDim.x + threadIdx.x; e < (int64_t)P.nu * lanes; e += (int64_t)nbx_ * blockDim.x) {
             const int64_t at = e / lanes;
             const float4 u = B.tmp4[(int64_t)f * P.nu + at];
+            if (__float_as_int(u.w) < 0) continue;   // no position
             float4 s;
             fix_cart(g, __float_as_int(u.x), __float_as_int(u.y), __float_as_int(u.z), s.x, s.y, s.z);
             int ilo[3], ihi[3];
@@ -2305,9 +2322,17 @@ __device__ __forceinline__ void b_prep_solvent_tiles(KP P, Bufs B, const T* xv, 
         mol_centre(g, xv + (int64_t)f * P.Nv * 3, (int64_t)v * P.nv, P.nv, c);
         double fr[3], n[3];
         wrap_point(g, c[0], c[1], c[2], fr, n);
+        int64_t kb = (int64_t)f * P.NP * P.Mv + v;
+        if (undefined3(fr)) {
+            // no centre (an atom's coordinate is no number): the molecule and
+            // what is placed from it (b_place_keys) are within no cutoff
+            B.mkey[kb] = -1;
+            atomicOr(&B.geo[f].voids, 1u);
+            if (P.K > 0) B.bflag[(int64_t)f * P.kb * P.Mv + v] |= BULK_VOID;
+            continue;
+        }
         int cell, c0, c1, c2;
         cell_of_frac(g, fr[0], fr[1], fr[2], cell, c0, c1, c2);
-        int64_t kb = (int64_t)f * P.NP * P.Mv + v;
         if (!B.near[(int64_t)f * P.cap + cell]) { B.mkey[kb] = -1; continue; }
         const int key = hilbert_key(tab, g.kbits, c0, c1, c2);
         B.mkey[kb] = key;
@@ -2529,6 +2554,14 @@ __global__ void __launch_bounds__(1024) k_chunk_table(KP P, Bufs B, int random)
     b_chunk_table(P, B, random, blockIdx.x, gridDim.x, blockIdx.y, gridDim.y);
 }
 
+// the molecule of frame f that a slot with the draw r is placed from
+__device__ __forceinline__ int64_t slot_source(const KP& P, const Bufs& B, int f, uint32_t r)
+{
+    const int64_t lk = (int64_t)f * P.kb;
+    const int nb = ldg(B.nbulk + lk);
+    return nb > 0 ? (int64_t)ldg(B.blist + lk * P.Mv + cm::draw_index(r, nb)) : cm::draw_index(r, P.Mv);
+}
+
 // randomize_solvent! (src/mddf.jl:65-88), first half: the new centre of every
 // slot; slots whose centre falls in a near cell get the Hilbert key of the (half-)cell
 // (the others cannot have an atom within the cutoff of the solute)
@@ -2547,7 +2580,12 @@ __device__ __forceinline__ void b_place_keys(KP P, Bufs B, const unsigned* tab, 
         int c0, c1, c2;
         cell_of_draws(g, r.y, r.z, r.w, sub, c0, c1, c2);
         const int cell = ((c2 >> sub) * g.nc[1] + (c1 >> sub)) * g.nc[0] + (c0 >> sub);
-        if (!B.near[(int64_t)f * P.cap + cell]) { B.mkey[e] = -1; continue; }
+        // (a copy of a molecule without a position has none)
+        if (!B.near[(int64_t)f * P.cap + cell] ||
+            (g.voids && (B.bflag[(int64_t)f * P.kb * P.Mv + slot_source(P, B, f, r.x)] & BULK_VOID))) {
+            B.mkey[e] = -1;
+            continue;
+        }
         const int key = hilbert_key(tab, g.kbits + sub, c0, c1, c2);
         B.mkey[e] = key;
         B.mrank[e] = atomicAdd(&B.mcnt[key_row(P, f, 1 + grp) + key], 1);
@@ -2572,10 +2610,7 @@ struct SlotMove {
     {
         const cm::u32x4 r = cm::philox4x32_10({(uint32_t)v, (uint32_t)k, g.frame, cm::TAG_SLOT}, P.key0, P.key1);
         const cm::u32x4 r2 = cm::philox4x32_10({(uint32_t)v, (uint32_t)k, g.frame, cm::TAG_SLOT + 1u}, P.key0, P.key1);
-        const int64_t lk = (int64_t)f * P.kb;
-        const int nb = ldg(B.nbulk + lk);
-        const int64_t jmol = nb > 0 ? (int64_t)ldg(B.blist + lk * P.Mv + cm::draw_index(r.x, nb)) : cm::draw_index(r.x, P.Mv);
-        x = xv + (int64_t)f * P.Nv * 3 + jmol * P.nv * 3;
+        x = xv + (int64_t)f * P.Nv * 3 + slot_source(P, B, f, r.x) * P.nv * 3;
         uc[0] = cm::u01(r.y); uc[1] = cm::u01(r.z); uc[2] = cm::u01(r.w);
         ua[0] = cm::u01(r2.x); ua[1] = cm::u01(r2.y); ua[2] = cm::u01(r2.z);
     }
@@ -6721,13 +6756,13 @@ void multi_launch(hipStream_t s, const MultiTab* tab, int hist, int lds_max, int
     hipLaunchKernelGGL(km_scatter, dim3(MG_256), dim3(BLOCK), 0, s, tab);
     hipLaunchKernelGGL(km_near_mark, dim3(MG_256), dim3(BLOCK), 0, s, tab);
     hipLaunchKernelGGL(km_dfield, dim3(MG_256), dim3(BLOCK), 0, s, tab);
+    hipLaunchKernelGGL(km_bulk_init, dim3(MG_256), dim3(BLOCK), 0, s, tab);
     hipLaunchKernelGGL(km_prep_solvent_tiles<T>, dim3(MG_256), dim3(BLOCK), 0, s, tab);
     hipLaunchKernelGGL(km_scan_sums<false>, dim3(MG_1024), dim3(1024), 0, s, tab);
     hipLaunchKernelGGL(km_scan_rows<false>, dim3(MG_1024), dim3(1024), 0, s, tab);
     hipLaunchKernelGGL(km_mol_scatter<false>, dim3(MG_256), dim3(BLOCK), 0, s, tab);
     hipLaunchKernelGGL(km_fill_real<T>, dim3(MG_256), dim3(BLOCK), 0, s, tab);
     hipLaunchKernelGGL(km_chunk_table<false>, dim3(MG_1024), dim3(1024), 0, s, tab);
-    hipLaunchKernelGGL(km_bulk_init, dim3(MG_256), dim3(BLOCK), 0, s, tab);
     int* ctr = (int*)((char*)tab + MT_CTR_OFF);
     hipLaunchKernelGGL(ev_real, dim3(g_real), dim3(64 * w_real), shm, s, tab, ctr);
     hipLaunchKernelGGL((km_resolve<T, T, false>), dim3(MG_RES), dim3(BLOCK), 0, s, tab);
