@@ -132,6 +132,7 @@ struct KP {                  // job parameters, by value
     int64_t Nu, Nv;
     int mpt;                 // molecules per chunk of the real pass (tiles family)
     int mpt_r;               // the same of the random passes
+    int mpt_auto;            // chunks may be larger than that, as each launch chooses (b_chunk_table)
     int mol_lane;            // tiles family: 3-atom solvent molecules (their three atoms evaluated together)
     int glds;                // molecule-pair kernels: group counts privatised in LDS
     int gnu, gnv;            // group counts of the solute / solvent side
@@ -210,9 +211,10 @@ struct Bufs {
     int* msum;               // [F][parts of kcap | NG x parts of kcapr] molecules per part of a row's keys
     int* msorted;            // [F][NP][Mv] slots in key order
     int* nnear;              // [F][1 + NG]
-    ull* resmask;            // one word per chunk of a launch: molecules left to the FP64 resolve (over mkey,
-                             // whose keys the scatter has read by then)
-    int* chunk_base;         // [F*rows + 2] chunk offsets of one launch, total, evaluation chunk counter
+    unsigned* resmask;       // per chunk of a launch: molecules left to the FP64 resolve, one word, two in chunks of
+                             // more than 32 (over mkey, whose keys the scatter has read by then)
+    int* chunk_base;         // chunk offsets of one launch, [F*rows] total, evaluation chunk counter, [F*rows + MPT_AT]
+                             // molecules per chunk
     // molecule pairs on the matrix cores (self: one side)
     ClSide cl[2];
     float* clA;              // [F][nT][4][16] rows of the A tiles: x, y, z, squared norm
@@ -255,6 +257,15 @@ __device__ __forceinline__ Geo ldc_geo(const Geo* p)
     Geo g;
     __builtin_memcpy(&g, (__attribute__((address_space(4))) const Geo*)p, sizeof(Geo));
     return g;
+}
+
+// Molecules per chunk of a launch, as b_chunk_table left them: a scalar load, from
+// another cache line than the counter that the launch's wavefronts increment.
+constexpr int MPT_AT = 64;
+__device__ __forceinline__ int chunk_molecules(const KP& P, const Bufs& B, bool random)
+{
+    if (!P.mpt_auto) return random ? P.mpt_r : P.mpt;
+    return *(__attribute__((address_space(4))) const int*)(B.chunk_base + P.F * (random ? P.NG : 1) + MPT_AT);
 }
 
 // first entry of a row of the sorted molecules: the real pass or random group grp of frame f
@@ -2517,12 +2528,58 @@ __global__ void k_mol_scatter(KP P, Bufs B, int random)
     b_mol_scatter(P, B, random, blockIdx.x, gridDim.x, blockIdx.y, gridDim.y);
 }
 
-// chunk offsets of the real pass or the random groups of every frame (one block)
+// molecules of nv atoms that 64 lanes hold, one atom each
+__host__ __device__ __forceinline__ int lane_molecules(int nv) { return 64 / nv; }
+
+// Chunk offsets of the real pass or the random groups of every frame (one
+// block), and the molecules per chunk.  A chunk costs some 3,000 instructions
+// besides its distances (box, rows of cells, staging).  Near a compact solute its
+// few hundred staged atoms outweigh them, and small chunks (P.mpt, P.mpt_r) have
+// fewer; near an extended one (fewer than CHUNK_SPARSE solute atoms per cutoff^3
+// of the volume that the near molecules fill) chunks of up to 512 atoms share
+// them, as long as the launch keeps CHUNKS_REAL or CHUNKS_RANDOM chunks for its
+// 4,096 wavefronts.  12,000 eight-atom molecules around a chain of 3,000 atoms
+// (4.5 per cutoff^3), 20 frames: random passes 1,133 us with 16 molecules a chunk,
+// 708 with 64; real pass 251 with 8, 169 with 18.  2,570 around a globule of 1,000
+// (6.5), 12 frames of 10 passes: 504 us in all with 16, 574 with 55.
+constexpr double CHUNK_SPARSE = 5.5;
+constexpr int CHUNKS_REAL = 8192, CHUNKS_RANDOM = 4096;
+// molecules per chunk that would leave a launch its chunks, were all of them near
+__host__ __device__ __forceinline__ int64_t chunk_most(const KP& P, bool random)
+{
+    return (int64_t)P.F * (random ? P.K : 1) * P.Mv / (random ? CHUNKS_RANDOM : CHUNKS_REAL);
+}
+__host__ __device__ __forceinline__ bool chunks_vary(const KP& P)
+{
+    return P.mpt_auto && (chunk_most(P, false) > P.mpt || chunk_most(P, true) > P.mpt_r);
+}
+
+// (AUTO: for launches that chunks_vary lets choose; without, a microsecond less)
+template <bool AUTO>
 __device__ __forceinline__ void b_chunk_table(KP P, Bufs B, int random, int bx_, int nbx_, int by_, int nby_)
 {
     __shared__ int wsum[16];
     __shared__ int carry;
-    const int nr = random ? P.NG : 1, n = P.F * nr, mpt = random ? P.mpt_r : P.mpt;
+    const int nr = random ? P.NG : 1, n = P.F * nr;
+    int mpt = random ? P.mpt_r : P.mpt;
+    if (AUTO && P.mpt_auto && chunk_most(P, random != 0) > mpt) {
+        __shared__ double part[16];
+        double t = 0.0;
+        for (int idx = threadIdx.x; idx < n; idx += blockDim.x) {
+            const int f = idx / nr, r = random ? 1 + idx - f * nr : 0;
+            t += (double)B.nnear[(int64_t)f * (1 + P.NG) + r];
+        }
+        for (int o = 32; o >= 1; o >>= 1) t += __shfl_xor(t, o, 64);
+        if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = t;
+        __syncthreads();
+        t = 0.0;
+        for (int w = 0; w < (int)(blockDim.x >> 6); w++) t += part[w];
+        const double* H = B.geo[0].cell.H;
+        const double vol = fabs(cm::cell_volume(H));
+        const double dens = (double)P.nu * P.Mv * P.F * (random ? P.K : 1) / (vol * fmax(t, 1.0));
+        if (dens * P.cutsys * P.cutsys * P.cutsys < CHUNK_SPARSE)
+            mpt = max(mpt, min(min(64, 8 * lane_molecules(P.nv)), (int)(t / (random ? CHUNKS_RANDOM : CHUNKS_REAL))));
+    }
     if (threadIdx.x == 0) carry = 0;
     __syncthreads();
     int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
@@ -2546,12 +2603,14 @@ __device__ __forceinline__ void b_chunk_table(KP P, Bufs B, int random, int bx_,
     if (threadIdx.x == 0) {
         B.chunk_base[n] = carry;
         B.chunk_base[n + 1] = 0;   // the evaluation's chunk counter
+        B.chunk_base[n + MPT_AT] = mpt;
     }
 }
 
+template <bool AUTO>
 __global__ void __launch_bounds__(1024) k_chunk_table(KP P, Bufs B, int random)
 {
-    b_chunk_table(P, B, random, blockIdx.x, gridDim.x, blockIdx.y, gridDim.y);
+    b_chunk_table<AUTO>(P, B, random, blockIdx.x, gridDim.x, blockIdx.y, gridDim.y);
 }
 
 // the molecule of frame f that a slot with the draw r is placed from
@@ -2736,6 +2795,26 @@ __device__ __forceinline__ Min2 gather_groups(const Min2 (&m)[GH], int lane)
     return k;
 }
 
+// The same for four tiles of 16 columns: lane l ends with column l.
+__device__ __forceinline__ Min2 gather_columns(const Min2* m, int lane)
+{
+    auto recv = [&](Min2& keep, const Min2& send, int o) {
+        keep.merge(__shfl_xor(send.b, o, 64), __shfl_xor(send.s, o, 64), __shfl_xor(send.c, o, 64));
+    };
+    auto pick = [](bool hi, const Min2& x, const Min2& y) {
+        Min2 r;
+        r.b = hi ? y.b : x.b; r.s = hi ? y.s : x.s; r.c = hi ? y.c : x.c;
+        return r;
+    };
+    const bool h4 = (lane & 16) != 0, h5 = (lane & 32) != 0;
+    Min2 k0 = pick(h5, m[0], m[2]), k1 = pick(h5, m[1], m[3]);
+    recv(k0, pick(h5, m[2], m[0]), 32);
+    recv(k1, pick(h5, m[3], m[1]), 32);
+    Min2 k = pick(h4, k0, k1);
+    recv(k, pick(h4, k1, k0), 16);
+    return k;
+}
+
 // LDS of the evaluation: the block's histograms, the launch's chunk table,
 // then one area per wavefront
 extern __shared__ float dyn[];
@@ -2748,14 +2827,17 @@ __device__ __forceinline__ void wave_sync()
     __builtin_amdgcn_wave_barrier();
 }
 
-constexpr int TQ_GEN = 4;           // solvent atoms per block of tiles (molecules of any size)
+// Column tiles: TQ solvent atoms of 16 G molecules each (TQ = 3: molecules of
+// three atoms), or 16 G consecutive atoms (TQ = ATOMS: molecules of any size; G =
+// 4 or 8)
+constexpr int ATOMS = 0;
 constexpr int EV_ROWS = 32;         // staged atoms per step (two row tiles)
 constexpr int TCAP = 288;           // staged solute atoms per round (at least 256, a multiple of 32)
 constexpr int SEG = 4;              // staging: consecutive atoms per lane
 
 // words of a wavefront's area: staged components and indices, the columns of
-// one block of tiles (-2 y' and |y'|^2 per atom), the segments of one step
-__host__ __device__ constexpr int eval_wave_words(int G, int TQ) { return 5 * TCAP + 4 * TQ * 16 * G + 2 * 64; }
+// the tiles (-2 y' and |y'|^2 per atom), the segments of one step
+__host__ __device__ constexpr int eval_wave_words(int G, int TQ) { return 5 * TCAP + 4 * (TQ == ATOMS ? 1 : TQ) * 16 * G + 2 * 64; }
 
 // Block histograms.  Millions of records per launch go into a few hundred md
 // and rdf bins: as global atomics they bounded the launch (the random passes of
@@ -2838,19 +2920,19 @@ __device__ __forceinline__ void ev_hist_record(const KP& P, const Bufs& B, const
 // where a chunk of a launch lies: frame, random group, its row of the sorted
 // molecules, first molecule, molecules, first atom (B.vw / B.vw_r, B.P)
 struct ChunkAt {
-    int f, grp, m0, nm;
+    int f, grp, m0, nm, mpt;
     int64_t row, atom;
     template <class CB>
     __device__ ChunkAt(const KP& P, const Bufs& B, bool random, int ch, CB base)
     {
         const int nr = random ? P.NG : 1;
+        mpt = chunk_molecules(P, B, random);
         int lo = 0, hi = P.F * nr;
         while (hi - lo > 1) {
             const int mid = (lo + hi) >> 1;
             if (base(mid) <= ch) lo = mid; else hi = mid;
         }
         const int fq = __builtin_amdgcn_readfirstlane(lo);
-        const int mpt = random ? P.mpt_r : P.mpt;
         f = fq / nr;
         grp = fq - f * nr;
         m0 = __builtin_amdgcn_readfirstlane((ch - base(fq)) * mpt);
@@ -2861,14 +2943,19 @@ struct ChunkAt {
 };
 
 // Minimum distances of the solvent molecules of one chunk, one wavefront.  The
-// chunk's molecules (at most 16 G) are consecutive in the sorted order, so their
-// atoms are contiguous; TQ solvent atoms of every molecule are evaluated
-// together (all three of 3-atom molecules, blocks of four otherwise).  Records
+// chunk's molecules are consecutive in the sorted order, so their atoms are
+// contiguous.  Molecules of three atoms (TQ 3, at most 16 G of them): a column is
+// a molecule, its three atoms are evaluated together.  Others: a column is an
+// atom, and after the last round a lane holds one (two with eight tiles);
+// molecules do not cross from one 64 lanes to the next.  (A column per molecule
+// with four of its atoms at a time needs 16 molecules for full tiles: 16 of 40
+// atoms are a box of half the solute.  5,000 solute atoms, 760 such molecules, 8
+// frames of 10 passes: 2.60 ms so, 0.35 ms now, with the resolve.)  Records
 // that FP32 decides are counted here; the molecules it cannot decide (a bin
 // edge, the cutoff or dbulk within the guard, or an argmin closer than the
 // guard) are left to k_resolve: one bit each in the chunk's word of resmask, and
-// the squared radii that hold every candidate in the w of the molecule's first
-// two atoms.
+// in the w of each atom the squared radius that holds its candidates, negative
+// when it has none.
 //
 // What bounds it: per step of 32 staged atoms and 16 molecules a solvent atom
 // costs two matrix instructions (64 cycles) and 12 vector ones (48 cycles) that
@@ -2884,11 +2971,12 @@ __device__ __forceinline__ void eval_chunk(const KP& P, const Bufs& B, const TU*
     // + n % 16 (the order in which the lanes of a row tile read them), their
     // indices, the columns [atom of the block][-2 y'x, -2 y'y, -2 y'z, |y'|^2]
     // [molecule], the segments of a staging step
+    constexpr bool FLAT = TQ == ATOMS;
     constexpr int MC = 16 * G;
     float* const lds = dyn + wofs;
     int* const si = (int*)(lds + 4 * TCAP);
     float* const yb = lds + 5 * TCAP;
-    int2* const sd = (int2*)(yb + 4 * TQ * MC);
+    int2* const sd = (int2*)(yb + 4 * (FLAT ? 1 : TQ) * MC);
     // (opaque per chunk: what depends on the lane alone is formed where it is
     // used, not held in registers over the whole launch)
     int lane = threadIdx.x & 63;
@@ -2900,398 +2988,531 @@ __device__ __forceinline__ void eval_chunk(const KP& P, const Bufs& B, const TU*
     // lane that does
     const int ml = (G == 4 ? ((lane >> 4) & 1) << 5 : 0) + (G == 1 ? 0 : (lane >> 5) << 4) + (lane & 15);
     const bool lead = G == 4 || (G == 2 ? (lane & 16) == 0 : lane < 16);
-    const int f = at.f, nm = at.nm;
+    const int f = at.f;
     const GeoC& g = *(const GeoC*)(B.geo + f);
-    float4* vwb = (RANDOM ? B.vw_r : B.vw) + at.atom;   // the chunk's atoms
-    const int na = nm * P.nv;
-    const bool active = lead && ml < nm;
-    const int slot = ldg(B.msorted + at.row + at.m0 + min(ml, nm - 1));
-    // box of the chunk's atoms about an atom in their middle; the first
-    // atom's w is the molecule's bound
-    const gptr<const f4v> vg = (gptr<const f4v>)vwb;
-    const f4v mid = vg[(nm >> 1) * P.nv];
-    int cix = __builtin_amdgcn_readfirstlane(__float_as_int(mid.x)), ciy = __builtin_amdgcn_readfirstlane(__float_as_int(mid.y)),
-        ciz = __builtin_amdgcn_readfirstlane(__float_as_int(mid.z));
-    // position relative to the chunk's (integer) centre
-    auto rel = [&](f4v y, float& x_, float& y_, float& z_) {
-        fix_cart(g, __float_as_int(y.x) - cix, __float_as_int(y.y) - ciy, __float_as_int(y.z) - ciz, x_, y_, z_);
-    };
-    float alx = INFINITY, aly = INFINITY, alz = INFINITY, ahx = -INFINITY, ahy = -INFINITY, ahz = -INFINITY, um = 0.f;
-    auto box = [&](const f4v& y) {
-        float x_, y_, z_;
-        rel(y, x_, y_, z_);
-        alx = fminf(alx, x_); aly = fminf(aly, y_); alz = fminf(alz, z_);
-        ahx = fmaxf(ahx, x_); ahy = fmaxf(ahy, y_); ahz = fmaxf(ahz, z_);
-        um = fmaxf(um, y.w);
-    };
-    if (TQ == 3) {
-        // 3-atom molecules: at most 3 G / 4 loads per lane, together
-        f4v y[(3 * G + 3) / 4];
+    // FLAT: a block is once or twice 64 lanes, an atom each (molecules do not cross
+    // from one 64 to the next): the lane's molecule in its 64, its atom there.  A
+    // chunk of several blocks evaluates them one after the other from the same
+    // staged atoms; where those do not fit the buffer, each block stages its own.
+    constexpr int NL = G / 4 > 0 ? G / 4 : 1;
+    const int mpl = FLAT ? lane_molecules(P.nv) : 0, apl = mpl * P.nv;
+    const int lm = FLAT ? lane / P.nv : 0, la = lane - lm * P.nv;
+    const int H = FLAT ? (at.nm + NL * mpl - 1) / (NL * mpl) : 1;
+    unsigned long long um_ = 0;   // the molecules left open, one bit each in molecule order
+    int h0 = 0, nb = H;
+    while (h0 < H) {
+        nb = FLAT ? min(nb, H - h0) : 1;
+        const int mc = FLAT ? NL * h0 * mpl : 0, nm = FLAT ? min(at.nm - mc, NL * nb * mpl) : at.nm;   // molecules from mc on
+        float4* vwb = (RANDOM ? B.vw_r : B.vw) + at.atom + mc * P.nv;   // their atoms
+        const int na = nm * P.nv;
+        const bool active = lead && ml < nm;
+        const int slot = FLAT ? 0 : ldg(B.msorted + at.row + at.m0 + min(ml, nm - 1));
+        // box of the atoms about one in their middle; the first atom's w is the
+        // molecule's bound
+        const gptr<const f4v> vg = (gptr<const f4v>)vwb;
+        const f4v mid = vg[(nm >> 1) * P.nv];
+        int cix = __builtin_amdgcn_readfirstlane(__float_as_int(mid.x)), ciy = __builtin_amdgcn_readfirstlane(__float_as_int(mid.y)),
+            ciz = __builtin_amdgcn_readfirstlane(__float_as_int(mid.z));
+        // position relative to the chunk's (integer) centre
+        auto rel = [&](f4v y, float& x_, float& y_, float& z_) {
+            fix_cart(g, __float_as_int(y.x) - cix, __float_as_int(y.y) - ciy, __float_as_int(y.z) - ciz, x_, y_, z_);
+        };
+        float alx = INFINITY, aly = INFINITY, alz = INFINITY, ahx = -INFINITY, ahy = -INFINITY, ahz = -INFINITY, um = 0.f;
+        auto box = [&](const f4v& y) {
+            float x_, y_, z_;
+            rel(y, x_, y_, z_);
+            alx = fminf(alx, x_); aly = fminf(aly, y_); alz = fminf(alz, z_);
+            ahx = fmaxf(ahx, x_); ahy = fmaxf(ahy, y_); ahz = fmaxf(ahz, z_);
+            um = fmaxf(um, y.w);
+        };
+        if (FLAT) {
+            for (int e = lane; e < na; e += 256) {
+                f4v y[4];
 #pragma unroll
-        for (int t = 0; t < (3 * G + 3) / 4; t++) y[t] = vg[min(64 * t + lane, na - 1)];
+                for (int t = 0; t < 4; t++) y[t] = vg[min(e + 64 * t, na - 1)];
 #pragma unroll
-        for (int t = 0; t < (3 * G + 3) / 4; t++) box(y[t]);
-    } else {
-        for (int e = lane; e < na; e += 256) {
-            f4v y[4];
-#pragma unroll
-            for (int t = 0; t < 4; t++) y[t] = vg[min(e + 64 * t, na - 1)];
-#pragma unroll
-            for (int t = 0; t < 4; t++) box(y[t]);
-        }
-    }
-    um = wave_max(um);
-    // the centre moves to the middle of the box (in whole units: exact), the
-    // box with it (to FP32 rounding, inside the staging radius' slack)
-    float bx, by, bz;   // half sides
-    {
-        const float lx = wave_min(alx), ly = wave_min(aly), lz = wave_min(alz);
-        const float hx = wave_max(ahx), hy = wave_max(ahy), hz = wave_max(ahz);
-        const float mx = 0.5f * (lx + hx), my = 0.5f * (ly + hy), mz = 0.5f * (lz + hz);
-        bx = sgpr_f(0.5f * (hx - lx) + 1e-4f); by = sgpr_f(0.5f * (hy - ly) + 1e-4f); bz = sgpr_f(0.5f * (hz - lz) + 1e-4f);
-        const float sc = ldexpf(1.0f, g.fix);
-        cix += __builtin_amdgcn_readfirstlane((int)rintf((g.Hi32[0] * mx + g.Hi32[3] * my + g.Hi32[6] * mz) * sc));
-        ciy += __builtin_amdgcn_readfirstlane((int)rintf((g.Hi32[1] * mx + g.Hi32[4] * my + g.Hi32[7] * mz) * sc));
-        ciz += __builtin_amdgcn_readfirstlane((int)rintf((g.Hi32[2] * mx + g.Hi32[5] * my + g.Hi32[8] * mz) * sc));
-    }
-    const float rs_full = g.rstage;
-    // Distances relative to the chunk centre c (a fixed-point position, no
-    // rounding of its own): |y' - s'|^2 = (|s'|^2 - 2 y'.s') + |y'|^2.  With u =
-    // 2^-24, Y >= |y'| and S >= |s'| for every staged atom, y' and s' are off by
-    // at most rho u Y and rho u S (fix_cart), which moves d^2 by at most
-    // 2 rho u (Y + S) d (d <= cutsys + 0.5 where it matters); the norms (3 u S^2,
-    // 3 u Y^2), the four products and three additions of a tile in whatever
-    // order (2 u Y S + 3 u (S^2 + 2 Y S)) and the last sum (u (Y + S)^2) add at
-    // most 7 u (Y + S)^2.  Both widen the frame's guard for this chunk (FP32
-    // here, every value rounded outward by the factors; S <= Y + the staging
-    // radius, which is at most um + 0.3).  The columns hold -2 y' (exact scaling).
-    float Gcf, cut2_hi_c, amb_c, gdir;   // gdir: the coordinates' rounding in a direct d^2, per d
-    {
-        const float Yb = __builtin_amdgcn_sqrtf(bx * bx + by * by + bz * bz) * (1.0f + 4e-6f) + 1e-3f;
-        const float YS = 2.0f * Yb + fminf(rs_full, um + 0.3f) * (1.0f + 1e-5f) + 1e-3f;
-        const float gd = 0x1p-24f * YS * (2.0f * g.rho * ((float)P.cutsys + 0.5f) + 7.0f * YS) * (1.0f + 1e-5f) + 1e-8f;
-        gdir = sgpr_f((g.gd1 + 0x1p-23f * g.rho * YS) * (1.0f + 1e-5f));
-        Gcf = sgpr_f((g.guard_up + gd) * (1.0f + 1e-6f));
-        cut2_hi_c = sgpr_f((P.c2hi32 + Gcf) * (1.0f + 1e-6f));
-        amb_c = sgpr_f(2.0f * Gcf + cut2_hi_c * 0x1p-20f);
-    }
-    // Staging radius.  Each molecule carries an upper bound U on its
-    // atoms' nearest solute distance (molecule_bound).  A solute atom that
-    // can decide anything for an atom p of the chunk (its FP64 nearest,
-    // or within the FP32 decision band of it) is within
-    // sqrt(U^2 + 2 G + amb) of p, hence of the AABB; staging out to
-    // sqrt(U^2 + 2 amb + 4 G) plus a slack over FP32 rounding keeps every
-    // such atom, and the farther ones cannot change a decision.
-    float rs = rs_full;
-    if (um < rs_full)
-        rs = sgpr_f(fminf(rs_full, fminf(__builtin_amdgcn_sqrtf(fmaf(um, um, 2.0f * amb_c + 4.0f * Gcf)) * (1.0f + 1e-5f) + 1e-2f, um + 0.3f)));
-    const float rs2 = rs * rs;
-    int ilo[3], ihi[3];
-    cell_range32(g, cix, ciy, ciz, bx + rs, by + rs, bz + rs, ilo, ihi);
-#pragma unroll
-    for (int k = 0; k < 3; k++) {
-        ilo[k] = __builtin_amdgcn_readfirstlane(ilo[k]);
-        ihi[k] = __builtin_amdgcn_readfirstlane(ihi[k]);
-    }
-    const int ny = ihi[1] - ilo[1] + 1, nz = ihi[2] - ilo[2] + 1;
-    const gptr<const int> st = (gptr<const int>)(B.start + (int64_t)f * (P.cap + 1));
-    const gptr<const f4v> srt = (gptr<const f4v>)(B.sorted + (int64_t)f * B.nitems);
-    // the lane's molecule over all rounds: minimum, second smallest and
-    // argmin pair, and the same for the reference atom
-    float mb = INFINITY, ms = INFINITY, rb = INFINITY, rsec = INFINITY;
-    float mdir = INFINITY, rdir = INFINITY;   // the argmin pairs' d^2 in the direct form
-    int mi = -1, ma = 0, ri = -1;
-    const unsigned long long lt_mask = (1ull << lane) - 1ull;
-    auto evaluate = [&](int n) {
-        // rows past n are far away and never the minimum
-        const int nsteps = (n + EV_ROWS - 1) / EV_ROWS;
-        if (lane < nsteps * EV_ROWS - n) {
-            const int q = n + lane, o = (q >> 4) * 64 + (q & 15);
-            lds[o] = 0.f; lds[o + 16] = 0.f; lds[o + 32] = 0.f; lds[o + 48] = 1e30f;
-            si[q] = -1;
-        }
-        Min2 wm, wr;
-        wm.init(); wr.init();
-        const int nvv = TQ == 3 ? 3 : P.nv;
-        for (int qb = 0; qb < nvv; qb += TQ) {
-            // columns of this block of atoms (zero where there is no molecule or atom)
-            for (int e = lane; e < MC * TQ; e += 64) {
-                const int m = e / TQ, qq = e - m * TQ;
-                float yx = 0.f, yy = 0.f, yz = 0.f;
-                if (m < nm && qb + qq < nvv) rel(vg[m * nvv + qb + qq], yx, yy, yz);
-                float* o = yb + qq * 4 * MC + m;
-                o[0] = -2.0f * yx; o[MC] = -2.0f * yy; o[2 * MC] = -2.0f * yz;
-                o[3 * MC] = fmaf(yx, yx, fmaf(yy, yy, yz * yz));
+                for (int t = 0; t < 4; t++) box(y[t]);
             }
-            wave_sync();
-#pragma unroll 1
-            for (int h = 0; h < G / GH; h++) {
-                const float* yh = yb + h * 16 * GH + (lane & 15);
-                float bc[GH][TQ], vb[GH][TQ], vs[GH][TQ];
-                int vc[GH][TQ];
+        } else {
+            // 3-atom molecules: at most 3 G / 4 loads per lane, together
+            f4v y[(3 * G + 3) / 4];
 #pragma unroll
-                for (int gg = 0; gg < GH; gg++)
+            for (int t = 0; t < (3 * G + 3) / 4; t++) y[t] = vg[min(64 * t + lane, na - 1)];
 #pragma unroll
-                    for (int qq = 0; qq < TQ; qq++) {
-                        const float c = yh[(qq * 4 + (lane >> 4)) * MC + gg * 16];
-                        bc[gg][qq] = lane >= 48 ? 1.0f : c;
-                        vb[gg][qq] = INFINITY; vs[gg][qq] = INFINITY; vc[gg][qq] = 0;
+            for (int t = 0; t < (3 * G + 3) / 4; t++) box(y[t]);
+        }
+        um = wave_max(um);
+        // the centre moves to the middle of the box (in whole units: exact), the
+        // box with it (to FP32 rounding, inside the staging radius' slack)
+        float bx, by, bz;   // half sides
+        {
+            const float lx = wave_min(alx), ly = wave_min(aly), lz = wave_min(alz);
+            const float hx = wave_max(ahx), hy = wave_max(ahy), hz = wave_max(ahz);
+            const float mx = 0.5f * (lx + hx), my = 0.5f * (ly + hy), mz = 0.5f * (lz + hz);
+            bx = sgpr_f(0.5f * (hx - lx) + 1e-4f); by = sgpr_f(0.5f * (hy - ly) + 1e-4f); bz = sgpr_f(0.5f * (hz - lz) + 1e-4f);
+            const float sc = ldexpf(1.0f, g.fix);
+            cix += __builtin_amdgcn_readfirstlane((int)rintf((g.Hi32[0] * mx + g.Hi32[3] * my + g.Hi32[6] * mz) * sc));
+            ciy += __builtin_amdgcn_readfirstlane((int)rintf((g.Hi32[1] * mx + g.Hi32[4] * my + g.Hi32[7] * mz) * sc));
+            ciz += __builtin_amdgcn_readfirstlane((int)rintf((g.Hi32[2] * mx + g.Hi32[5] * my + g.Hi32[8] * mz) * sc));
+        }
+        const float rs_full = g.rstage;
+        // Distances relative to the chunk centre c (a fixed-point position, no
+        // rounding of its own): |y' - s'|^2 = (|s'|^2 - 2 y'.s') + |y'|^2.  With u =
+        // 2^-24, Y >= |y'| and S >= |s'| for every staged atom, y' and s' are off by
+        // at most rho u Y and rho u S (fix_cart), which moves d^2 by at most
+        // 2 rho u (Y + S) d (d <= cutsys + 0.5 where it matters); the norms (3 u S^2,
+        // 3 u Y^2), the four products and three additions of a tile in whatever
+        // order (2 u Y S + 3 u (S^2 + 2 Y S)) and the last sum (u (Y + S)^2) add at
+        // most 7 u (Y + S)^2.  Both widen the frame's guard for this chunk (FP32
+        // here, every value rounded outward by the factors; S <= Y + the staging
+        // radius, which is at most um + 0.3).  The columns hold -2 y' (exact scaling).
+        float Gcf, cut2_hi_c, amb_c, gdir;   // gdir: the coordinates' rounding in a direct d^2, per d
+        {
+            const float Yb = __builtin_amdgcn_sqrtf(bx * bx + by * by + bz * bz) * (1.0f + 4e-6f) + 1e-3f;
+            const float YS = 2.0f * Yb + fminf(rs_full, um + 0.3f) * (1.0f + 1e-5f) + 1e-3f;
+            const float gd = 0x1p-24f * YS * (2.0f * g.rho * ((float)P.cutsys + 0.5f) + 7.0f * YS) * (1.0f + 1e-5f) + 1e-8f;
+            gdir = sgpr_f((g.gd1 + 0x1p-23f * g.rho * YS) * (1.0f + 1e-5f));
+            Gcf = sgpr_f((g.guard_up + gd) * (1.0f + 1e-6f));
+            cut2_hi_c = sgpr_f((P.c2hi32 + Gcf) * (1.0f + 1e-6f));
+            amb_c = sgpr_f(2.0f * Gcf + cut2_hi_c * 0x1p-20f);
+        }
+        // Staging radius.  Each molecule carries an upper bound U on its
+        // atoms' nearest solute distance (molecule_bound).  A solute atom that
+        // can decide anything for an atom p of the chunk (its FP64 nearest,
+        // or within the FP32 decision band of it) is within
+        // sqrt(U^2 + 2 G + amb) of p, hence of the AABB; staging out to
+        // sqrt(U^2 + 2 amb + 4 G) plus a slack over FP32 rounding keeps every
+        // such atom, and the farther ones cannot change a decision.
+        float rs = rs_full;
+        if (um < rs_full)
+            rs = sgpr_f(fminf(rs_full, fminf(__builtin_amdgcn_sqrtf(fmaf(um, um, 2.0f * amb_c + 4.0f * Gcf)) * (1.0f + 1e-5f) + 1e-2f, um + 0.3f)));
+        const float rs2 = rs * rs;
+        int ilo[3], ihi[3];
+        cell_range32(g, cix, ciy, ciz, bx + rs, by + rs, bz + rs, ilo, ihi);
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            ilo[k] = __builtin_amdgcn_readfirstlane(ilo[k]);
+            ihi[k] = __builtin_amdgcn_readfirstlane(ihi[k]);
+        }
+        const int ny = ihi[1] - ilo[1] + 1, nz = ihi[2] - ilo[2] + 1;
+        const gptr<const int> st = (gptr<const int>)(B.start + (int64_t)f * (P.cap + 1));
+        const gptr<const f4v> srt = (gptr<const f4v>)(B.sorted + (int64_t)f * B.nitems);
+        // FLAT: the lane's atoms over all rounds: minimum, second smallest, its solute
+        // atom and d^2 in the direct form
+        float fb[NL], fs[NL], fd[NL];
+        int fi[NL];
+        // the lane's molecule over all rounds: minimum, second smallest and
+        // argmin pair, and the same for the reference atom
+        float mb = INFINITY, ms = INFINITY, rb = INFINITY, rsec = INFINITY;
+        float mdir = INFINITY, rdir = INFINITY;   // the argmin pairs' d^2 in the direct form
+        int mi = -1, ma = 0, ri = -1;
+        const unsigned long long lt_mask = (1ull << lane) - 1ull;
+        // The records of the lanes' molecules (`on`: slot and molecule m of the
+        // chunk): minimum b, second smallest and argmin (solute atom i, atom a, d^2
+        // in the direct form), and of the reference atom.  Returns whether FP32 leaves
+        // the record open, and the squared radii w0 of every candidate's d^2 (FP32)
+        // and w1 of the reference atom's.
+        auto decide_record = [&](bool on, int slot_, int m, float b, float sec, int i, int a, float dir, float rb_, float rsec_,
+                                 int ri_, float rdir_, float& w0, float& w1) {
+            const int v = RANDOM ? slot_ - (slot_ / P.Mv) * P.Mv : slot_;   // solvent molecule (random passes: slot)
+            const int64_t jbase = (int64_t)v * P.nv;
+            Rec r = rec_zero();
+            bool undec = false, amb = false;   // left to the FP64 resolve (amb: an argmin FP32 cannot separate)
+            w0 = w1 = 0.f;
+            if (on) {
+                // a separated argmin decides with its direct d^2, whose guard shrinks
+                // with d: fixed-point units (E) and the rounding of both positions
+                // about the chunk centre, 2 rho u (Y + S) (gdir), times d, plus 2 rho + 4
+                // units of d^2 and the roundings of decide32's own sums
+                auto decide = [&](float d2, int& bn, int& bk) {
+                    const float Gd = fmaf(g.gd2, d2, gdir * (__builtin_amdgcn_sqrtf(d2) * (1.0f + 1e-6f))) + g.gd0;
+                    return decide32(P, Gd, d2, bn, bk);
+                };
+                int bn, bk;
+                if (b <= cut2_hi_c) {
+                    amb = !(sec - b > amb_c);
+                    const int dd = decide(dir, bn, bk);
+                    if (dd == 2) { r.within = 1; r.i = i; r.j = jbase + a; r.bin = bn; r.bulk = bk; }
+                    undec = dd == 0;
+                }
+                if (rb_ <= cut2_hi_c) {
+                    amb = amb || !(rsec_ - rb_ > amb_c);
+                    const int dd = decide(rdir_, bn, bk);
+                    if (dd == 2) { r.ref = 1; r.rbin = bn; }
+                    undec = undec || dd == 0;
+                }
+                undec = undec || amb;
+                if (undec) {
+                    const float band = amb_c + 2.0f * Gcf;
+                    w0 = fminf(b + band, cut2_hi_c);
+                    w1 = fminf(fmaxf(rb_, b) + band, cut2_hi_c);
+                } else {
+                    ev_hist_record<RANDOM>(P, B, &hist, r, a, jbase);
+                    if (!RANDOM && P.K > 0) B.bflag[(int64_t)f * P.kb * P.Mv + v] = inbulk(P, r) ? 1 : 0;
+                    if constexpr (VERIFY) {
+                        // verification: the record with its FP64 distances
+                        auto dist = [&](int i_, int a_) {
+                            double x0, x1, x2, y0, y1, y2;
+                            load3(xu + (int64_t)f * P.Nu * 3, i_, x0, x1, x2);
+                            if (RANDOM) load3(B.P + 3 * at.atom, (int64_t)m * P.nv + a_, y0, y1, y2);
+                            else load3(xv + (int64_t)f * P.Nv * 3, jbase + a_, y0, y1, y2);
+                            return sqrt(cm::canon_d2(B.geo[f].cell, x0, x1, x2, y0, y1, y2));
+                        };
+                        VRec o;
+                        o.within = r.within; o.i = r.i; o.j = r.j; o.ref = r.ref; o.pad = 0;
+                        o.d = r.within ? dist(r.i, a) : INFINITY;
+                        o.dref = r.ref ? dist(ri_, P.iref) : INFINITY;
+                        // slot: pass within the group times Mv plus the molecule
+                        B.vrec[at.row + slot_] = o;
                     }
+                }
+            }
+            return undec;
+        };
+        // the n staged atoms (FLAT: with block h, the first or last round of them)
+        auto evaluate = [&](int n, int h, bool first, bool last) {
+            const int nsteps = (n + EV_ROWS - 1) / EV_ROWS;
+            if (h == 0) {
+                // rows past n are far away and never the minimum
+                if (lane < nsteps * EV_ROWS - n) {
+                    const int q = n + lane, o = (q >> 4) * 64 + (q & 15);
+                    lds[o] = 0.f; lds[o + 16] = 0.f; lds[o + 32] = 0.f; lds[o + 48] = 1e30f;
+                    si[q] = -1;
+                }
+            }
+            // the candidate of a code (step and rows): eight staged atoms, the
+            // nearest of them (the tile's arithmetic is not repeated: when it
+            // matters the minimum is below every other value by more than the
+            // rounding of both forms, else the molecule is resolved in FP64)
+            auto candidate = [&](int code, float yx, float yy, float yz, float& best) {
+                const int k = (code >> 2) & 0x3fff, jl = code & 3;
+                best = INFINITY;
+                int bi = 0;
+#pragma unroll
+                for (int t = 0; t < 2; t++) {
+                    const float* o = lds + k * 128 + t * 64 + 4 * jl;
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        const float dx = yx - o[i], dy = yy - o[16 + i], dz = yz - o[32 + i];
+                        const float d2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+                        // (padding rows sit at the centre and are no candidates)
+                        const bool lt = d2 < best && o[48 + i] < 1e29f;
+                        best = lt ? d2 : best;
+                        bi = lt ? k * EV_ROWS + t * 16 + 4 * jl + i : bi;
+                    }
+                }
+                return si[bi];
+            };
+            if constexpr (FLAT) {
+                const int mh = NL * h * mpl, left = nm - mh;   // the block's first molecule, molecules from there on
+                auto on = [&](int k) { return lm < mpl && k * mpl + lm < left; };
+                if (first) {
+                    // the block's columns (zero where there is no atom)
+#pragma unroll
+                    for (int k = 0; k < NL; k++) {
+                        float yx = 0.f, yy = 0.f, yz = 0.f;
+                        if (on(k)) rel(vg[mh * P.nv + k * apl + lane], yx, yy, yz);
+                        float* o = yb + k * 256 + lane;
+                        o[0] = -2.0f * yx; o[64] = -2.0f * yy; o[128] = -2.0f * yz;
+                        o[192] = fmaf(yx, yx, fmaf(yy, yy, yz * yz));
+                        fb[k] = fs[k] = fd[k] = INFINITY;
+                        fi[k] = -1;
+                    }
+                }
+                wave_sync();
+                float bc[G], vb[G], vs[G];
+                int vc[G];
+#pragma unroll
+                for (int t = 0; t < G; t++) {
+                    const float c = yb[(t >> 2) * 256 + (lane >> 4) * 64 + (t & 3) * 16 + (lane & 15)];
+                    bc[t] = lane >= 48 ? 1.0f : c;
+                    vb[t] = INFINITY; vs[t] = INFINITY; vc[t] = 0;
+                }
 #pragma unroll 1
                 for (int k = 0; k < nsteps; k++) {
                     const float a0 = lds[k * 128 + lane], a1 = lds[k * 128 + 64 + lane];
 #pragma unroll
+                    for (int t = 0; t < G; t++) {
+                        const f4m v0 = pair_tile(a0, bc[t]), v1 = pair_tile(a1, bc[t]);
+                        const float b0 = vb[t];
+                        min2_4(vb[t], vs[t], v0);
+                        min2_4(vb[t], vs[t], v1);
+                        vc[t] = vb[t] < b0 ? k : vc[t];
+                    }
+                }
+#pragma unroll
+                for (int k = 0; k < NL; k++) {
+                    Min2 mt[4];
+#pragma unroll
+                    for (int t = 0; t < 4; t++) {
+                        mt[t].b = vb[4 * k + t]; mt[t].s = vs[4 * k + t]; mt[t].c = (vc[4 * k + t] << 2) | (lane >> 4);
+                    }
+                    Min2 w = gather_columns(mt, lane);
+                    const float* o = yb + k * 256 + lane;
+                    w.b += o[192];
+                    w.s += o[192];
+                    if (w.b < fb[k]) fi[k] = candidate(w.c, -0.5f * o[0], -0.5f * o[64], -0.5f * o[128], fd[k]);
+                    fs[k] = fminf(fmaxf(fb[k], w.b), fminf(fs[k], w.s));
+                    fb[k] = fminf(fb[k], w.b);
+                }
+                if (last) {
+#pragma unroll 1
+                    for (int k = 0; k < NL; k++) {
+                        const float b = k ? fb[NL - 1] : fb[0], sec = k ? fs[NL - 1] : fs[0], d = k ? fd[NL - 1] : fd[0];
+                        const int is = k ? fi[NL - 1] : fi[0];
+                        const bool has = on(k);
+                        // the atoms of a molecule into its first lane (c: lane of the minimum);
+                        // after the step with offset o a lane holds the next 2 o of its molecule
+                        Min2 w;
+                        w.b = has ? b : INFINITY; w.s = has ? sec : INFINITY; w.c = lane;
+                        for (int o = 1; o < P.nv; o <<= 1) {
+                            const float b2 = __shfl_down(w.b, o, 64), s2 = __shfl_down(w.s, o, 64);
+                            const int c2 = __shfl_down(w.c, o, 64);
+                            if (la + o < P.nv && lane + o < 64) w.merge(b2, s2, c2);
+                        }
+                        const int il = (lane + P.iref) & 63;
+                        const int i = __shfl(is, w.c, 64), ri_ = __shfl(is, il, 64);
+                        const float dir = __shfl(d, w.c, 64), rdir_ = __shfl(d, il, 64), rb_ = __shfl(b, il, 64), rsec_ = __shfl(sec, il, 64);
+                        const int m = mc + mh + k * mpl + lm;   // of the chunk
+                        const int slot_ = ldg(B.msorted + at.row + at.m0 + min(m, at.nm - 1));
+                        float w0, w1;
+                        const bool undec = decide_record(has && la == 0, slot_, m, w.b, w.s, i, w.c - lane, dir, rb_, rsec_, ri_, rdir_, w0, w1);
+                        // the radius of every atom of the molecules left open
+                        const int head = lane - la;
+                        const float x0 = __shfl(w0, head, 64), x1 = __shfl(w1, head, 64);
+                        if (__shfl(undec ? 1 : 0, head, 64) && has) {
+                            const bool isref = la == P.iref;
+                            const float wa = b <= x0 || (isref && b <= cut2_hi_c) ? (isref ? fmaxf(x0, x1) : x0) : -1.0f;
+                            ((float*)(vwb + mh * P.nv + k * apl + lane))[3] = wa;
+                        }
+                        const int fl = __shfl(undec ? 1 : 0, (lane * P.nv) & 63, 64);
+                        um_ |= __ballot(lane < mpl && fl != 0) << ((mc + mh + k * mpl) & 63);
+                    }
+                }
+            } else {
+                Min2 wm, wr;
+                wm.init(); wr.init();
+                // columns (zero where there is no molecule)
+                for (int e = lane; e < MC * TQ; e += 64) {
+                    const int m = e / TQ, qq = e - m * TQ;
+                    float yx = 0.f, yy = 0.f, yz = 0.f;
+                    if (m < nm) rel(vg[m * TQ + qq], yx, yy, yz);
+                    float* o = yb + qq * 4 * MC + m;
+                    o[0] = -2.0f * yx; o[MC] = -2.0f * yy; o[2 * MC] = -2.0f * yz;
+                    o[3 * MC] = fmaf(yx, yx, fmaf(yy, yy, yz * yz));
+                }
+                wave_sync();
+#pragma unroll 1
+                for (int hh = 0; hh < G / GH; hh++) {
+                    const float* yh = yb + hh * 16 * GH + (lane & 15);
+                    float bc[GH][TQ], vb[GH][TQ], vs[GH][TQ];
+                    int vc[GH][TQ];
+#pragma unroll
                     for (int gg = 0; gg < GH; gg++)
 #pragma unroll
                         for (int qq = 0; qq < TQ; qq++) {
-                            const f4m v0 = pair_tile(a0, bc[gg][qq]), v1 = pair_tile(a1, bc[gg][qq]);
-                            const float b0 = vb[gg][qq];
-                            min2_4(vb[gg][qq], vs[gg][qq], v0);
-                            min2_4(vb[gg][qq], vs[gg][qq], v1);
-                            vc[gg][qq] = vb[gg][qq] < b0 ? k : vc[gg][qq];
+                            const float c = yh[(qq * 4 + (lane >> 4)) * MC + gg * 16];
+                            bc[gg][qq] = lane >= 48 ? 1.0f : c;
+                            vb[gg][qq] = INFINITY; vs[gg][qq] = INFINITY; vc[gg][qq] = 0;
                         }
-                }
-                // + |y'|^2, the atoms of the block into the molecule; code: atom, step
-                Min2 mm[GH], mr[GH];
+#pragma unroll 1
+                    for (int k = 0; k < nsteps; k++) {
+                        const float a0 = lds[k * 128 + lane], a1 = lds[k * 128 + 64 + lane];
 #pragma unroll
-                for (int gg = 0; gg < GH; gg++) {
-                    mm[gg].init(); mr[gg].init();
+                        for (int gg = 0; gg < GH; gg++)
 #pragma unroll
-                    for (int qq = 0; qq < TQ; qq++) {
-                        if (qb + qq >= nvv) continue;
-                        const float y2 = yh[(qq * 4 + 3) * MC + gg * 16];
-                        const float b2 = vb[gg][qq] + y2, s2 = vs[gg][qq] + y2;
-                        const int code = ((qb + qq) << 16) | (vc[gg][qq] << 2) | (lane >> 4);
-                        mm[gg].merge(b2, s2, code);
-                        if (qb + qq == P.iref) { mr[gg].b = b2; mr[gg].s = s2; mr[gg].c = code; }
+                            for (int qq = 0; qq < TQ; qq++) {
+                                const f4m v0 = pair_tile(a0, bc[gg][qq]), v1 = pair_tile(a1, bc[gg][qq]);
+                                const float b0 = vb[gg][qq];
+                                min2_4(vb[gg][qq], vs[gg][qq], v0);
+                                min2_4(vb[gg][qq], vs[gg][qq], v1);
+                                vc[gg][qq] = vb[gg][qq] < b0 ? k : vc[gg][qq];
+                            }
                     }
+                    // + |y'|^2, the atoms into the molecule; code: atom, step
+                    Min2 mm[GH], mr[GH];
+#pragma unroll
+                    for (int gg = 0; gg < GH; gg++) {
+                        mm[gg].init(); mr[gg].init();
+#pragma unroll
+                        for (int qq = 0; qq < TQ; qq++) {
+                            const float y2 = yh[(qq * 4 + 3) * MC + gg * 16];
+                            const float b2 = vb[gg][qq] + y2, s2 = vs[gg][qq] + y2;
+                            const int code = (qq << 16) | (vc[gg][qq] << 2) | (lane >> 4);
+                            mm[gg].merge(b2, s2, code);
+                            if (qq == P.iref) { mr[gg].b = b2; mr[gg].s = s2; mr[gg].c = code; }
+                        }
+                    }
+                    const Min2 gm = gather_groups<GH>(mm, lane), gr = gather_groups<GH>(mr, lane);
+                    if (G < 4 || ((lane >> 4) & 1) == hh) { wm = gm; wr = gr; }
                 }
-                const Min2 gm = gather_groups<GH>(mm, lane), gr = gather_groups<GH>(mr, lane);
-                if (G < 4 || ((lane >> 4) & 1) == h) {
-                    wm.merge(gm.b, gm.s, gm.c);
-                    if (gr.b < INFINITY) wr = gr;   // (one block holds the reference atom)
-                }
+                wave_sync();
+                auto cand = [&](int code, float& best) {
+                    float yx, yy, yz;
+                    rel(vg[min(ml, nm - 1) * TQ + (code >> 16)], yx, yy, yz);
+                    return candidate(code, yx, yy, yz, best);
+                };
+                if (wm.b < mb) { mi = cand(wm.c, mdir); ma = wm.c >> 16; }
+                ms = fminf(fmaxf(mb, wm.b), fminf(ms, wm.s));
+                mb = fminf(mb, wm.b);
+                if (wr.b < rb) ri = cand(wr.c, rdir);
+                rsec = fminf(fmaxf(rb, wr.b), fminf(rsec, wr.s));
+                rb = fminf(rb, wr.b);
             }
             wave_sync();
-        }
-        // the candidate of a code: eight staged atoms of one step, the
-        // nearest of them (the tile's arithmetic is not repeated: when it
-        // matters the minimum is below every other value by more than the
-        // rounding of both forms, else the molecule is resolved in FP64)
-        auto candidate = [&](int code, float& best) {
-            const int q = code >> 16, k = (code >> 2) & 0x3fff, jl = code & 3;
-            float yx, yy, yz;
-            rel(vg[min(ml, nm - 1) * P.nv + q], yx, yy, yz);
-            best = INFINITY;
-            int bi = 0;
-#pragma unroll
-            for (int t = 0; t < 2; t++) {
-                const float* o = lds + k * 128 + t * 64 + 4 * jl;
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const float dx = yx - o[i], dy = yy - o[16 + i], dz = yz - o[32 + i];
-                    const float d2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-                    // (padding rows sit at the centre and are no candidates)
-                    const bool lt = d2 < best && o[48 + i] < 1e29f;
-                    best = lt ? d2 : best;
-                    bi = lt ? k * EV_ROWS + t * 16 + 4 * jl + i : bi;
-                }
-            }
-            return si[bi];
         };
-        if (wm.b < mb) { mi = candidate(wm.c, mdir); ma = wm.c >> 16; }
-        ms = fminf(fmaxf(mb, wm.b), fminf(ms, wm.s));
-        mb = fminf(mb, wm.b);
-        if (wr.b < rb) ri = candidate(wr.c, rdir);
-        rsec = fminf(fmaxf(rb, wr.b), fminf(rsec, wr.s));
-        rb = fminf(rb, wr.b);
-        wave_sync();
-    };
-    // Staging walks rows of cells (x fastest in memory): a slot is the part
-    // of one (y, z) row of the index box that lies in one periodic image
-    // along x, so its atoms are one contiguous range of the sorted list.
-    // With a diagonal cell, rows farther than rs from the AABB are
-    // dropped and each row is trimmed to the x range within rs (plus a
-    // slack over FP32 rounding); the per-atom AABB test below is exact.
-    // The rows are cut into segments of up to SEG consecutive atoms; in a step
-    // each lane takes one segment (listed in LDS by the rows' lanes), loads its
-    // atoms together and appends the ones within rs of the AABB at
-    // ballot/popcount offsets.  A step that would overflow the buffer evaluates
-    // what is staged first.  The staged set does not depend on the order (FP32
-    // ties between candidates go to the FP64 resolve).
-    int q0;
-    wrap_index(ilo[0], g.nc[0], q0);
-    int q1;
-    wrap_index(ihi[0], g.nc[0], q1);
-    const int npc = q1 - q0 + 1;
-    const int nslots = ny * nz * npc;
-    // (slack over the FP32 rounding of absolute coordinates)
-    const float slk = 1e-3f + 1e-6f * (fabsf(g.H32[0]) + fabsf(g.H32[4]) + fabsf(g.H32[8]));
-    const float rsl = rs + slk, rsl2 = rsl * rsl;
-    // (diagonal cells) the box's ends and the cells' sides
-    const float hcx = g.H32[0] * __builtin_amdgcn_rcpf((float)g.nc[0]), hcy = g.H32[4] * __builtin_amdgcn_rcpf((float)g.nc[1]),
-                hcz = g.H32[8] * __builtin_amdgcn_rcpf((float)g.nc[2]), icx = __builtin_amdgcn_rcpf(hcx);
-    const float ccx = g.Hfix[0] * (float)cix, ccy = g.Hfix[4] * (float)ciy, ccz = g.Hfix[8] * (float)ciz;
-    int nst = 0;            // staged atoms (uniform)
-    int sb = -64, s0 = 0, NS = 0;   // slots of the current 64, its next segment and number of segments
-    int cstart = 0, cnt = 0, nseg = 0, sexcl = 0, code = 0;   // the lane's row: atoms, segments, image
-    for (;;) {
-        while (s0 >= NS && sb + 64 < nslots) {
-            // the next 64 row slots
-            sb += 64;
-            s0 = 0;
-            const int sl = sb + lane;
-            cstart = 0; cnt = 0;
-            if (sl < nslots) {
-                const int r = sl / npc, pc = sl - r * npc;
-                const int iy = ilo[1] + r % ny, iz = ilo[2] + r / ny;
-                int x0 = ilo[0], x1 = ihi[0];
-                bool keep = true;
-                if (g.ortho) {
-                    const float dy = fmaxf(fabsf((iy + 0.5f) * hcy - ccy) - (by + 0.5f * hcy), 0.f);
-                    const float dz = fmaxf(fabsf((iz + 0.5f) * hcz - ccz) - (bz + 0.5f * hcz), 0.f);
-                    const float r2 = rsl2 - dy * dy - dz * dz;
-                    if (r2 < 0.f) {
-                        keep = false;
-                    } else {
-                        const float rx = __builtin_amdgcn_sqrtf(r2) * (1.0f + 1e-6f) + bx + slk;
-                        x0 = max(x0, (int)floorf((ccx - rx) * icx - 1e-3f));
-                        x1 = min(x1, (int)floorf((ccx + rx) * icx + 1e-3f));
+        // Staging walks rows of cells (x fastest in memory): a slot is the part
+        // of one (y, z) row of the index box that lies in one periodic image
+        // along x, so its atoms are one contiguous range of the sorted list.
+        // With a diagonal cell, rows farther than rs from the AABB are
+        // dropped and each row is trimmed to the x range within rs (plus a
+        // slack over FP32 rounding); the per-atom AABB test below is exact.
+        // The rows are cut into segments of up to SEG consecutive atoms; in a step
+        // each lane takes one segment (listed in LDS by the rows' lanes), loads its
+        // atoms together and appends the ones within rs of the AABB at
+        // ballot/popcount offsets.  A step that would overflow the buffer evaluates
+        // what is staged first.  The staged set does not depend on the order (FP32
+        // ties between candidates go to the FP64 resolve).
+        int q0;
+        wrap_index(ilo[0], g.nc[0], q0);
+        int q1;
+        wrap_index(ihi[0], g.nc[0], q1);
+        const int npc = q1 - q0 + 1;
+        const int nslots = ny * nz * npc;
+        // (slack over the FP32 rounding of absolute coordinates)
+        const float slk = 1e-3f + 1e-6f * (fabsf(g.H32[0]) + fabsf(g.H32[4]) + fabsf(g.H32[8]));
+        const float rsl = rs + slk, rsl2 = rsl * rsl;
+        // (diagonal cells) the box's ends and the cells' sides
+        const float hcx = g.H32[0] * __builtin_amdgcn_rcpf((float)g.nc[0]), hcy = g.H32[4] * __builtin_amdgcn_rcpf((float)g.nc[1]),
+                    hcz = g.H32[8] * __builtin_amdgcn_rcpf((float)g.nc[2]), icx = __builtin_amdgcn_rcpf(hcx);
+        const float ccx = g.Hfix[0] * (float)cix, ccy = g.Hfix[4] * (float)ciy, ccz = g.Hfix[8] * (float)ciz;
+        bool split = false;
+        int sb = -64, s0 = 0;   // slots of the current 64, its next segment
+        int NS = 0;             // segments of the current 64 slots
+        int cstart = 0, cnt = 0, nseg = 0, sexcl = 0, code = 0;   // the lane's row: atoms, segments, image
+        for (bool first = true;; first = false) {
+            int nst = 0;            // staged atoms (uniform)
+            // (FLAT: the rows are formed again after an evaluation, which has no
+            // registers to hold them)
+            bool full = false, again = FLAT && !first;
+            if (FLAT) { NS = 0; cstart = cnt = nseg = sexcl = code = 0; }
+            for (;;) {
+                while (again || (s0 >= NS && sb + 64 < nslots)) {
+                    // the next 64 row slots
+                    if (!again) { sb += 64; s0 = 0; }
+                    again = false;
+                    const int sl = sb + lane;
+                    cstart = 0; cnt = 0;
+                    if (sl < nslots) {
+                        const int r = sl / npc, pc = sl - r * npc;
+                        const int iy = ilo[1] + r % ny, iz = ilo[2] + r / ny;
+                        int x0 = ilo[0], x1 = ihi[0];
+                        bool keep = true;
+                        if (g.ortho) {
+                            const float dy = fmaxf(fabsf((iy + 0.5f) * hcy - ccy) - (by + 0.5f * hcy), 0.f);
+                            const float dz = fmaxf(fabsf((iz + 0.5f) * hcz - ccz) - (bz + 0.5f * hcz), 0.f);
+                            const float r2 = rsl2 - dy * dy - dz * dz;
+                            if (r2 < 0.f) {
+                                keep = false;
+                            } else {
+                                const float rx = __builtin_amdgcn_sqrtf(r2) * (1.0f + 1e-6f) + bx + slk;
+                                x0 = max(x0, (int)floorf((ccx - rx) * icx - 1e-3f));
+                                x1 = min(x1, (int)floorf((ccx + rx) * icx + 1e-3f));
+                            }
+                        }
+                        const int mx = q0 + pc;
+                        x0 = max(x0, mx * g.nc[0]);
+                        x1 = min(x1, mx * g.nc[0] + g.nc[0] - 1);
+                        if (keep && x0 <= x1) {
+                            int my, mz;
+                            const int cy = wrap_index(iy, g.nc[1], my), cz = wrap_index(iz, g.nc[2], mz);
+                            const int crow = (cz * g.nc[1] + cy) * g.nc[0] - mx * g.nc[0];
+                            cstart = st[crow + x0];
+                            cnt = st[crow + x1 + 1] - cstart;
+                            code = ((mx + 16) << 8) | ((my + 16) << 16) | ((mz + 16) << 24);
+                        }
                     }
+                    nseg = (cnt + SEG - 1) / SEG;
+                    const int sincl = wave_incl_scan(nseg);
+                    sexcl = sincl - nseg;
+                    NS = __builtin_amdgcn_readlane(sincl, 63);
+                    // (more than the buffer takes, before any is staged: about half of
+                    // the rows' atoms pass the test of the box)
+                    if (FLAT && nb > 1 && NS * SEG > 2 * TCAP) split = true;
+                    if (split) break;
                 }
-                const int mx = q0 + pc;
-                x0 = max(x0, mx * g.nc[0]);
-                x1 = min(x1, mx * g.nc[0] + g.nc[0] - 1);
-                if (keep && x0 <= x1) {
-                    int my, mz;
-                    const int cy = wrap_index(iy, g.nc[1], my), cz = wrap_index(iz, g.nc[2], mz);
-                    const int crow = (cz * g.nc[1] + cy) * g.nc[0] - mx * g.nc[0];
-                    cstart = st[crow + x0];
-                    cnt = st[crow + x1 + 1] - cstart;
-                    code = ((mx + 16) << 8) | ((my + 16) << 16) | ((mz + 16) << 24);
+                if (split || s0 >= NS) break;
+                f4v q[SEG];
+                bool pass[SEG];
+                int total = 0;
+                // segments s0 .. s0 + 63: first atom, row lane and atoms
+                for (int t = max(0, s0 - sexcl); t < nseg && sexcl + t < s0 + 64; t++)
+                    sd[sexcl + t - s0] = make_int2(cstart + SEG * t, code | min(SEG, cnt - SEG * t));
+                wave_sync();
+                int2 d = sd[lane];
+                wave_sync();
+                if (s0 + lane >= NS) d = make_int2(0, 0);
+                const int n = d.y & 255;
+#pragma unroll
+                for (int u = 0; u < SEG; u++) q[u] = srt[u < n ? d.x + u : 0];
+                // the image's origin relative to the centre
+                const int ox = ((((d.y >> 8) & 255) - 16) << g.fix) - cix, oy = ((((d.y >> 16) & 255) - 16) << g.fix) - ciy,
+                          oz = ((((d.y >> 24) & 255) - 16) << g.fix) - ciz;
+#pragma unroll
+                for (int u = 0; u < SEG; u++) {
+                    float x_, y_, z_;
+                    fix_cart(g, __float_as_int(q[u].x) + ox, __float_as_int(q[u].y) + oy, __float_as_int(q[u].z) + oz, x_, y_, z_);
+                    q[u].x = x_; q[u].y = y_; q[u].z = z_;
+                    const float dx = fmaxf(fabsf(q[u].x) - bx, 0.f), dy = fmaxf(fabsf(q[u].y) - by, 0.f),
+                                dz = fmaxf(fabsf(q[u].z) - bz, 0.f);
+                    pass[u] = u < n && dx * dx + dy * dy + dz * dz <= rs2;
+                    total += __popcll(__ballot(pass[u]));
+                }
+                full = nst + total > TCAP;
+                if (full) break;
+                s0 += 64;
+#pragma unroll
+                for (int u = 0; u < SEG; u++) {
+                    const unsigned long long m = __ballot(pass[u]);
+                    if (pass[u]) {
+                        const int a = nst + __popcll(m & lt_mask);
+                        const int o = (a >> 4) * 64 + (a & 15);
+                        lds[o] = q[u].x; lds[o + 16] = q[u].y; lds[o + 32] = q[u].z;
+                        lds[o + 48] = fmaf(q[u].x, q[u].x, fmaf(q[u].y, q[u].y, q[u].z * q[u].z));
+                        si[a] = __float_as_int(q[u].w);
+                    }
+                    nst += __popcll(m);
                 }
             }
-            nseg = (cnt + SEG - 1) / SEG;
-            const int sincl = wave_incl_scan(nseg);
-            sexcl = sincl - nseg;
-            NS = __builtin_amdgcn_readlane(sincl, 63);
-        }
-        const bool more = s0 < NS;
-        f4v q[SEG];
-        bool pass[SEG];
-        int total = 0;
-        if (more) {
-            // segments s0 .. s0 + 63: first atom, row lane and atoms
-            for (int t = max(0, s0 - sexcl); t < nseg && sexcl + t < s0 + 64; t++)
-                sd[sexcl + t - s0] = make_int2(cstart + SEG * t, code | min(SEG, cnt - SEG * t));
-            wave_sync();
-            int2 d = sd[lane];
-            wave_sync();
-            if (s0 + lane >= NS) d = make_int2(0, 0);
-            const int n = d.y & 255;
-#pragma unroll
-            for (int u = 0; u < SEG; u++) q[u] = srt[u < n ? d.x + u : 0];
-            // the image's origin relative to the centre
-            const int ox = ((((d.y >> 8) & 255) - 16) << g.fix) - cix, oy = ((((d.y >> 16) & 255) - 16) << g.fix) - ciy,
-                      oz = ((((d.y >> 24) & 255) - 16) << g.fix) - ciz;
-#pragma unroll
-            for (int u = 0; u < SEG; u++) {
-                float x_, y_, z_;
-                fix_cart(g, __float_as_int(q[u].x) + ox, __float_as_int(q[u].y) + oy, __float_as_int(q[u].z) + oz, x_, y_, z_);
-                q[u].x = x_; q[u].y = y_; q[u].z = z_;
-                const float dx = fmaxf(fabsf(q[u].x) - bx, 0.f), dy = fmaxf(fabsf(q[u].y) - by, 0.f),
-                            dz = fmaxf(fabsf(q[u].z) - bz, 0.f);
-                pass[u] = u < n && dx * dx + dy * dy + dz * dz <= rs2;
-                total += __popcll(__ballot(pass[u]));
+            if (full && nb > 1) split = true;
+            if (split) break;
+            if (FLAT || nst > 0) {
+#pragma unroll 1
+                for (int h = 0; h < nb; h++) evaluate(nst, h, first, !full);
             }
-            s0 += 64;
+            if (!full) break;
         }
-        const bool full = nst + total > TCAP;
-        if (nst > 0 && (!more || full)) {
-            evaluate(nst);
-            nst = 0;
-        }
-        if (!more) break;
-        if (full) {
-            // (loaded again, so that nothing is held across the evaluation)
-            s0 -= 64;
+        if (split) {
+            nb = 1;
             continue;
         }
+        h0 += nb;
+        if constexpr (!FLAT) {
+            float w0, w1;
+            const bool undec = decide_record(active, slot, ml, mb, ms, mi, ma, mdir, rb, rsec, ri, rdir, w0, w1);
+            if (undec) {
+                float* o = (float*)(vwb + ml * TQ);
 #pragma unroll
-        for (int u = 0; u < SEG; u++) {
-            const unsigned long long m = __ballot(pass[u]);
-            if (pass[u]) {
-                const int a = nst + __popcll(m & lt_mask);
-                const int o = (a >> 4) * 64 + (a & 15);
-                lds[o] = q[u].x; lds[o + 16] = q[u].y; lds[o + 32] = q[u].z;
-                lds[o + 48] = fmaf(q[u].x, q[u].x, fmaf(q[u].y, q[u].y, q[u].z * q[u].z));
-                si[a] = __float_as_int(q[u].w);
+                for (int q = 0; q < TQ; q++) o[4 * q + 3] = q == P.iref ? fmaxf(w0, w1) : w0;
             }
-            nst += __popcll(m);
+            um_ = __ballot(undec);
+            if (G == 2) um_ = (um_ & 0xffffull) | ((um_ >> 16) & 0xffff0000ull);
+            if (G == 4) um_ = (um_ & 0xffff00000000ffffull) | ((um_ & 0xffff0000ull) << 16) | ((um_ >> 16) & 0xffff0000ull);
         }
     }
-    const int v = RANDOM ? slot - (slot / P.Mv) * P.Mv : slot;   // solvent molecule (random passes: slot)
-    const int64_t jbase = (int64_t)v * P.nv;
-    Rec r = rec_zero();
-    bool undec = false, amb = false;   // left to the FP64 resolve (amb: an argmin FP32 cannot separate)
-    if (active) {
-        // a separated argmin decides with its direct d^2, whose guard shrinks
-        // with d: fixed-point units (E) and the rounding of both positions
-        // about the chunk centre, 2 rho u (Y + S) (gdir), times d, plus 2 rho + 4
-        // units of d^2 and the roundings of decide32's own sums
-        auto decide = [&](float d2, int& bn, int& bk) {
-            const float Gd = fmaf(g.gd2, d2, gdir * (__builtin_amdgcn_sqrtf(d2) * (1.0f + 1e-6f))) + g.gd0;
-            return decide32(P, Gd, d2, bn, bk);
-        };
-        int bn, bk;
-        if (mb <= cut2_hi_c) {
-            amb = !(ms - mb > amb_c);
-            const int dd = decide(mdir, bn, bk);
-            if (dd == 2) { r.within = 1; r.i = mi; r.j = jbase + ma; r.bin = bn; r.bulk = bk; }
-            undec = dd == 0;
-        }
-        if (rb <= cut2_hi_c) {
-            amb = amb || !(rsec - rb > amb_c);
-            const int dd = decide(rdir, bn, bk);
-            if (dd == 2) { r.ref = 1; r.rbin = bn; }
-            undec = undec || dd == 0;
-        }
-        undec = undec || amb;
-        if (undec) {
-            // every candidate of the record: d^2 (FP32) within these of the
-            // molecule's atoms, the reference atom's own beyond
-            const float band = amb_c + 2.0f * Gcf;
-            const float w0 = fminf(mb + band, cut2_hi_c), w1 = fminf(fmaxf(rb, mb) + band, cut2_hi_c);
-            const int o = ml * P.nv;
-            ((float*)(vwb + o))[3] = w0;
-            if (P.nv > 1) ((float*)(vwb + o + 1))[3] = w1;
-        } else {
-            ev_hist_record<RANDOM>(P, B, &hist, r, ma, jbase);
-            if (!RANDOM && P.K > 0) B.bflag[(int64_t)f * P.kb * P.Mv + v] = inbulk(P, r) ? 1 : 0;
-            if constexpr (VERIFY) {
-                // verification: the record with its FP64 distances
-                auto dist = [&](int i, int a) {
-                    double x0, x1, x2, y0, y1, y2;
-                    load3(xu + (int64_t)f * P.Nu * 3, i, x0, x1, x2);
-                    if (RANDOM) load3(B.P + 3 * at.atom, (int64_t)ml * P.nv + a, y0, y1, y2);
-                    else load3(xv + (int64_t)f * P.Nv * 3, jbase + a, y0, y1, y2);
-                    return sqrt(cm::canon_d2(B.geo[f].cell, x0, x1, x2, y0, y1, y2));
-                };
-                VRec o;
-                o.within = r.within; o.i = r.i; o.j = r.j; o.ref = r.ref; o.pad = 0;
-                o.d = r.within ? dist(r.i, ma) : INFINITY;
-                o.dref = r.ref ? dist(ri, P.iref) : INFINITY;
-                // slot: pass within the group times Mv plus the molecule
-                B.vrec[at.row + slot] = o;
-            }
-        }
-    }
-    // one bit per molecule, in molecule order
-    unsigned long long um_ = __ballot(undec);
-    if (G == 2) um_ = (um_ & 0xffffull) | ((um_ >> 16) & 0xffff0000ull);
-    if (G == 4) um_ = (um_ & 0xffff00000000ffffull) | ((um_ & 0xffff0000ull) << 16) | ((um_ >> 16) & 0xffff0000ull);
     if (lane == 0) {
-        B.resmask[ch] = um_;
+        if (at.mpt > 32) ((ull*)B.resmask)[ch] = um_;
+        else B.resmask[ch] = (unsigned)um_;
         if (um_) atomicAdd(&B.stats[0], (ull)__popcll(um_));
     }
 }
@@ -3370,12 +3591,14 @@ __global__ void __launch_bounds__(1024) k_eval_tiles(KP P, Bufs B, const TU* xu,
     ev_hist_flush<RANDOM>(P, B);
 }
 
-// FP64 records of the molecules FP32 left undecided (one or two per cent): a
-// block takes 64 consecutive chunks of a row, lists their marked molecules in
-// LDS and gives each 16 lanes (four solvent atoms times four rows of cells).
-// Every solute atom within the molecule's radii (FP32, wider than the guard) is
-// evaluated exactly, ties to the smallest (i, j).  Kept out of the evaluation,
-// whose registers and code it would double.
+// FP64 records of the molecules FP32 left undecided: a block takes a few
+// consecutive chunks of a row, lists their marked molecules in LDS and gives each
+// 16 lanes.  They walk the rows of cells within reach of the atoms that the
+// evaluation left a radius (of molecules of other than three atoms usually one or
+// two: the others are farther than the minimum by more than the guard).  Every
+// solute atom within the radius (FP32, wider than the guard) is evaluated exactly,
+// ties to the smallest (i, j).  Kept out of the evaluation, whose registers and
+// code it would double.
 constexpr int RES_CHUNKS = 64;
 
 // chunks a block of the resolve takes at a time: 64, in small launches as few
@@ -3390,6 +3613,45 @@ __host__ __device__ __forceinline__ int resolve_step(const KP& P, bool random)
 {
     const int64_t n = resolve_row_chunks(P, random) * P.F * (random ? P.NG : 1) / 1024;
     return n < 2 ? 2 : (n > RES_CHUNKS ? RES_CHUNKS : (int)n);
+}
+
+// cm::random_move of slot v of pass k by 16 lanes (sub), atoms at a stride: the
+// same operations in the same order, so the same positions (FP64, at yp).  Every
+// lane forms the centre, from the wrapped positions the others left there.
+template <class TV>
+__device__ __forceinline__ void place_by_lanes(const KP& P, const Bufs& B, const TV* xv, int f, int k, int v, double* yp, int sub)
+{
+    const cm::Cell64& c = B.geo[f].cell;
+    const SlotMove<TV> mv(P, B, B.geo[f], xv, f, k, v);
+    const MolSrc<TV> x(mv.x);
+    const double rx = x(P.iref, 0), ry = x(P.iref, 1), rz = x(P.iref, 2);
+    for (int a = sub; a < P.nv; a += 16) {
+        double ox, oy, oz;
+        cm::minimage(c, x(a, 0) - rx, x(a, 1) - ry, x(a, 2) - rz, &ox, &oy, &oz);
+        yp[3 * a] = rx + ox; yp[3 * a + 1] = ry + oy; yp[3 * a + 2] = rz + oz;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+    double cx = 0.0, cy = 0.0, cz = 0.0;
+    for (int a = 0; a < P.nv; a++) { cx += yp[3 * a]; cy += yp[3 * a + 1]; cz += yp[3 * a + 2]; }
+    cx = cx / (double)P.nv; cy = cy / (double)P.nv; cz = cz / (double)P.nv;
+    const double* H = c.H;
+    const double n0 = H[0] * mv.uc[0] + H[3] * mv.uc[1] + H[6] * mv.uc[2];
+    const double n1 = H[1] * mv.uc[0] + H[4] * mv.uc[1] + H[7] * mv.uc[2];
+    const double n2 = H[2] * mv.uc[0] + H[5] * mv.uc[1] + H[8] * mv.uc[2];
+    double A[9];
+    cm::eulermat_turns(mv.ua[0], mv.ua[1], mv.ua[2], A);
+    // (every lane has read the wrapped positions before one replaces them)
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+    for (int a = sub; a < P.nv; a += 16) {
+        const double dx = yp[3 * a] - cx, dy = yp[3 * a + 1] - cy, dz = yp[3 * a + 2] - cz;
+        yp[3 * a] = A[0] * dx + A[1] * dy + A[2] * dz + n0;
+        yp[3 * a + 1] = A[3] * dx + A[4] * dy + A[5] * dz + n1;
+        yp[3 * a + 2] = A[6] * dx + A[7] * dy + A[8] * dz + n2;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+    __builtin_amdgcn_wave_barrier();
 }
 
 template <class TU, class TV, bool RANDOM, bool VERIFY>
@@ -3412,58 +3674,76 @@ __device__ __forceinline__ void resolve_one(const KP& P, const Bufs& B, const TU
         jbase = v * P.nv;
         double* const yp = B.P + 3 * (atom + (int64_t)pos * P.nv);
         if (RANDOM && !P.place_all) {
-            // the molecule's FP64 positions, by one lane (k_place_near's move)
-            if (sub == 0) {
-                MolDst64 dst(yp);
-                const SlotMove<TV> mv(P, B, B.geo[f], xv, f, grp * P.KM + slot / P.Mv, (int)v);
-                cm::random_move(MolSrc<TV>(mv.x), dst, P.nv, P.iref, B.geo[f].cell, mv.uc, mv.ua);
+            // the molecule's FP64 positions (k_place_near's move): few atoms by one
+            // lane, more by all
+            const int pass = grp * P.KM + slot / P.Mv;
+            if (P.nv > 4) {
+                place_by_lanes(P, B, xv, f, pass, (int)v, yp, sub);
+            } else {
+                if (sub == 0) {
+                    MolDst64 dst(yp);
+                    const SlotMove<TV> mv(P, B, B.geo[f], xv, f, pass, (int)v);
+                    cm::random_move(MolSrc<TV>(mv.x), dst, P.nv, P.iref, B.geo[f].cell, mv.uc, mv.ua);
+                }
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+                __builtin_amdgcn_wave_barrier();
             }
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
-            __builtin_amdgcn_wave_barrier();
         }
-        const float w0 = vg[0].w, w1 = P.nv > 1 ? vg[1].w : w0;
-        for (int a = sub >> 2; a < P.nv; a += 4) {
-            const f4v y = vg[a];
-            const bool isref = a == P.iref;
-            const float R2 = isref ? fmaxf(w0, w1) : w0;
-            double y0, y1, y2;
-            if (RANDOM) load3((const double*)yp, a, y0, y1, y2);
-            else load3(xv + (int64_t)f * P.Nv * 3, jbase + a, y0, y1, y2);
-            const int ux = __float_as_int(y.x), uy = __float_as_int(y.y), uz = __float_as_int(y.z);
-            const float rr_ = __builtin_amdgcn_sqrtf(R2) * (1.0f + 1e-5f) + 1e-3f;
-            int jlo[3], jhi[3];
-            cell_range32(g, ux, uy, uz, rr_, rr_, rr_, jlo, jhi);
-            const int nyr = jhi[1] - jlo[1] + 1, rows = nyr * (jhi[2] - jlo[2] + 1);
-            for (int rr = sub & 3; rr < rows; rr += 4) {
-                int my, mz;
-                const int cy = wrap_index(jlo[1] + rr % nyr, g.nc[1], my), cz = wrap_index(jlo[2] + rr / nyr, g.nc[2], mz);
-                const int crow = (cz * g.nc[1] + cy) * g.nc[0];
-                for (int x0 = jlo[0]; x0 <= jhi[0];) {
-                    // the part of the row in one periodic image
-                    int mx;
-                    const int cx = wrap_index(x0, g.nc[0], mx);
-                    const int nx = min(jhi[0] - x0 + 1, g.nc[0] - cx);
-                    const int qx = ux - (mx << g.fix), qy = uy - (my << g.fix), qz = uz - (mz << g.fix);
-                    const int k1 = st[crow + cx + nx];
-                    for (int k = st[crow + cx]; k < k1; k += 8) {
-                        f4v s[8];
+        for (int ab = 0; ab < P.nv; ab += 16) {
+            const float wl = ab + sub < P.nv ? vg[ab + sub].w : -1.0f;
+            unsigned open = (unsigned)(__ballot(wl >= 0.0f) >> (lane & 48)) & 0xffffu;
+            while (open) {
+                // four, two or one of the open atoms at a time, `w` lanes each
+                const int left = __popc(open), w = left > 2 ? 4 : (left == 2 ? 8 : 16), wl0 = sub & (w - 1);
+                unsigned mine = open;
+                for (int q = 0; q < 16 / w; q++) {
+                    if (q < sub / w) mine &= mine - 1u;
+                    open &= open - 1u;
+                }
+                if (!mine) continue;
+                const int a = ab + __builtin_ctz(mine);
+                const f4v y = vg[a];
+                const bool isref = a == P.iref;
+                const float R2 = y.w;
+                double y0, y1, y2;
+                if (RANDOM) load3((const double*)yp, a, y0, y1, y2);
+                else load3(xv + (int64_t)f * P.Nv * 3, jbase + a, y0, y1, y2);
+                const int ux = __float_as_int(y.x), uy = __float_as_int(y.y), uz = __float_as_int(y.z);
+                const float rr_ = __builtin_amdgcn_sqrtf(R2) * (1.0f + 1e-5f) + 1e-3f;
+                int jlo[3], jhi[3];
+                cell_range32(g, ux, uy, uz, rr_, rr_, rr_, jlo, jhi);
+                const int nyr = jhi[1] - jlo[1] + 1, rows = nyr * (jhi[2] - jlo[2] + 1);
+                for (int rr = wl0; rr < rows; rr += w) {
+                    int my, mz;
+                    const int cy = wrap_index(jlo[1] + rr % nyr, g.nc[1], my), cz = wrap_index(jlo[2] + rr / nyr, g.nc[2], mz);
+                    const int crow = (cz * g.nc[1] + cy) * g.nc[0];
+                    for (int x0 = jlo[0]; x0 <= jhi[0];) {
+                        // the part of the row in one periodic image
+                        int mx;
+                        const int cx = wrap_index(x0, g.nc[0], mx);
+                        const int nx = min(jhi[0] - x0 + 1, g.nc[0] - cx);
+                        const int qx = ux - (mx << g.fix), qy = uy - (my << g.fix), qz = uz - (mz << g.fix);
+                        const int k1 = st[crow + cx + nx];
+                        for (int k = st[crow + cx]; k < k1; k += 8) {
+                            f4v s[8];
 #pragma unroll
-                        for (int u = 0; u < 8; u++) s[u] = srt[min(k + u, k1 - 1)];
+                            for (int u = 0; u < 8; u++) s[u] = srt[min(k + u, k1 - 1)];
 #pragma unroll
-                        for (int u = 0; u < 8; u++) {
-                            float dx, dy, dz;
-                            fix_cart(g, __float_as_int(s[u].x) - qx, __float_as_int(s[u].y) - qy, __float_as_int(s[u].z) - qz,
-                                     dx, dy, dz);
-                            if (k + u < k1 && fmaf(dx, dx, fmaf(dy, dy, dz * dz)) <= R2) {
-                                const int i = __float_as_int(s[u].w);
-                                double p0, p1, p2;
-                                load3(xuf, i, p0, p1, p2);
-                                const double d2 = cm::canon_d2(B.geo[f].cell, p0, p1, p2, y0, y1, y2);
-                                if (d2 <= P.cut2) rec_offer(r, i, jbase + a, sqrt(d2), isref);
+                            for (int u = 0; u < 8; u++) {
+                                float dx, dy, dz;
+                                fix_cart(g, __float_as_int(s[u].x) - qx, __float_as_int(s[u].y) - qy, __float_as_int(s[u].z) - qz,
+                                         dx, dy, dz);
+                                if (k + u < k1 && fmaf(dx, dx, fmaf(dy, dy, dz * dz)) <= R2) {
+                                    const int i = __float_as_int(s[u].w);
+                                    double p0, p1, p2;
+                                    load3(xuf, i, p0, p1, p2);
+                                    const double d2 = cm::canon_d2(B.geo[f].cell, p0, p1, p2, y0, y1, y2);
+                                    if (d2 <= P.cut2) rec_offer(r, i, jbase + a, sqrt(d2), isref);
+                                }
                             }
                         }
+                        x0 += nx;
                     }
-                    x0 += nx;
                 }
             }
         }
@@ -3488,7 +3768,7 @@ __device__ __forceinline__ void b_resolve(const KP& P, const Bufs& B, const TU* 
 {
     __shared__ int list[RES_CHUNKS * 64];
     __shared__ int nlist;
-    const int nr = RANDOM ? P.NG : 1, mpt = RANDOM ? P.mpt_r : P.mpt, step = resolve_step(P, RANDOM);
+    const int nr = RANDOM ? P.NG : 1, mpt = chunk_molecules(P, B, RANDOM), step = resolve_step(P, RANDOM);
     for (int fq = by_; fq < P.F * nr; fq += nby_) {
         const int f = fq / nr, grp = fq - f * nr;
         const int c0 = ldg(B.chunk_base + fq), c1 = ldg(B.chunk_base + fq + 1);
@@ -3498,7 +3778,7 @@ __device__ __forceinline__ void b_resolve(const KP& P, const Bufs& B, const TU* 
             // one wavefront lists the marked molecules' positions
             if (threadIdx.x < 64) {
                 const int ch = cb + threadIdx.x;
-                ull m = (int)threadIdx.x < step && ch < c1 ? B.resmask[ch] : 0ull;
+                ull m = (int)threadIdx.x < step && ch < c1 ? (mpt > 32 ? ((const ull*)B.resmask)[ch] : B.resmask[ch]) : 0ull;
                 const int n = __popcll(m), incl = wave_incl_scan(n);
                 int o = incl - n;
                 while (m) {
@@ -4452,7 +4732,7 @@ template <bool RANDOM>
 __global__ void __launch_bounds__(1024) km_chunk_table(const MultiTab* __restrict__ MT)
 {
     multi_blocks<RANDOM ? MS_CHUNKK : MS_CHUNK0, true>(MT, [&](const SysDev& S, int bx, int nbx, int by, int nby) {
-        b_chunk_table(S.P, S.B, RANDOM ? 1 : 0, bx, nbx, by, nby);
+        b_chunk_table<true>(S.P, S.B, RANDOM ? 1 : 0, bx, nbx, by, nby);
     });
 }
 
@@ -4858,7 +5138,8 @@ struct cm_job {
     DevBuf near, mkey, mrank, mcnt, mstart, msum, msorted, nnear, chunk_base;
     DevBuf xin_u, xin_v;
     double cell_frac = 0.5;   // tiles family: fine cell side as a fraction of the cutoff
-    int tile_c = 4;           // tiles family: 64 / (solvent molecules per chunk of the real pass): 1, 2, 4 or 8
+    int tile_c = 4;           // tiles family: 64 / (molecules per chunk of the real pass; atoms unless 3 per molecule): 1, 2, 4 or 8
+    bool tuned_c = false;     // tile_c was set (cm_job_set_tuning): chunks keep that size
     int eval_grid = 0;        // tiles family: workgroups of the persistent evaluation kernel (0: fill the device)
     int cus = 256;            // compute units of the device
     int lds_max = 65536;      // LDS bytes one block may use
@@ -5007,8 +5288,14 @@ int64_t cells_for(const cm_job* J, const double* cell9, int64_t* keys)
     return n;
 }
 
-// groups of 16 molecules an evaluating wavefront holds for mpt molecules per chunk
-int chunk_groups(int mpt) { return mpt > 32 ? 4 : (mpt > 16 ? 2 : 1); }
+// tiles of 16 columns an evaluating wavefront holds (eval_chunk's G): molecules
+// of three atoms, or atoms
+int chunk_groups(const KP& P, bool random)
+{
+    const int mpt = random ? P.mpt_r : P.mpt;
+    if (P.mol_lane) return mpt > 32 ? 4 : (mpt > 16 ? 2 : 1);
+    return mpt > lane_molecules(P.nv) ? 8 : 4;
+}
 
 // Wavefronts per block of an evaluation and its LDS: as many (up to 16) as fit
 // one CU's LDS together with the histograms and the chunk table
@@ -5053,15 +5340,14 @@ void launch_tiles_one(hipStream_t s, int grid, const cm_job* J, const KP& P, con
 template <class TU, class TV, bool RANDOM>
 void launch_tiles(hipStream_t s, int grid, const cm_job* J, const KP& P, const Bufs& B, const void* xu, const void* xv)
 {
-    const int g = chunk_groups(RANDOM ? P.mpt_r : P.mpt);
+    const int g = chunk_groups(P, RANDOM);
     if (P.mol_lane) {
         if (g == 4) launch_tiles_one<TU, TV, RANDOM, 4, 3>(s, grid, J, P, B, xu, xv);
         else if (g == 2) launch_tiles_one<TU, TV, RANDOM, 2, 3>(s, grid, J, P, B, xu, xv);
         else launch_tiles_one<TU, TV, RANDOM, 1, 3>(s, grid, J, P, B, xu, xv);
     } else {
-        if (g == 4) launch_tiles_one<TU, TV, RANDOM, 4, TQ_GEN>(s, grid, J, P, B, xu, xv);
-        else if (g == 2) launch_tiles_one<TU, TV, RANDOM, 2, TQ_GEN>(s, grid, J, P, B, xu, xv);
-        else launch_tiles_one<TU, TV, RANDOM, 1, TQ_GEN>(s, grid, J, P, B, xu, xv);
+        if (g == 8) launch_tiles_one<TU, TV, RANDOM, 8, ATOMS>(s, grid, J, P, B, xu, xv);
+        else launch_tiles_one<TU, TV, RANDOM, 4, ATOMS>(s, grid, J, P, B, xu, xv);
     }
 }
 
@@ -5205,7 +5491,7 @@ Bufs batch_bufs(const cm_job* J, Geo* geo)
     B.mcnt = (int*)J->mcnt.p;
     B.mstart = (int*)J->mstart.p;
     B.msum = (int*)J->msum.p;
-    B.resmask = (ull*)J->mkey.p;
+    B.resmask = (unsigned*)J->mkey.p;
     B.msorted = (int*)J->msorted.p;
     B.nnear = (int*)J->nnear.p;
     B.chunk_base = (int*)J->chunk_base.p;
@@ -5299,6 +5585,7 @@ int run_batch(cm_job* J, int F, const int64_t* frame_index, const void* xu_dev, 
     P.cap = (int)cap;
     P.kcap = (int)kcap;
     P.kcapr = (int)(kcap << (3 * P.ksub));
+    P.mpt_auto = chunks_vary(P) ? 1 : 0;
     const bool tiles = J->atoms_family;
     // geometry on the host: cells, inverse, spacings (and the fine grid of the tiles family)
     J->hgeo.assign(F, Geo());
@@ -5405,7 +5692,7 @@ int run_batch(cm_job* J, int F, const int64_t* frame_index, const void* xu_dev, 
             hipLaunchKernelGGL(k_mol_scatter, grid_slots(P.Mv, F), dim3(BLOCK), 0, s, P, B, 0);
             if (f32) hipLaunchKernelGGL(k_fill_real<float>, dim3(grid_for(n)), dim3(BLOCK), 0, s, P, B, vf);
             else hipLaunchKernelGGL(k_fill_real<double>, dim3(grid_for(n)), dim3(BLOCK), 0, s, P, B, vd);
-            hipLaunchKernelGGL(k_chunk_table, dim3(1), dim3(1024), 0, s, P, B, 0);
+            hipLaunchKernelGGL(P.mpt_auto ? k_chunk_table<true> : k_chunk_table<false>, dim3(1), dim3(1024), 0, s, P, B, 0);
         } else {
             int64_t n = (int64_t)F * P.Mv;
             if (f32) hipLaunchKernelGGL(k_prep_solvent<float>, dim3(grid_for(n)), dim3(BLOCK), 0, s, P, B, vf);
@@ -5456,7 +5743,7 @@ int run_batch(cm_job* J, int F, const int64_t* frame_index, const void* xu_dev, 
             hipLaunchKernelGGL(k_mol_scatter, gs, dim3(BLOCK), 0, s, P, B, 1);
             if (f32) hipLaunchKernelGGL(k_place_near<float>, gs, dim3(BLOCK), 0, s, P, B, vf);
             else hipLaunchKernelGGL(k_place_near<double>, gs, dim3(BLOCK), 0, s, P, B, vd);
-            hipLaunchKernelGGL(k_chunk_table, dim3(1), dim3(1024), 0, s, P, B, 1);
+            hipLaunchKernelGGL(P.mpt_auto ? k_chunk_table<true> : k_chunk_table<false>, dim3(1), dim3(1024), 0, s, P, B, 1);
         } else {
             hipLaunchKernelGGL(k_mols_near, grid_slots((P.Mv + NEAR_SLOTS - 1) / NEAR_SLOTS, F * P.K), dim3(BLOCK), 0, s, P, B);
         }
@@ -5517,8 +5804,8 @@ int alloc_batch(cm_job* J, int F, int64_t cap, int64_t kcap, int dtype_size, boo
         }
     } else {
         if ((r = ensure(J, J->near, near_bytes(F, cap)))) return r;
-        // (also one 8-byte word per chunk of a launch: chunks hold 8 molecules
-        // or more, or are the only one of their row)
+        // (also the chunks' resmask: four bytes, eight in chunks of more than 32
+        // molecules; a row may end in a chunk of fewer)
         if ((r = ensure(J, J->mkey, (size_t)4 * F * NP * Mv + (size_t)8 * F * (1 + J->kp.NG)))) return r;
         if ((r = ensure(J, J->mrank, (size_t)4 * F * NP * Mv))) return r;
         KP P = J->kp;
@@ -5529,7 +5816,7 @@ int alloc_batch(cm_job* J, int F, int64_t cap, int64_t kcap, int dtype_size, boo
         if ((r = ensure(J, J->msum, (size_t)4 * F * (scan_parts(P.kcap) + P.NG * scan_parts(P.kcapr))))) return r;
         if ((r = ensure(J, J->msorted, (size_t)4 * F * NP * Mv))) return r;
         if ((r = ensure(J, J->nnear, (size_t)4 * F * (1 + P.NG)))) return r;
-        if ((r = ensure(J, J->chunk_base, (size_t)4 * (F * std::max(J->K, 1) + 2)))) return r;
+        if ((r = ensure(J, J->chunk_base, (size_t)4 * (F * std::max(J->K, 1) + MPT_AT + 1)))) return r;
     }
     if (J->K > 0) {
         if ((r = ensure(J, J->P, (size_t)24 * F * J->K * J->Nv))) return r;
@@ -5712,14 +5999,23 @@ int validate_desc(const cm_job_desc& d)
     return CM_OK;
 }
 
-// Molecules per chunk (one wavefront each): 64 / tile_c in the real pass.  KM
-// random passes place KM times the molecules in the same space, so their
-// chunks hold up to four times as many in no more space.
+// Molecules per chunk (one wavefront each) of the real pass: 64 / tile_c, or for
+// molecules of other than three atoms what 64 / tile_c atoms make.  KM random
+// passes place KM times the molecules in the same space, so their chunks hold
+// up to four times as many in no more space (up to 128 atoms: eight tiles).
 void set_chunks(cm_job* J)
 {
     KP& P = J->kp;
-    P.mpt = 64 / J->tile_c;
-    P.mpt_r = std::min(64, P.mpt * (P.KM >= 8 ? 4 : (P.KM >= 3 ? 2 : 1)));
+    const int share = P.KM >= 8 ? 4 : (P.KM >= 3 ? 2 : 1);
+    if (P.mol_lane) {
+        P.mpt = 64 / J->tile_c;
+        P.mpt_r = std::min(64, P.mpt * share);
+    } else {
+        const int at = 64 / J->tile_c, at_r = at * share;
+        P.mpt = std::max(1, at / P.nv);
+        P.mpt_r = std::max(1, std::min(64, at_r > 64 ? 2 * lane_molecules(P.nv) : at_r / P.nv));
+        P.mpt_auto = J->tuned_c ? 0 : 1;
+    }
 }
 
 // (re)initialises a job on its stream for a validated description; device
@@ -5746,6 +6042,7 @@ void job_params(cm_job* J, const cm_job_desc& d)
     J->launch_ms.clear();
     J->cell_frac = 0.5;
     J->eval_grid = 0;
+    J->tuned_c = false;
     // tiles family: one solute molecule, solvent molecules that fit a wavefront
     J->atoms_family = (d.nmols_u == 1 && !d.autocorrelation && d.natoms_per_mol_v <= 64);
     J->K = d.coordination_number_only ? 0 : d.n_random_samples;
@@ -5790,7 +6087,13 @@ void job_params(cm_job* J, const cm_job_desc& d)
         P.NG = J->K > 0 ? (J->K + P.KM - 1) / P.KM : 0;
         P.ksub = J->K >= 8 * std::max(P.NG, 1) ? 1 : 0;
     }
-    J->tile_c = 4;
+    // Molecules a chunk of the real pass: 16 of one, two or three atoms, 8 and 6 of
+    // four and five, beyond that 64 atoms.  Larger chunks stage solute atoms for
+    // molecules they are not near (5,000 solute atoms, 8 frames, evaluation and
+    // resolve: 12,600 single atoms 44 us with 16, 53 with 32, 78 with 64; 5,000
+    // four-atom molecules 105 with 8, 118 with 16), smaller ones stage the same
+    // atoms more often (6,500 eight-atom molecules 151 with 8, 177 with 4).
+    J->tile_c = P.nv == 1 || P.mol_lane ? 4 : (P.nv <= 5 ? 2 : 1);
     set_chunks(J);
     // Molecule pairs on the matrix cores: molecules of up to CL_ATOMS atoms
     // on both sides, the rows of one tile.  Larger ones would need minima over
@@ -6240,10 +6543,13 @@ int cm_job_set_tuning(cm_job* J, double cell_fraction, int32_t columns, int32_t 
     if (!(cell_fraction >= 0.2 && cell_fraction <= 1.0)) return fail(CM_EINVAL, "cell_fraction must be in [0.2, 1]");
     if (columns != 0 && columns != 1 && columns != 2 && columns != 4 && columns != 8)
         return fail(CM_EINVAL, "columns must be 0 (default), 1, 2, 4 or 8");
-    if (!J->kp.mol_lane && columns > 0 && (64 / columns) / J->kp.nv < 1) return fail(CM_EINVAL, "too many columns for the solvent molecule size");
+    const bool tuned = columns > 0;
+    if (!tuned) columns = J->tile_c;
+    if (!J->kp.mol_lane && (64 / columns) / J->kp.nv < 1) return fail(CM_EINVAL, "too many columns for the solvent molecule size");
     if (eval_workgroups < 0) return fail(CM_EINVAL, "eval_workgroups must be >= 0");
     J->cell_frac = cell_fraction;
-    if (columns > 0) J->tile_c = columns;
+    J->tuned_c = tuned;
+    J->tile_c = columns;
     set_chunks(J);
     J->eval_grid = eval_workgroups;
     return CM_OK;
@@ -6734,18 +7040,26 @@ int multi_hist_words(const KP& P)
 
 // the stage launches of one round (every argument but the table address is
 // fixed per kernel variant, so the sequence can be captured and replayed)
-template <class T, int TQ, int G, int GR>
-void multi_launch(hipStream_t s, const MultiTab* tab, int hist, int lds_max, int cus)
+// (g, gr: chunk_groups of its jobs)
+template <class T, int TQ, bool RANDOM>
+auto multi_eval(int g) -> void (*)(const MultiTab*, int*)
 {
-    auto ev_real = km_eval_tiles<T, T, false, G, TQ>;
-    auto ev_rand = km_eval_tiles<T, T, true, GR, TQ>;
+    if constexpr (TQ == ATOMS) return g == 8 ? km_eval_tiles<T, T, RANDOM, 8, TQ> : km_eval_tiles<T, T, RANDOM, 4, TQ>;
+    else return g == 4 ? km_eval_tiles<T, T, RANDOM, 4, TQ> : (g == 2 ? km_eval_tiles<T, T, RANDOM, 2, TQ> : km_eval_tiles<T, T, RANDOM, 1, TQ>);
+}
+
+template <class T, int TQ>
+void multi_launch(int g, int gr, hipStream_t s, const MultiTab* tab, int hist, int lds_max, int cus)
+{
+    auto ev_real = multi_eval<T, TQ, false>(g);
+    auto ev_rand = multi_eval<T, TQ, true>(gr);
     // (the chunk tables of multi_tickets are static LDS)
-    auto waves = [&](int g) {
-        return (int)std::max<int64_t>(1, std::min<int64_t>(16, (lds_max - 2048 - 4 * (int64_t)hist) / (4 * (int64_t)eval_wave_words(g, TQ))));
+    auto waves = [&](int n) {
+        return (int)std::max<int64_t>(1, std::min<int64_t>(16, (lds_max - 2048 - 4 * (int64_t)hist) / (4 * (int64_t)eval_wave_words(n, TQ))));
     };
-    const int w_real = waves(G), w_rand = waves(GR);
-    const size_t shm = 4 * ((size_t)hist + (size_t)w_real * eval_wave_words(G, TQ));
-    const size_t shm_r = 4 * ((size_t)hist + (size_t)w_rand * eval_wave_words(GR, TQ));
+    const int w_real = waves(g), w_rand = waves(gr);
+    const size_t shm = 4 * ((size_t)hist + (size_t)w_real * eval_wave_words(g, TQ));
+    const size_t shm_r = 4 * ((size_t)hist + (size_t)w_rand * eval_wave_words(gr, TQ));
     // persistent grids of the two evaluations
     const int g_real = persistent_grid(ev_real, 64 * w_real, shm, cus);
     const int g_rand = persistent_grid(ev_rand, 64 * w_rand, shm_r, cus);
@@ -6777,36 +7091,24 @@ void multi_launch(hipStream_t s, const MultiTab* tab, int hist, int lds_max, int
     hipLaunchKernelGGL((km_resolve<T, T, true>), dim3(MG_RES), dim3(BLOCK), 0, s, tab);
 }
 
-// groups of molecules per wavefront of the jobs of a variant (multi_variant)
-template <class T, int TQ>
-void multi_launch_g(int g, int gr, hipStream_t s, const MultiTab* tab, int hist, int lds_max, int cus)
-{
-    if (g == 4) multi_launch<T, TQ, 4, 4>(s, tab, hist, lds_max, cus);
-    else if (g == 2 && gr == 4) multi_launch<T, TQ, 2, 4>(s, tab, hist, lds_max, cus);
-    else if (g == 2) multi_launch<T, TQ, 2, 2>(s, tab, hist, lds_max, cus);
-    else if (gr == 4) multi_launch<T, TQ, 1, 4>(s, tab, hist, lds_max, cus);
-    else if (gr == 2) multi_launch<T, TQ, 1, 2>(s, tab, hist, lds_max, cus);
-    else multi_launch<T, TQ, 1, 1>(s, tab, hist, lds_max, cus);
-}
-
 void multi_launch_any(int dtype, const cm_job* J, hipStream_t s, const MultiTab* tab, int cus)
 {
-    const int g = chunk_groups(J->kp.mpt), gr = chunk_groups(J->kp.mpt_r);
+    const int g = chunk_groups(J->kp, false), gr = chunk_groups(J->kp, true);
     const int hist = multi_hist_words(J->kp), lds_max = J->lds_max;
     if (dtype == CM_F32) {
-        if (J->kp.mol_lane) multi_launch_g<float, 3>(g, gr, s, tab, hist, lds_max, cus);
-        else multi_launch_g<float, TQ_GEN>(g, gr, s, tab, hist, lds_max, cus);
+        if (J->kp.mol_lane) multi_launch<float, 3>(g, gr, s, tab, hist, lds_max, cus);
+        else multi_launch<float, ATOMS>(g, gr, s, tab, hist, lds_max, cus);
     } else {
-        if (J->kp.mol_lane) multi_launch_g<double, 3>(g, gr, s, tab, hist, lds_max, cus);
-        else multi_launch_g<double, TQ_GEN>(g, gr, s, tab, hist, lds_max, cus);
+        if (J->kp.mol_lane) multi_launch<double, 3>(g, gr, s, tab, hist, lds_max, cus);
+        else multi_launch<double, ATOMS>(g, gr, s, tab, hist, lds_max, cus);
     }
 }
 
 // jobs that share the kernels of a round's launches
 int multi_variant(int dtype, const cm_job* J)
 {
-    return (dtype == CM_F32 ? 1 : 0) | (J->kp.mol_lane ? 2 : 0) | (chunk_groups(J->kp.mpt) << 2) | (chunk_groups(J->kp.mpt_r) << 5) |
-           (multi_hist_words(J->kp) << 8);
+    return (dtype == CM_F32 ? 1 : 0) | (J->kp.mol_lane ? 2 : 0) | (chunk_groups(J->kp, false) << 2) |
+           (chunk_groups(J->kp, true) << 6) | (multi_hist_words(J->kp) << 10);
 }
 
 // one job's part of a multi-job submission
@@ -6903,6 +7205,7 @@ int multi_run_group(MultiRunner& R, std::vector<MJob>& grp, int dtype)
                 S.P.cap = (int)m.cap;
                 S.P.kcap = (int)m.kcap;
                 S.P.kcapr = (int)(m.kcap << (3 * S.P.ksub));
+                S.P.mpt_auto = chunks_vary(S.P) ? 1 : 0;
                 S.B = batch_bufs(J, gd + goff);
                 S.B.dfield = (unsigned*)((char*)J->near.p + near_flags_bytes(F, m.cap));
                 S.xu = (const char*)fr.d_x_solute + (size_t)f0 * J->Nu * 3 * ds;

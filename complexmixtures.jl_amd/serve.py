@@ -253,9 +253,9 @@ def service_breakdown(reqs, service):
 
 
 def tuning_candidates(natoms_per_mol_v):
-    """Cell fractions x columns per row: a row is a whole molecule for 3-atom
-    solvent molecules (2-8 columns: 32-8 molecules per chunk), one solvent
-    atom otherwise (1-2 columns)."""
+    """Cell fractions x columns: 64 / columns solvent molecules per chunk for
+    3-atom molecules (2-8 columns: 32-8 molecules), 64 / columns atoms
+    otherwise (1-2 columns)."""
     cols = (2, 4, 8) if natoms_per_mol_v == 3 else (1, 2)
     return [dict(cell_fraction=cf, columns=c) for cf in (0.35, 0.5, 0.75, 1.0) for c in cols]
 

@@ -189,10 +189,12 @@ int cm_multi_stats(int64_t *rounds, int64_t *launches);
 
 /* Tuning of the single-solute kernels (no counterpart in the reference; the
  * reference's Options.lcell plays this role for CellListMap): fine cell side
- * as a fraction of the cutoff (0.2-1.0), columns (1, 2, 4 or 8: 64 / columns
- * solvent molecules per wavefront of the real pass, up to four times as many
- * in the random passes; 0 keeps the default, 4) and workgroups of the
- * persistent evaluation kernel (0 = as many as the device holds at once).
+ * as a fraction of the cutoff (0.2-1.0), columns (1, 2, 4 or 8: a wavefront of
+ * the real pass takes 64 / columns solvent molecules of three atoms, or the
+ * molecules that 64 / columns atoms make, refused where that is none; up to four
+ * times as many in the random passes; 0 keeps the default: 4 for three atoms,
+ * else chosen by the library) and workgroups of the persistent evaluation
+ * kernel (0 = as many as the device holds at once).
  * Results do not depend on these. */
 int cm_job_set_tuning(cm_job *job, double cell_fraction, int32_t columns, int32_t eval_workgroups);
 

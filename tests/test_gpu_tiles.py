@@ -58,3 +58,41 @@ def test_molecules_per_chunk(pkg, oracle, columns):
     opts = pkg.Options(bulk_range=(8.0, 11.0), n_random_samples=10, seed=19, silent=True)
     a, _ = oracle_raw(pkg, oracle, traj, opts)
     assert_raw_equal(a, gpu_raw(pkg, traj, opts, job_kw={"tuning": dict(columns=columns)}))
+
+
+@pytest.mark.parametrize("nu,nmols,nv,passes,frames", [
+    (3, 400, 8, 330, 2), (90, 500, 4, 200, 2), (40, 300, 1, 220, 3), (60, 150, 14, 200, 2), (30, 100, 24, 130, 3),
+    (12, 60, 40, 330, 2), (130, 4, 63, 1100, 8)])
+@pytest.mark.parametrize("triclinic", [False, True])
+def test_chunks_of_several_blocks(pkg, oracle, nu, nmols, nv, passes, frames, triclinic):
+    """Enough random slots around a sparse solute for chunks of up to 512 atoms: several blocks of 128 atoms from one
+    staging, and (130 atoms) more staged atoms than the buffer takes, each block on its own."""
+    traj = _system(pkg, nu, nmols, nv, nframes=frames, seed=5, triclinic=triclinic)
+    traj.xu[:] = np.random.default_rng(nu).uniform(0.0, 26.0, size=traj.xu.shape[1:])
+    opts = pkg.Options(dbulk=9.0, n_random_samples=passes, seed=21, silent=True, irefatom=min(2, nv))
+    a, _ = oracle_raw(pkg, oracle, traj, opts, nthreads=8)
+    assert_raw_equal(a, gpu_raw(pkg, traj, opts))
+
+
+def test_real_chunks_of_several_blocks(pkg, oracle):
+    """48 frames of 900 molecules: chunks of five molecules, two blocks of 64 lanes, in the real pass."""
+    traj = _system(pkg, 20, 900, 14, nframes=48, seed=6)
+    traj.xu[:] = np.random.default_rng(6).uniform(0.0, 26.0, size=traj.xu.shape[1:])
+    opts = pkg.Options(dbulk=9.0, seed=22, silent=True)
+    a, _ = oracle_raw(pkg, oracle, traj, opts, coordination_number_only=True, nthreads=8)
+    assert_raw_equal(a, gpu_raw(pkg, traj, opts, coordination_number_only=True))
+
+
+@pytest.mark.parametrize("columns,nv", [(1, 8), (2, 8), (4, 8), (8, 8), (1, 14), (2, 14), (4, 14), (8, 14), (1, 63), (2, 63),
+                                        (0, 63)])
+def test_atoms_per_chunk(pkg, oracle, columns, nv):
+    """64 / columns atoms per chunk of molecules of other than three; where that holds no molecule, the setting is refused."""
+    traj = _system(pkg, 300, 120, nv, seed=7)
+    opts = pkg.Options(dbulk=9.0, n_random_samples=10, seed=23, silent=True)
+    kw = {"job_kw": {"tuning": dict(columns=columns)}}
+    if columns and 64 // columns < nv:
+        with pytest.raises(pkg.ArgumentError):
+            gpu_raw(pkg, traj, opts, **kw)
+        return
+    a, _ = oracle_raw(pkg, oracle, traj, opts)
+    assert_raw_equal(a, gpu_raw(pkg, traj, opts, **kw))
