@@ -1230,30 +1230,6 @@ struct PairCtx {
         }
     }
 
-    // the record of a cross pair from FP64 distances alone (not counted here)
-    __device__ void cross_exhaustive(int u, int v) const
-    {
-        Rec r = rec_zero();
-        const int64_t ub = (int64_t)u * P.nu, vb = (int64_t)v * P.nv;
-#pragma unroll 1
-        for (int a = 0; a < P.nv; a++) {
-            double y0, y1, y2;
-            load3(xvf, vb + a, y0, y1, y2);
-#pragma unroll 1
-            for (int i = 0; i < P.nu; i++) {
-                double x0, x1, x2;
-                load3(xuf, ub + i, x0, x1, x2);
-                const double d2 = cm::canon_d2(g.cell, x0, x1, x2, y0, y1, y2);
-                if (d2 <= P.cut2) rec_offer(r, i, vb + a, sqrt(d2), a == P.iref);
-            }
-        }
-        rec_complete(P, r);
-        hist_record_mols(P, sh, shg, B.cnt_gu, B.cnt_gv, r);
-        if (P.K > 0 && r.within)
-            for (int qq = dp[u]; qq < dp[u + 1]; qq++)
-                B.bflag[((int64_t)f * P.kb + di[qq]) * P.Mv + v] = inbulk(P, r) ? 1 : 0;
-    }
-
     __device__ void rdf_hit(int bin) const
     {
         if (bin < P.nbins) atomicAdd(&sh[P.nbins + bin], 1u);
@@ -1353,18 +1329,18 @@ struct PairCtx {
                 }
             }
         }
-        rec_complete(P, r1);
-        rec_complete(P, r2);
-        hist_record_mols(P, sh, shg, B.cnt_gu, B.cnt_gv, r1);
-        hist_record_mols(P, sh, shg, B.cnt_gu, B.cnt_gv, r2);
-        if (P.K > 0) {
-            if (r1.within)
-                for (int qq = dp[u]; qq < dp[u + 1]; qq++)
-                    B.bflag[((int64_t)f * P.kb + di[qq]) * P.Mv + v] = inbulk(P, r1) ? 1 : 0;
-            if (r2.within)
-                for (int qq = dp[v]; qq < dp[v + 1]; qq++)
-                    B.bflag[((int64_t)f * P.kb + di[qq]) * P.Mv + u] = inbulk(P, r2) ? 1 : 0;
-        }
+        exact_record(u, v, r1);
+        exact_record(v, u, r2);
+    }
+
+    // counts and dbulk flags of the FP64 record of solvent molecule v about u
+    __device__ void exact_record(int u, int v, Rec r) const
+    {
+        rec_complete(P, r);
+        hist_record_mols(P, sh, shg, B.cnt_gu, B.cnt_gv, r);
+        if (P.K > 0 && r.within)
+            for (int qq = dp[u]; qq < dp[u + 1]; qq++)
+                B.bflag[((int64_t)f * P.kb + di[qq]) * P.Mv + v] = inbulk(P, r) ? 1 : 0;
     }
 
     // one queued pair {u, v, cell of u, shift code or -1}: every shift of the
@@ -3850,7 +3826,7 @@ struct ClArgs {
     Bufs B;
     const TU* xu;
     const TV* xv;
-    int S;
+    int S, Sg;
 };
 
 // Sort key of a molecule, the 2^bits grid cell of its centre, and the largest
@@ -4135,18 +4111,60 @@ __device__ __forceinline__ float2 row_pair(float x)
 
 // Out of line, with the kernel's arguments read where they are used and the
 // histograms by their LDS address (flat atomics took five times as long; glds:
-// words before the group histograms, 0: none): the FP64 record of a deferred
-// pair (input indices) ...
+// words before the group histograms, 0: none): the FP64 record of a deferred ...
 using CArgs = __attribute__((address_space(4))) const char*;
 using LdsU = __attribute__((address_space(3))) unsigned*;
+// ... pair (input indices; u < 0: none), by `width` lanes that take its atom pairs
+// in turn (sub: this lane's place among them).  One lane a pair walks them all:
+// 100 us and more for the few pairs that a wavefront of a small job ends with
+// (30 frames of 500 eight-atom molecules in a 60 A box: 164 us, 101 us so)
 template <class TU, class TV, bool SELF>
-__device__ __attribute__((noinline)) void cl_exact(CArgs k, int f, int u, int v, LdsU sh_, int glds)
+__device__ __attribute__((noinline)) void cl_exact(CArgs k, int f, int u, int v, int sub, int width, LdsU sh_, int glds)
 {
     unsigned *const sh = (unsigned*)sh_, *const shg = glds ? sh + glds : nullptr;
-    const ClArgs<TU, TV>& a = *(const ClArgs<TU, TV>*)k;
-    const PairCtx<TU, TV, 0> ctx(a.P, a.B, f, a.xu, a.xv, sh, shg);
-    if (SELF) ctx.self_exhaustive(u, v);
-    else ctx.cross_exhaustive(u, v);
+    const ClArgs<TU, TV>& A = *(const ClArgs<TU, TV>*)k;
+    const KP& P = A.P;
+    const TU* x = A.xu + (int64_t)f * P.Nu * 3;
+    const TV* y = (SELF ? (const TV*)A.xu : A.xv) + (int64_t)f * P.Nv * 3;
+    const int64_t ub = (int64_t)u * P.nu, vb = (int64_t)v * P.nv;
+    Rec r1 = rec_zero(), r2 = rec_zero();
+    const cm::Cell64& c = A.B.geo[f].cell;
+    auto offer = [&](int i, int a, double y0, double y1, double y2) {
+        double x0, x1, x2;
+        load3(x, ub + i, x0, x1, x2);
+        const double d2 = cm::canon_d2(c, x0, x1, x2, y0, y1, y2);
+        if (d2 <= P.cut2) {
+            const double d = sqrt(d2);
+            rec_offer(r1, i, vb + a, d, a == P.iref);
+            if (SELF) rec_offer(r2, a, ub + i, d, i == P.iref);
+        }
+    };
+    const int na = u < 0 ? 0 : P.nv;
+    double y0, y1, y2;
+    if (width <= P.nu) {
+        // every lane has some of an atom's pairs
+#pragma unroll 1
+        for (int a = 0; a < na; a++) {
+            load3(y, vb + a, y0, y1, y2);
+#pragma unroll 1
+            for (int i = sub; i < P.nu; i += width) offer(i, a, y0, y1, y2);
+        }
+    } else {
+#pragma unroll 1
+        for (int p = sub; p < na * P.nu; p += width) {
+            const int a = p / P.nu;
+            load3(y, vb + a, y0, y1, y2);
+            offer(p - a * P.nu, a, y0, y1, y2);
+        }
+    }
+    for (int o = 1; o < width; o <<= 1) {
+        rec_merge(r1, rec_shfl_xor(r1, o));
+        if (SELF) rec_merge(r2, rec_shfl_xor(r2, o));
+    }
+    if (u < 0 || sub != 0) return;
+    const PairCtx<TU, TV, 0> ctx(P, A.B, f, A.xu, A.xv, sh, shg);
+    ctx.exact_record(u, v, r1);
+    if (SELF) ctx.exact_record(v, u, r2);
 }
 
 // ... and the updates of a decided pair where there is more than the plain
@@ -4165,7 +4183,7 @@ __device__ __attribute__((noinline)) void cl_main(CArgs k, int f, int u, int v, 
 // the k-th eighth of the (frame, cluster) items in frame-major order, so its L2
 // holds one or two frames at a time.
 template <class TU, class TV, int RPM, int NVT, bool SELF>
-__global__ void __launch_bounds__(NVT > 8 ? 512 : 1024) k_cl_eval(KP P_, Bufs B_, const TU* xu_, const TV* xv_, int S)
+__global__ void __launch_bounds__(NVT > 8 ? 512 : 1024) k_cl_eval(KP P_, Bufs B_, const TU* xu_, const TV* xv_, int S, int Sg_)
 {
     constexpr int mp = 16 / RPM, RL = RPM / 4;   // molecules per tile, lane groups per molecule
     constexpr int QB = NVT <= 4 ? 2 : (NVT <= 8 ? 3 : 4);
@@ -4194,11 +4212,13 @@ __global__ void __launch_bounds__(NVT > 8 ? 512 : 1024) k_cl_eval(KP P_, Bufs B_
 
     auto deferred = [&](int n) {
         wave_sync();
-        if (lane < n) {
-            CArgs ka = k0;
-            asm volatile("" : "+s"(ka));
-            cl_exact<TU, TV, SELF>(ka, fcur, dq[2 * (dn - n + lane)], dq[2 * (dn - n + lane) + 1], (LdsU)sh, shg ? 2 * P.nbins : 0);
-        }
+        int w = 1;   // lanes per pair
+        CArgs ka = k0;
+        asm volatile("" : "+s"(ka));
+        const ClArgs<TU, TV>& E = *(const ClArgs<TU, TV>*)ka;
+        while (2 * w * n <= 64 && w < E.P.nu * E.P.nv) w *= 2;
+        const int e = lane / w, o = 2 * (dn - n + min(e, n - 1));
+        cl_exact<TU, TV, SELF>(ka, fcur, e < n ? dq[o] : -1, dq[o + 1], lane & (w - 1), w, (LdsU)sh, shg ? 2 * P.nbins : 0);
         wave_sync();
         dn -= n;
         nexact += n;
@@ -4213,6 +4233,9 @@ __global__ void __launch_bounds__(NVT > 8 ? 512 : 1024) k_cl_eval(KP P_, Bufs B_
         const int f = __builtin_amdgcn_readfirstlane((int)(fbv / A.P.nB));
         const int b = __builtin_amdgcn_readfirstlane((int)(fbv - (int64_t)f * A.P.nB));
         const int64_t fb = (int64_t)f * A.P.nB + b;
+        // split items (S > 1): the super tiles in reach go round Sg of them, the
+        // tiles of those round S / Sg (Sg from the arguments where it is used: held
+        // over the launch it cost 2 % of large ones)
         const int s = (int)(it - fb * S);
         if (f != fcur) {
             while (dn > 0) deferred(min(dn, 64));
@@ -4324,7 +4347,7 @@ __global__ void __launch_bounds__(NVT > 8 ? 512 : 1024) k_cl_eval(KP P_, Bufs B_
         const float rc = (float)A.P.cutsys + 2e-3f + 1e-6f * ((float)g.sp[0] + (float)g.sp[1] + (float)g.sp[2]);
         const gptr<const float> ca = (gptr<const float>)(A.B.clA + (int64_t)f * A.P.nT * 64);
         const int nS = A.P.nS;
-        int turn = 0;   // tiles in reach so far: split items (S > 1) take every S-th
+        int turn = 0, sturn = 0;   // tiles, super tiles in reach so far (split items)
         int sb = -64;
         unsigned long long smask = 0, tm = 0;
         int tile = 0, sets = 0, tn = -1;
@@ -4353,6 +4376,11 @@ __global__ void __launch_bounds__(NVT > 8 ? 512 : 1024) k_cl_eval(KP P_, Bufs B_
                         in = cl_reach(gr, rc, si[0], si[1], bm, bh, sets);
                     }
                     smask = __ballot(in);
+                    if (S > 1 && R.Sg > 1) {
+                        const int rank = sturn + __popcll(smask & lt);
+                        sturn = __builtin_amdgcn_readfirstlane((sturn + __popcll(smask)) % R.Sg);
+                        smask = __ballot(in && rank % R.Sg == s % R.Sg);
+                    }
                     continue;
                 }
                 int mine = -1;
@@ -4384,9 +4412,9 @@ __global__ void __launch_bounds__(NVT > 8 ? 512 : 1024) k_cl_eval(KP P_, Bufs B_
                 wave_sync();
                 tm = __ballot(ok);
                 if (S > 1) {
-                    const int rank = turn + __popcll(tm & lt);
-                    turn = __builtin_amdgcn_readfirstlane((turn + __popcll(tm)) % S);
-                    tm = __ballot(ok && rank % S == s);
+                    const int rank = turn + __popcll(tm & lt), St = S / R.Sg;
+                    turn = __builtin_amdgcn_readfirstlane((turn + __popcll(tm)) % St);
+                    tm = __ballot(ok && rank % St == s / R.Sg);
                 }
             }
             if (tm) {
@@ -5540,12 +5568,17 @@ void launch_cl_one(hipStream_t s, const cm_job* J, const KP& P, const Bufs& B, c
     const size_t lds = (size_t)(head + 4 * (int64_t)CL_WORDS * waves);
     int nb = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kern, 64 * waves, lds) != hipSuccess || nb < 1) nb = 1;
-    // small systems: S wavefronts split a cluster's tiles, so that every
-    // wavefront of the device has about two items
+    // Few clusters: S wavefronts split a cluster's tiles, so that every wavefront
+    // of the device has about two items of four tiles or more; first by super
+    // tiles (a wavefront tests the tiles of its own only), eight each.  Ten frames
+    // of 40 ions in 8,000 waters, 30 clusters of up to 2,000 tiles: 249 us with 16
+    // wavefronts a cluster, 76 us so.
     const int64_t items = (int64_t)P.F * P.nB, want = 2 * (int64_t)nb * J->cus * waves;
-    const int S = (int)std::min<int64_t>(16, std::max<int64_t>(1, want / std::max<int64_t>(items, 1)));
+    const int64_t most = std::max(P.nT / 4, std::min(16, P.nT));
+    const int S0 = (int)std::min<int64_t>(most, std::max<int64_t>(1, want / std::max<int64_t>(items, 1)));
+    const int Sg = std::min(S0, std::max(1, P.nS / 8)), S = (S0 + Sg - 1) / Sg * Sg;
     const int64_t blocks = std::min<int64_t>((int64_t)nb * J->cus, (items * S + waves - 1) / waves);
-    hipLaunchKernelGGL(kern, dim3((unsigned)((blocks + 7) / 8 * 8)), dim3(64 * waves), lds, s, P, B, (const T*)xu, (const T*)xv, S);
+    hipLaunchKernelGGL(kern, dim3((unsigned)((blocks + 7) / 8 * 8)), dim3(64 * waves), lds, s, P, B, (const T*)xu, (const T*)xv, S, Sg);
 }
 
 template <class T, int RPM>

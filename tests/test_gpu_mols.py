@@ -96,3 +96,25 @@ def test_group_histograms_in_and_beyond_lds(pkg, oracle, binstep):
     """17 groups of 400, 800 and 1,600 bins: 27, 54 and 109 kB, of which 64 kB may lie in LDS."""
     traj = _traj(pkg, 14, 12, 3, 150, seed=8)
     _check(pkg, oracle, traj, dbulk=8.0, binstep=binstep, n_random_samples=3)
+
+
+@pytest.mark.parametrize("nu,mu,nv,mv", [(1, 1100, 1, 5), (3, 1500, 1, 20), (4, 2100, 3, 33), (8, 700, 8, 17), (14, 300, 2, 16)])
+def test_many_tiles_few_clusters(pkg, oracle, nu, mu, nv, mv):
+    """One to three clusters a frame: their super tiles, and those tiles, split over many wavefronts."""
+    _check(pkg, oracle, _traj(pkg, nu, mu, nv, mv, box=40.0, nframes=1, seed=9, angle=80.0), dbulk=9.0, n_random_samples=2)
+
+
+@pytest.mark.parametrize("nu,nv", [(1, 1), (2, 3), (5, 8), (14, 3), (16, 16)])
+@pytest.mark.parametrize("mv", [3, 40])
+def test_exact_ties_between_species(pkg, oracle, nu, nv, mv):
+    """Whole Angstroms on both sides: every pair in reach is left to FP64, few (several lanes a pair) and many."""
+    t = _traj(pkg, nu, 6, nv, mv, nframes=2, seed=10, broken=False)
+    t.xu[:], t.xv[:] = np.round(t.xu), np.round(t.xv)
+    _check(pkg, oracle, t, dbulk=8.0, n_random_samples=3, irefatom=nv)
+
+
+@pytest.mark.parametrize("n,m", [(2, 7), (8, 30), (14, 9)])
+def test_exact_ties_of_larger_molecules(pkg, oracle, n, m):
+    t = _traj(pkg, 0, 0, n, m, nframes=2, seed=11, broken=False)
+    t.xv[:] = np.round(t.xv)
+    _check(pkg, oracle, t, dbulk=8.0, n_random_samples=3, irefatom=n)
