@@ -146,7 +146,8 @@ struct KP {                  // job parameters, by value
     int ksub;                // bits per dimension the random groups' keys have beyond them
     int kcapr;               // sort keys of a random group: kcap << 3 ksub
     // molecule pairs on the matrix cores: rows per solute molecule in an A
-    // tile (0: not used); A tiles, super tiles and B clusters per frame
+    // tile (0: not used; 1: single atoms on both sides); A tiles, super tiles and B
+    // clusters per frame
     int rpm, nT, nS, nB;
     int place_all;           // verification: every slot of a random pass placed (molecule pairs), FP64 positions kept (tiles)
 };
@@ -4187,7 +4188,11 @@ __global__ void __launch_bounds__(NVT > 8 ? 512 : 1024) k_cl_eval(KP P_, Bufs B_
 {
     constexpr int mp = 16 / RPM, RL = RPM / 4;   // molecules per tile, lane groups per molecule
     constexpr int QB = NVT <= 4 ? 2 : (NVT <= 8 ? 3 : 4);
-    constexpr int CBITS = 2 + QB + (RPM == 4 ? 0 : (RPM == 8 ? 1 : 2));   // code: row of the lane, solvent atom, lane group
+    // (RPM 1: single atoms on both sides, a row is a molecule and a lane holds four
+    // pairs, with nothing to choose between: 30,000 atoms in a 97 A box, 6 frames,
+    // 551 us in rows of four, 271 us so; the cell walk 373)
+    constexpr bool ONE = RPM == 1;
+    constexpr int CBITS = ONE ? 0 : 2 + QB + (RPM == 4 ? 0 : (RPM == 8 ? 1 : 2));   // code: row of the lane, solvent atom, lane group
     constexpr int CMASK = (1 << CBITS) - 1;
     CArgs k0 = (CArgs)__builtin_amdgcn_kernarg_segment_ptr();
     const KP& P = *(const KP*)k0;
@@ -4314,7 +4319,7 @@ __global__ void __launch_bounds__(NVT > 8 ? 512 : 1024) k_cl_eval(KP P_, Bufs B_
                     v = (int)(ov & ~CL_DRAWN);
                 }
                 if (dm == 2 && !def) {
-                    const int row = (code & 3) + (RPM == 4 ? 0 : 4 * (code >> (2 + QB)));
+                    const int row = ONE ? 0 : (code & 3) + (RPM == 4 ? 0 : 4 * (code >> (2 + QB)));
                     const int q = cl_atom((code >> 2) & ((1 << QB) - 1), Q.P.iref), i = SELF ? cl_atom(row, Q.P.iref) : row;
                     const int nb = Q.P.nbins;
                     if (plain && !drawn) {
@@ -4429,6 +4434,7 @@ __global__ void __launch_bounds__(NVT > 8 ? 512 : 1024) k_cl_eval(KP P_, Bufs B_
             }
             if (t >= 0) {
                 float bb = INFINITY, ms = INFINITY, rv = INFINITY, ru = INFINITY;
+                f4m one = {INFINITY, INFINITY, INFINITY, INFINITY};   // ONE: the lane's pairs
                 int xs = st & 7, ys = (st >> 3) & 7, zs = st >> 6;
                 for (;;) {
                     const float at = kk == 3 ? 1.0f : nt0, ct = kk == 3 ? nt0 : 0.f, bt = kk == 3 ? 0.f : 2.0f * nt0;
@@ -4439,6 +4445,11 @@ __global__ void __launch_bounds__(NVT > 8 ? 512 : 1024) k_cl_eval(KP P_, Bufs B_
                         const f4m c = QUAD ? __builtin_amdgcn_mfma_f32_16x16x4f32(nt0, Z[q], f4m{Y[q], Y[q], Y[q], Y[q]}, 0, 0, 0)
                                            : __builtin_amdgcn_mfma_f32_16x16x4f32(at, Y[q] + ct, f4m{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
                         f4m d = __builtin_amdgcn_mfma_f32_16x16x4f32(a, Z[q] + bt, c, 0, 0, 0);
+                        if constexpr (ONE) {
+#pragma unroll
+                            for (int r = 0; r < 4; r++) one[r] = fminf(one[r], d[r]);
+                            continue;
+                        }
 #pragma unroll
                         for (int r = 0; r < 4; r++) d[r] = __int_as_float((__float_as_int(d[r]) & ~CMASK) | (r | (q << 2)));
                         min2_4(bb, ms, d);
@@ -4458,6 +4469,25 @@ __global__ void __launch_bounds__(NVT > 8 ? 512 : 1024) k_cl_eval(KP P_, Bufs B_
                              dz + (__builtin_ctz(zs) - 1) * (1 << g.fix), tx, ty, tz);
                     nt0 = kk == 0 ? tx : (kk == 1 ? ty : (kk == 2 ? tz : fmaf(tx, tx, fmaf(ty, ty, tz * tz))));
                 }
+                if constexpr (ONE) {
+                    // (two images of a molecule within reach: the nearer one)
+#pragma unroll 1
+                    for (int r = 0; r < 4; r++) {
+                        const float x = one[0];
+                        one = f4m{one[1], one[2], one[3], INFINITY};
+                        unsigned long long m = __ballot(x <= thr);
+                        if (SELF && t == b) m &= __ballot(4 * kk + r > col);
+                        if (__builtin_amdgcn_inverse_ballot_w64(m)) {
+                            const int k = qn + __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0));
+                            qv[k] = x; qv[CL_Q + k] = x;
+                            if (SELF) qv[2 * CL_Q + k] = x;
+                            qi[3 * CL_Q + k] = t * mp + 4 * kk + r;
+                            qi[4 * CL_Q + k] = col;
+                        }
+                        qn += __popcll(m);
+                        if (r < 3 && qn >= 64) count(64);
+                    }
+                }
                 // lane groups holding the other rows of the molecule
                 if constexpr (RPM > 4) {
                     bb = __int_as_float(__float_as_int(bb) | ((kk & (RL - 1)) << (2 + QB)));
@@ -4475,18 +4505,20 @@ __global__ void __launch_bounds__(NVT > 8 ? 512 : 1024) k_cl_eval(KP P_, Bufs B_
                     merge([](float x) { return row_pair<16>(x); });
                     if constexpr (RPM > 8) merge([](float x) { return row_pair<32>(x); });
                 }
-                const int up = t * mp + (RPM == 4 ? kk : (RPM == 8 ? kk >> 1 : 0));
-                unsigned long long m = __ballot((RPM == 4 || (kk & (RL - 1)) == 0) && bb <= thr);
-                if (SELF && t * mp / 16 == b) m &= __ballot((up & 15) > col);
-                const bool hit = __builtin_amdgcn_inverse_ballot_w64(m);
-                if (hit) {
-                    const int k = qn + __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0));
-                    qv[k] = bb; qv[CL_Q + k] = rv;
-                    if (SELF) qv[2 * CL_Q + k] = ru;
-                    qi[3 * CL_Q + k] = up;
-                    qi[4 * CL_Q + k] = col | (ms - bb > ambx ? 0 : 256);
+                if constexpr (!ONE) {
+                    const int up = t * mp + (RPM == 4 ? kk : (RPM == 8 ? kk >> 1 : 0));
+                    unsigned long long m = __ballot((RPM == 4 || (kk & (RL - 1)) == 0) && bb <= thr);
+                    if (SELF && t * mp / 16 == b) m &= __ballot((up & 15) > col);
+                    const bool hit = __builtin_amdgcn_inverse_ballot_w64(m);
+                    if (hit) {
+                        const int k = qn + __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0));
+                        qv[k] = bb; qv[CL_Q + k] = rv;
+                        if (SELF) qv[2 * CL_Q + k] = ru;
+                        qi[3 * CL_Q + k] = up;
+                        qi[4 * CL_Q + k] = col | (ms - bb > ambx ? 0 : 256);
+                    }
+                    qn += __popcll(m);
                 }
-                qn += __popcll(m);
             }
             const bool last = tn < 0 && t < 0 && !more;
             if (qn >= 64 || last) count(min(qn, 64));
@@ -5569,14 +5601,16 @@ void launch_cl_one(hipStream_t s, const cm_job* J, const KP& P, const Bufs& B, c
     int nb = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kern, 64 * waves, lds) != hipSuccess || nb < 1) nb = 1;
     // Few clusters: S wavefronts split a cluster's tiles, so that every wavefront
-    // of the device has about two items of four tiles or more; first by super
-    // tiles (a wavefront tests the tiles of its own only), eight each.  Ten frames
-    // of 40 ions in 8,000 waters, 30 clusters of up to 2,000 tiles: 249 us with 16
-    // wavefronts a cluster, 76 us so.
+    // of the device has about two items of four tiles or more; beyond 16 by super
+    // tiles first, eight or more each (a wavefront tests the tiles of its own only;
+    // below, the tiles divide more evenly).  Ten frames of 40 ions in 8,000 waters,
+    // 30 clusters of up to 2,000 tiles: 249 us with 16 wavefronts a cluster, 76 us
+    // so; 2,000 waters, 10 frames, 1,250 clusters: 132 us with six by tiles, 144
+    // with four by super tiles and two by tiles.
     const int64_t items = (int64_t)P.F * P.nB, want = 2 * (int64_t)nb * J->cus * waves;
     const int64_t most = std::max(P.nT / 4, std::min(16, P.nT));
     const int S0 = (int)std::min<int64_t>(most, std::max<int64_t>(1, want / std::max<int64_t>(items, 1)));
-    const int Sg = std::min(S0, std::max(1, P.nS / 8)), S = (S0 + Sg - 1) / Sg * Sg;
+    const int Sg = std::min((S0 + 15) / 16, std::max(1, P.nS / 8)), S = (S0 + Sg - 1) / Sg * Sg;
     const int64_t blocks = std::min<int64_t>((int64_t)nb * J->cus, (items * S + waves - 1) / waves);
     hipLaunchKernelGGL(kern, dim3((unsigned)((blocks + 7) / 8 * 8)), dim3(64 * waves), lds, s, P, B, (const T*)xu, (const T*)xv, S, Sg);
 }
@@ -5599,7 +5633,10 @@ void launch_cl_rpm(hipStream_t s, const cm_job* J, const KP& P, const Bufs& B, c
 template <class T>
 void launch_cl(hipStream_t s, const cm_job* J, const KP& P, const Bufs& B, const void* xu, const void* xv)
 {
-    if (P.rpm == 4) launch_cl_rpm<T, 4>(s, J, P, B, xu, xv);
+    if (P.rpm == 1) {
+        if (P.self_) launch_cl_one<T, 1, 1, true>(s, J, P, B, xu, xv);
+        else launch_cl_one<T, 1, 1, false>(s, J, P, B, xu, xv);
+    } else if (P.rpm == 4) launch_cl_rpm<T, 4>(s, J, P, B, xu, xv);
     else if (P.rpm == 8) launch_cl_rpm<T, 8>(s, J, P, B, xu, xv);
     else launch_cl_rpm<T, 16>(s, J, P, B, xu, xv);
 }
@@ -6134,7 +6171,7 @@ void job_params(cm_job* J, const cm_job_desc& d)
     // thread, 289 of them or more a pair).  The no-allocation entry point keeps
     // the walk as well: its admission rule counts the walk's buffers.
     if (!J->atoms_family && !J->arena && P.nu <= CL_ATOMS && P.nv <= CL_ATOMS) {
-        P.rpm = P.nu <= 4 ? 4 : (P.nu <= 8 ? 8 : 16);
+        P.rpm = P.nu == 1 && P.nv == 1 ? 1 : (P.nu <= 4 ? 4 : (P.nu <= 8 ? 8 : 16));
         P.nT = (int)(((int64_t)P.Mu * P.rpm + 15) / 16);
         P.nS = (P.nT + CL_SUP - 1) / CL_SUP;
         P.nB = (P.Mv + 15) / 16;

@@ -118,3 +118,14 @@ def test_exact_ties_of_larger_molecules(pkg, oracle, n, m):
     t = _traj(pkg, 0, 0, n, m, nframes=2, seed=11, broken=False)
     t.xv[:] = np.round(t.xv)
     _check(pkg, oracle, t, dbulk=8.0, n_random_samples=3, irefatom=n)
+
+
+@pytest.mark.parametrize("mu,mv", [(0, 16), (0, 17), (0, 33), (0, 900), (2, 3), (15, 16), (16, 17), (17, 400), (600, 33)])
+@pytest.mark.parametrize("angle,dtype", [(90.0, np.float32), (75.0, np.float64)])
+def test_single_atoms(pkg, oracle, mu, mv, angle, dtype):
+    """Single atoms on both sides: a row of a tile is a molecule; also whole Angstroms (FP64) and two images in reach."""
+    _check(pkg, oracle, _traj(pkg, 1, mu, 1, mv, angle=angle, dtype=dtype, seed=12), dbulk=9.0, n_random_samples=3)
+    t = _traj(pkg, 1, mu, 1, mv, box=20.0, angle=angle, dtype=dtype, seed=13, broken=False)
+    for x in (t.xu, t.xv):
+        x[:] = np.round(x)
+    _check(pkg, oracle, t, bulk_range=(7.0, 9.5))
