@@ -15,6 +15,7 @@ once; an FMA is the exact float64 product plus the addend, rounded to
 float32 (the float64 sum adds at most 2^-53 relative before that rounding).
 """
 import numpy as np
+import pytest
 
 U = 2.0 ** -24
 
@@ -173,3 +174,85 @@ def test_direct_distance_guard_about_a_centre():
     fixed = 3 * E * E + 1e-9 + 2 * np.sqrt(3) * E * r + (2 * rho + 4) * u * exact
     assert (err <= fixed + 2 * rho * u * (S + Y) * r).all()
     assert (err > fixed).any()
+
+
+def _pair_guard(S, Y, cutoff, rho):
+    """Gx of the molecule-pair kernel for tile radius S and cluster radius Y."""
+    cut = cutoff + 0.5
+    W, E2 = cut + S + Y, cut + 2.0 * S
+    return (U * (4.0 * max(Y * (Y + 2.0 * W), (cut + S) ** 2) + 4.0 * (Y * Y + W * W) + 4.0 * E2 * E2 +
+                 S * (3.0 * S + 2.0 * (cut + S)) + 3.5 * cut * (S + Y + rho * W)) + 1e-7) * (1.0 + 1e-4)
+
+
+def _cell(box, angle):
+    """Lattice vectors as columns, the kernel's FP32 vectors per unit, and rho."""
+    import math
+    c, s = math.cos(math.radians(angle)), math.sin(math.radians(angle))
+    H = np.array([[1.0, c, c], [0.0, s, c * (1 - c) / s], [0.0, 0.0, 0.0]])
+    H[2, 2] = math.sqrt(1.0 - H[0, 2] ** 2 - H[1, 2] ** 2)
+    H *= box
+    if angle == 90.0:
+        H = np.diag(np.diag(H))
+        return H, 3.0
+    V = np.linalg.det(H)
+    sp = [V / np.linalg.norm(np.cross(H[:, (k + 1) % 3], H[:, (k + 2) % 3])) for k in range(3)]
+    kappa = max(sum(abs(H[r, k]) / sp[k] for k in range(3)) for r in range(3))
+    return H, 5.0 * math.sqrt(3.0) * kappa
+
+
+def _chain(c, a, b, order):
+    """c + a . b over four components by FMAs in an order of the additions."""
+    for k in order:
+        c = fma32(a[k], b[k], c)
+    return c
+
+
+@pytest.mark.parametrize("angle", [90.0, 75.0])
+@pytest.mark.parametrize("bits", [0, 4, 5, 6, 8])
+def test_molecule_pair_distance_within_guard(angle, bits):
+    """The two chained products of the molecule-pair kernel (|t - y'|^2 as the
+    start of |t - y' + s'|^2, t between the centres of tile and cluster) in both
+    layouts of the operands and both orders of their sums, with the candidate's
+    code in the lowest bits: within the kernel's guard for pairs within the cutoff,
+    tiles and clusters of 0.5 to 60 A radius."""
+    rng = np.random.default_rng([2030, int(angle), bits])
+    box, fix, cutoff, n = 240.0, 27, 10.0, 20000
+    H, rho = _cell(box, angle)
+    Hfix = (H * 2.0 ** -fix).astype(np.float32)
+    unit = lambda m: (lambda v: v / np.linalg.norm(v, axis=1)[:, None])(rng.normal(size=(m, 3)))
+    inside = lambda R: unit(n) * (R * rng.uniform(size=n) ** (1 / 3))[:, None]
+    worst = 0.0
+    for S, Y in [(0.5, 0.5), (3.0, 6.0), (6.0, 3.0), (12.0, 25.0), (60.0, 4.0), (4.0, 60.0), (60.0, 60.0)]:
+        sr, yr = inside(S), inside(Y)
+        e = unit(n) * (rng.uniform(size=n) * cutoff)[:, None]
+        ti = np.rint(np.linalg.solve(H, (yr + e - sr).T).T * 2.0 ** fix).astype(np.int64)   # centres, tile minus cluster
+        d2 = ((ti * 2.0 ** -fix @ H.T + sr - yr) ** 2).sum(1)
+        keep = d2 <= cutoff * cutoff
+        s, y = [f32(sr[keep, k]) for k in range(3)], [f32(yr[keep, k]) for k in range(3)]
+        a, b, c = (f32(ti[keep, k]) for k in range(3))
+        t = [f32(Hfix[0, 0] * a), f32(Hfix[1, 1] * b), f32(Hfix[2, 2] * c)]
+        if angle != 90.0:
+            t[0] = fma32(Hfix[0, 1], b, fma32(Hfix[0, 2], c, t[0]))
+            t[1] = fma32(Hfix[1, 0], a, fma32(Hfix[1, 2], c, t[1]))
+            t[2] = fma32(Hfix[2, 0], a, fma32(Hfix[2, 1], b, t[2]))
+        norm = lambda v: fma32(v[0], v[0], fma32(v[1], v[1], f32(v[2] * v[2])))
+        s2, y2, t2 = norm(s), norm(y), norm(t)
+        one, zero = np.ones_like(s2), np.zeros_like(s2)
+        m2y = [f32(-2.0 * v) for v in y]
+        z = [f32(m2y[k] + f32(2.0 * t[k])) for k in range(3)]
+        G = _pair_guard(S, Y, cutoff, rho)
+        pk = 2.0 ** (bits - 23)
+        for order in ((0, 1, 2, 3), (3, 2, 1, 0)):
+            for quad in (True, False):
+                first = _chain(y2, t + [t2], m2y + [one], order) if quad else _chain(zero, t + [one], m2y + [f32(y2 + t2)], order)
+                got = _chain(first, s + [s2], z + [one], order)
+                code = got.view(np.int32)
+                coded = (code & ~((1 << bits) - 1) | rng.integers(0, 1 << bits, size=code.shape)).astype(np.int32).view(np.float32)
+                # as decided: the code cleared, half its range added back
+                val = ((code & ~((1 << bits) - 1)).astype(np.int32).view(np.float32) * f32(1.0 + 0.5 * pk)).astype(np.float64)
+                bound = G + val * (0.5 * pk + 2.0 ** -21) + 1e-7
+                worst = max(worst, (np.abs(val - d2[keep]) / bound).max())
+                assert (np.abs(val - d2[keep]) <= bound).all()
+                # the value compared and queued carries the code
+                assert (np.abs(coded.astype(np.float64) - d2[keep]) <= G + d2[keep] * (pk + 2.0 ** -21) + 1e-7).all()
+    assert worst > 0.02, worst
