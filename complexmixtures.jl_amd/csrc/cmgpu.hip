@@ -14,13 +14,16 @@
 //   k_scan_sums, k_scan_rows, k_mol_scatter, k_chunk_table
 //                       near molecules sorted by the Hilbert key of their cell
 //                       (the real pass; the random passes of a frame together),
-//                       cut into chunks of whole molecules, one wavefront each
+//                       cut into chunks of whole molecules, one wavefront each:
+//                       fewer near a compact solute, more about an extended one
 //   k_fill_real         atoms of the near molecules in sorted order, fixed point
 //   k_eval_tiles        per chunk: AABB, solute atoms within reach of it staged
-//                       in LDS, distances on the matrix cores, minimum and second
-//                       smallest per atom, minimum per molecule, records that
-//                       FP32 decides into LDS histograms
-//   k_resolve           the other molecules (about one in two hundred) in FP64
+//                       in LDS, distances on the matrix cores (columns: molecules
+//                       of three atoms, or atoms), minimum and second smallest per
+//                       atom, minimum per molecule, records that FP32 decides into
+//                       LDS histograms
+//   k_resolve           the other molecules in FP64: 0.2 % of those within the cutoff of
+//                       a globule in a cubic cell, 0.7 % in a triclinic one
 //   k_bulk_compact      ordered list of bulk molecules (inbulk, src/mddf.jl:55-57)
 //   k_place_keys, k_place_near
 //                       Philox placement (src/rigid_body.jl:107-137): centres
@@ -32,8 +35,8 @@
 // to 16 atoms:
 //   k_cl_keys, k_cl_scan, k_cl_order
 //                       molecule radii, molecules in Hilbert order
-//   k_cl_build          tiles of 16 solute rows, clusters of 16 solvent
-//                       molecules, their boxes
+//   k_cl_build          tiles of 16 solute rows (1, 4, 8 or 16 a molecule),
+//                       clusters of 16 solvent molecules, their boxes
 //   k_cl_eval           per cluster: every tile whose box is within the cutoff,
 //                       distances on the matrix cores, pairs within the cutoff
 //                       queued and counted, what FP32 leaves open in FP64
@@ -44,6 +47,10 @@
 // drawn solute molecule), k_eval_mols_rand (their placement and records).
 //
 // k_flush turns integer hits into FP64 accumulators times the frame weight.
+//
+// Coordinates that are not numbers (or infinite) take part in no distance: a
+// solute atom without a position is in no cell and no tile, a solvent molecule of
+// which any atom has none is near nothing (tiles), and its placed copies with it.
 //
 // Exactness.  Candidate pairs are evaluated in FP32, from fixed-point fractions
 // of the cell (tiles: differences are exact) or from coordinates in the frame of
@@ -193,7 +200,7 @@ struct Bufs {
     // random passes
     double* P;               // [F][K][Nv][3]
     float4* vw_r;            // [F][K][Nv]
-    float4* vcen_r;          // mols, [F*K][Mv]: slots to evaluate, their centres and numbers (count: slot_counts)          // [F][K][Mv]
+    float4* vcen_r;          // [F][K][Mv] slots to evaluate, their centres and numbers (count: slot_counts)
     unsigned char* bflag;    // [F][kb][Mv]
     int* blist;              // [F][kb][Mv]
     int* nbulk;              // [F][kb]
@@ -1672,11 +1679,11 @@ __global__ void k_bulk_init(KP P, Bufs B)
     b_bulk_init(P, B, blockIdx.x, gridDim.x, blockIdx.y, gridDim.y);
 }
 
-// ordered compaction of the bulk flags, one block per (frame, list)
 // Slots listed per (frame, pass) of the molecule-pair family.  The counts take the
 // place of drawn_idx, which the real pass was the last to read.
 __device__ __forceinline__ int* slot_counts(const Bufs& B) { return B.drawn_idx; }
 
+// ordered compaction of the bulk flags, one block per (frame, list)
 __device__ __forceinline__ void b_bulk_compact(KP P, Bufs B, int bx_, int nbx_, int by_, int nby_, bool mols = false)
 {
     if (mols)
@@ -2048,10 +2055,6 @@ __device__ __forceinline__ void cell_range32(const GEO& g, int cx, int cy, int c
     }
 }
 
-// cells near the solute: every cell within rnear of a solute atom (index
-// box).  A block takes 256 consecutive atoms of one frame (neighbours along
-// the chain, whose cell ranges overlap): the marks go into a bitmap of the
-// frame's cells in LDS first, and the block writes each marked cell once.
 // Lanes an atom in k_near_mark.  Few atoms: eight, each with an eighth of the
 // serial walk over the atom's cells (30 atoms: 25 -> 11 us).  From a block's worth
 // on, one: the cell ranges that every lane forms are extra (1,000 atoms: 36 us,
@@ -2059,6 +2062,10 @@ __device__ __forceinline__ void cell_range32(const GEO& g, int cx, int cy, int c
 __host__ __device__ __forceinline__ int near_lanes(int nu) { return nu < 256 ? 8 : 1; }
 constexpr int NEAR_WORDS = 8192;   // LDS bitmap words (frames of up to 262,144 cells; larger: direct stores)
 
+// cells near the solute: every cell within rnear of a solute atom (index
+// box).  A block takes 256 consecutive atoms of one frame (neighbours along
+// the chain, whose cell ranges overlap): the marks go into a bitmap of the
+// frame's cells in LDS first, and the block writes each marked cell once.
 __device__ __forceinline__ void b_near_mark(KP P, Bufs B, int bx_, int nbx_, int by_, int nby_)
 {
     __shared__ unsigned bits[NEAR_WORDS];
@@ -2336,8 +2343,8 @@ __global__ void k_prep_solvent_tiles(KP P, Bufs B, const T* xv)
     b_prep_solvent_tiles<T>(P, B, xv, tab, blockIdx.x, gridDim.x, blockIdx.y, gridDim.y);
 }
 
-// real pass: atoms of the near molecules in sorted order, FP32, in the frame of
-// the centre's cell
+// real pass: atoms of the near molecules in sorted order, in fixed point (fix_point),
+// by the periodic image of the molecule's centre
 template <class T>
 __device__ __forceinline__ void b_fill_real(KP P, Bufs B, const T* xv, int bx_, int nbx_, int by_, int nby_)
 {
@@ -3793,16 +3800,19 @@ int64_t resolve_parts(const KP& P, bool random)
 // molecule pairs on the matrix cores (molecules of up to CL_ATOMS atoms)
 // ---------------------------------------------------------------------------
 // Solute molecules, sorted along a Hilbert curve, fill the 16 rows of A tiles:
-// RPM rows per molecule (4, 8 or 16), 16 / RPM molecules per tile; solvent
+// RPM rows per molecule (1 where both sides are single atoms, else 4, 8 or 16),
+// 16 / RPM molecules per tile; solvent
 // molecules in the same kind of order fill the 16 columns of B clusters, one
 // column tile per atom.  Positions are FP32 relative to the tile's (cluster's)
 // fixed-point centre.  A wavefront takes one B cluster and every A tile whose box
 // is within the cutoff of its box: one matrix instruction per solvent atom q
-// gives 256 distances, four per lane, so a lane holds one molecule pair (RPM 4)
-// or a part of one, and keeps its minimum, second smallest value and the minima
-// over the reference atoms.  The pairs within the cutoff (about one in six) go
-// to an LDS queue and are counted 64 at a time; the ones FP32 cannot decide go
-// on to a second queue and are formed again in FP64, 64 at a time.
+// gives 256 distances, four per lane, so a lane holds one molecule pair (RPM 4),
+// a part of one, or four of single atoms, and keeps its minimum, second smallest
+// value and the minima over the reference atoms.  The pairs within the cutoff
+// (about one in six) go to an LDS queue and are counted 64 at a time; the ones FP32
+// cannot decide go on to a second queue and are formed again in FP64, 64 at a time,
+// the last of a wavefront's with the lanes shared out among them.  Where the
+// clusters are fewer than the wavefronts, S of these share one, its tiles in turn.
 //
 // The cell walk evaluates a pair in one thread, some 25 vector instructions per
 // distance with the tests of its neighbourhood; here a distance costs 2.25 (its
@@ -4538,15 +4548,14 @@ __global__ void __launch_bounds__(NVT > 8 ? 512 : 1024) k_cl_eval(KP P_, Bufs B_
     if (shg) groups_flush(P, shg, B_.cnt_gu, B_.cnt_gv);
 }
 
-// Fills n16 16-byte words and then ntail single bytes with zeros (a kernel,
+// Ranges of memory, each filled with copies of its own word, all in one launch:
+// nine of a small call's thirty launches were fills, some 4 us each.  (A kernel,
 // not hipMemsetAsync: memset nodes captured in HIP graphs have given wrong
-// results on replays here, and a caller may capture these launches).
-// Several ranges in one launch (each its own word): nine of a small call's
-// thirty launches were fills, some 4 us each.
+// results on replays here, and a caller may capture these launches.)
 struct FillList {
-    static constexpr int MAX = 6;
+    static constexpr int MAX = 6;   // (the longest list has five)
     int n = 0;
-    unsigned char* p[MAX];   // 16-byte aligned
+    unsigned char* p[MAX];   // 16-byte aligned: every buffer here starts on a 256-byte boundary
     int64_t bytes[MAX];
     unsigned word[MAX];
     void add(void* q, size_t b, unsigned w = 0)
@@ -4920,8 +4929,6 @@ int fail(int code, const std::string& msg)
         if (e_ != hipSuccess) return fail(CM_EHIP, std::string(#x) + ": " + hipGetErrorString(e_)); \
     } while (0)
 
-// x: blocks over n molecules or slots; y: one per (frame, pass) pair, up to
-// the grid limit (the kernels stride over y beyond it)
 // blocks per frame of k_near_mark: every lane an item while that is few blocks
 // (each clears and writes out its bitmap), then as many as there are atoms for
 int near_blocks(int nu)
@@ -4930,6 +4937,8 @@ int near_blocks(int nu)
     return std::max(1, std::min(all, std::max(4, (nu + BLOCK - 1) / BLOCK)));
 }
 
+// x: blocks over n molecules or slots; y: one per (frame, pass) pair, up to
+// the grid limit (the kernels stride over y beyond it)
 dim3 grid_slots(int n, int pairs)
 {
     return dim3((unsigned)std::max(1, (n + BLOCK - 1) / BLOCK), (unsigned)std::max(1, std::min(pairs, 65535)));
@@ -4943,8 +4952,8 @@ int grid_for(int64_t n)
     return (int)b;
 }
 
-// zeroes `bytes` bytes at p (16-byte aligned: every buffer here starts on a
-// 256-byte boundary) on stream s
+// one launch of k_fill over the ranges of L on stream s, a lane per 16 bytes of
+// the longest up to 2,048 blocks
 int fill_async(const FillList& L, hipStream_t s)
 {
     if (!L.n) return CM_OK;
@@ -6169,7 +6178,9 @@ void job_params(cm_job* J, const cm_job_desc& d)
     // on both sides, the rows of one tile.  Larger ones would need minima over
     // several tiles; their walk already spends its time on distances (one
     // thread, 289 of them or more a pair).  The no-allocation entry point keeps
-    // the walk as well: its admission rule counts the walk's buffers.
+    // the walk as well: tiles and clusters take more of its fixed scratch per frame
+    // (three-atom molecules against themselves 165 to 180 bytes a molecule, the
+    // walk 104), so jobs near its limit would be refused.
     if (!J->atoms_family && !J->arena && P.nu <= CL_ATOMS && P.nv <= CL_ATOMS) {
         P.rpm = P.nu == 1 && P.nv == 1 ? 1 : (P.nu <= 4 ? 4 : (P.nu <= 8 ? 8 : 16));
         P.nT = (int)(((int64_t)P.Mu * P.rpm + 15) / 16);
